@@ -73,8 +73,9 @@ static const cuthip_variant_info_t kMatMulGgufVariants[] = {
      "streaming GEMV / skinny GEMM (M <= 8): 32 weight rows per workgroup, split-K over the waves, "
      "in-register unpack feeding 32x32x16 f16 MFMA, fp32 per-sub-block scaling; beyond 8 rows of A the choice by shape"},
     {"MatMulGgufSkinnyMfma", 64, 4, 32, 32, "same pipeline with a 32-row activation tile (8 < M <= 32 per pass)"},
-    {"MatMulGgufGemmLds", 256, 1, 128, 128,
-     "prefill GEMM: weights dequantized to fp16 tiles in LDS, 32x32x16 f16 MFMA, fp32 accumulate"},
+    {"MatMulGgufGemmLds", 512, 1, 128, 128,
+     "tens to hundreds of rows in one launch: blocks through LDS row images, decoded to fp16 in the registers that feed "
+     "32x32x16 f16 MFMA, up to four 32-row tiles of A per workgroup (long K split over workgroups through the workspace)"},
     {"MatMulGgufGemvRows8", 64, 4, 8, 8,
      "decode GEMV (M <= 8): 8 weight rows x 128-byte runs per wave instruction, four 64-element pieces per row as "
      "MFMA columns, register ring of loads, no cross-wave reduction unless K is split"},

@@ -92,7 +92,7 @@ __device__ inline void q4k_scales(uint32_t s0, uint32_t s1, uint32_t s2, uint32_
 // Unary / binary epilogues of the matmul: the operator set and the formulas of cut_writeOutput
 // (operators/impl/matmul/MatMulQ8Common.cuh:58-109), selected by the reference's operator codes.
 // Only six unary (NEG, TANH, RELU, SIGMOID, GELU, SILU) and six binary (ADD, SUB, MUL, DIV, MIN, MAX) operators are part
-// of the matmul kernels' epilogues.  The tiled GEMMs store 128 and more accumulators per lane through fully unrolled
+// of the matmul kernels' epilogues.  The dense GEMMs store 128 and more accumulators per lane through fully unrolled
 // loops; with the whole operator set inlined at every store those loops no longer unroll, and the accumulator arrays
 // they index leave the registers (measured: 710 -> 39 TFLOP/s).  The entry points run such a
 // matmul unfused and apply the operator in a second, elementwise launch (launch_long_epilogue).

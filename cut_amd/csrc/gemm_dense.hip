@@ -2,7 +2,7 @@
 //   pass 1  dequantizes the GGUF weight tensor once into an fp16 [N, K] workspace
 //           (the dequant kernel of this library, HBM-bound: ~25 us for 14336 x 4096),
 //   pass 2  C[m,n] = sum_k A[m,k] * W16[n,k] as a dense fp16 MFMA GEMM.
-// The single-launch GEMM (gemm.hip) decodes every weight once per 256 rows of
+// The row-tile matmul (gemm_rows.hpp) decodes every weight once per 128 rows of
 // activations, i.e. M/256 times; for M in the thousands the decode ALU work, not
 // the MFMA, bounds it.  Here each weight is decoded exactly once and the GEMM's
 // inner loop contains nothing but MFMAs, LDS fragment reads and copy instructions.
@@ -31,7 +31,7 @@
 // multiplied after the barrier, under the first fragment reads of the next slice.
 //
 // Numerics: weights rounded to fp16 once (2^-11 relative), fp32 activations rounded
-// to fp16 once, fp32 accumulation: the same error budget as the single-launch GEMM.
+// to fp16 once, fp32 accumulation: the same error budget as the row-tile matmul.
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -673,30 +673,27 @@ size_t dense_f16_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16) {
   return dense_gemm_workspace(M, K, N, a_f16) - align256((size_t)N * K * 2);
 }
 
-// Cost models in microseconds for the automatic choice between the two-pass path and the single-launch GEMM, fitted to
-// a sweep over the weight shapes of an 8B model (all formats, M = 16 .. 2048, HIP-graph replay, MI355X):
-//   two-pass      3 + N K (bytes per weight + 2) / 6.0 MB   the dequantization (reads the blocks, writes fp16)
-//                 + 17 + max(2 ceil128(M) N K / 1.25 PFLOP/s,  the dense GEMM (tiles are at least 128 rows high; up to 256 rows
-//                            2 N K / 3.5 MB)                  it is bound by reading the fp16 weights: 128 and 256 x 28672 x 4096
-//                                                             both take 147-148 us on Q6_K, 14336 x 4096 76 and 79)
-//   single launch K x c_fmt x max(1, tiles / 256)            c = 14.7 ns (Q4_K, Q4_0), 17 ns (Q8_0: 256 x 28672 x 4096 122 us,
-//                 512 rows 220, 256 x 14336 x 4096 73-76), 19.5 ns (Q6_K: 256 x 28672 x 4096 133-139 us,
-//                 512 x 14336 x 4096 139):
-//                 a workgroup decodes its K-long strip of weights once per 128 rows of A, and nothing overlaps that
-//                 walk until every CU holds more than one 128 x 128 tile.
-// Measured against them (Q4_K, M x N x K): 64 x 4096 x 4096 38 / 62 us, 512 x 14336 x 4096 99 / 105, 512 x 28672 x 4096
-// 173 / 203, 256 x 28672 x 4096 147 / 107; Q6_K 64 x 14336 x 4096 79 / 104.
-//                 + 5 where the GEMM splits K (a third launch sums the partial products): 1024 x 1024 x 4096 36 us
-double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N) {
+// Cost in microseconds of the two-pass path, for the automatic choice between it and the row-tile matmul; fitted to 432
+// launches (four formats, 64 .. 2048 rows, nine weight shapes from 2048 x 2048 to 28672 x 4096, both activation types,
+// HIP-graph replay, MI355X; 8 % rms):
+//   10 + N K (bytes per weight + 2) / 5.5 MB  the dequantization (reads the blocks, writes fp16)
+//   + 6.6 per round of tiles over the 256 CUs + K x the tile's area x its cost per multiply-add, a round that fills the chip
+//     1.4 times one that leaves it nearly empty (clocks, memory)
+//   + the partial products of a K split, + the conversion of fp32 activations
+// The row-tile matmul decodes every weight once per 128 rows and this path once, so the line runs at about 450 rows on wide
+// matrices (14336 x 4096, us, row tiles / two passes: Q8_0 384 rows 96 / 106, 448 rows 97 / 86; Q4_K 640 rows 91 / 96,
+// 768 rows 119 / 112) and higher on narrow ones (4096 x 4096 Q4_K: 1024 rows 46 / 60, 2048 rows 89 / 73; 1024 x 4096: never).
+double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16) {
   const double nk = (double)N * K, bpw = (double)fmt_bytes(fmt) / fmt_elems(fmt);
-  const double split = pick_dense_shape(M, K, N).ksplit > 1 ? 5.0 : 0.0;
-  const double mfma = 2.0 * (double)((M + 127) / 128 * 128) * nk / 1.25e9, stream = 2.0 * nk / 3.5e6;
-  return 3.0 + nk * (bpw + 2.0) / 6.0e6 + 17.0 + (mfma > stream ? mfma : stream) + split;
-}
-double single_launch_rows_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N) {
-  const double c = fmt == CUTHIP_Q6_K ? 19.5e-3 : fmt == CUTHIP_Q8_0 ? 17.0e-3 : 14.7e-3;
-  const double tiles = (double)((M + 127) / 128) * ((N + 127) / 128);
-  return K * c * (tiles > 256.0 ? tiles / 256.0 : 1.0);
+  const DenseShape sh = pick_dense_shape(M, K, N);
+  const double weight = sh.bn == 224 ? 0.96 : sh.bn == 448 ? 1.0 : sh.bm == 256 ? 1.03 : sh.ksplit == 1 ? 0.88 : 0.97;
+  const uint64_t tiles = (uint64_t)((M + sh.bm - 1) / sh.bm) * ((N + sh.bn - 1) / sh.bn) * sh.ksplit;
+  const double full = (double)((tiles - 1) / 256), last = (double)(tiles - 1) - 256.0 * full + 1.0;
+  double us = 9.6 + nk * (bpw + 2.0) / 5.46e6 + 6.6 * (full + 1.0) +
+              (double)K / sh.ksplit * sh.bm * sh.bn * weight * 2.64e-7 * (full * 1.41 + 1.0 + 0.41 * last / 256.0);
+  if (sh.ksplit > 1) us += 8.0 * sh.ksplit * M * N / 7.4e6;
+  if (!a_f16) us += 1.5 + 6.0 * M * K / 5e6;
+  return us;
 }
 
 // use_blaslt: the dense GEMM goes to hipBLASLt (no epilogue there: the caller checks)

@@ -1,7 +1,7 @@
 // Streaming matmul on Q4_K blocks for a handful of activation rows (5 <= M <= 32):
 //   C[m,n] = sum_k A[m,k] * dequant(W)[n,k]
 // between the 8-row GEMV (whose matrix-core path spends three quarters of every product on mismatched pieces)
-// and the tiled GEMM (which decodes every weight to fp16 through LDS, three vector instructions per weight).
+// and the row-tile matmul (which rounds every weight to fp16).
 // Supersedes MatMulQ4GemvKPar8.cu / MatMulQ4TiledReg.cu (operators/impl/matmul) at these batch sizes.
 //
 // Two waves share 16 weight rows and each walks half of the workgroup's K range in steps of one 256-element
@@ -22,7 +22,7 @@
 // keeps kStreamDepth steps of weight loads in flight in a register ring and waits only for the step it multiplies.
 //
 // Measured (MI355X, HIP-graph replay, Q4_K 14336 x 4096): 15.0 us at 9-16 rows (two passes of the 8-row GEMV: 25),
-// 21 us at 17-32 rows (tiled GEMM with K split: 30); at 8 rows and fewer the 8-row GEMV is the faster one (13 us):
+// 21 us at 17-32 rows (row-tile matmul: 16, on rounded weights); at 8 rows and fewer the 8-row GEMV is the faster one (13 us):
 // both spend about 0.05 vector instructions per weight on the unpack, which bounds them well before HBM does.
 #include <type_traits>
 

@@ -121,17 +121,17 @@ GemvShape pick_gemv_shape(uint32_t N, uint32_t nsteps, int mt) {
   return GemvShape{kp, w};
 }
 
-int launch_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
-                uint32_t strideA, uint32_t strideC, Epilogue epi, hipStream_t stream, void *scratch, size_t scratch_bytes);
+int launch_rows_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
+                     uint32_t strideA, uint32_t strideC, Epilogue epi, hipStream_t stream, void *scratch, size_t scratch_bytes);
+double rows_gemm_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16, size_t scratch_bytes);
+bool rows_gemm_fits(int fmt, uint32_t K, uint32_t strideA, int a_f16);
 
 bool dense_gemm_fits(uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A);
 size_t dense_gemm_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16);
-double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N);
-double single_launch_rows_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N);
+double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16);
 int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K,
                       uint32_t N, uint32_t strideA, uint32_t strideC, Epilogue epi, void *workspace, hipStream_t stream,
                       int use_blaslt);
-uint32_t tiled_gemm_ksplit(uint32_t M, uint32_t K, uint32_t N, size_t scratch_bytes);
 bool stream_gemm_fits(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A);
 size_t stream_gemm_scratch(uint32_t M, uint32_t K, uint32_t N);
 int launch_stream_gemm(const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
@@ -167,43 +167,34 @@ static cuthip::GemvParams gemv_params(int fmt, const void *W, const void *A, int
   return p;
 }
 
-constexpr uint32_t kPassesMaxRows = 40;   // up to here 8-row passes of the decode kernels can beat one tiled GEMM launch
+constexpr uint32_t kPassesMaxRows = 40;   // up to here 8-row passes of the decode kernels are considered
 
-// Costs in microseconds fitted to a sweep over the weight shapes of an 8B model (HIP-graph replay, MI355X): an 8-row
-// pass of the decode kernels 6.5 + weight bytes / 4.3 MB (x 1.45 on rows of K >= 8192, x 1.05 for Q6_K: 14336 x 4096 18.6 us,
-// 28672 x 4096 34.4; x 1.55 for both), one launch of
-// the tiled GEMM on the blocks 62 + weight bytes / 7 MB (its cost is the decode of the whole matrix whatever M is; on
-// rows of K >= 8192 it has too few tiles and is never the better one).
 static double weight_bytes(int fmt, uint32_t K, uint32_t N) { return (double)N * K / cuthip::fmt_elems(fmt) * cuthip::fmt_bytes(fmt); }
+// Microseconds of 8-row passes of the decode kernels, fitted to a sweep over the weight shapes of an 8B model (HIP-graph
+// replay, MI355X): 6.5 + weight bytes / 4.3 MB each (x 1.45 on rows of K >= 8192, x 1.05 for Q6_K: 14336 x 4096 18.6 us,
+// 28672 x 4096 34.4; x 1.55 for both).
 static double passes_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N) {
   const double f = K >= 8192 ? (fmt == CUTHIP_Q6_K ? 1.55 : 1.45) : (fmt == CUTHIP_Q6_K ? 1.05 : 1.0);
   return ((M + 7) / 8) * (6.5 + weight_bytes(fmt, K, N) / 4.3e6) * f;
 }
-// The tiled GEMM with its K split over workgroups (scratch memory at hand, so few 128 x 128 tiles that the launch rule
-// of gemm.hip splits): 9.5 us for the two launches + 0.66 us (Q4_K; Q6_K x 1.84, Q8_0 x 1.31) per slice of 64 that a
-// CU walks (x 0.85 with the 64-row tiles of up to 64 rows) + the partial products written and read back at 6 MB/us.
-// 14336 x 4096 Q4_K: 27 us at 32 rows, 29 at 64, 38 at 128, 62 at 256 (unsplit 65 at every M up to 128; 216 on
-// K = 14336); 4096 x 1024: 19 at 256 rows, 20 at 512, 28 at 1024.
-// Beyond 256 rows only for matrices of fewer than 32 M weights: on 4096 x 14336 at 512 rows the model says 89 us and
-// the launch takes 102, against 93 for the two-pass path.
-static bool tiled_split_applies(uint32_t M, uint32_t K, uint32_t N, const void *scratch, size_t scratch_bytes) {
-  return scratch && (uintptr_t)scratch % 16 == 0 && M > 8 && (M <= 256 || (uint64_t)N * K < 32000000ull) &&
-         cuthip::tiled_gemm_ksplit(M, K, N, scratch_bytes) > 1;
-}
-static double tiled_split_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, size_t scratch_bytes) {
+// 9-40 rows in passes of 8.  The passes multiply the weights as they are (1e-5 of the result's norm), one launch of the
+// row-tile matmul rounds them to fp16 first (3e-4).  It is the faster one at every shape (12 x 14336 x 4096 on Q6_K 24 us
+// against 31, on Q4_K 16 against 26), so the line is one of precision, not of time: passes are kept wherever a matmul of
+// 128 x 128 tiles that decodes through LDS - what such calls would otherwise have run before there were 32-row tiles -
+// costs as much: without scratch memory for a K split 62 us + weight bytes / 7 MB (and always from K = 8192), with it
+// 9.5 us + 0.66 us (Q4_0 0.73, Q8_0 0.86, Q6_K 1.21; x 0.85, its tiles of 64 rows) per slice of 64 that a CU walks + the
+// partial products at 6 MB/us.  A call keeps the accuracy that it had.
+static bool passes_preferred(int fmt, uint32_t M, uint32_t K, uint32_t N, const void *scratch, size_t scratch_bytes) {
+  if (M <= 8 || M > kPassesMaxRows) return false;
+  const double passes = passes_cost_us(fmt, M, K, N);
+  const uint64_t tiles = ((uint64_t)N + 127) / 128;
+  const uint32_t slices = (K + 63) / 64;
+  uint32_t ks = 1;   // K ranges of at least eight slices that fill the chip
+  if (scratch && (uintptr_t)scratch % 16 == 0)
+    while (ks < 16 && tiles * ks < 384 && slices / (2 * ks) >= 8 && (uint64_t)2 * ks * M * N * 4 <= scratch_bytes) ks *= 2;
+  if (ks == 1) return K >= 8192 || passes <= 62.0 + weight_bytes(fmt, K, N) / 7e6;
   const double f = fmt == CUTHIP_Q6_K ? 1.84 : fmt == CUTHIP_Q8_0 ? 1.31 : fmt == CUTHIP_Q4_0 ? 1.1 : 1.0;
-  const double tiles = (double)((M + 127) / 128) * ((N + 127) / 128), slices = (K + 63) / 64;
-  const uint32_t ks = cuthip::tiled_gemm_ksplit(M, K, N, scratch_bytes);
-  const double tile_rows = M <= 64 ? 0.85 : 1.0;   // 64-row tiles: half the matrix-core work per slice
-  return 9.5 + 0.66 * f * tile_rows * tiles * slices / 256.0 + (double)ks * M * N * 8.0 / 6e6;
-}
-// split: bytes of scratch the tiled GEMM may split K through, 0 = none (or the launch would not split)
-static double single_launch_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, size_t split) {
-  return split ? tiled_split_cost_us(fmt, M, K, N, split) : 62.0 + weight_bytes(fmt, K, N) / 7e6;
-}
-static bool passes_preferred(int fmt, uint32_t M, uint32_t K, uint32_t N, size_t split) {
-  return M > 8 && M <= kPassesMaxRows &&
-         ((K >= 8192 && !split) || passes_cost_us(fmt, M, K, N) <= single_launch_cost_us(fmt, M, K, N, split));
+  return passes <= 9.5 + 0.66 * f * 0.85 * (double)tiles * slices / 256.0 + (double)ks * M * N * 8.0 / 6e6;
 }
 
 // Argument checks shared by the matmul entry points: 0 = go on, 1 = empty problem (success), < 0 = error.
@@ -253,13 +244,13 @@ static int check_matmul_args(int fmt, const void *W, const void *A, int a_dtype,
 
 static bool stream_preferred(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A,
                              const void *scratch, size_t scratch_bytes) {
-  // (few weight rows: too few workgroups for it; 1024 x 4096 at 16-32 rows 11.6-13.3 us against 10.6-11.2 for the tiled GEMM)
+  // (few weight rows: too few workgroups for it; 1024 x 4096 at 16-32 rows 11.6-13.3 us against 8.2-8.4 for the row-tile matmul)
   if (M < 9 || M > 32 || N < 2048 || !cuthip::stream_gemm_fits(fmt, M, K, N, strideA, a_f16, A)) return false;
   const size_t need = cuthip::stream_gemm_scratch(M, K, N);
   return need == 0 || (scratch && (uintptr_t)scratch % 16 == 0 && scratch_bytes >= need);
 }
 
-// cuthip_matmul_gguf with optional scratch memory (the workspace of cuthip_matmul_gguf_ws, or none): the tiled GEMM
+// cuthip_matmul_gguf with optional scratch memory (the workspace of cuthip_matmul_gguf_ws, or none): the row-tile matmul
 // splits K through it where it has too few tiles for the chip
 static int matmul_gguf_scratch(int fmt, const void *W, const void *A, int a_dtype, void *C, int c_dtype, uint32_t M,
                                uint32_t K, uint32_t N, uint32_t strideA, uint32_t strideC, int epilogue,
@@ -286,7 +277,7 @@ static int matmul_gguf_scratch(int fmt, const void *W, const void *A, int a_dtyp
     set_error("cuthip_matmul_gguf: K too large");
     return CUTHIP_ERR_INVALID;
   }
-  // variant table: 0 streaming GEMV (M <= 8; beyond, as -1), 1 skinny passes of 32 rows, 2 LDS-tiled GEMM,
+  // variant table: 0 streaming GEMV (M <= 8; beyond, as -1), 1 skinny passes of 32 rows, 2 the row-tile matmul,
   // 3 the 8-row GEMV, 4 / 5 dequantize + dense GEMM (workspace entry point only), 6 the streaming MFMA kernel (Q4_K, M <= 32)
   Epilogue epi{epilogue, epilogue_op, epilogue == CUTHIP_EPI_BINARY ? D : nullptr};
   if (epilogue == CUTHIP_EPI_SWIGLU_PAIRS && variant != -1 && variant != 3) {
@@ -299,9 +290,9 @@ static int matmul_gguf_scratch(int fmt, const void *W, const void *A, int a_dtyp
   }
   // the table's default entry is valid for every M: beyond the 8 rows its GEMV takes it is the choice by shape
   if (variant == 0 && M > 8) variant = -1;
-  // 9-32 rows on Q4_K: the streaming MFMA kernel (9-16 rows of 14336 x 4096: 15.8 us against 25 for two 8-row
-  // passes; 17-32 rows: 21 us against 30 for the tiled GEMM with K split), wherever the scratch memory it needs
-  // for long rows or two activation tiles is at hand
+  // 9-32 rows on Q4_K: the streaming MFMA kernel (9-16 rows of 14336 x 4096: 15.8 us against 25 for two 8-row passes,
+  // and like them on weights that are not rounded), wherever the scratch memory it needs for long rows or two activation
+  // tiles is at hand
   if (variant == -1 && stream_preferred(fmt, M, K, N, strideA, a_dtype == CUTHIP_F16, A, scratch, scratch_bytes)) variant = 6;
   // variant 6: the streaming MFMA kernel (Q4_K, up to 32 rows); scratch only where K has to be split over workgroups
   if (variant == 6) {
@@ -312,10 +303,8 @@ static int matmul_gguf_scratch(int fmt, const void *W, const void *A, int a_dtyp
     return launch_stream_gemm(W, A, a_dtype == CUTHIP_F16, C, c_dtype == CUTHIP_F16, M, K, N, strideA, strideC, epi, scratch,
                               scratch_bytes, reinterpret_cast<hipStream_t>(stream));
   }
-  // 9-40 rows, automatic choice: passes of 8 rows through the decode kernels.  Measured on 14336 x 4096: 14 us per
-  // pass, against 69-87 us for the 32-row skinny kernel and 73-80 us for one launch of the tiled GEMM, whose cost
-  // is the decode of the whole weight matrix whatever M is.
-  if (variant == -1 && passes_preferred(fmt, M, K, N, tiled_split_applies(M, K, N, scratch, scratch_bytes) ? scratch_bytes : 0)) {
+  // 9-40 rows, automatic choice: passes of 8 rows through the decode kernels
+  if (variant == -1 && passes_preferred(fmt, M, K, N, scratch, scratch_bytes)) {
     const size_t asz = a_dtype == CUTHIP_F16 ? 2 : 4, csz = c_dtype == CUTHIP_F16 ? 2 : 4;
     for (uint32_t m0 = 0; m0 < M; m0 += 8) {
       const uint8_t *a = reinterpret_cast<const uint8_t *>(A) + (size_t)m0 * strideA * asz;
@@ -327,13 +316,14 @@ static int matmul_gguf_scratch(int fmt, const void *W, const void *A, int a_dtyp
     }
     return CUTHIP_OK;
   }
-  if (variant == 2 || (variant == -1 && M > 8)) {   // 9..40 rows come here when one tiled launch beats the passes
+  const bool rows_fits = rows_gemm_fits(fmt, K, strideA, a_dtype == CUTHIP_F16);   // (else the 32-row skinny passes)
+  if ((variant == 2 || (variant == -1 && M > 8)) && rows_fits) {
     if ((uint64_t)N * row_bytes > 0xFFFFFFFFFFFFull) {
       set_error("cuthip_matmul_gguf: weight matrix too large");
       return CUTHIP_ERR_INVALID;
     }
-    return launch_gemm(fmt, W, A, a_dtype == CUTHIP_F16, C, c_dtype == CUTHIP_F16, M, K, N, strideA, strideC, epi,
-                       reinterpret_cast<hipStream_t>(stream), scratch, scratch_bytes);
+    return launch_rows_gemm(fmt, W, A, a_dtype == CUTHIP_F16, C, c_dtype == CUTHIP_F16, M, K, N, strideA, strideC, epi,
+                            reinterpret_cast<hipStream_t>(stream), scratch, scratch_bytes);
   }
   GemvParams p = gemv_params(fmt, W, A, a_dtype, C, c_dtype, M, K, N, strideA, strideC, epi);
   // variant 3 (and the automatic choice for M <= 8): 8 rows x 128-byte runs per wave instruction
@@ -632,19 +622,19 @@ int cuthip_matmul_gguf_ws(int fmt, const void *W, const void *A, int a_dtype, vo
     return matmul_gguf_scratch(fmt, W, A, a_dtype, C, c_dtype, M, K, N, strideA, strideC, epilogue, epilogue_op, D, 6, stream,
                                workspace, workspace_bytes);
   // Beyond 8 rows, with a workspace at hand: dequantize + dense GEMM where its modelled cost is below that of what
-  // would run otherwise (8-row passes up to 40 rows where those beat the single-launch GEMM, else that GEMM); against
-  // either only by a margin (a tenth, a twentieth): the models are rough.  From 1024 rows always.
+  // would run otherwise: 8-row passes (by a tenth: the model is rough) or the row-tile matmul.
   const bool fits = dense_gemm_fits(M, K, N, strideA, a_f16, A);
   const size_t need = dense_gemm_workspace(M, K, N, a_f16);
   const bool ws_ok = workspace && (uintptr_t)workspace % 256 == 0 && workspace_bytes >= need;
-  const size_t split = tiled_split_applies(M, K, N, workspace, workspace ? workspace_bytes : 0) ? workspace_bytes : 0;
+  const bool passes = variant == -1 && passes_preferred(fmt, M, K, N, workspace, workspace ? workspace_bytes : 0);
   bool dense_first = false;
   if (variant == -1 && M > 8 && fits && ws_ok) {
-    const double t4 = dense_cost_us(fmt, M, K, N);
-    const double tiled = split ? tiled_split_cost_us(fmt, M, K, N, split) : single_launch_rows_cost_us(fmt, M, K, N);
-    dense_first = (M >= 1024 && !split) || (passes_preferred(fmt, M, K, N, split) ? t4 < 0.9 * passes_cost_us(fmt, M, K, N) : t4 < 0.95 * tiled);
+    const double t4 = dense_cost_us(fmt, M, K, N, a_f16);
+    // (K of at most 512 from 1024 rows on: nothing is at stake, and the choice stays bit for bit variant 4 as it always was)
+    dense_first = (M >= 1024 && K <= 512) ||
+                  (passes ? t4 < 0.9 * passes_cost_us(fmt, M, K, N) : t4 < rows_gemm_cost_us(fmt, M, K, N, a_f16, workspace_bytes));
   }
-  if (variant == -1 && !dense_first && passes_preferred(fmt, M, K, N, split)) {   // 8-row passes, each with the workspace (K split on long rows)
+  if (variant == -1 && !dense_first && passes) {   // 8-row passes, each with the workspace (K split on long rows)
     const size_t asz = a_f16 ? 2 : 4, csz = c_dtype == CUTHIP_F16 ? 2 : 4;
     for (uint32_t m0 = 0; m0 < M; m0 += 8) {
       const uint8_t *a = reinterpret_cast<const uint8_t *>(A) + (size_t)m0 * strideA * asz;

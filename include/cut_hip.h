@@ -59,7 +59,7 @@ typedef enum {
  * other code is refused with CUTHIP_ERR_INVALID (the reference's shader would silently store the unfused value).
  * NEG, TANH, RELU, SIGMOID, GELU, SILU and ADD, SUB, MUL, DIV, MIN, MAX (what the runner's graphs fuse) run inside the
  * matmul kernels; the others are applied by a second, elementwise launch on the same stream (inlined at every store
- * of the tiled GEMMs the whole set costs those kernels their register allocation): same
+ * of the dense GEMMs the whole set costs those kernels their register allocation): same
  * result up to the rounding of C to its dtype in between, and for MOD, POW, FLOOR_DIV D must not alias C. */
 typedef enum {
   CUTHIP_UNARY_NEG = 100, CUTHIP_UNARY_ABS = 101, CUTHIP_UNARY_SQRT = 102, CUTHIP_UNARY_SQUARE = 103,
@@ -219,7 +219,7 @@ int cuthip_dequant(int fmt, const void *blocks, void *out, int out_dtype, uint32
  * variant: index into the CUTHIP_OP_MATMUL_GGUF table, or -1 = choose by shape
  *          (M <= 8 -> streaming GEMV; 9..16 rows of Q4_K with K <= 4096 -> variant 6, the
  *          streaming MFMA kernel; other 9..40 -> passes of 8 rows through the GEMV; else
- *          the LDS-tiled MFMA GEMM); variants 4 and 5 need cuthip_matmul_gguf_ws, which
+ *          the row-tile MFMA matmul); variants 4 and 5 need cuthip_matmul_gguf_ws, which
  *          also gives variants 2 and 6 the scratch memory they split K through. */
 int cuthip_matmul_gguf(int fmt, const void *W, const void *A, int a_dtype, void *C, int c_dtype, uint32_t M, uint32_t K,
                        uint32_t N, uint32_t strideA, uint32_t strideC, int epilogue, int epilogue_op, const void *D,

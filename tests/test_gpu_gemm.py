@@ -52,6 +52,34 @@ def test_gemm_ragged_k_and_fp32_activations(ops, name, K):
     assert normwise_rel_err(got, want) < 8e-4  # activations and weights both rounded to fp16
 
 
+@pytest.mark.parametrize("name,K", [("Q8_0", 32), ("Q8_0", 1312), ("Q8_0", 1024), ("Q4_0", 544), ("Q4_0", 2048), ("Q4_K", 256), ("Q4_K", 1280),
+                                    ("Q4_K", 2048), ("Q6_K", 768), ("Q6_K", 2048)])
+@pytest.mark.parametrize("a_type", [np.float16, np.float32])
+def test_row_tiles_at_their_edges(ops, tuning, name, K, a_type):
+    """The row-tile matmul at both sides of every number of 32-row tiles (one to four per workgroup, then several
+    workgroups), with a last weight panel of one row (N = 65: panels of 64 and of 128) and enough panels for the wider
+    workgroup at one and two tiles (N = 8200), K shorter than one unit of 128 and not a multiple of it, K ranges that come out uneven,
+    with and without room for a K split, and rows of A that start two bytes off.  Bound: weights rounded to fp16, 2^-11
+    at most each and independent, so below 2^-11 of the norm; fp32 activations are rounded as well: 2^-11 x sqrt(2)."""
+    fmt = oracle.FORMATS[name]
+    tol = 5e-4 if a_type == np.float16 else 7e-4
+    for N, rows in ((65, (9, 32, 33, 64, 65, 96, 97, 128, 129, 300)), (8200, (31, 64))):
+        W = quantized_weights(fmt, N, K, seed=K + N)
+        w = torch.from_numpy(W).cuda()
+        A = gauss_acts((max(rows), K + 1), seed=K, dtype=a_type)[:, 1:]
+        buf = torch.zeros((max(rows), K + 1), dtype=torch.float16 if a_type == np.float16 else torch.float32, device="cuda")
+        buf[:, 1:] = torch.from_numpy(np.ascontiguousarray(A)).cuda()
+        want = oracle.matmul_gguf(fmt, W, np.ascontiguousarray(A).astype(np.float32), N, f64=True)
+        for M in rows:
+            for split in (None, "1", "2", "7"):
+                tuning("gemm_ksplit", split)
+                ws = ops.matmul_gguf_workspace(fmt, M, K, N, buf.dtype, "cuda") if split != "1" else None
+                a = buf[:M, 1:] if split == "2" else buf[:M, 1:].contiguous()
+                got = ops.matmul_gguf(a, w, fmt, N, K, out_dtype=torch.float32, variant=2, workspace=ws).cpu().numpy()
+                err = normwise_rel_err(got, want[:M])
+                assert err < tol, (N, M, split, err)
+
+
 def test_gemm_variants_agree(ops):
     """The same problem through the GEMM (variant 2) and the skinny passes
     (variant 1): the reference checks batched against per-row the same way
