@@ -165,147 +165,171 @@ constexpr int kAttnMaxHd = 128;   // head dimension limit (as the reference's sh
 constexpr int kAttnRow = kAttnMaxHd + 8;   // LDS row in halfs: +16 bytes keeps the 64 rows off each other's banks
 
 // partial layout per (query head h, split s): [m, l, o[headDim]] floats at ((h * nsplit + s) * (2 + headDim))
-// HD: the head dimension when it is the common 128 (loops over it unroll and their LDS reads overlap), 0 = any
+// Bound: HBM on long contexts (K and V once), latency on short ones.  Split s takes the 64-position chunks s, s + nsplit,
+// s + 2 nsplit, ...: a workgroup that has several keeps (m, l, o) of its heads in registers and requests the next chunk
+// while it works on the present one, so that memory does not idle between workgroups and a long context leaves 64
+// records per head to merge instead of 256 (attn_splits draws the line).  A 16,384-position context of 8 KV heads of 128:
+// partials and merge 30.6 us before, about 20 now.
+// HD: the head dimension where it is 128 or 64 (loops over it unroll and their LDS reads overlap), 0 = any
+// NG: query heads of a KV head in groups of four (one per wave); gridDim.z covers the heads beyond 4 * NG
 // The arguments that the first loads need (up to and including headDimArg: 14 dwords) lead the list: with
 // kernel-argument preloading they arrive in SGPRs with the wave, and the loads of q, K and V wait for no scalar load.
-template <int HD>
+template <int HD, int NG>
 __global__ void __launch_bounds__(256) attn_partial_kernel(const void *q, const half_t *kCache, const half_t *vCache,
                                                            const uint32_t *params, uint32_t alignedKvDim, uint32_t maxSeqLen,
                                                            uint32_t nHeads, uint32_t nKvHeads, int q_f16, uint32_t headDimArg,
                                                            float *partial, float scale, uint32_t nsplit) {
   const uint32_t headDim = HD ? (uint32_t)HD : headDimArg;
-  __shared__ __attribute__((aligned(16))) half_t Ks[kAttnChunk * kAttnRow];
-  __shared__ __attribute__((aligned(16))) half_t Vs[kAttnChunk * kAttnRow];
-  __shared__ __attribute__((aligned(16))) float Qs[4 * kAttnMaxHd];
+  constexpr uint32_t kRow = (HD ? HD : kAttnMaxHd) + 8;   // LDS row in halfs: +16 bytes keeps the 64 rows off each other's banks
+  __shared__ __attribute__((aligned(16))) half_t Ks[kAttnChunk * kRow];
+  __shared__ __attribute__((aligned(16))) half_t Vs[kAttnChunk * kRow];
+  __shared__ __attribute__((aligned(16))) float Qs[4 * NG * kAttnMaxHd];
   __shared__ __attribute__((aligned(16))) float Ps[4 * kAttnChunk];
-  const uint32_t kvH = blockIdx.x, split = blockIdx.y, nRep = nHeads / nKvHeads;
+  const uint32_t kvH = blockIdx.x, split = blockIdx.y, nRep = nHeads / nKvHeads, rep0 = blockIdx.z * 4 * NG;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t seqLen = min(params[1], maxSeqLen);   // a length beyond the cache capacity attends the capacity only
-  const uint32_t t0 = split * kAttnChunk;
-  const uint32_t nvalid = t0 < seqLen ? min((uint32_t)kAttnChunk, seqLen - t0) : 0u;
 
   // Every load of the start-up is requested before the first of them is used, so that the kernel begins with one
-  // memory round trip: the query of the first pass (raw bits, converted later: a conversion right behind the load is a
-  // use, and the compiler then waits for it on the spot), then the chunk of K and V.  Written as a loop with the
+  // memory round trip: the queries (raw bits, converted later: a conversion right behind the load is a use, and the
+  // compiler then waits for it on the spot), then the first chunk of K and V.  Written as a loop with the
   // store right behind each load, the staging waited for four round trips in turn, and the query for two more.
-  uint32_t q_raw[2] = {0u, 0u};
-  {
-    const uint32_t h0 = kvH * nRep + (wave < nRep ? wave : 0);
-    const size_t qi = (size_t)h0 * headDim + min(lane, headDim - 1);   // lanes beyond the head dimension read a valid element
-    const size_t qj = (size_t)h0 * headDim + min(lane + 64, headDim - 1);
+  uint32_t q_raw[NG][2];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const uint32_t rep = rep0 + 4 * g + wave, h = kvH * nRep + (rep < nRep ? rep : 0);
+    const size_t qi = (size_t)h * headDim + min(lane, headDim - 1);   // lanes beyond the head dimension read a valid element
+    const size_t qj = (size_t)h * headDim + min(lane + 64, headDim - 1);
     if (q_f16) {
-      q_raw[0] = reinterpret_cast<const uint16_t *>(q)[qi];
-      q_raw[1] = reinterpret_cast<const uint16_t *>(q)[qj];
+      q_raw[g][0] = reinterpret_cast<const uint16_t *>(q)[qi];
+      q_raw[g][1] = reinterpret_cast<const uint16_t *>(q)[qj];
     } else {
-      q_raw[0] = reinterpret_cast<const uint32_t *>(q)[qi];
-      q_raw[1] = reinterpret_cast<const uint32_t *>(q)[qj];
+      q_raw[g][0] = reinterpret_cast<const uint32_t *>(q)[qi];
+      q_raw[g][1] = reinterpret_cast<const uint32_t *>(q)[qj];
     }
   }
-  // stage the chunk of K and V (16-byte pieces; rows past the sequence are zero).  The loads do not wait for the
-  // sequence length (every row below the cache capacity is readable); rows past the sequence are zeroed afterwards.
-  const uint32_t pieces = headDim / 8;
-  if constexpr (HD != 0) {
-    constexpr int IT = kAttnChunk * (HD / 8) / 256;
-    static_assert(IT * 256 == kAttnChunk * (HD / 8), "one 16-byte piece per thread and round");
-    u32x4 kraw[IT], vraw[IT];
+  // a chunk of K and V in 16-byte pieces, IT per thread.  The first chunk's loads do not wait for the sequence length
+  // (every row below the cache capacity is readable); rows past the sequence are zeroed on their way into LDS.
+  const uint32_t pieces = headDim / 8, npieces = kAttnChunk * pieces;
+  constexpr int IT = kAttnChunk * ((HD ? HD : kAttnMaxHd) / 8) / 256;
+  static_assert(HD == 0 || IT * 256 == kAttnChunk * (HD / 8), "one 16-byte piece per thread and round");
+  u32x4 kraw[IT], vraw[IT];
+  auto fetch = [&](uint32_t t0) {
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const uint32_t i = tid + 256u * it, r = i / (HD / 8), c8 = i % (HD / 8);
+      const uint32_t i = min(tid + 256u * it, npieces - 1), r = i / pieces, c8 = i % pieces;
       const size_t off = (size_t)min(t0 + r, maxSeqLen - 1) * alignedKvDim + kvH * headDim + c8 * 8;
       kraw[it] = ld_u32x4(reinterpret_cast<const uint8_t *>(kCache + off));
       vraw[it] = ld_u32x4(reinterpret_cast<const uint8_t *>(vCache + off));
     }
-    __builtin_amdgcn_sched_barrier(0);
+  };
+  uint32_t t0 = split * kAttnChunk;
+  fetch(t0);
+  __builtin_amdgcn_sched_barrier(0);
+  const uint32_t seqLen = min(params[1], maxSeqLen);   // a length beyond the cache capacity attends the capacity only
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      if (lane + 64 * e < headDim)   // each wave reads only its own queries
+        Qs[(4 * g + wave) * kAttnMaxHd + lane + 64 * e] =
+            q_f16 ? (float)__builtin_bit_cast(half_t, (uint16_t)q_raw[g][e]) : __builtin_bit_cast(float, q_raw[g][e]);
+
+  float m_run[NG], l_run[NG], o_run[NG][2];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    m_run[g] = -INFINITY;
+    l_run[g] = o_run[g][0] = o_run[g][1] = 0.0f;
+  }
+  for (bool first = true;; first = false) {
+    const uint32_t nvalid = t0 < seqLen ? min((uint32_t)kAttnChunk, seqLen - t0) : 0u;   // 0 only in the first chunk
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const uint32_t i = tid + 256u * it, r = i / (HD / 8), c8 = i % (HD / 8);
+      const uint32_t i = tid + 256u * it, r = i / pieces, c8 = i % pieces;
+      if (HD == 0 && i >= npieces) break;
       const bool past = r >= nvalid;
-      *reinterpret_cast<u32x4 *>(Ks + r * kAttnRow + c8 * 8) = past ? u32x4{0, 0, 0, 0} : kraw[it];
-      *reinterpret_cast<u32x4 *>(Vs + r * kAttnRow + c8 * 8) = past ? u32x4{0, 0, 0, 0} : vraw[it];
+      *reinterpret_cast<u32x4 *>(Ks + r * kRow + c8 * 8) = past ? u32x4{0, 0, 0, 0} : kraw[it];
+      *reinterpret_cast<u32x4 *>(Vs + r * kRow + c8 * 8) = past ? u32x4{0, 0, 0, 0} : vraw[it];
     }
-  } else {
-    for (uint32_t i = tid; i < kAttnChunk * pieces; i += 256) {
-      uint32_t r = i / pieces, c8 = i % pieces;
-      size_t off = (size_t)min(t0 + r, maxSeqLen - 1) * alignedKvDim + kvH * headDim + c8 * 8;
-      u32x4 kv = ld_u32x4(reinterpret_cast<const uint8_t *>(kCache + off));
-      u32x4 vv = ld_u32x4(reinterpret_cast<const uint8_t *>(vCache + off));
-      if (r >= nvalid) {
-        kv = u32x4{0, 0, 0, 0};
-        vv = u32x4{0, 0, 0, 0};
+    __syncthreads();   // K, V staged
+    const uint32_t t_next = t0 + nsplit * kAttnChunk;
+    const bool more = t_next < seqLen;
+    if (more) fetch(t_next);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g > 0 && rep0 + 4 * g >= nRep) break;
+      // score of position t0 + lane: q is read as broadcast 16-byte pieces
+      float sc = 0.0f;
+      const half_t *krow = Ks + lane * kRow;
+      const f32x4 *qv = reinterpret_cast<const f32x4 *>(Qs + (4 * g + wave) * kAttnMaxHd);
+#pragma unroll
+      for (uint32_t d = 0; d < headDim; d += 8) {
+        half8_t k8 = *reinterpret_cast<const half8_t *>(krow + d);
+        f32x4 qa = qv[d / 4], qb = qv[d / 4 + 1];
+        sc = fmaf(qa.x, (float)k8[0], sc); sc = fmaf(qa.y, (float)k8[1], sc);
+        sc = fmaf(qa.z, (float)k8[2], sc); sc = fmaf(qa.w, (float)k8[3], sc);
+        sc = fmaf(qb.x, (float)k8[4], sc); sc = fmaf(qb.y, (float)k8[5], sc);
+        sc = fmaf(qb.z, (float)k8[6], sc); sc = fmaf(qb.w, (float)k8[7], sc);
       }
-      *reinterpret_cast<u32x4 *>(Ks + r * kAttnRow + c8 * 8) = kv;
-      *reinterpret_cast<u32x4 *>(Vs + r * kAttnRow + c8 * 8) = vv;
+      sc = lane < nvalid ? sc * scale : -INFINITY;
+      const float mc = wave_max(sc), m = first ? mc : fmaxf(m_run[g], mc);
+      const float p = lane < nvalid ? expf(sc - m) : 0.0f;
+      const float l = wave_sum(p);
+      Ps[wave * kAttnChunk + lane] = p;   // zero for positions past the sequence
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (!first) {
+        const float keep = expf(m_run[g] - m);
+        l_run[g] *= keep;
+        o_run[g][0] *= keep;
+        o_run[g][1] *= keep;
+      }
+      m_run[g] = m;
+      l_run[g] += l;
+      // weighted V: lane owns the adjacent dims 2 * lane and 2 * lane + 1 (one 4-byte LDS read per position),
+      // four weights per 16-byte read; rows past the sequence are zero and carry zero weight.  Heads of 64: lanes
+      // 0-31 take the first 32 positions, lanes 32-63 the others, added at the end.
+      float o0 = o_run[g][0], o1 = o_run[g][1];
+      typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+      constexpr uint32_t kSpan = HD == 64 ? kAttnChunk / 2 : kAttnChunk;
+      const uint32_t tb = HD == 64 ? (lane >> 5) * kSpan : 0u;
+      const f32x4 *pv = reinterpret_cast<const f32x4 *>(Ps + wave * kAttnChunk + tb);
+      const half_t *vcol = Vs + tb * kRow + (HD == 64 ? 2 * (lane & 31) : min(2 * lane, (uint32_t)kAttnMaxHd - 2));
+#pragma unroll
+      for (uint32_t t = 0; t < kSpan; t += 4) {
+        f32x4 p4 = pv[t / 4];
+        half2v v0 = *reinterpret_cast<const half2v *>(vcol + (t + 0) * kRow);
+        half2v v1 = *reinterpret_cast<const half2v *>(vcol + (t + 1) * kRow);
+        half2v v2 = *reinterpret_cast<const half2v *>(vcol + (t + 2) * kRow);
+        half2v v3 = *reinterpret_cast<const half2v *>(vcol + (t + 3) * kRow);
+        o0 = fmaf(p4.x, (float)v0.x, o0); o1 = fmaf(p4.x, (float)v0.y, o1);
+        o0 = fmaf(p4.y, (float)v1.x, o0); o1 = fmaf(p4.y, (float)v1.y, o1);
+        o0 = fmaf(p4.z, (float)v2.x, o0); o1 = fmaf(p4.z, (float)v2.y, o1);
+        o0 = fmaf(p4.w, (float)v3.x, o0); o1 = fmaf(p4.w, (float)v3.y, o1);
+      }
+      o_run[g][0] = o0;
+      o_run[g][1] = o1;
     }
+    if (!more) break;
+    __syncthreads();   // every wave is done with this chunk
+    t0 = t_next;
   }
-  float q_pre[2];
 #pragma unroll
-  for (int e = 0; e < 2; ++e)
-    q_pre[e] = q_f16 ? (float)__builtin_bit_cast(half_t, (uint16_t)q_raw[e]) : __builtin_bit_cast(float, q_raw[e]);
-  // query heads of this KV head are handled four at a time, one per wave
-  for (uint32_t rep0 = 0; rep0 < nRep; rep0 += 4) {
-    const uint32_t rep = rep0 + wave;
-    const bool live = rep < nRep;
-    const uint32_t h = kvH * nRep + (live ? rep : 0);
-    if (rep0 == 0) {
-      // the first pass' query goes to LDS ahead of the staging barrier (each wave reads only its own), so that the
-      // pass costs one workgroup barrier, not two
-#pragma unroll
-      for (int e = 0; e < 2; ++e)
-        if (lane + 64 * e < headDim) Qs[wave * kAttnMaxHd + lane + 64 * e] = q_pre[e];
-      __syncthreads();   // K, V staged
-    } else {
-      __syncthreads();   // Qs, Ps free again
-      for (uint32_t d = lane; d < headDim; d += 64) Qs[wave * kAttnMaxHd + d] = ld_act(q, q_f16, (size_t)h * headDim + d);
-      __syncthreads();
+  for (int g = 0; g < NG; ++g) {
+    float o0 = o_run[g][0], o1 = o_run[g][1];
+    if (HD == 64) {
+      o0 += __shfl_xor(o0, 32);
+      o1 += __shfl_xor(o1, 32);
     }
-    // score of position t0 + lane: q is read as broadcast 16-byte pieces
-    float sc = 0.0f;
-    const half_t *krow = Ks + lane * kAttnRow;
-    const f32x4 *qv = reinterpret_cast<const f32x4 *>(Qs + wave * kAttnMaxHd);
-#pragma unroll
-    for (uint32_t d = 0; d < headDim; d += 8) {
-      half8_t k8 = *reinterpret_cast<const half8_t *>(krow + d);
-      f32x4 qa = qv[d / 4], qb = qv[d / 4 + 1];
-      sc = fmaf(qa.x, (float)k8[0], sc); sc = fmaf(qa.y, (float)k8[1], sc);
-      sc = fmaf(qa.z, (float)k8[2], sc); sc = fmaf(qa.w, (float)k8[3], sc);
-      sc = fmaf(qb.x, (float)k8[4], sc); sc = fmaf(qb.y, (float)k8[5], sc);
-      sc = fmaf(qb.z, (float)k8[6], sc); sc = fmaf(qb.w, (float)k8[7], sc);
+    const uint32_t rep = rep0 + 4 * g + wave;
+    if (rep >= nRep) continue;
+    float *dst = partial + ((size_t)(kvH * nRep + rep) * nsplit + split) * (2 + headDim);
+    if (lane == 0) {
+      dst[0] = m_run[g];   // -inf for a split past the sequence
+      dst[1] = l_run[g];
     }
-    sc = lane < nvalid ? sc * scale : -INFINITY;
-    float m = wave_max(sc);
-    float p = lane < nvalid ? expf(sc - m) : 0.0f;
-    float l = wave_sum(p);
-    Ps[wave * kAttnChunk + lane] = p;   // zero for positions past the sequence
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    // weighted V: lane owns the adjacent dims 2 * lane and 2 * lane + 1 (one 4-byte LDS read per position),
-    // four weights per 16-byte read; rows past the sequence are zero and carry zero weight
-    float o0 = 0.0f, o1 = 0.0f;
-    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-    const f32x4 *pv = reinterpret_cast<const f32x4 *>(Ps + wave * kAttnChunk);
-    const uint32_t dcol = min(2 * lane, (uint32_t)kAttnMaxHd - 2);
-#pragma unroll
-    for (uint32_t t = 0; t < (uint32_t)kAttnChunk; t += 4) {
-      f32x4 p4 = pv[t / 4];
-      half2v v0 = *reinterpret_cast<const half2v *>(Vs + (t + 0) * kAttnRow + dcol);
-      half2v v1 = *reinterpret_cast<const half2v *>(Vs + (t + 1) * kAttnRow + dcol);
-      half2v v2 = *reinterpret_cast<const half2v *>(Vs + (t + 2) * kAttnRow + dcol);
-      half2v v3 = *reinterpret_cast<const half2v *>(Vs + (t + 3) * kAttnRow + dcol);
-      o0 = fmaf(p4.x, (float)v0.x, o0); o1 = fmaf(p4.x, (float)v0.y, o1);
-      o0 = fmaf(p4.y, (float)v1.x, o0); o1 = fmaf(p4.y, (float)v1.y, o1);
-      o0 = fmaf(p4.z, (float)v2.x, o0); o1 = fmaf(p4.z, (float)v2.y, o1);
-      o0 = fmaf(p4.w, (float)v3.x, o0); o1 = fmaf(p4.w, (float)v3.y, o1);
-    }
-    if (live) {
-      float *dst = partial + ((size_t)h * nsplit + split) * (2 + headDim);
-      if (lane == 0) {
-        dst[0] = nvalid ? m : -INFINITY;
-        dst[1] = l;
-      }
-      if (2 * lane + 1 < headDim) {
-        dst[2 + 2 * lane] = o0;
-        dst[2 + 2 * lane + 1] = o1;
-      }
+    if (2 * lane + 1 < headDim) {
+      dst[2 + 2 * lane] = o0;
+      dst[2 + 2 * lane + 1] = o1;
     }
   }
 }
@@ -468,66 +492,82 @@ __global__ void __launch_bounds__(256) attn_partial_wide_kernel(const void *q, c
   }
 }
 
-// One workgroup of 128 threads per query head: the (max, sum) pairs of the splits are taken one per lane, so the
-// merge weights need two wave reductions instead of a serial walk over the splits; thread d then sums dimension d.
-constexpr int kAttnMaxSplit = 1024;   // splits per head the merge kernel holds weights for (context of 65,536)
+// One workgroup per query head.  GROUPS = 1 (128 threads, up to 32 splits): thread d holds dimension d of every split.
+// GROUPS = 8 (1024 threads): group g takes the splits g, g + 8, ..., so that each thread has an eighth of the records to
+// wait for, and the groups meet in LDS (one group walked 256 records in 13.3 us).  Bound: the latency of its loads.
+constexpr int kAttnMaxSplit = 1024;   // splits per head the merge kernel holds weights for
 
-__global__ void __launch_bounds__(128) attn_merge_kernel(const float *partial, const uint32_t *params, void *out, int out_f16,
-                                                         uint32_t headDim, uint32_t nsplit) {
-  __shared__ float Ws[kAttnMaxSplit];
-  __shared__ float red[4];
-  const uint32_t h = blockIdx.x, tid = threadIdx.x;
+template <int GROUPS>
+__global__ void __launch_bounds__(128 * GROUPS) attn_merge_kernel(const float *partial, void *out, int out_f16, uint32_t headDim,
+                                                                  uint32_t nsplit) {
+  constexpr uint32_t kPre = GROUPS == 1 ? 32 : 8;   // records a thread requests at the start
+  __shared__ float Ws[GROUPS == 1 ? 1 : kAttnMaxSplit];
+  __shared__ float red[GROUPS == 1 ? 1 : 2 * GROUPS], reds[GROUPS == 1 ? 1 : 2 * GROUPS];
+  __shared__ float os[GROUPS == 1 ? 1 : GROUPS][kAttnMaxHd];
+  const uint32_t h = blockIdx.x, tid = threadIdx.x, d = tid & 127, g = tid >> 7, lane = tid & 63;
   // every split has a record (empty ones carry max = -inf, sum = 0), so the merge does not need the sequence length
   // and its loads do not wait for it
-  (void)params;
-  const uint32_t used = nsplit;
   const uint32_t rec = 2 + headDim;
   const float *base = partial + (size_t)h * nsplit * rec;
-  // up to 32 splits (a context of 2048): this thread's dimension of every split is requested now, together with the
-  // (max, sum) pairs, so that the whole merge costs one memory round trip instead of three
-  constexpr uint32_t kPre = 32;
-  const bool pre = used <= kPre;
+  // this thread's dimension of the first splits is requested together with the (max, sum) pairs, so that a merge of up
+  // to 32 (64) splits costs one memory round trip instead of three
   float ov[kPre];
 #pragma unroll
-  for (uint32_t s = 0; s < kPre; ++s) ov[s] = (pre && s < used && tid < headDim) ? base[(size_t)s * rec + 2 + tid] : 0.0f;
-  if (pre) {
-    // up to 32 splits: every wave holds all (max, sum) pairs, one per lane, and folds them by itself: no LDS, no
-    // workgroup barrier; the weight of split s comes out of lane s
-    const uint32_t ls = tid & 63;
-    const bool have = ls < used;
-    const float ms = have ? base[(size_t)ls * rec] : -INFINITY, lsum = have ? base[(size_t)ls * rec + 1] : 0.0f;
+  for (uint32_t u = 0; u < kPre; ++u) {
+    const uint32_t s = g + GROUPS * u;
+    ov[u] = (s < nsplit && d < headDim) ? base[(size_t)s * rec + 2 + d] : 0.0f;
+  }
+  float o = 0.0f, L;
+  if (GROUPS == 1 || nsplit <= 64) {
+    // every wave holds all (max, sum) pairs, one per lane, and folds them by itself: no workgroup barrier; the weight of
+    // split s comes out of lane s (every lane takes part in the shuffles; threads beyond the head dimension hold zeros)
+    const bool have = lane < nsplit;
+    const float ms = have ? base[(size_t)lane * rec] : -INFINITY, lsum = have ? base[(size_t)lane * rec + 1] : 0.0f;
     const float M = wave_max(ms);
     const float w = ms == -INFINITY ? 0.0f : expf(ms - M);   // an empty split (and an empty sequence: M = -inf) weighs nothing
-    const float L = wave_sum(lsum * w);
-    float o = 0.0f;   // every lane takes part in the shuffles; threads beyond the head dimension hold zeros
+    L = wave_sum(lsum * w);
 #pragma unroll
-    for (uint32_t s = 0; s < kPre; ++s) o = fmaf(ov[s], __shfl(w, (int)s), o);
-    if (tid < headDim) st_act(out, out_f16, (size_t)h * headDim + tid, L > 0.0f ? o / L : 0.0f);
-    return;
-  }
-  float m = -INFINITY;
-  for (uint32_t s = tid; s < used; s += 128) m = fmaxf(m, base[(size_t)s * rec]);
-  m = wave_max(m);
-  if ((tid & 63) == 0) red[tid >> 6] = m;
-  __syncthreads();
-  const float M = fmaxf(red[0], red[1]);
-  float l = 0.0f;
-  for (uint32_t s = tid; s < used; s += 128) {
-    float ms = base[(size_t)s * rec];
-    float w = ms == -INFINITY ? 0.0f : expf(ms - M);   // an empty split (and an empty sequence: M = -inf) weighs nothing
-    Ws[s] = w;
-    l = fmaf(base[(size_t)s * rec + 1], w, l);
-  }
-  l = wave_sum(l);
-  if ((tid & 63) == 0) red[2 + (tid >> 6)] = l;
-  __syncthreads();
-  const float L = red[2] + red[3];
-  if (tid < headDim) {
-    float o = 0.0f;
+    for (uint32_t u = 0; u < kPre; ++u) o = fmaf(ov[u], __shfl(w, (int)(g + GROUPS * u)), o);
+  } else {
+    float m = tid < nsplit ? base[(size_t)tid * rec] : -INFINITY;   // at most 1024 splits: one pair per thread
+    const float ls = tid < nsplit ? base[(size_t)tid * rec + 1] : 0.0f;
+    const float wm = wave_max(m);
+    if (lane == 0) red[tid >> 6] = wm;
+    __syncthreads();
+    const float M = wave_max(lane < 2 * GROUPS ? red[lane] : -INFINITY);
+    const float w = m == -INFINITY ? 0.0f : expf(m - M);
+    Ws[tid] = w;
+    const float l = wave_sum(ls * w);
+    if (lane == 0) reds[tid >> 6] = l;
+    __syncthreads();
+    L = wave_sum(lane < 2 * GROUPS ? reds[lane] : 0.0f);
+#pragma unroll
+    for (uint32_t u = 0; u < kPre; ++u) {
+      const uint32_t s = g + GROUPS * u;   // < 64 < nsplit
+      o = fmaf(ov[u], Ws[s], o);
+    }
+    if (d < headDim) {
 #pragma unroll 8
-    for (uint32_t s = 0; s < used; ++s) o = fmaf(base[(size_t)s * rec + 2 + tid], Ws[s], o);
-    st_act(out, out_f16, (size_t)h * headDim + tid, L > 0.0f ? o / L : 0.0f);
+      for (uint32_t s = g + GROUPS * kPre; s < nsplit; s += GROUPS) o = fmaf(base[(size_t)s * rec + 2 + d], Ws[s], o);
+    }
   }
+  if constexpr (GROUPS > 1) {
+    os[g][d] = o;
+    __syncthreads();
+    if (g > 0) return;
+#pragma unroll
+    for (int k = 1; k < GROUPS; ++k) o += os[k][d];
+  }
+  if (d < headDim) st_act(out, out_f16, (size_t)h * headDim + d, L > 0.0f ? o / L : 0.0f);
+}
+
+static int launch_attn_merge(const void *records, uint32_t nsplit, uint32_t n_heads, uint32_t head_dim, void *out, int out_f16,
+                             hipStream_t s) {
+  if (nsplit <= 32)
+    hipLaunchKernelGGL(attn_merge_kernel<1>, dim3(n_heads), dim3(128), 0, s, (const float *)records, out, out_f16, head_dim, nsplit);
+  else
+    hipLaunchKernelGGL(attn_merge_kernel<8>, dim3(n_heads), dim3(1024), 0, s, (const float *)records, out, out_f16, head_dim, nsplit);
+  return check_hip(hipGetLastError(), "attention merge launch");
 }
 
 // ---- SiLU(gate) * up on the output of a fused gate+up matmul: in = [gate(n) | up(n)] ----
@@ -787,19 +827,33 @@ static int attn_check_args(const char *who, const void *q, int q_dtype, const vo
   return CUTHIP_OK;
 }
 
+// Splits of the context (records per head): one chunk of 64 positions each while that gives at most kAttnWgs workgroups
+// (two per CU; twice as many where a workgroup serves more than four heads), several beyond, so that every workgroup is
+// resident and streams.  Eight layers of an 8B model in all, us, with 8 KV heads of 128 and a context of 16,384 / 8,192 /
+// 4,096: one chunk per workgroup 420 / 344 / 300, at most 1024 workgroups 401 / 344 / 298, 512 384 / 332 / 300, 256
+// 411 / 340 / 305; 32 KV heads at 8,192: 560 / 512 / 496 / 573; 4 KV heads (eight query heads each) at 16,384: 363 / 363 /
+// 372 / 400.  (One chunk each, one group of threads per merge and no prefetch: 464 / 363 / 318; 534; 446.)
+constexpr uint32_t kAttnWgs = 512;
+static uint32_t attn_splits(uint32_t max_seq_len, uint32_t n_heads, uint32_t n_kv_heads) {
+  const uint32_t chunks = (max_seq_len + kAttnChunk - 1) / kAttnChunk, wgs = n_heads / n_kv_heads > 4 ? 2 * kAttnWgs : kAttnWgs;
+  const uint32_t per = (uint32_t)(((uint64_t)chunks * n_kv_heads + wgs - 1) / wgs);
+  return (chunks + per - 1) / per;
+}
+
 // The two launches of the split-context attention; `partial` holds cuthip_attn_decode_workspace_bytes() bytes.
 static int attn_launch(const void *q, int q_dtype, const void *k_cache, const void *v_cache, const uint32_t *runtime_params,
                        void *out, int out_dtype, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
                        uint32_t aligned_kv_dim, float scale, uint32_t max_seq_len, void *partial, hipStream_t s) {
-  uint32_t nsplit = (max_seq_len + kAttnChunk - 1) / kAttnChunk;
-  auto partial_kernel = head_dim == 128 ? attn_partial_kernel<128> : attn_partial_kernel<0>;
-  hipLaunchKernelGGL(partial_kernel, dim3(n_kv_heads, nsplit), dim3(256), 0, s, q, (const half_t *)k_cache,
+  const uint32_t nsplit = attn_splits(max_seq_len, n_heads, n_kv_heads), n_rep = n_heads / n_kv_heads;
+  const bool two = n_rep > 4;
+  auto kernel = head_dim == 128  ? (two ? attn_partial_kernel<128, 2> : attn_partial_kernel<128, 1>)
+                : head_dim == 64 ? (two ? attn_partial_kernel<64, 2> : attn_partial_kernel<64, 1>)
+                                 : (two ? attn_partial_kernel<0, 2> : attn_partial_kernel<0, 1>);
+  hipLaunchKernelGGL(kernel, dim3(n_kv_heads, nsplit, (n_rep + 7) / 8), dim3(256), 0, s, q, (const half_t *)k_cache,
                      (const half_t *)v_cache, runtime_params, aligned_kv_dim, max_seq_len, n_heads, n_kv_heads,
                      (int)(q_dtype == CUTHIP_F16), head_dim, (float *)partial, scale, nsplit);
   if (int rc = check_hip(hipGetLastError(), "attention launch")) return rc;
-  hipLaunchKernelGGL(attn_merge_kernel, dim3(n_heads), dim3(128), 0, s, (const float *)partial, runtime_params, out,
-                     out_dtype == CUTHIP_F16, head_dim, nsplit);
-  return check_hip(hipGetLastError(), "attention merge launch");
+  return launch_attn_merge(partial, nsplit, n_heads, head_dim, out, out_dtype == CUTHIP_F16, s);
 }
 
 int cuthip_attn_decode(const void *q, int q_dtype, const void *k_cache, const void *v_cache, const uint32_t *runtime_params,
@@ -868,9 +922,7 @@ int cuthip_attn_merge(const void *records, uint32_t nsplit, uint32_t n_heads, ui
               n_heads, head_dim, kAttnMaxHd);
     return CUTHIP_ERR_INVALID;
   }
-  hipLaunchKernelGGL(attn_merge_kernel, dim3(n_heads), dim3(128), 0, (hipStream_t)stream, (const float *)records,
-                     (const uint32_t *)nullptr, out, out_dtype == CUTHIP_F16, head_dim, nsplit);
-  return check_hip(hipGetLastError(), "attention merge launch");
+  return launch_attn_merge(records, nsplit, n_heads, head_dim, out, out_dtype == CUTHIP_F16, (hipStream_t)stream);
 }
 
 }  // extern "C"

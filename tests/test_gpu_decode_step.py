@@ -132,6 +132,28 @@ def test_attention_decode(ops, n_heads, n_kv, hd, seq, max_ctx):
     assert normwise_rel_err(out.cpu().numpy(), want) < 2e-6
 
 
+# several chunks of 64 positions per workgroup (two and three, a last chunk that is short or missing), heads of 64 / 128 /
+# other, five and nine query heads per KV head, merges of 33 and 130 records; tolerance: fp32 sums in any order, as above
+@pytest.mark.parametrize("n_heads,n_kv,hd,seq,max_ctx", [(32, 32, 64, 1090, 1100), (32, 32, 64, 577, 1100), (32, 32, 64, 3, 1100),
+                                                       (80, 16, 16, 4200, 4200), (64, 16, 128, 4401, 4480), (18, 2, 128, 100, 130),
+                                                       (4, 1, 128, 8250, 8256), (9, 1, 64, 8256, 8256), (66, 33, 40, 1100, 1100)])
+def test_attention_decode_several_chunks_per_workgroup(ops, n_heads, n_kv, hd, seq, max_ctx):
+    rng = np.random.default_rng(n_heads + seq)
+    q = rng.standard_normal(n_heads * hd).astype(np.float16)
+    K = (rng.standard_normal((max_ctx, n_kv * hd)) * 0.5).astype(np.float16)
+    V = rng.standard_normal((max_ctx, n_kv * hd)).astype(np.float16)
+    scale = 1 / math.sqrt(hd)
+    want = oracle.attention_decode(q.astype(np.float32), K.view(np.uint16), V.view(np.uint16), seq, n_heads, n_kv, hd, scale)
+    K[seq:], V[seq:] = np.float16(60000.0), np.float16(np.nan)   # what lies past the sequence must not matter
+    ws = ops.attn_decode_workspace(n_heads, hd, max_ctx, "cuda")
+    out = torch.full((n_heads * hd,), np.nan, dtype=torch.float32, device="cuda")
+    for qd in (q, q.astype(np.float32)):
+        for n in (seq, 0):
+            ops.attn_decode(dev(qd), dev(K), dev(V), dev(np.array([n - 1, n], np.int32)), n_heads, n_kv, hd, scale, ws, out)
+            torch.cuda.synchronize()
+            assert normwise_rel_err(out.cpu().numpy(), want) < 2e-6 if n else bool((out == 0).all())
+
+
 def test_silu_mul_and_argmax(ops):
     rng = np.random.default_rng(5)
     gu = (rng.standard_normal(2 * 14336) * 3).astype(np.float16)
