@@ -94,6 +94,8 @@ CUTHIP_EXTERN_PAIR(CUTHIP_Q4_K, CUTHIP_Q4_K)
 CUTHIP_EXTERN_PAIR(CUTHIP_Q4_K, CUTHIP_Q6_K)
 CUTHIP_EXTERN_PAIR(CUTHIP_Q6_K, CUTHIP_Q4_K)
 CUTHIP_EXTERN_PAIR(CUTHIP_Q6_K, CUTHIP_Q6_K)
+CUTHIP_EXTERN_PAIR(CUTHIP_Q8_0, CUTHIP_Q8_0)
+CUTHIP_EXTERN_PAIR(CUTHIP_Q4_0, CUTHIP_Q4_0)
 #undef CUTHIP_EXTERN_PAIR
 
 static int launch_rows8_any(int fmt, const GemvParams &p, hipStream_t stream, bool *taken) {
@@ -570,6 +572,8 @@ int cuthip_matmul_gguf_pair(int fmt_a, const void *Wa, uint32_t Na, void *Ca, in
     else if (fmt_a == CUTHIP_Q4_K && fmt_b == CUTHIP_Q6_K) taken = launch_rows8_pair_fmt<CUTHIP_Q4_K, CUTHIP_Q6_K>(pa, pb, s, &rc);
     else if (fmt_a == CUTHIP_Q6_K && fmt_b == CUTHIP_Q4_K) taken = launch_rows8_pair_fmt<CUTHIP_Q6_K, CUTHIP_Q4_K>(pa, pb, s, &rc);
     else if (fmt_a == CUTHIP_Q6_K && fmt_b == CUTHIP_Q6_K) taken = launch_rows8_pair_fmt<CUTHIP_Q6_K, CUTHIP_Q6_K>(pa, pb, s, &rc);
+    else if (fmt_a == CUTHIP_Q8_0 && fmt_b == CUTHIP_Q8_0) taken = launch_rows8_pair_fmt<CUTHIP_Q8_0, CUTHIP_Q8_0>(pa, pb, s, &rc);
+    else if (fmt_a == CUTHIP_Q4_0 && fmt_b == CUTHIP_Q4_0) taken = launch_rows8_pair_fmt<CUTHIP_Q4_0, CUTHIP_Q4_0>(pa, pb, s, &rc);
     if (taken) return rc;
   }
   // other formats or shapes: the same two products as two launches

@@ -1261,8 +1261,9 @@ template <int FMT> int launch_rows8_fmt(const GemvParams &p, hipStream_t stream)
   return launch_rows8_shape<FMT, 8>(p, s.rwg, s.kw, stream);
 }
 
-// Pair launch for the K-quant formats at the shapes a decode step uses; returns false (nothing launched) for
-// anything else, and the caller issues two launches.
+// Pair launch at the shapes a decode step uses; returns false (nothing launched) for anything else, and the caller issues
+// two launches.  A layer of 2048 hidden elements at 8 bits (2560 and 512 rows) took 7.0 + 4.9 us in two launches, both mostly
+// start-up; its decode step of 16 layers went from 690 to 599 us with the pair.
 template <int FA, int FB> bool launch_rows8_pair_fmt(const GemvParams &pa, const GemvParams &pb, hipStream_t stream, int *rc) {
   if (pa.M != 1 || pb.M != 1 || pa.K != pb.K || pa.pro || pb.pro) return false;
   if (rows8_lds_bytes<FA>(pa, 1) > kRows8LdsBudget || rows8_lds_bytes<FB>(pb, 1) > kRows8LdsBudget) return false;
@@ -1272,6 +1273,8 @@ template <int FA, int FB> bool launch_rows8_pair_fmt(const GemvParams &pa, const
   else if (s.kw == 2) *rc = launch_rows8_pair<FA, FB, 2, 2, D, 4>(pa, pb, stream);
   // four steps per wave: a ring of two (1.730 against 1.750 ms per token of an 8B decode step with a ring of four)
   else if (s.kw == 4 && pa.nsteps <= 16) *rc = launch_rows8_pair<FA, FB, 1, 4, 2, 2>(pa, pb, stream);
+  // K up to 8192: five to eight steps per wave, and up to four groups of activations per thread
+  else if (s.kw == 4 && pa.nsteps <= 32) *rc = launch_rows8_pair<FA, FB, 1, 4, 2, 4>(pa, pb, stream);
   else return false;
   return true;
 }

@@ -324,8 +324,8 @@ typedef struct {
  * (Q4_K and Q6_K in the common GGUF mixes) and so cannot be concatenated like
  * gate and up; the reference fuses wqkv only when the loader could concatenate
  * them and otherwise issues one matmul per projection
- * (interface/runner/llama/llama.cpp:1710-1756).  One launch for the K-quant
- * formats at decode shapes, otherwise the same two products as two launches.
+ * (interface/runner/llama/llama.cpp:1710-1756).  One launch for pairs of K-quant
+ * formats and for two tensors of one format at decode shapes, otherwise the same two products as two launches.
  * No epilogue; dtypes and alignment as cuthip_matmul_gguf. */
 int cuthip_matmul_gguf_pair(int fmt_a, const void *Wa, uint32_t Na, void *Ca, int fmt_b, const void *Wb, uint32_t Nb,
                             void *Cb, const void *A, int a_dtype, int c_dtype, uint32_t K,

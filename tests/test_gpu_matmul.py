@@ -443,6 +443,26 @@ def test_pair_launch_equals_two_matmuls(ops, fa, fb, Na, Nb, K):
         assert normwise_rel_err(c.cpu().numpy()[None, :], single.cpu().numpy()) < 2e-6
 
 
+@pytest.mark.parametrize("fmt_name", ["Q8_0", "Q4_0", "Q4_K", "Q6_K"])
+@pytest.mark.parametrize("Na,Nb,K", [(2560, 512, 2048), (2560, 512, 2048 + 256), (1000, 333, 4096 + 256), (1001, 127, 8192), (24, 17, 512),
+                                     (9, 7, 256)])
+def test_pair_launch_of_one_format(ops, fmt_name, Na, Nb, K):
+    """Both tensors of one format: every split of K of the joint launch (1, 2 and 4 ranges, up to 8 steps per range) and row
+    counts that end inside a group of eight, with the outputs' surroundings left alone."""
+    fmt = oracle.FORMATS[fmt_name]
+    A = gauss_acts((1, K), seed=63, dtype=np.float16)
+    wa, wb = quantized_weights(fmt, Na, K, seed=64), quantized_weights(fmt, Nb, K, seed=65)
+    both = torch.full((Na + Nb + 8,), 7.0, dtype=torch.float32, device="cuda")
+    ops.matmul_gguf_pair(torch.from_numpy(A).cuda().view(-1), torch.from_numpy(wa).cuda(), fmt, Na, both[:Na], torch.from_numpy(wb).cuda(),
+                         fmt, Nb, both[Na:Na + Nb], K)
+    torch.cuda.synchronize()
+    got = both.cpu().numpy()
+    assert np.all(got[Na + Nb:] == 7.0)
+    for w, n, c in ((wa, Na, got[:Na]), (wb, Nb, got[Na:Na + Nb])):
+        want = oracle.matmul_gguf(fmt, w, A.astype(np.float32), n, f64=True)
+        assert normwise_rel_err(c[None, :], want) < TOL_F16_ACT
+
+
 @pytest.mark.parametrize("name", list(oracle.FORMATS))
 @pytest.mark.parametrize("M,N,K", [(2, 4096, 14336), (4, 4096, 14336), (8, 4096, 14336), (3, 4096, 14336), (3, 100, 8192), (5, 9, 8192 + 32),
                                    (2, 100, 8192 + 256)])
