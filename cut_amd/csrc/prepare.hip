@@ -10,30 +10,32 @@
 //     unrounded scale), nibbles kept, written in the [K, N/2] orientation.
 //   * fp32 rows -> Q8_0 blocks (quantizeRowsQ8_0, llama.cpp:488-505).
 //
-// All of it is byte shuffling bound by HBM.  A workgroup copies the block runs
-// of 128 weight rows into LDS with coalesced 2-byte loads (GGUF blocks are only
-// 2-byte aligned; the LDS image pads every block so that its quants are dword
-// aligned), then every thread reads one dword (four consecutive k) of 4 (int8)
-// or 8 (nibble) neighbouring rows, transposes the 4 x 4 bytes with v_perm_b32
-// and writes four dwords, so the transposed rows are written in runs of 128
-// (64) bytes.
+// All of it is byte shuffling bound by HBM.  A workgroup takes 256 elements of k of 128 (int8) or 256 (nibbles) weight
+// rows, so that it writes runs of 128 bytes, whole cache lines.  It requests the blocks in 16-byte pieces (GGUF blocks are
+// only 2-byte aligned), all of them before the first use, and puts the quants into LDS without the scales between them;
+// then a thread reads a 16-byte piece of 4 (int8) or 8 (nibble) neighbouring rows, transposes 4 x 4 bytes at a time with
+// v_perm_b32 and writes 16 (32) dwords.  14336 x 4096, us: Q8_0 52 -> 25, Q4_0 34 -> 15, Q4_K 38 -> 13.5 (before: 2-byte
+// loads, one dword per row read from LDS, runs of 64 bytes for nibbles), all three 154 -> 67, 3.9 TB/s.
 #include <cstdint>
 
 #include "common.hpp"
 
 namespace cuthip {
 
-constexpr int kPrepRows = 128;      // weight rows per tile
 constexpr int kPrepThreads = 256;
+constexpr int kPrepK = 256;   // k extent of a tile
 
 enum PrepMode { PREP_Q8_0 = 0, PREP_Q4_0 = 1, PREP_Q4_K_AFFINE = 2, PREP_NIBBLES = 3 };
 
-// k extent of a tile and the bytes one weight row contributes to it
-template <int MODE> struct PrepGeom;
-template <> struct PrepGeom<PREP_Q8_0> { static constexpr int KT = 128, RUN = 4 * 34, PITCH = 4 * 36 + 4; };
-template <> struct PrepGeom<PREP_Q4_0> { static constexpr int KT = 256, RUN = 8 * 18, PITCH = 8 * 20 + 4; };
-template <> struct PrepGeom<PREP_Q4_K_AFFINE> { static constexpr int KT = 256, RUN = 144, PITCH = RUN; };
-template <> struct PrepGeom<PREP_NIBBLES> { static constexpr int KT = 256, RUN = 128, PITCH = RUN + 4; };
+// ROWS: weight rows of a tile.  PIECES: 16-byte pieces of a row's LDS image.  A row takes PIECES (made odd) x 16 bytes there
+// and row r sits at (r % G) * 32 + r / G, G = rows of a transposition item: the 32 lanes that read row G * lane + j of
+// their items then touch every bank once.
+template <int MODE> struct PrepGeom {
+  static constexpr int G = MODE == PREP_Q8_0 ? 4 : 8, ROWS = 32 * G;
+  static constexpr int PIECES = MODE == PREP_Q8_0 ? 16 : MODE == PREP_Q4_K_AFFINE ? 9 : 8, PITCH = 16 * (PIECES | 1);
+  static constexpr bool SCALES = MODE == PREP_Q8_0 || MODE == PREP_Q4_0;   // blocks of 32 with one fp16 scale
+  static __device__ uint32_t slot(uint32_t row) { return (row % G) * 32 + row / G; }
+};
 
 struct PrepParams {
   const uint8_t *src;
@@ -41,128 +43,142 @@ struct PrepParams {
   uint16_t *S;
   uint32_t N, K, strideB, scaleStride;
   uint32_t src_row_bytes;
+  uint32_t tiles, ktiles, tiles_per_xcd;   // set by the launch
 };
 
-// Where the quant byte of element k (a multiple of 4) of a row sits in its LDS image, and the shift that brings its
-// nibble down.  Q4_K: piece g = k / 64, low nibbles are its first 32 elements, high nibbles the rest.  GGML Q4_0 order
-// (also the packed tensor of the separated reader): low nibble of byte j of a block is element j, high nibble element
-// j + 16.  The Q4_0 image keeps each block at 20 bytes ([d][2 bytes unused][qs:16]) so that the quants are dword aligned.
-template <int MODE> __device__ inline uint32_t prep_quant_offset(uint32_t k) {
-  if (MODE == PREP_Q4_K_AFFINE) return 16 + 32 * (k >> 6) + (k & 31);
-  if (MODE == PREP_Q4_0) return (k >> 5) * 20 + 4 + (k & 15);
-  return (k >> 5) * 16 + (k & 15);
-}
-template <int MODE> __device__ inline uint32_t prep_quant_shift(uint32_t k) {
-  return MODE == PREP_Q4_K_AFFINE ? ((k & 32) ? 4u : 0u) : ((k & 16) ? 4u : 0u);
+// 4 x 4 bytes: byte i of in[j] -> byte j of out[i]
+__device__ __forceinline__ void transpose4(const uint32_t (&in)[4], uint32_t (&out)[4]) {
+  const uint32_t t0 = __builtin_amdgcn_perm(in[1], in[0], 0x05010400u), t1 = __builtin_amdgcn_perm(in[3], in[2], 0x05010400u);
+  const uint32_t t2 = __builtin_amdgcn_perm(in[1], in[0], 0x07030602u), t3 = __builtin_amdgcn_perm(in[3], in[2], 0x07030602u);
+  out[0] = __builtin_amdgcn_perm(t1, t0, 0x05040100u);
+  out[1] = __builtin_amdgcn_perm(t1, t0, 0x07060302u);
+  out[2] = __builtin_amdgcn_perm(t3, t2, 0x05040100u);
+  out[3] = __builtin_amdgcn_perm(t3, t2, 0x07060302u);
 }
 
 template <int MODE> __global__ void __launch_bounds__(kPrepThreads) prepare_sep_kernel(PrepParams p) {
   using G = PrepGeom<MODE>;
-  __shared__ __attribute__((aligned(16))) uint8_t raw[kPrepRows * G::PITCH];
+  __shared__ __attribute__((aligned(16))) uint8_t raw[G::ROWS * G::PITCH];
+  __shared__ uint16_t sc[G::SCALES ? 8 * G::ROWS : 1];
   const uint32_t tid = threadIdx.x;
-  const uint32_t n0 = blockIdx.x * kPrepRows, k0 = blockIdx.y * G::KT;
-  const uint32_t run_off = blockIdx.y * G::RUN;
-  const uint32_t valid = min((uint32_t)G::RUN, p.src_row_bytes - run_off);   // the last tile of a row may be short
-  constexpr uint32_t W = G::RUN / 2;
-  for (uint32_t i = tid; i < kPrepRows * W; i += kPrepThreads) {
-    const uint32_t row = i / W, w = i - row * W, n = n0 + row;
-    uint16_t v = 0;
-    if (n < p.N && 2 * w < valid) v = (uint16_t)ld_u16(p.src + (size_t)n * p.src_row_bytes + run_off + 2 * w);
-    uint32_t dst = 2 * w;
-    if (MODE == PREP_Q4_0) dst = (w / 9) * 20 + ((w % 9) ? 2 * (w % 9) + 2 : 0);   // scale at 0, quants from byte 4
-    if (MODE == PREP_Q8_0) dst = (w / 17) * 36 + ((w % 17) ? 2 * (w % 17) + 2 : 0);  // [d][2 bytes unused][q:32]
-    *reinterpret_cast<uint16_t *>(raw + row * G::PITCH + dst) = v;
-  }
-  __syncthreads();
-  const uint32_t kt = min((uint32_t)G::KT, p.K - k0);
+  // an XCD (block index modulo 8) walks along k before it goes to the next rows: the cache lines that two neighbouring
+  // tiles of a row share are read once into its L2
+  const uint32_t tile = (blockIdx.x & 7u) * p.tiles_per_xcd + (blockIdx.x >> 3);
+  if (tile >= p.tiles) return;
+  const uint32_t nt = tile / p.ktiles, n0 = nt * G::ROWS, k0 = (tile - nt * p.ktiles) * kPrepK;
+  const uint32_t kt = min((uint32_t)kPrepK, p.K - k0);   // a multiple of 32
 
-  if constexpr (MODE == PREP_Q8_0) {
-    // item = (4 consecutive k, 4 rows): one dword of LDS per row (the image keeps every block at 36 bytes so that the
-    // quants are dword aligned), a 4 x 4 byte transpose, four dwords B[k + i, n .. n+3]
-    const bool words = (p.strideB & 3u) == 0;
-    for (uint32_t i = tid; i < (uint32_t)(G::KT / 4) * (kPrepRows / 4); i += kPrepThreads) {
-      const uint32_t k = (i / (kPrepRows / 4)) * 4, r4 = (i % (kPrepRows / 4)) * 4, n = n0 + r4;
-      if (k >= kt || n >= p.N) continue;
-      const uint32_t off = (k >> 5) * 36 + 4 + (k & 31);
-      uint32_t pr[4];
+  // Rows past N and blocks past K read the last one instead and are not written.
+  if constexpr (G::SCALES) {
+    constexpr uint32_t BYTES = MODE == PREP_Q8_0 ? 34 : 18, Q = MODE == PREP_Q8_0 ? 2 : 1;   // Q: 16-byte pieces of quants
+    constexpr int IT = 8 * G::ROWS / kPrepThreads;
+    const uint32_t blk = tid & 7u, b = k0 / 32 + min(blk, kt / 32 - 1);
+    u32x4 q[IT][Q];
+    uint32_t d[IT];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) pr[j] = *reinterpret_cast<const uint32_t *>(raw + (r4 + j) * G::PITCH + off);
-      const uint32_t t0 = __builtin_amdgcn_perm(pr[1], pr[0], 0x05010400u), t1 = __builtin_amdgcn_perm(pr[3], pr[2], 0x05010400u);
-      const uint32_t t2 = __builtin_amdgcn_perm(pr[1], pr[0], 0x07030602u), t3 = __builtin_amdgcn_perm(pr[3], pr[2], 0x07030602u);
-      const uint32_t out[4] = {__builtin_amdgcn_perm(t1, t0, 0x05040100u), __builtin_amdgcn_perm(t1, t0, 0x07060302u),
-                               __builtin_amdgcn_perm(t3, t2, 0x05040100u), __builtin_amdgcn_perm(t3, t2, 0x07060302u)};
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t n = min(n0 + it * 32u + (tid >> 3), p.N - 1);
+      const uint8_t *src = p.src + (size_t)n * p.src_row_bytes + b * BYTES;
+      d[it] = ld_u16(src);
 #pragma unroll
-      for (uint32_t e = 0; e < 4; ++e) {
-        if (k + e >= kt) break;
-        uint8_t *dst = p.B + (size_t)(k0 + k + e) * p.strideB + n;
-        if (words && n + 3 < p.N) {
-          *reinterpret_cast<uint32_t *>(dst) = out[e];
-        } else {
-          for (uint32_t j = 0; j < 4 && n + j < p.N; ++j) dst[j] = (uint8_t)(out[e] >> (8 * j));
-        }
-      }
+      for (uint32_t u = 0; u < Q; ++u) q[it][u] = ld_u32x4(src + 2 + 16 * u);
     }
-    for (uint32_t i = tid; i < (G::KT / 32) * kPrepRows; i += kPrepThreads) {
-      const uint32_t blk = i / kPrepRows, row = i % kPrepRows, n = n0 + row;
-      if (n < p.N && blk * 32 < kt)
-        p.S[(size_t)(k0 / 32 + blk) * p.scaleStride + n] = *reinterpret_cast<const uint16_t *>(raw + row * G::PITCH + blk * 36);
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t row = it * 32u + (tid >> 3);
+#pragma unroll
+      for (uint32_t u = 0; u < Q; ++u) *reinterpret_cast<u32x4 *>(raw + G::slot(row) * G::PITCH + (blk * Q + u) * 16) = q[it][u];
+      sc[blk * G::ROWS + row] = (uint16_t)d[it];
     }
   } else {
-    // item = (4 consecutive k, 8 rows): one dword of LDS per row holds the four quants (k .. k+3 share a nibble half
-    // and four neighbouring bytes), row pairs are merged into bytes (even row in the low nibble) and a 4 x 4 byte
-    // transpose (v_perm_b32) turns [row pair][k] into the four output dwords B[k + i, n/2 .. n/2+3]
-    const bool words = (p.strideB & 3u) == 0;
-    for (uint32_t i = tid; i < (uint32_t)(G::KT / 4) * (kPrepRows / 8); i += kPrepThreads) {
-      const uint32_t k = (i / (kPrepRows / 8)) * 4, r8 = (i % (kPrepRows / 8)) * 8, n = n0 + r8;
-      if (k >= kt || n >= p.N) continue;
-      const uint32_t off = prep_quant_offset<MODE>(k), sh = prep_quant_shift<MODE>(k);
-      uint32_t pr[4];
+    constexpr uint32_t RUN = G::PIECES * 16;
+    constexpr int IT = (G::ROWS * G::PIECES + kPrepThreads - 1) / kPrepThreads;
+    static_assert(IT * kPrepThreads == G::ROWS * G::PIECES, "whole rounds of pieces");
+    const uint32_t last = MODE == PREP_NIBBLES ? kt / 32 - 1 : G::PIECES - 1;
+    const uint8_t *src = p.src + (size_t)(k0 / kPrepK) * RUN;
+    u32x4 q[IT];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t lo = (*reinterpret_cast<const uint32_t *>(raw + (r8 + 2 * j) * G::PITCH + off) >> sh) & 0x0F0F0F0Fu;
-        const uint32_t hi = (*reinterpret_cast<const uint32_t *>(raw + (r8 + 2 * j + 1) * G::PITCH + off) >> sh) & 0x0F0F0F0Fu;
-        pr[j] = lo | (hi << 4);   // byte i: rows (r8 + 2j, r8 + 2j + 1) at k + i; rows past N are zero
-      }
-      const uint32_t t0 = __builtin_amdgcn_perm(pr[1], pr[0], 0x05010400u), t1 = __builtin_amdgcn_perm(pr[3], pr[2], 0x05010400u);
-      const uint32_t t2 = __builtin_amdgcn_perm(pr[1], pr[0], 0x07030602u), t3 = __builtin_amdgcn_perm(pr[3], pr[2], 0x07030602u);
-      const uint32_t out[4] = {__builtin_amdgcn_perm(t1, t0, 0x05040100u), __builtin_amdgcn_perm(t1, t0, 0x07060302u),
-                               __builtin_amdgcn_perm(t3, t2, 0x05040100u), __builtin_amdgcn_perm(t3, t2, 0x07060302u)};
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t i = it * kPrepThreads + tid, row = i / G::PIECES, c = i - row * G::PIECES;
+      q[it] = ld_u32x4(src + (size_t)min(n0 + row, p.N - 1) * p.src_row_bytes + min(c, last) * 16);
+    }
 #pragma unroll
-      for (uint32_t e = 0; e < 4; ++e) {
-        if (k + e >= kt) break;
-        uint8_t *dst = p.B + (size_t)(k0 + k + e) * p.strideB + n / 2;
-        if (words && n + 7 < p.N) {
-          *reinterpret_cast<uint32_t *>(dst) = out[e];
-        } else {
-          for (uint32_t j = 0; j < 4 && n + 2 * j < p.N; ++j) dst[j] = (uint8_t)(out[e] >> (8 * j));
-        }
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t i = it * kPrepThreads + tid, row = i / G::PIECES, c = i - row * G::PIECES;
+      *reinterpret_cast<u32x4 *>(raw + G::slot(row) * G::PITCH + c * 16) = q[it];
+    }
+  }
+  __syncthreads();
+
+  const bool words = (p.strideB & 3u) == 0;
+  const uint32_t lane = tid & 31u;   // rows G * lane .. of the tile
+  const uint32_t col = (MODE == PREP_Q8_0 ? n0 : n0 / 2) + 4 * lane, cols = MODE == PREP_Q8_0 ? p.N : p.N / 2;
+  auto put = [&](uint32_t k, uint32_t v) {   // columns col .. col + 3 of row k0 + k
+    uint8_t *dst = p.B + (size_t)(k0 + k) * p.strideB + col;
+    if (words && col + 3 < cols) {
+      *reinterpret_cast<uint32_t *>(dst) = v;
+    } else {
+      for (uint32_t j = 0; j < 4 && col + j < cols; ++j) dst[j] = (uint8_t)(v >> (8 * j));
+    }
+  };
+  // Q8_0: piece c holds k = 16 c ..; nibbles: 32 k of block c, low half first (Q4_K: of 64 k, 16 low and 16 high ones)
+  constexpr uint32_t QUANTS = MODE == PREP_Q8_0 ? 16 : 8, FIRST = MODE == PREP_Q4_K_AFFINE ? 1 : 0;
+  for (uint32_t c = tid >> 5; c < QUANTS; c += kPrepThreads / 32) {
+    const uint32_t k = MODE == PREP_Q8_0 ? 16 * c : MODE == PREP_Q4_K_AFFINE ? 64 * (c >> 1) + 16 * (c & 1) : 32 * c;
+    if (k >= kt) break;
+    u32x4 q[G::G];
+#pragma unroll
+    for (int j = 0; j < G::G; ++j) q[j] = *reinterpret_cast<const u32x4 *>(raw + (j * 32 + lane) * G::PITCH + (FIRST + c) * 16);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      uint32_t in[4], out[4];
+      if constexpr (MODE == PREP_Q8_0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) in[j] = q[j][w];
+        transpose4(in, out);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) put(k + 4 * w + e, out[e]);
+      } else {
+        constexpr uint32_t kLow = 0x0F0F0F0Fu, HIGH = MODE == PREP_Q4_K_AFFINE ? 32 : 16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) in[j] = (q[2 * j][w] & kLow) | ((q[2 * j + 1][w] & kLow) << 4);   // even row in the low nibble
+        transpose4(in, out);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) put(k + 4 * w + e, out[e]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) in[j] = ((q[2 * j][w] >> 4) & kLow) | (q[2 * j + 1][w] & ~kLow);
+        transpose4(in, out);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) put(k + HIGH + 4 * w + e, out[e]);
       }
     }
-    if constexpr (MODE == PREP_Q4_0) {
-      for (uint32_t i = tid; i < (G::KT / 32) * kPrepRows; i += kPrepThreads) {
-        const uint32_t blk = i / kPrepRows, row = i % kPrepRows, n = n0 + row;
-        if (n < p.N && blk * 32 < kt)
-          p.S[(size_t)(k0 / 32 + blk) * p.scaleStride + n] = *reinterpret_cast<const uint16_t *>(raw + row * G::PITCH + blk * 20);
-      }
+  }
+  if constexpr (G::SCALES) {
+#pragma unroll
+    for (int it = 0; it < 8 * G::ROWS / kPrepThreads; ++it) {
+      const uint32_t i = it * kPrepThreads + tid, blk = i / G::ROWS, n = n0 + i % G::ROWS;
+      if (n < p.N && blk * 32 < kt) p.S[(size_t)(k0 / 32 + blk) * p.scaleStride + n] = sc[i];
     }
-    if constexpr (MODE == PREP_Q4_K_AFFINE) {
-      const uint32_t blocksK = p.K / 32;
-      for (uint32_t i = tid; i < 8 * kPrepRows; i += kPrepThreads) {
-        const uint32_t j = i / kPrepRows, row = i % kPrepRows, n = n0 + row;
-        if (n >= p.N) continue;
-        const uint8_t *r = raw + row * G::PITCH, *q = r + 4;
-        const float d = f16bits_to_f32(*reinterpret_cast<const uint16_t *>(r));
-        const float dmin = f16bits_to_f32(*reinterpret_cast<const uint16_t *>(r + 2));
-        uint32_t sc, m;   // get_scale_min_k4 (llama.cpp:547-555)
+  }
+  if constexpr (MODE == PREP_Q4_K_AFFINE) {   // one thread per row: scales and minima of its eight sub-blocks
+    static_assert(G::ROWS == kPrepThreads, "one row per thread");
+    const uint32_t n = n0 + tid, blocksK = p.K / 32;
+    if (n < p.N) {
+      const u32x4 h = *reinterpret_cast<const u32x4 *>(raw + G::slot(tid) * G::PITCH);
+      const float d = f16bits_to_f32(h.x & 0xFFFFu), dmin = f16bits_to_f32(h.x >> 16);
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) {
+        const uint32_t sh = 8 * (j & 3);
+        uint32_t s, m;   // get_scale_min_k4 (llama.cpp:547-555) on the packed bytes h.y, h.z, h.w
         if (j < 4) {
-          sc = q[j] & 63u;
-          m = q[j + 4] & 63u;
+          s = (h.y >> sh) & 63u;
+          m = (h.z >> sh) & 63u;
         } else {
-          sc = (q[j + 4] & 15u) | ((uint32_t)(q[j - 4] >> 6) << 4);
-          m = (uint32_t)(q[j + 4] >> 4) | ((uint32_t)(q[j] >> 6) << 4);
+          s = ((h.w >> sh) & 15u) | (((h.y >> (sh + 6)) & 3u) << 4);
+          m = ((h.w >> (sh + 4)) & 15u) | (((h.z >> (sh + 6)) & 3u) << 4);
         }
         // both products are exact in fp32 (11 x 6 bits), so the subtraction is the only rounding whether or not it is fused
-        const float scale = d * (float)sc;
+        const float scale = d * (float)s;
         const float minv = 8.0f * scale - dmin * (float)m;
         const size_t b = k0 / 32 + j;
         p.S[b * p.scaleStride + n] = (uint16_t)f32_to_f16bits_any(scale);
@@ -172,14 +188,17 @@ template <int MODE> __global__ void __launch_bounds__(kPrepThreads) prepare_sep_
   }
 }
 
-template <int MODE> static int launch_prepare(const PrepParams &p, hipStream_t stream) {
+template <int MODE> static int launch_prepare(PrepParams p, hipStream_t stream) {
   using G = PrepGeom<MODE>;
-  dim3 grid((p.N + kPrepRows - 1) / kPrepRows, (p.K + G::KT - 1) / G::KT);
-  if (grid.y > 65535u) {
+  p.ktiles = (p.K - 1) / kPrepK + 1;
+  const uint64_t tiles = (uint64_t)((p.N - 1) / G::ROWS + 1) * p.ktiles;
+  if ((p.K - 1) / (MODE == PREP_Q8_0 ? 128 : 256) >= 65535u || tiles > 0x7FFFFFF0ull) {
     set_error("prepare: K = %u is too long for one launch", p.K);
     return CUTHIP_ERR_INVALID;
   }
-  hipLaunchKernelGGL(prepare_sep_kernel<MODE>, grid, dim3(kPrepThreads), 0, stream, p);
+  p.tiles = (uint32_t)tiles;
+  p.tiles_per_xcd = (p.tiles + 7) / 8;
+  hipLaunchKernelGGL(prepare_sep_kernel<MODE>, dim3(8 * p.tiles_per_xcd), dim3(kPrepThreads), 0, stream, p);
   return check_hip(hipGetLastError(), "prepare launch");
 }
 
@@ -241,7 +260,7 @@ int cuthip_prepare_sep(int fmt, const void *blocks, uint32_t N, uint32_t K, void
     set_error("cuthip_prepare_sep: B must be 4-byte aligned, blocks and scales 2-byte aligned");
     return CUTHIP_ERR_INVALID;
   }
-  PrepParams p;
+  PrepParams p{};
   p.src = reinterpret_cast<const uint8_t *>(blocks);
   p.B = reinterpret_cast<uint8_t *>(B);
   p.S = scales;
@@ -275,13 +294,13 @@ int cuthip_transpose_q4_nibble(const void *packed, void *packedT, uint32_t N, ui
     set_error("cuthip_transpose_q4_nibble: output must be 4-byte aligned, input 2-byte aligned");
     return CUTHIP_ERR_INVALID;
   }
-  PrepParams p;
+  PrepParams p{};
   p.src = reinterpret_cast<const uint8_t *>(packed);
   p.B = reinterpret_cast<uint8_t *>(packedT);
   p.S = nullptr;
   p.N = N; p.K = K; p.strideB = strideOutHalf; p.scaleStride = 0;
   p.src_row_bytes = strideInHalf;
-  // a tile reads 128 bytes of each row; only K / 2 of a padded row are nibbles, the kernel stops at K
+  // only K / 2 bytes of a padded row are nibbles: the kernel stops at K
   return launch_prepare<PREP_NIBBLES>(p, (hipStream_t)stream);
 }
 

@@ -513,8 +513,13 @@ def prepare_sep(w_blocks: torch.Tensor, fmt, N: int, K: int, stride_b: int | Non
     sb = stride_b if stride_b is not None else (width + 3) & ~3
     ss = scale_stride if scale_stride is not None else (N + 3) & ~3
     rows_s = (2 if f == _l.Q4_K else 1) * (K // 32)
-    B = torch.zeros((K, sb), dtype=torch.uint8 if q4 else torch.int8, device=w_blocks.device)
-    S = torch.zeros((rows_s, ss), dtype=torch.float16, device=w_blocks.device)
+    B = torch.empty((K, sb), dtype=torch.uint8 if q4 else torch.int8, device=w_blocks.device)
+    S = torch.empty((rows_s, ss), dtype=torch.float16, device=w_blocks.device)
+    # the kernel writes every column up to the width; the padding beyond it is zero
+    if sb > width:
+        B[:, width:].zero_()
+    if ss > N:
+        S[:, N:].zero_()
     _l.check(_l.load().cuthip_prepare_sep(f, w_blocks.data_ptr(), N, K, B.data_ptr(), sb, S.data_ptr(), ss, _stream_ptr()))
     return B, S
 

@@ -121,6 +121,33 @@ def test_prepared_q8_feeds_the_matmul(ops):
     assert normwise_rel_err(got, ref) < 1e-3
 
 
+@pytest.mark.parametrize("name", ["Q8_0", "Q4_0", "Q4_K"])
+@pytest.mark.parametrize("N,K", [(2, 256), (126, 512), (128, 256 * 9), (254, 256), (264, 768), (1026, 2304)])
+@pytest.mark.parametrize("shift", [0, 2, 6])
+def test_separated_at_tile_edges_and_odd_addresses(ops, name, N, K, shift):
+    """Row counts around one and several tiles, block runs at addresses that are only 2-byte aligned, rows of B whose length
+    is no multiple of four bytes, and more tiles than one per XCD; the bytes around the output rows stay as they were."""
+    fmt = oracle.FORMATS[name]
+    blocks = finite_random_blocks(fmt, N * K // oracle.BLOCK_ELEMS[fmt], seed=N + K + shift)
+    if name == "Q8_0":
+        v, sc = oracle.split_q8_0(blocks, N, K)
+        want, want_s = np.ascontiguousarray(v.T).view(np.uint8), sc.T
+    elif name == "Q4_0":
+        p, sc = oracle.split_q4_0(blocks, N, K)
+        want, want_s = oracle.transpose_q4_nibble(p, N, K), sc.T
+    else:
+        want, want_s = oracle.requantize_q4k_to_affine(blocks, N, K)
+    width = want.shape[1]
+    raw = torch.zeros(blocks.size + 16, dtype=torch.uint8, device="cuda")
+    raw[shift:shift + blocks.size] = dev(blocks).view(-1).view(torch.uint8)
+    for stride in (width, width + 1, width + 4):
+        B, S = ops.prepare_sep(raw[shift:shift + blocks.size], name, N, K, stride_b=stride, scale_stride=N + 1)
+        B, S = host(B).view(np.uint8), host(S.view(torch.int16)).view(np.uint16)
+        np.testing.assert_array_equal(B[:, :width], want)
+        np.testing.assert_array_equal(S[:, :N], want_s)
+        assert not B[:, width:].any() and not S[:, N:].any()
+
+
 @pytest.mark.parametrize("n", [32, 96, 4096, 32 * 1001])
 def test_quantize_rows_q8_0(ops, n):
     rng = np.random.default_rng(n)
