@@ -21,6 +21,11 @@ struct RowsLayout { uint32_t t, nw, per, ksplit; double cost; };
 // so that e.g. Q4_K 64 x 14336 x 4096 runs as 224 workgroups of nw = 2 (20.9 us; nw = 4 with two K ranges 22.0, with one 25.5),
 // 64 x 28672 x 4096 as 224 of nw = 4 (31.7; nw = 2 in two rounds 42.8), 64 x 4096 x 4096 as 64 x 4 of nw = 2 (13.1; 2 ranges
 // 13.9), 128 x 4096 x 14336 as 32 x 8 of nw = 4 (34.1; 4 ranges 37.1, 16 ranges 44.5).  fp32 activations: a tenth more.
+// Q8_0 on fp32 activations, four tiles, a K that the ranges do not cover exactly: the one instance that spills more than a
+// couple of registers, and its reloads wait for every load in flight: 646 x 3584 x 9600 took 230 us where the model without
+// this rule said 82.
+static bool rows_spills(int fmt, uint32_t t, bool af32) { return fmt == CUTHIP_Q8_0 && af32 && t == 4; }
+
 static double unit_us(int fmt, uint32_t t, uint32_t nw) {
   static const double q4[2][4] = {{0.82, 1.27, 0, 0}, {0.67, 0.94, 1.35, 1.67}};
   static const double q6_k[2][4] = {{1.47, 1.84, 0, 0}, {1.27, 1.54, 1.85, 2.03}};
@@ -30,26 +35,33 @@ static double unit_us(int fmt, uint32_t t, uint32_t nw) {
 }
 
 static RowsLayout rows_layout(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16, size_t scratch_bytes) {
-  const uint32_t tmax = rows_max_tiles(fmt, !a_f16), t32 = (M - 1) / 32 + 1, mt = (t32 - 1) / tmax + 1, t = (t32 - 1) / mt + 1;
-  const uint32_t units = (K - 1) / 128 + 1, mtiles = (t32 - 1) / t + 1;
+  const uint32_t tmax = rows_max_tiles(fmt, !a_f16), t32 = (M - 1) / 32 + 1, units = (K - 1) / 128 + 1;
   const uint32_t want = (uint32_t)g_tuning.gemm_ksplit;   // forced by a test or a sweep
   RowsLayout best{0, 0, 0, 0, 1e30};
-  for (uint32_t nw = t <= 2 ? 2 : 4; nw <= 4; nw += 2) {
-    const uint32_t kw = 8 / nw;
-    const uint64_t tiles = (uint64_t)((N - 1) / (32 * nw) + 1) * mtiles;
-    for (uint32_t ks = 1; ks <= 16; ++ks) {
-      if (ks > 1 && (uint64_t)ks * M * N * 4 > scratch_bytes) break;
-      if (want && ks != want && (uint64_t)want * M * N * 4 <= scratch_bytes) continue;
-      uint32_t per = (units - 1) / (ks * kw) + 1;
-      if (fmt == CUTHIP_Q4_K || fmt == CUTHIP_Q6_K) per = (per + 1) & ~1u;   // whole blocks of 256
-      const uint32_t ranges = (units - 1) / (per * kw) + 1;                  // no empty range
-      const double full = (double)((tiles * ranges - 1) / 256), last = (double)(tiles * ranges) - 256.0 * full;
-      const double f = 0.73 - 0.1 * (t - 1), unit = unit_us(fmt, t, nw) * (a_f16 ? 1.0 : 1.1);
-      double cost = 2.6 + 2.25 * (full + 1.0) + per * unit * (full * (1.0 + f) + 1.0 + f * last / 256.0);
-      if (ranges > 1) cost += 1.8 + 0.15 * ranges + 8.0 * ranges * M * N / 3.9e6;
-      if (cost < best.cost) best = RowsLayout{t, nw, per, ranges, cost};
+  auto consider = [&](uint32_t t) {
+    const uint32_t mtiles = (t32 - 1) / t + 1;
+    for (uint32_t nw = t <= 2 ? 2 : 4; nw <= 4; nw += 2) {
+      const uint32_t kw = 8 / nw;
+      const uint64_t tiles = (uint64_t)((N - 1) / (32 * nw) + 1) * mtiles;
+      for (uint32_t ks = 1; ks <= 16; ++ks) {
+        if (ks > 1 && (uint64_t)ks * M * N * 4 > scratch_bytes) break;
+        if (want && ks != want && (uint64_t)want * M * N * 4 <= scratch_bytes) continue;
+        uint32_t per = (units - 1) / (ks * kw) + 1;
+        if (fmt == CUTHIP_Q4_K || fmt == CUTHIP_Q6_K) per = (per + 1) & ~1u;   // whole blocks of 256
+        const uint32_t ranges = (units - 1) / (per * kw) + 1;                  // no empty range
+        const double full = (double)((tiles * ranges - 1) / 256), last = (double)(tiles * ranges) - 256.0 * full;
+        const double f = 0.73 - 0.1 * (t - 1);
+        double unit = unit_us(fmt, t, nw) * (a_f16 ? 1.0 : 1.1);
+        if (rows_spills(fmt, t, !a_f16) && (K % 128 != 0 || per * kw * ranges != units)) unit *= 2.4;
+        double cost = 2.6 + 2.25 * (full + 1.0) + per * unit * (full * (1.0 + f) + 1.0 + f * last / 256.0);
+        if (ranges > 1) cost += 1.8 + 0.15 * ranges + 8.0 * ranges * M * N / 3.9e6;
+        if (cost < best.cost) best = RowsLayout{t, nw, per, ranges, cost};
+      }
     }
-  }
+  };
+  auto even = [&](uint32_t most) { return (t32 - 1) / ((t32 - 1) / most + 1) + 1; };   // tiles per workgroup, evenly spread
+  consider(even(tmax));
+  if (rows_spills(fmt, best.t, !a_f16)) consider(even(best.t - 1));
   return best;
 }
 
