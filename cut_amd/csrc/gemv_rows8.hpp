@@ -922,7 +922,7 @@ __device__ __forceinline__ void rows8_body(const GemvParams &p, const uint32_t b
     writer = c.g == 0;
   }
   float carry_sq = 0.0f;
-  float am_v = -INFINITY;          // this lane's candidate for the arg-max of the wave's 8 rows (writer lanes only)
+  float am_v = -INFINITY;          // this lane's candidate for the arg-max of its 8 rows (writer lanes only)
   uint32_t am_i = 0xFFFFFFFFu;
   // SwiGLU over row pairs: weight rows 2i / 2i+1 are gate_i / up_i, C[m, i] = silu(gate) * up.  The partner row
   // sits four lanes up (same piece, same K half); in the folded path it is the next thread.
@@ -958,8 +958,11 @@ __device__ __forceinline__ void rows8_body(const GemvParams &p, const uint32_t b
               carry_sq = v * v;
             }
             if (MT == 1) {
-              am_v = p.c_f16 ? (float)(half_t)v : v;   // the value as C holds it
-              am_i = n0 + r8;
+              const float stored = p.c_f16 ? (float)(half_t)v : v;   // the value as C holds it; a NaN is no candidate
+              if (stored == stored) {
+                am_v = stored;
+                am_i = n0 + r8;
+              }
             }
           }
         }
@@ -1015,7 +1018,26 @@ __device__ __forceinline__ void rows8_body(const GemvParams &p, const uint32_t b
             p.next_x16[nn] = (half_t)(v * p.next_norm_w[nn]);
             carry_sq = v * v;
           }
+          if (MT == 1) {
+            const float stored = p.c_f16 ? (float)(half_t)v : v;   // as above
+            if (stored == stored) {
+              am_v = stored;
+              am_i = nn;
+            }
+          }
         }
+      }
+      if (MT == 1 && p.argmax_parts) {   // (uniform) largest of the row group's eight threads, the first one on a tie
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1) {
+          const float ov = __shfl_xor(am_v, o);
+          const uint32_t oi = __shfl_xor(am_i, o);
+          if (ov > am_v || (ov == am_v && oi < am_i)) {
+            am_v = ov;
+            am_i = oi;
+          }
+        }
+        if (rr == 0 && nn < p.N) p.argmax_parts[nn / 8] = ArgmaxPart{am_v, am_i};
       }
     }
   }

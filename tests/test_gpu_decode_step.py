@@ -26,6 +26,56 @@ def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
+@pytest.mark.parametrize("dt_in", [torch.float16, torch.float32])
+@pytest.mark.parametrize("dt_out", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n", [8, 2040, 2048, 2056, 5 * 2048 + 8, 13, 4099])
+def test_silu_mul_eight_at_a_time(ops, dt_in, dt_out, n):
+    """The 16-byte path against the element path (an output that is not 16-byte aligned) bit for bit, large and small gates
+    and infinities among them, and nothing written behind the output."""
+    gu = dev(gauss_acts((2 * n,), seed=n, dtype=np.float32) * 8).to(dt_in)
+    gu[:3] = torch.tensor([60000.0, -60000.0, float("inf")])
+    a = torch.full((n + 8,), 3.0, dtype=dt_out, device="cuda")
+    b = torch.full((n + 9,), 3.0, dtype=dt_out, device="cuda")
+    ops.silu_mul(gu, a[:n])
+    ops.silu_mul(gu, b[1:n + 1])
+    torch.cuda.synchronize()
+    assert torch.equal(a[:n].view(torch.uint8), b[1:n + 1].clone().view(torch.uint8))
+    assert bool((a[n:] == 3.0).all()) and bool((b[n + 1:] == 3.0).all()) and float(b[0]) == 3.0
+    want = torch.nn.functional.silu(gu[3:n].double()) * gu[n + 3:].double()
+    # fp32 arithmetic with the fast exponential (relative error below 2^-20), one rounding to the output type
+    torch.testing.assert_close(a[3:n].double(), want, rtol=2.0 ** -10 if dt_out == torch.float16 else 4e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("name", list(oracle.FORMATS))
+@pytest.mark.parametrize("N,K", [(1, 2048), (4097, 2048), (8200, 1024), (9000, 512), (32001, 256), (1000, 8192), (28700, 512)])
+def test_head_argmax_with_k_split_over_the_waves(ops, name, N, K):
+    """Per-group winners out of the folded epilogue: against the scan of the logits (no workspace), with row counts that
+    end inside a group, a maximum that stands twice (the first row wins) and rows whose logits are not numbers."""
+    fmt = oracle.FORMATS[name]
+    rb = oracle.n_bytes(fmt, K)
+    W = quantized_weights(fmt, N, K, seed=N % 97).reshape(N, rb).copy()
+    d_at = rb - 2 if name == "Q6_K" else 0   # the fp16 scale of a row's last (first) block
+    a = dev(gauss_acts((1, K), seed=73, dtype=np.float16)).view(-1)
+    out, idx = torch.empty(N, dtype=torch.float32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+
+    def run(ws, dtype):
+        logits = out.to(dtype)
+        ops.matmul_gguf_argmax(a, dev(W.reshape(-1)), fmt, N, K, logits, idx, workspace=ws)
+        torch.cuda.synchronize()
+        return logits.float().cpu().numpy(), int(idx.item())
+    best = int(np.argmax(run(None, torch.float32)[0]))
+    if N > 16:
+        W[(best + N // 2) % N] = W[best]                                     # a tie
+        nan_row = (best // 8) * 8 + (best + 1) % 8
+        if nan_row < N and nan_row != best:
+            W[nan_row, d_at:d_at + 2] = (0x00, 0x7E)                         # in the group of the maximum
+    for dtype in (torch.float32, torch.float16):
+        l0, i0 = run(None, dtype)
+        l1, i1 = run(ops.lm_head_workspace(N, "cuda"), dtype)
+        assert np.array_equal(l0, l1, equal_nan=True)
+        assert i0 == i1 == int(np.nanargmax(l0))
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("rows,dim", [(1, 4096), (3, 1000), (2, 64)])
 def test_rmsnorm(ops, dtype, rows, dim):
