@@ -292,6 +292,30 @@ def test_tiled_gemm_splits_k_through_the_workspace(ops, tuning, name, K, M):
     assert normwise_rel_err(got3, unsplit) < 1e-6
 
 
+@pytest.mark.parametrize("c_f16", [False, True])
+@pytest.mark.parametrize("split", [2, 3, 5, 8, 9])
+@pytest.mark.parametrize("N,pad", [(4, 0), (300, 0), (300, 12), (302, 0), (300, 2)])
+def test_reduce_of_a_k_split(ops, tuning, N, pad, split, c_f16):
+    """The reduce behind a K split: every instance (2, 4, 8 ranges at a time and more), rows with and without a gap, rows
+    that allow no vector accesses, each kind of operator; against the unsplit launch (the same products in another
+    order of fp32 additions, and one rounding to fp16 where C is fp16)."""
+    M, K = 17, 256 * 18
+    W = quantized_weights(oracle.Q4_0, N, K, seed=N + split)
+    w, a = torch.from_numpy(W).cuda(), torch.from_numpy(gauss_acts((M, K), seed=3, dtype=np.float16)).cuda()
+    dt = torch.float16 if c_f16 else torch.float32
+    ws = torch.empty(split * M * N * 4, dtype=torch.uint8, device="cuda")
+    d = torch.empty((M, N + pad), dtype=dt, device="cuda").normal_()[:, :N]
+    for more in ({}, {"binary": "add", "d": d}, {"unary": "silu"}):
+        got, want = (torch.full((M, N + pad), 7.0, dtype=dt, device="cuda") for _ in range(2))
+        tuning("gemm_ksplit", "1")
+        ops.matmul_gguf(a, w, oracle.Q4_0, N, K, out=want[:, :N], variant=2, **more)
+        tuning("gemm_ksplit", str(split))
+        ops.matmul_gguf(a, w, oracle.Q4_0, N, K, out=got[:, :N], variant=2, workspace=ws, **more)
+        err = normwise_rel_err(got[:, :N].float().cpu().numpy(), want[:, :N].float().cpu().numpy())
+        assert err < (1e-3 if c_f16 else 1e-6)
+        assert torch.all(got[:, N:] == 7.0)
+
+
 @pytest.mark.parametrize("mfma16", ["1", "0"])
 @pytest.mark.parametrize("tile", ["256,224", "128,448", "256,256", "128,256", "128,256,2", "256,256,4"])
 def test_dense_gemm_every_tile_shape_and_both_kernels(ops, tuning, tile, mfma16):
