@@ -90,6 +90,23 @@ def test_rmsnorm(ops, dtype, rows, dim):
     assert normwise_rel_err(got16.float().cpu().numpy(), want) < 4e-4   # one fp16 rounding of the output
 
 
+@pytest.mark.parametrize("xdtype", [np.float32, np.float16])
+@pytest.mark.parametrize("dim", [8, 504, 2040, 2048, 2056, 4096, 4104, 8184, 8192, 8200])
+def test_rmsnorm_row_lengths(ops, xdtype, dim):
+    """The edges of what a thread holds (one, two, four groups of eight elements, rows beyond them), in place as well."""
+    rng = np.random.default_rng(dim)
+    x = rng.standard_normal((5, dim)).astype(xdtype)
+    w = rng.uniform(0.5, 1.5, dim).astype(np.float32)
+    want = oracle.rmsnorm(x.astype(np.float32), w, 1e-5)
+    got = ops.rmsnorm(dev(x), dev(w), 1e-5, out_dtype=torch.float32).cpu().numpy()
+    np.testing.assert_allclose(got, want, rtol=2e-6, atol=1e-7)
+    shifted = torch.empty(dim + 1, dtype=torch.float32, device="cuda")[1:].copy_(dev(w))   # weights that allow no 16-byte loads
+    np.testing.assert_allclose(ops.rmsnorm(dev(x), shifted, 1e-5, out_dtype=torch.float32).cpu().numpy(), want, rtol=2e-6, atol=1e-7)
+    inplace = dev(x)
+    ops.rmsnorm(inplace, dev(w), 1e-5, out=inplace)
+    assert normwise_rel_err(inplace.float().cpu().numpy(), want) < (4e-4 if xdtype == np.float16 else 2e-6)
+
+
 def _tables(max_pos, head_dim, theta=500000.0):
     half = head_dim // 2
     inv = 1.0 / theta ** (np.arange(half, dtype=np.float64) * 2 / head_dim)
