@@ -554,18 +554,19 @@ __global__ void __launch_bounds__(256) attn_partial_wide_kernel(const void *q, c
   }
 }
 
-// One workgroup per query head.  GROUPS = 1 (128 threads, up to 32 splits): thread d holds dimension d of every split.
-// GROUPS = 8 (1024 threads): group g takes the splits g, g + 8, ..., so that each thread has an eighth of the records to
-// wait for, and the groups meet in LDS (one group walked 256 records in 13.3 us).  Bound: the latency of its loads.
+// One workgroup per query head, GROUPS groups of 128 threads: group g takes the splits g, g + GROUPS, ..., thread d of it
+// dimension d of each, and the groups meet in LDS.  Bound: the latency of its loads.  Up to 32 splits: four groups (one
+// group, with 32 loads per thread, made the step of an 8B shape at position 2047 1513 us instead of 1487).  More: eight
+// groups (one group walked 256 records in 13.3 us).
 constexpr int kAttnMaxSplit = 1024;   // splits per head the merge kernel holds weights for
 
 template <int GROUPS>
 __global__ void __launch_bounds__(128 * GROUPS) attn_merge_kernel(const float *partial, void *out, int out_f16, uint32_t headDim,
                                                                   uint32_t nsplit) {
-  constexpr uint32_t kPre = GROUPS == 1 ? 32 : 8;   // records a thread requests at the start
-  __shared__ float Ws[GROUPS == 1 ? 1 : kAttnMaxSplit];
-  __shared__ float red[GROUPS == 1 ? 1 : 2 * GROUPS], reds[GROUPS == 1 ? 1 : 2 * GROUPS];
-  __shared__ float os[GROUPS == 1 ? 1 : GROUPS][kAttnMaxHd];
+  constexpr uint32_t kPre = 8;   // records a thread requests at the start
+  __shared__ float Ws[GROUPS < 8 ? 1 : kAttnMaxSplit];
+  __shared__ float red[2 * GROUPS], reds[2 * GROUPS];
+  __shared__ float os[GROUPS][kAttnMaxHd];
   const uint32_t h = blockIdx.x, tid = threadIdx.x, d = tid & 127, g = tid >> 7, lane = tid & 63;
   // every split has a record (empty ones carry max = -inf, sum = 0), so the merge does not need the sequence length
   // and its loads do not wait for it
@@ -580,7 +581,7 @@ __global__ void __launch_bounds__(128 * GROUPS) attn_merge_kernel(const float *p
     ov[u] = (s < nsplit && d < headDim) ? base[(size_t)s * rec + 2 + d] : 0.0f;
   }
   float o = 0.0f, L;
-  if (GROUPS == 1 || nsplit <= 64) {
+  if (GROUPS < 8 || nsplit <= GROUPS * kPre) {   // fewer groups are launched for up to 32 splits only
     // every wave holds all (max, sum) pairs, one per lane, and folds them by itself: no workgroup barrier; the weight of
     // split s comes out of lane s (threads beyond the head dimension hold zeros)
     const bool have = lane < nsplit;
@@ -615,20 +616,18 @@ __global__ void __launch_bounds__(128 * GROUPS) attn_merge_kernel(const float *p
       for (uint32_t s = g + GROUPS * kPre; s < nsplit; s += GROUPS) o = fmaf(base[(size_t)s * rec + 2 + d], Ws[s], o);
     }
   }
-  if constexpr (GROUPS > 1) {
-    os[g][d] = o;
-    __syncthreads();
-    if (g > 0) return;
+  os[g][d] = o;
+  __syncthreads();
+  if (g > 0) return;
 #pragma unroll
-    for (int k = 1; k < GROUPS; ++k) o += os[k][d];
-  }
+  for (int k = 1; k < GROUPS; ++k) o += os[k][d];
   if (d < headDim) st_act(out, out_f16, (size_t)h * headDim + d, L > 0.0f ? o / L : 0.0f);
 }
 
 static int launch_attn_merge(const void *records, uint32_t nsplit, uint32_t n_heads, uint32_t head_dim, void *out, int out_f16,
                              hipStream_t s) {
   if (nsplit <= 32)
-    hipLaunchKernelGGL(attn_merge_kernel<1>, dim3(n_heads), dim3(128), 0, s, (const float *)records, out, out_f16, head_dim, nsplit);
+    hipLaunchKernelGGL(attn_merge_kernel<4>, dim3(n_heads), dim3(512), 0, s, (const float *)records, out, out_f16, head_dim, nsplit);
   else
     hipLaunchKernelGGL(attn_merge_kernel<8>, dim3(n_heads), dim3(1024), 0, s, (const float *)records, out, out_f16, head_dim, nsplit);
   return check_hip(hipGetLastError(), "attention merge launch");

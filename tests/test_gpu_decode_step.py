@@ -221,6 +221,24 @@ def test_attention_decode_several_chunks_per_workgroup(ops, n_heads, n_kv, hd, s
             assert normwise_rel_err(out.cpu().numpy(), want) < 2e-6 if n else bool((out == 0).all())
 
 
+@pytest.mark.parametrize("records", [1, 3, 4, 5, 8, 31, 32, 33, 64, 65])
+@pytest.mark.parametrize("hd", [128, 40])
+def test_attention_merge_of_few_and_many_records(ops, records, hd):
+    """Numbers of records around the groups of the merge and around the line between its two instances."""
+    n_heads, n_kv, max_ctx = 4, 2, 64 * records
+    rng = np.random.default_rng(records)
+    q = rng.standard_normal(n_heads * hd).astype(np.float32)
+    K = (rng.standard_normal((max_ctx, n_kv * hd)) * 0.5).astype(np.float16)
+    V = rng.standard_normal((max_ctx, n_kv * hd)).astype(np.float16)
+    ws = ops.attn_decode_workspace(n_heads, hd, max_ctx, "cuda")
+    out = torch.empty(n_heads * hd, dtype=torch.float32, device="cuda")
+    for seq in (max_ctx, max_ctx // 2 + 1):
+        want = oracle.attention_decode(q, K.view(np.uint16), V.view(np.uint16), seq, n_heads, n_kv, hd, 0.1)
+        ops.attn_decode(dev(q), dev(K), dev(V), dev(np.array([seq - 1, seq], np.int32)), n_heads, n_kv, hd, 0.1, ws, out)
+        torch.cuda.synchronize()
+        assert normwise_rel_err(out.cpu().numpy(), want) < 2e-6   # fp32 sums in any order, as above
+
+
 def test_silu_mul_and_argmax(ops):
     rng = np.random.default_rng(5)
     gu = (rng.standard_normal(2 * 14336) * 3).astype(np.float16)
