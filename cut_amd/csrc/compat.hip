@@ -10,13 +10,14 @@
 // The layout is column-major in n, so a wave streams whole k-rows: each lane
 // owns 16 consecutive columns (one 16-byte load of int8, or 8 bytes of
 // nibbles), a wave 1024 columns, and the k range is split over the four waves
-// of a workgroup and over workgroups (grid.y).  Per 32-row block a lane
+// of a workgroup and over workgroups.  Per 32-row block a lane
 // accumulates sum(x * q) per column and applies the block's scale once; the
 // "- 8" and the affine minimum become multiples of the block's sum(x).  The
 // waves of a workgroup are reduced through LDS; if the k range is split over
 // several workgroups the partial sums go to a caller-provided workspace and a
 // second kernel adds them and applies the epilogue.
 #include <cstdint>
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -35,8 +36,8 @@ struct SepParams {
   float *C;         // output, or the workspace [nsplit][M][N] when nsplit > 1
   Epilogue epi;
   uint32_t M, K, N, strideA, strideB, strideC, scaleStride;
-  uint32_t m0;      // first row of A handled by this launch
-  uint32_t nsplit;
+  uint32_t m0;                      // first row of A of this launch
+  uint32_t nsplit, tiles, passes;   // K ranges, column tiles, groups of MT rows of A
   int affine;
 };
 
@@ -50,8 +51,14 @@ __global__ void __launch_bounds__(64 * kSepWaves, 2) sep_gemv_kernel(SepParams p
   __shared__ float xs[XL * 64 * kSepWaves];
   __shared__ f32x4 red[kSepWaves - 1][MT][kSepCols / 4][64];   // lane-contiguous 16-byte slots: no bank conflicts
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t c0 = blockIdx.x * kSepTile + lane * kSepCols;
-  const uint32_t kwg = blockIdx.y * (kSepWaves * kSepKC);   // first k-row of this workgroup
+  // Ids id, id + 8, ... share an XCD: the passes over one piece of the weights run there one after the other, and all but
+  // the first find it in that XCD's L2.
+  const uint32_t slot = blockIdx.x >> 3, group = slot / p.passes, pass = slot - group * p.passes;
+  const uint32_t piece = __builtin_amdgcn_readfirstlane(group * 8 + (blockIdx.x & 7));
+  const uint32_t split = __builtin_amdgcn_readfirstlane(piece / p.tiles), m0 = p.m0 + __builtin_amdgcn_readfirstlane(pass * MT);
+  if (split >= p.nsplit) return;   // the last group of eight may be short
+  const uint32_t c0 = (piece - split * p.tiles) * kSepTile + lane * kSepCols;
+  const uint32_t kwg = split * (kSepWaves * kSepKC);        // first k-row of this workgroup
   const uint32_t k0 = kwg + wave * kSepKC;                  // this wave's block
   const uint32_t blocksK = p.K / 32;
   const uint32_t ncols = c0 < p.N ? min((uint32_t)kSepCols, p.N - c0) : 0u;
@@ -96,7 +103,7 @@ __global__ void __launch_bounds__(64 * kSepWaves, 2) sep_gemv_kernel(SepParams p
 #pragma unroll
   for (int u = 0; u < XL; ++u) {
     const int i = tid + u * 64 * kSepWaves, m = i / (kSepWaves * kSepKC), kk = i % (kSepWaves * kSepKC);
-    const uint32_t row = p.m0 + m, k = kwg + kk;
+    const uint32_t row = m0 + m, k = kwg + kk;
     const bool ok = m < MT && row < p.M && k < p.K;
     xv[u] = p.A[ok ? (size_t)row * p.strideA + k : (size_t)0];
     if (!ok) xv[u] = 0.0f;
@@ -211,10 +218,10 @@ __global__ void __launch_bounds__(64 * kSepWaves, 2) sep_gemv_kernel(SepParams p
         }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      const uint32_t row = p.m0 + m;
+      const uint32_t row = m0 + m;
       if (row >= p.M) continue;
       if (p.nsplit > 1) {   // workspace [split][M][N]
-        float *dst = p.C + ((size_t)blockIdx.y * p.M + row) * p.N + c0;
+        float *dst = p.C + ((size_t)split * p.M + row) * p.N + c0;
         if ((!RAGGED || ncols == kSepCols) && ((uintptr_t)dst & 15u) == 0) {
 #pragma unroll
           for (int c4 = 0; c4 < kSepCols / 4; ++c4)
@@ -244,46 +251,69 @@ __global__ void __launch_bounds__(256) sep_reduce_kernel(const float *ws, float 
   store_out(C, epi, 0, (size_t)row * strideC + n, v);
 }
 
-// The same for four consecutive columns per thread (N a multiple of 4, 16-byte aligned workspace): 16 partial sums
-// requested at a time instead of eight single floats, added in the same order.
-__global__ void __launch_bounds__(256) sep_reduce4_kernel(const float *ws, float *C, Epilogue epi, uint32_t M, uint32_t N,
-                                                          uint32_t strideC, uint32_t m0, uint32_t mcount, uint32_t nsplit) {
-  const uint32_t n4 = N / 4, i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= mcount * n4) return;
-  const uint32_t row = m0 + i / n4, n = (i % n4) * 4;
-  const float *src = ws + (size_t)row * N + n;
+// The same for four consecutive columns per lane (N a multiple of 4, 16-byte aligned workspace).  Bound: the latency of its
+// loads.  Eight waves share the columns: wave w adds the ranges w, w + 8, ..., up to 16 of them requested at a time (ranges
+// past the last repeat it and are dropped), and the eight sums meet in LDS.  One wave that walked all ranges of a column
+// waited seven times and more for the 112 ranges of K = 14336.
+constexpr int kRedWaves = 8;
+__global__ void __launch_bounds__(64 * kRedWaves) sep_reduce4_kernel(const float *ws, float *C, Epilogue epi, uint32_t M, uint32_t N,
+                                                                     uint32_t strideC, uint32_t m0, uint32_t nsplit, uint32_t tiles) {
+  __shared__ f32x4 sums[kRedWaves - 1][64];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t r = blockIdx.x / tiles, n = (blockIdx.x - r * tiles) * 256 + 4 * lane, row = m0 + r;
+  const float *src = ws + (size_t)row * N + min(n, N - 4);
   const size_t step = (size_t)M * N;
   f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-  uint32_t s = 0;
-  for (; s + 16 <= nsplit; s += 16) {
-    f32x4 t[16];
+  auto take = [&](uint32_t s, auto count) __attribute__((always_inline)) {
+    constexpr int U = decltype(count)::value;
+    f32x4 t[U];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) t[u] = *reinterpret_cast<const f32x4 *>(src + (s + u) * step);
+    for (int u = 0; u < U; ++u) t[u] = *reinterpret_cast<const f32x4 *>(src + min(s + kRedWaves * u, nsplit - 1) * step);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v += t[u];
-  }
-  for (; s < nsplit; ++s) v += *reinterpret_cast<const f32x4 *>(src + s * step);
+    for (int u = 0; u < U; ++u)
+      if (s + kRedWaves * u < nsplit) v += t[u];
+  };
+  if (nsplit <= 4 * kRedWaves) take(wave, std::integral_constant<int, 4>{});
+  else
+    for (uint32_t s = wave; s < nsplit; s += 16 * kRedWaves) take(s, std::integral_constant<int, 16>{});
+  if (wave > 0) sums[wave - 1][lane] = v;
+  __syncthreads();
+  if (wave > 0 || n >= N) return;
+#pragma unroll
+  for (int w = 0; w < kRedWaves - 1; ++w) v += sums[w][lane];
 #pragma unroll
   for (int c = 0; c < 4; ++c) store_out(C, epi, 0, (size_t)row * strideC + n + c, v[c]);
 }
 
-template <bool Q4, int MT> static int launch_sep(SepParams p, uint32_t mcount, float *C, void *workspace, hipStream_t stream) {
-  dim3 grid((p.N + kSepTile - 1) / kSepTile, p.nsplit);
-  float *out = p.nsplit == 1 ? C : reinterpret_cast<float *>(workspace);
-  p.C = out;
-  // whole lanes: every lane holds 16 columns and its scales are 16-byte aligned
-  if (p.N % kSepCols == 0 && (uintptr_t)p.S % 16 == 0 && p.scaleStride % 8 == 0)
-    hipLaunchKernelGGL((sep_gemv_kernel<Q4, MT, false>), grid, dim3(64 * kSepWaves), 0, stream, p);
-  else hipLaunchKernelGGL((sep_gemv_kernel<Q4, MT, true>), grid, dim3(64 * kSepWaves), 0, stream, p);
-  if (int rc = check_hip(hipGetLastError(), "separated-layout matmul launch")) return rc;
-  if (p.nsplit > 1) {
+// One launch for all rows of A (and one for the sum over the K ranges).  With a launch and a reduce for every four rows the
+// weights came from memory every time: a layer of seven matrices (hidden 4096, feed-forward 14336, int8) took 235 us at 8 rows
+// and 951 at 31, now 148 and 370; one row, from the shorter reduce, 94 -> 92 (host work bound).
+template <bool Q4, int MT> static int launch_sep(SepParams p, void *workspace, hipStream_t stream) {
+  float *C = p.C;
+  const float *ws = reinterpret_cast<const float *>(workspace);
+  if (p.nsplit > 1) p.C = reinterpret_cast<float *>(workspace);
+  p.tiles = (p.N - 1) / kSepTile + 1;
+  const uint64_t pieces = ((uint64_t)p.tiles * p.nsplit + 7) / 8 * 8, red_tiles = (p.N - 1) / 256 + 1;
+  // threads of a launch are counted in 32 bits: rows in as many launches as that takes
+  const uint64_t most = 0xFFFFFFFFull / (64 * kRedWaves * std::max<uint64_t>(pieces, red_tiles)) / MT * MT;
+  const uint32_t step = (uint32_t)std::max<uint64_t>(MT, std::min<uint64_t>(most, p.M));
+  for (p.m0 = 0; p.m0 < p.M; p.m0 += step) {
+    const uint32_t mc = std::min(step, p.M - p.m0);
+    p.passes = (mc - 1) / MT + 1;
+    const dim3 grid((uint32_t)pieces * p.passes);
+    // whole lanes: every lane holds 16 columns and its scales are 16-byte aligned
+    if (p.N % kSepCols == 0 && (uintptr_t)p.S % 16 == 0 && p.scaleStride % 8 == 0)
+      hipLaunchKernelGGL((sep_gemv_kernel<Q4, MT, false>), grid, dim3(64 * kSepWaves), 0, stream, p);
+    else hipLaunchKernelGGL((sep_gemv_kernel<Q4, MT, true>), grid, dim3(64 * kSepWaves), 0, stream, p);
+    if (int rc = check_hip(hipGetLastError(), "separated-layout matmul launch")) return rc;
+    if (p.nsplit == 1) continue;
     if (p.N % 4 == 0 && (uintptr_t)workspace % 16 == 0)
-      hipLaunchKernelGGL(sep_reduce4_kernel, dim3((mcount * (p.N / 4) + 255) / 256), dim3(256), 0, stream,
-                         reinterpret_cast<const float *>(workspace), C, p.epi, p.M, p.N, p.strideC, p.m0, mcount, p.nsplit);
+      hipLaunchKernelGGL(sep_reduce4_kernel, dim3((uint32_t)red_tiles * mc), dim3(64 * kRedWaves), 0, stream, ws, C, p.epi, p.M, p.N,
+                         p.strideC, p.m0, p.nsplit, (uint32_t)red_tiles);
     else
-      hipLaunchKernelGGL(sep_reduce_kernel, dim3((mcount * p.N + 255) / 256), dim3(256), 0, stream,
-                         reinterpret_cast<const float *>(workspace), C, p.epi, p.M, p.N, p.strideC, p.m0, mcount, p.nsplit);
-    return check_hip(hipGetLastError(), "separated-layout reduce launch");
+      hipLaunchKernelGGL(sep_reduce_kernel, dim3((mc * p.N + 255) / 256), dim3(256), 0, stream, ws, C, p.epi, p.M, p.N, p.strideC,
+                         p.m0, mc, p.nsplit);
+    if (int rc = check_hip(hipGetLastError(), "separated-layout reduce launch")) return rc;
   }
   return CUTHIP_OK;
 }
@@ -500,21 +530,11 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
     set_error("%s: workspace of %zu bytes, need %zu", who, workspace_bytes, (size_t)p.nsplit * M * N * sizeof(float));
     return CUTHIP_ERR_INVALID;
   }
-  // passes of up to 4 rows of A (each pass streams the weights once; 8 rows would spill registers)
-  for (uint32_t m0 = 0; m0 < M; m0 += 4) {
-    uint32_t mc = min(4u, M - m0);
-    p.m0 = m0;
-    int rc;
-    if (q4) {
-      rc = mc == 1 ? launch_sep<true, 1>(p, mc, C, workspace, stream) : mc == 2 ? launch_sep<true, 2>(p, mc, C, workspace, stream)
-                                                                                 : launch_sep<true, 4>(p, mc, C, workspace, stream);
-    } else {
-      rc = mc == 1 ? launch_sep<false, 1>(p, mc, C, workspace, stream) : mc == 2 ? launch_sep<false, 2>(p, mc, C, workspace, stream)
-                                                                                  : launch_sep<false, 4>(p, mc, C, workspace, stream);
-    }
-    if (rc) return rc;
-  }
-  return CUTHIP_OK;
+  // passes of up to 4 rows of A (8 rows would spill registers)
+  if (q4) return M == 1 ? launch_sep<true, 1>(p, workspace, stream) : M == 2 ? launch_sep<true, 2>(p, workspace, stream)
+                                                                             : launch_sep<true, 4>(p, workspace, stream);
+  return M == 1 ? launch_sep<false, 1>(p, workspace, stream) : M == 2 ? launch_sep<false, 2>(p, workspace, stream)
+                                                                      : launch_sep<false, 4>(p, workspace, stream);
 }
 
 }  // namespace cuthip

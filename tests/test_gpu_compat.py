@@ -74,6 +74,23 @@ def test_q4_against_oracle(ops, affine, M, K, N):
     assert normwise_rel_err(run(ops, A, Bp, S, N, q4=True, affine=affine), want) < 2e-5
 
 
+@pytest.mark.parametrize("M", [1, 7, 31])
+@pytest.mark.parametrize("K,N", [(128, 1040), (160, 16), (4096, 260), (4128, 2064), (14336, 272), (4128, 1030), (16416, 64)])
+def test_row_passes_and_reduce_edges(ops, M, K, N):
+    """Rows of A in one, two and eight passes (the last one short), column tiles and K ranges whose product is no multiple
+    of eight, 1, 2, 32, 33, 112 and 129 ranges in the reduce, rows that allow no vector accesses there, and the residual
+    add; fp32 sums in any order, as above."""
+    rng = np.random.default_rng(M * K + N)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    S = rng.uniform(0.001, 0.02, (K // 32, N)).astype(np.float16).astype(np.float32)
+    want = oracle.matmul_sep_q8(A, B, S, f64=True)
+    assert normwise_rel_err(run(ops, A, B, S, N), want) < 2e-6
+    D = dev(rng.standard_normal((M, N)).astype(np.float32))
+    got = ops.matmul_sep(dev(A), dev(B), dev(S.astype(np.float16)), N, out=torch.full((M, N), 7.0, device="cuda"), binary="add", d=D)
+    assert normwise_rel_err((got - D).cpu().numpy(), want) < 4e-6
+
+
 def test_affine_layout_from_q4k_requantizer(ops):
     """Q4_K blocks -> requantizeQ4KToAffine (oracle restatement of llama.cpp:573-619) -> separated affine matmul
     agrees with the matmul over the decoded affine weights."""
