@@ -8,6 +8,11 @@ extern template int launch_rows_fmt<CUTHIP_Q4_0>(const RowsParams &, int, int, u
 extern template int launch_rows_fmt<CUTHIP_Q4_K>(const RowsParams &, int, int, uint32_t, uint32_t, hipStream_t);
 extern template int launch_rows_fmt<CUTHIP_Q6_K>(const RowsParams &, int, int, uint32_t, uint32_t, hipStream_t);
 
+// Q8_0 on fp32 activations, four tiles, a K that the ranges do not cover exactly: the one instance that spills more than a
+// couple of registers, and its reloads wait for every load in flight: 646 x 3584 x 9600 took 230 us where the model without
+// this rule said 82.
+static bool rows_spills(int fmt, uint32_t t, bool af32) { return fmt == CUTHIP_Q8_0 && af32 && t == 4; }
+
 struct RowsLayout { uint32_t t, nw, per, ksplit; double cost; };
 
 // How the launch is cut: t 32-row tiles of A and 32 nw weight rows per workgroup, K in ksplit x (8 / nw) ranges of per
@@ -21,11 +26,6 @@ struct RowsLayout { uint32_t t, nw, per, ksplit; double cost; };
 // so that e.g. Q4_K 64 x 14336 x 4096 runs as 224 workgroups of nw = 2 (20.9 us; nw = 4 with two K ranges 22.0, with one 25.5),
 // 64 x 28672 x 4096 as 224 of nw = 4 (31.7; nw = 2 in two rounds 42.8), 64 x 4096 x 4096 as 64 x 4 of nw = 2 (13.1; 2 ranges
 // 13.9), 128 x 4096 x 14336 as 32 x 8 of nw = 4 (34.1; 4 ranges 37.1, 16 ranges 44.5).  fp32 activations: a tenth more.
-// Q8_0 on fp32 activations, four tiles, a K that the ranges do not cover exactly: the one instance that spills more than a
-// couple of registers, and its reloads wait for every load in flight: 646 x 3584 x 9600 took 230 us where the model without
-// this rule said 82.
-static bool rows_spills(int fmt, uint32_t t, bool af32) { return fmt == CUTHIP_Q8_0 && af32 && t == 4; }
-
 static double unit_us(int fmt, uint32_t t, uint32_t nw) {
   static const double q4[2][4] = {{0.82, 1.27, 0, 0}, {0.67, 0.94, 1.35, 1.67}};
   static const double q6_k[2][4] = {{1.47, 1.84, 0, 0}, {1.27, 1.54, 1.85, 2.03}};
