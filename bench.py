@@ -436,7 +436,7 @@ def main():
 
     def ffn_step_ws(b):
         # 9 rows and more: the three matmuls through cuthip_matmul_gguf_ws, whose workspace lets the streaming MFMA
-        # kernel and the tiled GEMM split K
+        # kernel and the row-tile matmul split K
         xb = torch.from_numpy(rng.standard_normal((b, N_EMBD), dtype=np.float32).astype(np.float16)).to(dev)
         hb = torch.from_numpy(rng.standard_normal((b, N_FF), dtype=np.float32).astype(np.float16)).to(dev)
         yb_ff = torch.empty((b, N_FF), dtype=torch.float16, device=dev)
