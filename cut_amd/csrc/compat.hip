@@ -7,7 +7,8 @@
 //   C[m,n] = sum_k A[m,k] * w[k,n]          (MatMulQ8Common.cuh / MatMulQ4Common.cuh:126-153)
 // A, C, D are fp32 as in the reference.
 //
-// The layout is column-major in n, so a wave streams whole k-rows: each lane
+// From three rows of A on the matrix cores take over where the columns allow it (sep_rows.hip).  The vector kernel here:
+// the layout is column-major in n, so a wave streams whole k-rows: each lane
 // owns 16 consecutive columns (one 16-byte load of int8, or 8 bytes of
 // nibbles), a wave 1024 columns, and the k range is split over the four waves
 // of a workgroup and over workgroups.  Per 32-row block a lane
@@ -21,6 +22,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "sep_rows.hpp"
 
 namespace cuthip {
 
@@ -293,9 +295,19 @@ __global__ void __launch_bounds__(64 * kRedWaves) sep_reduce4_kernel(const float
   for (int c = 0; c < 4; ++c) store_out(C, epi, 0, (size_t)row * strideC + n + c, v[c]);
 }
 
-// One launch for all rows of A (and one for the sum over the K ranges).  With a launch and a reduce for every four rows the
-// weights came from memory every time: a layer of seven matrices (hidden 4096, feed-forward 14336, int8) took 235 us at 8 rows
-// and 951 at 31, now 148 and 370; one row, from the shorter reduce, 94 -> 92 (host work bound).
+// Sums [nsplit][M][N] of K ranges into mc rows of C from m0 on, through the epilogue.
+static int launch_sep_reduce(const float *ws, float *C, const Epilogue &epi, uint32_t M, uint32_t N, uint32_t strideC, uint32_t m0,
+                             uint32_t mc, uint32_t nsplit, hipStream_t stream) {
+  const uint32_t tiles = (N - 1) / 256 + 1;
+  if (N % 4 == 0 && (uintptr_t)ws % 16 == 0)
+    hipLaunchKernelGGL(sep_reduce4_kernel, dim3(tiles * mc), dim3(64 * kRedWaves), 0, stream, ws, C, epi, M, N, strideC, m0, nsplit, tiles);
+  else
+    hipLaunchKernelGGL(sep_reduce_kernel, dim3((mc * N + 255) / 256), dim3(256), 0, stream, ws, C, epi, M, N, strideC, m0, mc, nsplit);
+  return check_hip(hipGetLastError(), "separated-layout reduce launch");
+}
+
+// One launch for all rows of A (and one for the sum over the K ranges): with a launch and a reduce for every four rows the
+// weights came from memory every time.
 template <bool Q4, int MT> static int launch_sep(SepParams p, void *workspace, hipStream_t stream) {
   float *C = p.C;
   const float *ws = reinterpret_cast<const float *>(workspace);
@@ -310,19 +322,14 @@ template <bool Q4, int MT> static int launch_sep(SepParams p, void *workspace, h
     const bool flat = p.M > MT || p.nsplit > 65535u;
     p.passes = flat ? (mc - 1) / MT + 1 : 0;
     const dim3 grid = flat ? dim3((uint32_t)pieces * p.passes) : dim3(p.tiles, p.nsplit);
-    // whole lanes: every lane holds 16 columns and its scales are 16-byte aligned
-    if (p.N % kSepCols == 0 && (uintptr_t)p.S % 16 == 0 && p.scaleStride % 8 == 0)
-      hipLaunchKernelGGL((sep_gemv_kernel<Q4, MT, false>), grid, dim3(64 * kSepWaves), 0, stream, p);
+    // whole lanes: every lane holds 16 columns and its scales are 16-byte aligned (more than two such rows are sep_rows.hip's)
+    bool whole = false;
+    if constexpr (MT <= 2) whole = p.N % kSepCols == 0 && (uintptr_t)p.S % 16 == 0 && p.scaleStride % 8 == 0;
+    if (whole) hipLaunchKernelGGL((sep_gemv_kernel<Q4, MT, MT <= 2 ? false : true>), grid, dim3(64 * kSepWaves), 0, stream, p);
     else hipLaunchKernelGGL((sep_gemv_kernel<Q4, MT, true>), grid, dim3(64 * kSepWaves), 0, stream, p);
     if (int rc = check_hip(hipGetLastError(), "separated-layout matmul launch")) return rc;
     if (p.nsplit == 1) continue;
-    if (p.N % 4 == 0 && (uintptr_t)workspace % 16 == 0)
-      hipLaunchKernelGGL(sep_reduce4_kernel, dim3((uint32_t)red_tiles * mc), dim3(64 * kRedWaves), 0, stream, ws, C, p.epi, p.M, p.N,
-                         p.strideC, p.m0, p.nsplit, (uint32_t)red_tiles);
-    else
-      hipLaunchKernelGGL(sep_reduce_kernel, dim3((mc * p.N + 255) / 256), dim3(256), 0, stream, ws, C, p.epi, p.M, p.N, p.strideC,
-                         p.m0, mc, p.nsplit);
-    if (int rc = check_hip(hipGetLastError(), "separated-layout reduce launch")) return rc;
+    if (int rc = launch_sep_reduce(ws, C, p.epi, p.M, p.N, p.strideC, p.m0, mc, p.nsplit, stream)) return rc;
   }
   return CUTHIP_OK;
 }
@@ -540,6 +547,16 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
   if (p.nsplit > 1 && (!workspace || workspace_bytes < (size_t)p.nsplit * M * N * sizeof(float))) {
     set_error("%s: workspace of %zu bytes, need %zu", who, workspace_bytes, (size_t)p.nsplit * M * N * sizeof(float));
     return CUTHIP_ERR_INVALID;
+  }
+  // One or two rows stay on the vector ALU: 14336 x 4096, us, both launches, vector kernel / matrix cores: int8 one row 16.9 / 19.2,
+  // two 19.2 / 19.4, three 22.3 / 19.7; nibbles 13.3 / 16.6, 15.6 / 17.0, 19.3 / 17.2.
+  if (M > 2) {
+    SepRowsParams r{A, p.B, p.S, C, reinterpret_cast<float *>(workspace), p.epi, M, K, N, strideA, strideB, strideC, scaleStride};
+    sep_rows_cut(r);
+    if (sep_rows_fits(r) && (r.nsplit == 1 || (uintptr_t)workspace % 16 == 0)) {
+      if (int rc = launch_sep_rows(r, q4, affine != 0, stream)) return rc;
+      return r.nsplit == 1 ? CUTHIP_OK : launch_sep_reduce(r.partial, C, p.epi, M, N, strideC, 0, M, r.nsplit, stream);
+    }
   }
   // passes of up to 4 rows of A (8 rows would spill registers)
   if (q4) return M == 1 ? launch_sep<true, 1>(p, workspace, stream) : M == 2 ? launch_sep<true, 2>(p, workspace, stream)

@@ -91,6 +91,53 @@ def test_row_passes_and_reduce_edges(ops, M, K, N):
     assert normwise_rel_err((got - D).cpu().numpy(), want) < 4e-6
 
 
+@pytest.mark.parametrize("kind", ["q8", "q4", "affine"])
+@pytest.mark.parametrize("M,K,N", [(3, 32, 8), (16, 160, 264), (17, 4128, 520), (31, 4096, 256), (33, 96, 136), (70, 2080, 248), (4, 2048, 20)])
+def test_rows_on_the_matrix_cores(ops, kind, M, K, N):
+    """Streaming variants from three rows on: lanes and sides of a column tile without columns, waves and ranges without
+    blocks, short last row tiles and passes, one launch through the operators and several ranges; columns that are no
+    multiple of eight stay on the vector kernel.  Exact products and fp32 sums: the bounds of the vector kernel."""
+    rng = np.random.default_rng(M * K + N)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = rng.integers(-127, 128, (K, N)).astype(np.int8) if kind == "q8" else rng.integers(0, 256, (K, N // 2)).astype(np.uint8)
+    S = rng.uniform(0.001, 0.02, ((2 if kind == "affine" else 1) * (K // 32), N)).astype(np.float16).astype(np.float32)
+    if kind == "affine":
+        S[K // 32:] = rng.uniform(-0.1, 0.1, (K // 32, N)).astype(np.float16).astype(np.float32)
+    how = dict(q4=kind != "q8", affine=kind == "affine", variant=1)
+    if kind == "q8":
+        w = B * S.astype(np.float64).repeat(32, 0)
+    else:
+        q = np.stack((B & 15, B >> 4), -1).reshape(K, N).astype(np.float64) - 8
+        w = q * S[:K // 32].astype(np.float64).repeat(32, 0)
+        if kind == "affine":
+            w += S[K // 32:].astype(np.float64).repeat(32, 0)
+    want = A.astype(np.float64) @ w
+    assert normwise_rel_err(run(ops, A, B, S, N, **how), want) < 2e-6
+    D = rng.standard_normal((M, N)).astype(np.float32)
+    got = ops.matmul_sep(dev(A), dev(B), dev(S.astype(np.float16)), N, binary="add", d=dev(D), **how).cpu().numpy()
+    assert normwise_rel_err(got - D, want) < 4e-6
+
+
+def test_rows_on_the_matrix_cores_extreme_activations(ops):
+    """Magnitudes from the smallest normal numbers to the largest, and an infinity: it reaches its own row alone, as infinity
+    where the weight is not zero."""
+    M, K, N = 5, 64, 32
+    rng = np.random.default_rng(5)
+    A = (rng.standard_normal((M, K)) * np.array([1e-30, 1e-8, 1.0, 1e8, 1e30])[:, None]).astype(np.float32)
+    B = rng.integers(1, 128, (K, N)).astype(np.int8)
+    B[9, 4:7] = (0, -3, 5)
+    S = np.full((K // 32, N), 0.0078125, np.float32)
+    want = A.astype(np.float64) @ (B * S.astype(np.float64).repeat(32, 0))
+    got = run(ops, A, B, S, N)
+    for m in range(M):
+        assert normwise_rel_err(got[m], want[m]) < 2e-6
+    A[2, 9] = np.inf
+    inf = run(ops, A, B, S, N)
+    np.testing.assert_array_equal(np.delete(inf, 2, 0), np.delete(got, 2, 0))
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_array_equal(inf[2], np.where(B[9] == 0, np.nan, np.inf * B[9].astype(np.float32)))
+
+
 def test_affine_layout_from_q4k_requantizer(ops):
     """Q4_K blocks -> requantizeQ4KToAffine (oracle restatement of llama.cpp:573-619) -> separated affine matmul
     agrees with the matmul over the decoded affine weights."""
