@@ -335,12 +335,11 @@ template <bool Q4, int MT> static int launch_sep(SepParams p, void *workspace, h
 }
 
 // ---- prefill on the separated layout: dequantize to fp16 [N][K], then the dense GEMM ------------------------------
-// The GEMV above takes 4 rows of A a pass and multiplies in fp32; from kSepDenseRows rows on the tensors are turned into the
-// fp16 [N][K] operand of the dense GEMM first (one launch: value = float(q) * scale (+ min), rounded to nearest even,
-// 64 x 64 tiles transposed through LDS so that both the reads along n and the writes along k are contiguous) and the
-// product goes through the same hand-written GEMM as cuthip_matmul_dense_f16.  The line is one of precision as well, so it
-// stays where large matrices cross it (us, GEMV at 31 rows / dense at 32: int8 14336 x 4096 92 / 81, 4096 x 4096 35 / 31,
-// 512 x 512 13 / 13; narrow ones would cross it later: 1024 x 4096 16 / 23).
+// From kSepDenseRows rows on the operands are fp16, rounded once: decoded as they are needed (sep_rows.hip), or, where that is
+// estimated to be slower, turned into the fp16 [N][K] operand of the dense GEMM first (one launch: value = float(q) * scale
+// (+ min), rounded to nearest even, 64 x 64 tiles transposed through LDS so that both the reads along n and the writes along k
+// are contiguous), then the hand-written GEMM of cuthip_matmul_dense_f16.  The line at 32 rows is one of precision, not of
+// time (14336 x 4096, int8: exact products of 31 rows 30 us, rounded ones of 32 rows 25).
 constexpr uint32_t kSepDenseRows = 32;
 
 bool dense_gemm_fits(uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A);
@@ -348,6 +347,11 @@ size_t dense_f16_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16);
 int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K,
                       uint32_t N, uint32_t strideA, uint32_t strideC, Epilogue epi, void *workspace, hipStream_t stream,
                       int use_blaslt);
+
+int launch_cvt_rows(const float *A, half_t *A16, uint32_t M, uint32_t K, uint32_t strideA, hipStream_t stream);
+int launch_splitk_reduce(const float *partial, uint32_t ksplit, uint32_t M, uint32_t N, void *C, uint32_t strideC, Epilogue epi,
+                         int c_f16, hipStream_t stream);
+double sep_two_pass_us(uint32_t M, uint32_t K, uint32_t N);
 
 static size_t sep_w16_bytes(uint32_t K, uint32_t N) { return ((size_t)N * K * 2 + 255) & ~(size_t)255; }
 static bool sep_dense_fits(uint32_t K, uint32_t N, uint32_t M) {
@@ -457,7 +461,7 @@ __global__ void __launch_bounds__(256) sep_dequant_kernel(const uint8_t *B, cons
 // names at the reference's indices (MatMulQ8Variants.generated.h:20-32, MatMulQ4Variants.generated.h:20-29); its
 // eight / five shaders collapse onto the two kernels here:
 //   tiled shaders (Q8 0, 2, 6; Q4 0) and -1            -> the choice by shape the reference's own default makes
-//   GEMV shaders (Q8 1, 3, 4, 5; Q4 1, 2, 3)            -> the streaming kernel, whatever M is
+//   GEMV shaders (Q8 1, 3, 4, 5; Q4 1, 2, 3)            -> the streaming kernels, whatever M is
 //   cooperative-matrix shaders (Q8 7; Q4 4)            -> dequantize to fp16, then the dense MFMA GEMM
 // The reference's int8-activation shaders (Q8 5 GemvDot, 6 TiledDot) run here with fp32 / fp16 activations, i.e.
 // closer to the fp32 loop than the reference's own result for those indices.
@@ -521,6 +525,18 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
     return CUTHIP_ERR_INVALID;
   }
   if (dense_ok && (route == kSepDense || (route == kSepAuto && M >= kSepDenseRows))) {
+    const Epilogue epi{epilogue, epilogue_op, epilogue == CUTHIP_EPI_BINARY ? D : nullptr};
+    if (route == kSepAuto) {   // decoding the weights as they are needed, where that is estimated to be the cheaper way
+      const size_t a16 = sep_w16_bytes(K, M);   // fp16 [M][K]
+      SepRowsParams r{A, reinterpret_cast<const uint8_t *>(B), reinterpret_cast<const uint16_t *>(S), C,
+                      reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(workspace) + a16), epi, M, K, N, strideA, strideB, strideC,
+                      scaleStride, reinterpret_cast<const half_t *>(workspace)};
+      if (sep_rows16_cut(r, q4, affine != 0, workspace_bytes - a16) && r.cost_us < sep_two_pass_us(M, K, N)) {
+        if (int rc = launch_cvt_rows(A, reinterpret_cast<half_t *>(workspace), M, K, strideA, stream)) return rc;
+        if (int rc = launch_sep_rows16(r, q4, affine != 0, stream)) return rc;
+        return r.nsplit == 1 ? CUTHIP_OK : launch_splitk_reduce(r.partial, r.nsplit, M, N, C, strideC, epi, 0, stream);
+      }
+    }
     half_t *w16 = reinterpret_cast<half_t *>(workspace);
     dim3 grid((N + 63) / 64, (K + 63) / 64);
     if (q4)
@@ -530,7 +546,6 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
       hipLaunchKernelGGL(sep_dequant_kernel<false>, grid, dim3(256), 0, stream, reinterpret_cast<const uint8_t *>(B),
                          reinterpret_cast<const uint16_t *>(S), w16, K, N, strideB, scaleStride, 0);
     if (int rc = check_hip(hipGetLastError(), "separated-layout dequant launch")) return rc;
-    Epilogue epi{epilogue, epilogue_op, epilogue == CUTHIP_EPI_BINARY ? D : nullptr};
     return launch_dense_gemm(-1, w16, A, 0, C, 0, M, K, N, strideA, strideC, epi,
                              reinterpret_cast<uint8_t *>(workspace) + sep_w16_bytes(K, N), stream,
                              0);
@@ -552,8 +567,7 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
   // two 19.2 / 19.4, three 22.3 / 19.7; nibbles 13.3 / 16.6, 15.6 / 17.0, 19.3 / 17.2.
   if (M > 2) {
     SepRowsParams r{A, p.B, p.S, C, reinterpret_cast<float *>(workspace), p.epi, M, K, N, strideA, strideB, strideC, scaleStride};
-    sep_rows_cut(r);
-    if (sep_rows_fits(r) && (r.nsplit == 1 || (uintptr_t)workspace % 16 == 0)) {
+    if (sep_rows_cut(r, (uintptr_t)workspace % 16 == 0 ? workspace_bytes : 0)) {
       if (int rc = launch_sep_rows(r, q4, affine != 0, stream)) return rc;
       return r.nsplit == 1 ? CUTHIP_OK : launch_sep_reduce(r.partial, C, p.epi, M, N, strideC, 0, M, r.nsplit, stream);
     }

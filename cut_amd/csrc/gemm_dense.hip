@@ -517,6 +517,12 @@ __global__ void __launch_bounds__(256) cvt_rows_kernel(const float *src, half_t 
   *reinterpret_cast<half8v *>(dst + (size_t)row * K + c * 8) = o;
 }
 
+int launch_cvt_rows(const float *A, half_t *A16, uint32_t M, uint32_t K, uint32_t strideA, hipStream_t stream) {
+  const uint32_t chunks = (K / 8 + 255) / 256;
+  hipLaunchKernelGGL(cvt_rows_kernel, dim3(M * chunks), dim3(256), 0, stream, A, A16, K, strideA, chunks);
+  return check_hip(hipGetLastError(), "activation convert launch");
+}
+
 // C = epilogue(sum over the K ranges of the fp32 partial products), one output per thread
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *partial, uint32_t ksplit, uint32_t M, uint32_t N,
                                                             void *C, uint32_t strideC, Epilogue epi, int c_f16) {
@@ -706,22 +712,29 @@ size_t dense_f16_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16) {
 // matrices (14336 x 4096, us, row tiles / two passes: Q8_0 384 rows 83 / 103, 448 rows 94 / 83; Q4_K 512 rows 78 / 85, 768 rows
 // 116 / 107) and higher on narrow ones (4096 x 4096 Q4_K: 1024 rows 45 / 56, 2048 rows 85 / 72; 1024 x 4096: never).  The last
 // factor puts it there: on panels that are a multiple of eight the other terms come out a few per cent high at 450 to 800 rows.
-double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16) {
+static double two_pass_us(double decode_us, uint32_t M, uint32_t K, uint32_t N, int a_f16) {
   static const struct { double mac, f; } kTile[5] = {{1.42e-7, 1.38}, {1.06e-7, 2.0}, {1.12e-7, 2.0}, {1.76e-7, 1.14}, {2.48e-7, 0.43}};
-  const double nk = (double)N * K, bpw = (double)fmt_bytes(fmt) / fmt_elems(fmt);
   const DenseShape sh = pick_dense_shape(M, K, N);
   const int shape = sh.bn == 224 ? 0 : sh.bn == 448 ? 1 : sh.bm == 256 ? 2 : sh.ksplit == 1 ? 3 : 4;
   const uint32_t mtiles = (M - 1) / sh.bm + 1, ntiles = (N - 1) / sh.bn + 1;
   const bool spread = mtiles > 1 && ntiles % 8 != 0;
   const uint64_t tiles = (uint64_t)mtiles * ntiles * sh.ksplit;
   const double full = (double)((tiles - 1) / 256), last = (double)tiles - 256.0 * full, f = kTile[shape].f;
-  double us = 5.0 + nk * (bpw + 2.0) / 5.14e6 + 5.54 * (full + 1.0) + 0.168e-6 * M * N * (a_f16 ? 2 : 4) +
+  double us = decode_us + 5.54 * (full + 1.0) + 0.168e-6 * M * N * (a_f16 ? 2 : 4) +
               (double)K / sh.ksplit * sh.bm * sh.bn * kTile[shape].mac * (full * (1.0 + f) + 1.0 + f * last / 256.0) *
                   (!spread ? 1.0 : shape < 3 ? 1.22 : 1.39);
   if (sh.ksplit > 1) us += 1.2 + 8.0 * sh.ksplit * M * N / 7.12e6;
   if (!a_f16) us += 2.3 + 6.0 * M * K / 7.54e6;
   return us * (spread ? 1.0 : 0.96);
 }
+
+double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16) {
+  return two_pass_us(5.0 + (double)N * K * ((double)fmt_bytes(fmt) / fmt_elems(fmt) + 2.0) / 5.14e6, M, K, N, a_f16);
+}
+
+// The same from the separated layout and fp32 activations: the transposing dequantization runs at 1.33 weights per ps
+// (14336 x 4096 45 us); 270 launches of 32 .. 512 rows on nine weight shapes come out 10 per cent above the fit.
+double sep_two_pass_us(uint32_t M, uint32_t K, uint32_t N) { return 1.1 * two_pass_us(4.0 + (double)N * K / 1.33e6, M, K, N, 0); }
 
 // What a call of 9 to 40 rows has to save before it gives up weights that are not rounded (8-row passes, 1e-5 of the
 // result's norm) for fp16 ones (3e-4): passes stay while this is not below 0.9 of their cost.  A line of precision, not an
@@ -752,10 +765,7 @@ int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C,
   p.strideA = strideA;
   if (!a_f16) {
     half_t *a16 = reinterpret_cast<half_t *>(after_w);
-    uint32_t chunks = (K / 8 + 255) / 256;
-    hipLaunchKernelGGL(cvt_rows_kernel, dim3(M * chunks), dim3(256), 0, stream, reinterpret_cast<const float *>(A), a16, K,
-                       strideA, chunks);
-    if (int rc = check_hip(hipGetLastError(), "activation convert launch")) return rc;
+    if (int rc = launch_cvt_rows(reinterpret_cast<const float *>(A), a16, M, K, strideA, stream)) return rc;
     p.A = reinterpret_cast<const uint8_t *>(a16);
     p.strideA = K;
   }

@@ -12,12 +12,17 @@ struct SepRowsParams {
   float *partial;   // [nsplit][M][N], 16-byte aligned, when nsplit > 1
   Epilogue epi;
   uint32_t M, K, N, strideA, strideB, strideC, scaleStride;
-  uint32_t nsplit, per;     // K ranges over workgroups, blocks per wave    } set by sep_rows_cut
-  uint32_t tiles, passes;   // column tiles, groups of 16 or 32 rows of A   }
+  const half_t *A16;   // sep_rows16: [M][K], 16-byte aligned
+  uint32_t t;                           // 16-row tiles of A per pass            } set by the two that cut
+  uint32_t nsplit, per, tiles, passes;  // K ranges over workgroups, blocks per wave, column tiles, passes over the rows }
+  double cost_us;                       // sep_rows16: estimate                  }
 };
 
-void sep_rows_cut(SepRowsParams &p);          // nsplit is never more than K / 128 rounded up
-bool sep_rows_fits(const SepRowsParams &p);   // after sep_rows_cut
+// How the launch is cut; false if it does not fit.  partial_bytes: room for the sums of several K ranges (nsplit is never
+// more than K / 128 rounded up).
+bool sep_rows_cut(SepRowsParams &p, size_t partial_bytes);
+bool sep_rows16_cut(SepRowsParams &p, bool q4, bool affine, size_t partial_bytes);
 int launch_sep_rows(const SepRowsParams &p, bool q4, bool affine, hipStream_t stream);
+int launch_sep_rows16(const SepRowsParams &p, bool q4, bool affine, hipStream_t stream);
 
 }  // namespace cuthip

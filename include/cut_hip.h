@@ -382,19 +382,20 @@ int cuthip_matmul_gguf_pro(int fmt, const void *W, const void *A, int a_dtype, v
  * epilogue / epilogue_op / D as in cuthip_matmul_gguf (MatMulFusion).
  * workspace: device scratch of cuthip_matmul_sep_workspace_bytes(M, K, N)
  * bytes, 256-byte aligned (may be NULL when that is 0).  Below 32 rows of A
- * (or when K is not a multiple of 128) the weights are streamed once per 4 rows
- * and the workspace holds split-K partial sums; from 32 rows on the tensors are
- * first dequantized to fp16 [N][K] in the workspace (one launch) and multiplied
- * by the dense GEMM of cuthip_matmul_dense_f16 (fp16 operands, fp32 accumulate:
- * within 1e-3 of the fp32 loop, normwise).  That path rounds the fp32 activations
+ * (or when K is not a multiple of 128) the weights are streamed once per 32 rows
+ * (N not a multiple of 8: per 4 rows) and the workspace holds split-K partial sums;
+ * from 32 rows on the products are those of fp16 operands, fp32 accumulate (within
+ * 1e-3 of the fp32 loop, normwise): with weights decoded as they are needed, or, where
+ * that is estimated to be slower, first dequantized to fp16 [N][K] in the workspace
+ * (one launch) and multiplied by the dense GEMM of cuthip_matmul_dense_f16.  Both round the fp32 activations
  * and the products q * scale to fp16 once each, where the reference's kernels
  * keep fmaf(a, q * scale, acc) in fp32: activations beyond the fp16 range
  * (|a| > 65504) become infinite there; the GEMV variants (Q8 1, Q4 1) take any fp32.
  * variant: the MatMulOpNode `spec` argument, an index into the CUTHIP_OP_MATMUL_Q8 / CUTHIP_OP_MATMUL_Q4 tables,
  * which hold the reference's variant names at the reference's indices (MatMulQ8Variants.generated.h:20-32, default 2;
  * MatMulQ4Variants.generated.h:20-29, default 0; "indices are ABI", MatMulOp.cpp:353-356), or -1 = choose by shape.
- * The reference's shaders collapse onto two kernels here: its tiled shaders (Q8 0, 2, 6; Q4 0) choose by shape as -1
- * does; its GEMV shaders (Q8 1, 3, 4, 5; Q4 1, 2, 3) stream the weights once per 4 rows whatever M is; its
+ * The reference's shaders collapse onto these routes here: its tiled shaders (Q8 0, 2, 6; Q4 0) choose by shape as -1
+ * does; its GEMV shaders (Q8 1, 3, 4, 5; Q4 1, 2, 3) stream the weights in fp32 whatever M is; its
  * cooperative-matrix shaders (Q8 7; Q4 4) dequantize to fp16 and run the dense MFMA GEMM whatever M is (an error if
  * K is not a multiple of 128 or the workspace is too small).  The int8-activation shaders of the reference (Q8 5, 6)
  * run with unquantized activations here.  Any other index: CUTHIP_ERR_UNKNOWN_VARIANT.

@@ -118,6 +118,41 @@ def test_rows_on_the_matrix_cores(ops, kind, M, K, N):
     assert normwise_rel_err(got - D, want) < 4e-6
 
 
+@pytest.mark.parametrize("ks", ["", "1", "3"])
+@pytest.mark.parametrize("kind", ["q8", "q4", "affine"])
+@pytest.mark.parametrize("M,K,N", [(32, 128, 8), (33, 384, 264), (64, 640, 136), (65, 1152, 520), (130, 256, 1032)])
+def test_rows_on_rounded_operands(ops, kind, ks, M, K, N):
+    """The default from 32 rows: two, three and four row tiles in one pass and several, sides and lanes without columns, waves
+    without blocks, one range and several.  Against the float64 product of the operands rounded to fp16 once each: fp32 sums."""
+    from cut_amd import lib
+    rng = np.random.default_rng(M * K + N)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    S = rng.uniform(0.001, 0.02, ((2 if kind == "affine" else 1) * (K // 32), N)).astype(np.float16).astype(np.float64)
+    if kind == "affine":
+        S[K // 32:] = rng.uniform(-0.1, 0.1, (K // 32, N)).astype(np.float16)
+    scale = S[:K // 32].repeat(32, 0)
+    if kind == "q8":
+        B = rng.integers(-128, 128, (K, N)).astype(np.int8)
+        w = B * scale
+    else:
+        B = rng.integers(0, 256, (K, N // 2)).astype(np.uint8)
+        w = (np.stack((B & 15, B >> 4), -1).reshape(K, N).astype(np.float64) - 8) * scale
+        if kind == "affine":
+            w += S[K // 32:].repeat(32, 0)
+    want = A.astype(np.float16).astype(np.float64) @ w.astype(np.float16).astype(np.float64)
+    D = rng.standard_normal((M, N)).astype(np.float32)
+    how = dict(q4=kind != "q8", affine=kind == "affine")
+    dll = lib.load()
+    lib.check(dll.cuthip_set_tuning(b"gemm_ksplit", ks.encode()))
+    try:
+        got = run(ops, A, B, S, N, **how)
+        added = ops.matmul_sep(dev(A), dev(B), dev(S.astype(np.float16)), N, binary="add", d=dev(D), **how).cpu().numpy()
+    finally:
+        lib.check(dll.cuthip_set_tuning(b"gemm_ksplit", b""))
+    assert normwise_rel_err(got, want) < 2e-6
+    assert normwise_rel_err(added - D, want) < 4e-6
+
+
 def test_rows_on_the_matrix_cores_extreme_activations(ops):
     """Magnitudes from the smallest normal numbers to the largest, and an infinity: it reaches its own row alone, as infinity
     where the weight is not zero."""
