@@ -190,7 +190,7 @@ static int set_tuning_key(const char *key, const char *value) {
   } else if (!strcmp(key, "dense_tile")) {
     if (clear) { g_tuning.dense_bm = g_tuning.dense_bn = 0; g_tuning.dense_ks = 1; return CUTHIP_OK; }
     const int got = sscanf(value, "%d,%d,%d", &a, &b, &c);
-    if (got >= 2 && ((b == 256 && (a == 256 || a == 128)) || (b == 448 && a == 128) || (b == 224 && a == 256)) &&
+    if (got >= 2 && ((b == 256 && (a == 256 || a == 128)) || (b == 448 && a == 128) || (a == 256 && (b == 128 || b == 160 || b == 192 || b == 224))) &&
         (c == 1 || c == 2 || c == 4 || c == 8)) {
       g_tuning.dense_bm = a; g_tuning.dense_bn = b; g_tuning.dense_ks = c; return CUTHIP_OK;
     }

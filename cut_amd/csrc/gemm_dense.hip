@@ -34,6 +34,7 @@
 // to fp16 once, fp32 accumulation: the same error budget as the row-tile matmul.
 #include <stdio.h>
 #include <stdlib.h>
+#include <algorithm>
 
 #include "common.hpp"
 #include "gemm_store.hpp"
@@ -58,10 +59,23 @@ struct DenseParams {
   // and every pf_asplit-th row of its activation tile; the workgroups that run beside it on the same XCD and share the
   // panel (the tile) touch the other rows.
   uint32_t pf_dist, pf_wsplit, pf_asplit;
+  uint32_t per_xcd;       // tiles of an XCD
   int vec_store;          // C (and a binary epilogue's operand) allow 16-byte accesses
 };
 
 [[maybe_unused]] constexpr int kDBK = 64;   // K elements per LDS stage
+
+// Which tile of C and which K range a workgroup takes.  Ids id, id + 8, ... share an XCD: each XCD gets an eighth of the tiles,
+// the M-tiles of one weight panel after the other, so that the 32 workgroups that run there together share panels and activations
+// in its L2 whatever the number of panels.
+__device__ __forceinline__ bool dense_tile(const DenseParams &p, uint32_t &mt, uint32_t &nt, uint32_t &split, uint32_t &aphase) {
+  split = __builtin_amdgcn_readfirstlane(blockIdx.x / (8 * p.per_xcd));
+  const uint32_t id = blockIdx.x - split * 8 * p.per_xcd, tile = (id & 7) * p.per_xcd + (id >> 3);
+  nt = __builtin_amdgcn_readfirstlane(tile / p.mtiles);
+  mt = tile - nt * p.mtiles;
+  aphase = __builtin_amdgcn_readfirstlane(nt % p.pf_asplit);
+  return nt < p.ntiles;   // the last XCD may have fewer
+}
 
 // WM: waves along M (4 / WM along N); a wave owns a (BM / WM) x (BN / WN) sub-tile
 template <int BM, int BN, int WM = 2>
@@ -89,20 +103,8 @@ __global__ void __launch_bounds__(256, 1) gemm_dense_kernel(DenseParams p) {
   // them the M-tiles of the same weight panels.
   // (the quotients come out of the vector ALU: readfirstlane moves what depends on them back to SGPRs, where the
   // scalar-base loads below need their addresses)
-  const uint32_t tiles = p.mtiles * p.ntiles, split = __builtin_amdgcn_readfirstlane(blockIdx.x / tiles);
-  uint32_t id = blockIdx.x - split * tiles, mt, nt, aphase = 0;
-  if (p.ntiles % 8 == 0) {
-    uint32_t xcd = id & 7, slot = id >> 3;
-    nt = (slot / p.mtiles) * 8 + xcd;
-    mt = slot % p.mtiles;
-    aphase = (slot / p.mtiles) % p.pf_asplit;
-  } else {
-    nt = id / p.mtiles;
-    mt = id % p.mtiles;
-  }
-  mt = __builtin_amdgcn_readfirstlane(mt);
-  nt = __builtin_amdgcn_readfirstlane(nt);
-  aphase = __builtin_amdgcn_readfirstlane(aphase);
+  uint32_t mt, nt, split, aphase;
+  if (!dense_tile(p, mt, nt, split, aphase)) return;
   const uint32_t m0 = mt * BM, n0 = nt * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave: in an SGPR
   const int wm = wave / WN, wn = wave % WN;
@@ -321,20 +323,8 @@ __global__ void __launch_bounds__(256, 1) gemm_dense16_kernel(DenseParams p) {
   uint8_t *const sA0 = lds, *const sA1 = lds + BM * 128, *const sB0 = lds + BM * 256, *const sB1 = lds + BM * 256 + BN * 128;
   __shared__ uint32_t pf_sink[4 * 64];
 
-  const uint32_t tiles = p.mtiles * p.ntiles, split = __builtin_amdgcn_readfirstlane(blockIdx.x / tiles);
-  uint32_t id = blockIdx.x - split * tiles, mt, nt, aphase = 0;
-  if (p.ntiles % 8 == 0) {
-    uint32_t xcd = id & 7, slot = id >> 3;
-    nt = (slot / p.mtiles) * 8 + xcd;
-    mt = slot % p.mtiles;
-    aphase = (slot / p.mtiles) % p.pf_asplit;
-  } else {
-    nt = id / p.mtiles;
-    mt = id % p.mtiles;
-  }
-  mt = __builtin_amdgcn_readfirstlane(mt);
-  nt = __builtin_amdgcn_readfirstlane(nt);
-  aphase = __builtin_amdgcn_readfirstlane(aphase);
+  uint32_t mt, nt, split, aphase;
+  if (!dense_tile(p, mt, nt, split, aphase)) return;
   const uint32_t m0 = mt * BM, n0 = nt * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
@@ -614,26 +604,24 @@ int launch_splitk_reduce(const float *partial, uint32_t ksplit, uint32_t M, uint
 template <int BM, int BN, int WM = 2> static int launch_dense_bm(DenseParams p, hipStream_t stream) {
   p.mtiles = (p.M + BM - 1) / BM;
   p.ntiles = (p.N + BN - 1) / BN;
-  // Who runs beside whom: with the XCD-aware order an XCD's 32 CUs hold 32 consecutive slots = the M-tiles of
-  // 32 / mtiles weight panels.  Otherwise every workgroup warms all its own lines.
+  // Who runs beside whom: an XCD's 32 CUs hold 32 consecutive tiles = the M-tiles of 32 / mtiles weight panels.
   p.pf_dist = 3;
-  p.pf_wsplit = p.pf_asplit = 1;
-  if (p.ntiles % 8 == 0) {
-    p.pf_wsplit = p.mtiles < 32 ? p.mtiles : 32;
-    const uint32_t panels = 32 / p.pf_wsplit, per_xcd = p.ntiles / 8;
-    p.pf_asplit = panels < per_xcd ? panels : per_xcd;
-    if (p.pf_asplit == 0) p.pf_asplit = 1;
-  }
+  p.per_xcd = (uint32_t)(((uint64_t)p.mtiles * p.ntiles + 7) / 8);
+  p.pf_wsplit = std::min(p.mtiles, 32u);
+  p.pf_asplit = std::max(1u, std::min(32 / p.pf_wsplit, p.ntiles / 8));
   if (g_tuning.dense_pf >= 0) p.pf_dist = (uint32_t)g_tuning.dense_pf;
-  uint64_t grid = (uint64_t)p.mtiles * p.ntiles * p.ksplit;
+  uint64_t grid = (uint64_t)p.per_xcd * 8 * p.ksplit;
   if (grid > 0x7FFFFFFFull) {
     set_error("cuthip_matmul_gguf_ws: problem too large for one launch");
     return CUTHIP_ERR_INVALID;
   }
   // the 16 x 16 x 32 kernel unless the tuning key dense_mfma16 = 0 asks for the 32 x 32 x 16 one (kept for comparison)
   const bool mfma16 = g_tuning.dense_mfma16 != 0;
-  if (mfma16) hipLaunchKernelGGL((gemm_dense16_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL((gemm_dense_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
+  constexpr bool kBoth = WM == 2 || BN == 224;
+  if constexpr (kBoth) {
+    if (!mfma16) hipLaunchKernelGGL((gemm_dense_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
+  }
+  if (mfma16 || !kBoth) hipLaunchKernelGGL((gemm_dense16_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
   return check_hip(hipGetLastError(), "dense gemm launch");
 }
 
@@ -650,49 +638,51 @@ bool dense_gemm_fits(uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a
   return true;
 }
 
-// Tile shape and number of K ranges.  Candidates in the order of their measured cost per multiply-add on whole rounds
-// (2048 x 14336 x 4096, every shape forced in turn on one box): 256 x 224 (four waves along M) 0.96, 128 x 448 1.00,
-// 256 x 256 1.03, 128 x 256 1.24.  A shape costs rounds over the 256 CUs x tile area x that factor; tiles that hang
-// over the edge of C count in full.  When the best shape leaves most of the chip idle, K is split over 128 x 256
-// tiles instead (partials in the workspace, summed by a second kernel).
-struct DenseShape { int bm, bn; uint32_t ksplit; };
-static DenseShape pick_dense_shape(uint32_t M, uint32_t K, uint32_t N) {
-  if (g_tuning.dense_bn && K % ((uint32_t)g_tuning.dense_ks * 128) == 0)   // forced by a test or a sweep
-    return DenseShape{g_tuning.dense_bm, g_tuning.dense_bn, (uint32_t)g_tuning.dense_ks};
-  static const struct { int bm, bn; double cost; } cands[] = {{256, 224, 0.96}, {128, 448, 1.00}, {256, 256, 1.03}, {128, 256, 1.24}};
-  int best = 0;
-  double best_t = 0.0;
-  uint64_t best_tiles = 0;
-  for (int c = 0; c < 4; ++c) {
-    const uint64_t tiles = (uint64_t)((M + cands[c].bm - 1) / cands[c].bm) * ((N + cands[c].bn - 1) / cands[c].bn);
-    const double t = (double)((tiles + 255) / 256) * cands[c].bm * cands[c].bn * cands[c].cost;
-    if (c == 0 || t < best_t) {
-      best = c;
-      best_t = t;
-      best_tiles = tiles;
+// scratch the vendor GEMM may use (variant 5) behind the dequantized weights and the converted activations, and room for the
+// partial products of a K split
+constexpr size_t kDenseScratch = (size_t)32 << 20;
+
+// Tile shape and number of K ranges: the cheapest by a model of the GEMM's time, fitted to 680 launches (400 .. 2048 rows, 12
+// weight shapes from 1024 x 4096 to 32000 x 2048, every tile forced in turn, graph replay; 6 % rms, the shape chosen is 0.7 % slower
+// than the best of them on average).  Microseconds: a part for each round of 256 workgroups, K x the tile's area x its cost per
+// multiply-add, once more a little of it for a full chip (clocks), C; a K split writes and reads its partial products and is a
+// second launch.  Edge tiles count in full, so that narrower tiles win where they fit the rows of W or the CUs better (us, widest
+// tiles in the order of one panel per eight XCDs -> this): 2048 x 5120 x 4096 107 -> 73 (256 x 160), 1024 x 5120 x 4096 105 -> 57
+// (256 x 128), 512 x 11008 x 4096 117 -> 59, 2048 x 11008 x 4096 222 -> 167 (256 x 192), 2048 x 2560 x 2560 63 -> 40,
+// 700 x 5632 x 2048 59 -> 34; 2048 x 14336 x 4096 stays with 256 x 224.
+struct DenseShape { int bm, bn; uint32_t ksplit; double us; };
+static DenseShape pick_dense_shape(uint32_t M, uint32_t K, uint32_t N, int c_bytes) {
+  static const struct { int bm, bn; double mac, full; } kTiles[] = {
+      {256, 224, 2.87e-7, 0.17e-7}, {256, 192, 2.87e-7, 0.39e-7}, {256, 160, 3.01e-7, 0.47e-7}, {256, 128, 3.33e-7, 0.41e-7},
+      {128, 448, 2.96e-7, 0.24e-7}, {256, 256, 2.59e-7, 0.26e-7}, {128, 256, 3.58e-7, 0.42e-7}};
+  const double mn = (double)M * N;
+  DenseShape best{0, 0, 1, 1e30};
+  for (const auto &t : kTiles) {
+    for (uint32_t ks = 1; ks <= 8; ks *= 2) {
+      if (g_tuning.dense_bn && (t.bm != g_tuning.dense_bm || t.bn != g_tuning.dense_bn || ks != (uint32_t)g_tuning.dense_ks) &&
+          K % ((uint32_t)g_tuning.dense_ks * 128) == 0)
+        continue;   // forced by a test or a sweep
+      const uint64_t tiles = (uint64_t)((M - 1) / t.bm + 1) * ((N - 1) / t.bn + 1) * ks;
+      if (ks > 1 && (K % (ks * 128) != 0 || (!g_tuning.dense_bn && (t.bm != 128 || t.bn != 256 || tiles > 256 || ks * mn * 4 > (double)kDenseScratch)))) break;
+      const double full = (double)((tiles - 1) / 256), part = (tiles - 256.0 * full) / 256.0;
+      double us = 0.3 + 5.25 * (full + 1.0) + 0.37e-6 * mn * c_bytes + (double)K / ks * t.bm * t.bn * (t.mac * (full + 1.0) + t.full * (full + part));
+      if (ks > 1) us += 5.2 + 0.95e-6 * ks * mn;
+      if (us < best.us) best = DenseShape{t.bm, t.bn, ks, us};
     }
   }
-  if (best_tiles >= 192) return DenseShape{cands[best].bm, cands[best].bn, 1};
-  const uint64_t tiles128 = (uint64_t)((M + 127) / 128) * ((N + 255) / 256);
-  uint32_t s = 1;
-  while (s < 8 && tiles128 * s < 192 && K % (2 * s * 128) == 0) s *= 2;
-  if (s == 1) return DenseShape{cands[best].bm, cands[best].bn, 1};
-  return DenseShape{128, 256, s};
+  return best;
 }
 
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
-
-// scratch the vendor GEMM may use (variant 5) behind the dequantized weights and the converted activations
-constexpr size_t kBlasLtScratch = (size_t)32 << 20;
 
 bool blaslt_available();
 int launch_blaslt_gemm(const void *Wd, const void *A16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA,
                        uint32_t strideC, void *workspace, size_t workspace_bytes, hipStream_t stream);
 
 size_t dense_gemm_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16) {
-  DenseShape sh = pick_dense_shape(M, K, N);
-  const size_t partial = sh.ksplit > 1 ? (size_t)sh.ksplit * M * N * 4 : 0;
-  return align256((size_t)N * K * 2) + align256(a_f16 ? 0 : (size_t)M * K * 2) + (partial > kBlasLtScratch ? partial : kBlasLtScratch);
+  const uint32_t ks = g_tuning.dense_bn ? (uint32_t)g_tuning.dense_ks : 1u;   // (what is chosen fits; a forced split may not)
+  const size_t partial = ks > 1 ? (size_t)ks * M * N * 4 : 0;
+  return align256((size_t)N * K * 2) + align256(a_f16 ? 0 : (size_t)M * K * 2) + std::max(partial, kDenseScratch);
 }
 
 // workspace of the GEMM on resident fp16 weights: converted activations (fp32 input only) + split-K partials / scratch
@@ -700,49 +690,36 @@ size_t dense_f16_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16) {
   return dense_gemm_workspace(M, K, N, a_f16) - align256((size_t)N * K * 2);
 }
 
-// Cost in microseconds of the two-pass path, for the automatic choice between it and one launch on the blocks; fitted to 3,756
-// launches (four formats, 64 .. 4096 rows, 22 weight shapes from 512 x 512 to 32,000 x 2048, both activation types, HIP-graph
-// replay, MI355X; 5.5 % rms where it is near the row-tile matmul):
-//   5 + N K (bytes per weight + 2) / 5.14 MB  the dequantization (reads the blocks, writes fp16)
-//   + 5.5 per round of tiles over the 256 CUs + K x the tile's area x its cost per multiply-add, f more for a round that fills
-//     the chip (clocks, memory); where the panels are no multiple of eight, and a panel's tiles are spread over the XCDs, 1.22
-//     (128 x 256 tiles: 1.39) times as much
-//   + C at 6 TB/s, the partial products of a K split, the conversion of fp32 activations
-// The row-tile matmul decodes every weight once per 128 rows and this path once, so the line runs at about 450 rows on wide
-// matrices (14336 x 4096, us, row tiles / two passes: Q8_0 384 rows 83 / 103, 448 rows 94 / 83; Q4_K 512 rows 78 / 85, 768 rows
-// 116 / 107) and higher on narrow ones (4096 x 4096 Q4_K: 1024 rows 45 / 56, 2048 rows 85 / 72; 1024 x 4096: never).  The last
-// factor puts it there: on panels that are a multiple of eight the other terms come out a few per cent high at 450 to 800 rows.
+// Cost in microseconds of the two-pass path, for the automatic choice between it and one launch on the blocks: the
+// dequantization (reads the blocks, writes fp16 at 5.14 TB/s together), the conversion of fp32 activations, the GEMM.
 static double two_pass_us(double decode_us, uint32_t M, uint32_t K, uint32_t N, int a_f16) {
-  static const struct { double mac, f; } kTile[5] = {{1.42e-7, 1.38}, {1.06e-7, 2.0}, {1.12e-7, 2.0}, {1.76e-7, 1.14}, {2.48e-7, 0.43}};
-  const DenseShape sh = pick_dense_shape(M, K, N);
-  const int shape = sh.bn == 224 ? 0 : sh.bn == 448 ? 1 : sh.bm == 256 ? 2 : sh.ksplit == 1 ? 3 : 4;
-  const uint32_t mtiles = (M - 1) / sh.bm + 1, ntiles = (N - 1) / sh.bn + 1;
-  const bool spread = mtiles > 1 && ntiles % 8 != 0;
-  const uint64_t tiles = (uint64_t)mtiles * ntiles * sh.ksplit;
-  const double full = (double)((tiles - 1) / 256), last = (double)tiles - 256.0 * full, f = kTile[shape].f;
-  double us = decode_us + 5.54 * (full + 1.0) + 0.168e-6 * M * N * (a_f16 ? 2 : 4) +
-              (double)K / sh.ksplit * sh.bm * sh.bn * kTile[shape].mac * (full * (1.0 + f) + 1.0 + f * last / 256.0) *
-                  (!spread ? 1.0 : shape < 3 ? 1.22 : 1.39);
-  if (sh.ksplit > 1) us += 1.2 + 8.0 * sh.ksplit * M * N / 7.12e6;
+  double us = decode_us + pick_dense_shape(M, K, N, a_f16 ? 2 : 4).us;
   if (!a_f16) us += 2.3 + 6.0 * M * K / 7.54e6;
-  return us * (spread ? 1.0 : 0.96);
+  return us;
 }
 
 double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16) {
-  return two_pass_us(5.0 + (double)N * K * ((double)fmt_bytes(fmt) / fmt_elems(fmt) + 2.0) / 5.14e6, M, K, N, a_f16);
+  // The factor sets this sum against the estimate of the row-tile matmul: over 1,040 calls of 224 .. 2048 rows on ten weight shapes
+  // (four formats, both activation types) the sum comes out 6 per cent high and that estimate 6 per cent low; Q6_K, whose 210-byte
+  // blocks are slower to take apart, is held at the row tiles where the two are level (640 x 11008 x 4096 94 us either way).  The
+  // choice is 0.3 per cent slower than the better of the two on average.  The row-tile matmul decodes every weight once per 128
+  // rows and this path once, so the line runs at about 450 rows on wide matrices and 32000 x 2048, at 600 on 4096 x 14336, at
+  // 1,300 on 4096 x 4096.
+  return (fmt == CUTHIP_Q6_K ? 1.01 : 0.88) *
+         two_pass_us(5.0 + (double)N * K * ((double)fmt_bytes(fmt) / fmt_elems(fmt) + 2.0) / 5.14e6, M, K, N, a_f16);
 }
 
 // The same from the separated layout and fp32 activations: the transposing dequantization runs at 1.33 weights per ps
-// (14336 x 4096 45 us); 270 launches of 32 .. 512 rows on nine weight shapes come out 10 per cent above the fit.
-double sep_two_pass_us(uint32_t M, uint32_t K, uint32_t N) { return 1.1 * two_pass_us(4.0 + (double)N * K / 1.33e6, M, K, N, 0); }
+// (14336 x 4096 45 us).
+double sep_two_pass_us(uint32_t M, uint32_t K, uint32_t N) { return two_pass_us(4.0 + (double)N * K / 1.33e6, M, K, N, 0); }
 
 // What a call of 9 to 40 rows has to save before it gives up weights that are not rounded (8-row passes, 1e-5 of the
 // result's norm) for fp16 ones (3e-4): passes stay while this is not below 0.9 of their cost.  A line of precision, not an
 // estimate of time: dense_cost_us, refitted on 64 rows and more, comes out 5 to 8 us lower at K = 256 .. 768 and, used here,
 // took the exact weights from calls of 17 to 32 rows (24 x 2048 x 512 on Q8_0: 2.7e-7 of the norm became 2.1e-4, 17.8 us 12.6).
-double dense_line_us(int fmt, uint32_t M, uint32_t K, uint32_t N) {
+double dense_line_us(int fmt, uint32_t K, uint32_t N) {
   const double nk = (double)N * K, bpw = (double)fmt_bytes(fmt) / fmt_elems(fmt);
-  const double split = pick_dense_shape(M, K, N).ksplit > 1 ? 5.0 : 0.0;
+  const double split = (N - 1) / 256 + 1 < 192 && K % 256 == 0 ? 5.0 : 0.0;   // too few tiles of one row of them: a K split
   return 3.0 + nk * (bpw + 2.0) / 6.0e6 + 17.0 + 2.0 * nk / 3.5e6 + split;
 }
 
@@ -771,7 +748,7 @@ int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C,
   }
   if (use_blaslt) {
     uint8_t *scratch = after_w + align256(a_f16 ? 0 : (size_t)M * K * 2);
-    const int rc = launch_blaslt_gemm(w16, p.A, C, c_f16, M, K, N, p.strideA, strideC, scratch, kBlasLtScratch, stream);
+    const int rc = launch_blaslt_gemm(w16, p.A, C, c_f16, M, K, N, p.strideA, strideC, scratch, kDenseScratch, stream);
     // 1 = asked for by variant index: its errors are the caller's; 2 = automatic choice: a shape the library has no
     // kernel for goes on to the GEMM below (nothing has been enqueued for it yet)
     if (rc == CUTHIP_OK || use_blaslt == 1 || rc != CUTHIP_ERR_INVALID) return rc;
@@ -782,13 +759,16 @@ int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C,
   p.mtiles = p.ntiles = 0;
   p.c_f16 = c_f16;
   p.vec_store = store8_aligned(C, strideC, c_f16, epi) ? 1 : 0;
-  const DenseShape sh = pick_dense_shape(M, K, N);
+  const DenseShape sh = pick_dense_shape(M, K, N, c_f16 ? 2 : 4);
   p.ksplit = sh.ksplit;
   p.kper = K / sh.ksplit;
   p.partial = reinterpret_cast<float *>(after_w + align256(a_f16 ? 0 : (size_t)M * K * 2));
   int rc;
   if (sh.bn == 448) rc = launch_dense_bm<128, 448>(p, stream);
   else if (sh.bn == 224) rc = launch_dense_bm<256, 224, 4>(p, stream);
+  else if (sh.bn == 192) rc = launch_dense_bm<256, 192, 4>(p, stream);
+  else if (sh.bn == 160) rc = launch_dense_bm<256, 160, 4>(p, stream);
+  else if (sh.bn == 128) rc = launch_dense_bm<256, 128, 4>(p, stream);
   else if (sh.bm == 256) rc = launch_dense_bm<256, 256>(p, stream);
   else rc = launch_dense_bm<128, 256>(p, stream);
   if (rc) return rc;

@@ -135,7 +135,7 @@ double lds_gemm_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16);
 bool dense_gemm_fits(uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A);
 size_t dense_gemm_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16);
 double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16);
-double dense_line_us(int fmt, uint32_t M, uint32_t K, uint32_t N);
+double dense_line_us(int fmt, uint32_t K, uint32_t N);
 int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K,
                       uint32_t N, uint32_t strideA, uint32_t strideC, Epilogue epi, void *workspace, hipStream_t stream,
                       int use_blaslt);
@@ -666,7 +666,7 @@ int cuthip_matmul_gguf_ws(int fmt, const void *W, const void *A, int a_dtype, vo
   SingleLaunch single{};
   const SingleLaunch *chosen = nullptr;
   if (variant == -1 && M > 8 && fits && ws_ok) {
-    passes = passes && dense_line_us(fmt, M, K, N) >= 0.9 * passes_cost_us(fmt, M, K, N);
+    passes = passes && dense_line_us(fmt, K, N) >= 0.9 * passes_cost_us(fmt, M, K, N);
     if (!passes) {
       single = single_launch_choice(fmt, M, K, N, strideA, a_f16, workspace_bytes);
       dense_first = dense_cost_us(fmt, M, K, N, a_f16) < single.cost;
