@@ -16,6 +16,24 @@ import torch
 
 from . import lib as _l
 
+_native = None
+
+
+def _host():
+    """The native host side of the operators that are launched most (csrc/host_ops.cpp): checks, outputs and the C-ABI call.
+    A decode step of the two-layer test model, 15 launches one by one: 107 us in Python and ctypes, 68 with it; seven
+    matmuls on the separated layout 94 -> 86 (bound by the kernels then)."""
+    global _native
+    if _native is None:
+        _l.load()   # says how to build what is missing
+        try:
+            from . import _host_ops
+        except ImportError as e:
+            raise _l.CutHipError(f"cut_amd/_host_ops.so is missing or does not load: build it with `make -C cut_amd/csrc` ({e})") from e
+        _host_ops.setup(_l.CutHipError, _l.FORMATS, _l.UNARY, _l.BINARY)
+        _native = _host_ops
+    return _native
+
 
 def _stream_ptr() -> int:
     # the handle alone: a Stream object around it costs 2.8 us more, on every launch
@@ -40,20 +58,7 @@ def n_bytes(fmt, rows: int, cols: int) -> int:
 def dequantize(raw: torch.Tensor, fmt, rows: int, cols: int, dtype: torch.dtype = torch.float32,
                out: torch.Tensor | None = None) -> torch.Tensor:
     """raw: 1-D uint8/int8 device tensor of GGUF blocks -> [rows, cols]."""
-    f = _fmt(fmt)
-    if not raw.is_cuda or raw.element_size() != 1 or not raw.is_contiguous():
-        raise _l.CutHipError("dequantize: raw must be a contiguous 1-byte device tensor")
-    need = n_bytes(f, rows, cols)
-    if raw.numel() < need:
-        raise _l.CutHipError(f"dequantize: raw holds {raw.numel()} bytes, {need} needed")
-    if dtype not in (torch.float32, torch.float16):
-        raise _l.CutHipError("dequantize: output dtype must be float32 or float16")
-    if out is None:
-        out = torch.empty((rows, cols), dtype=dtype, device=raw.device)
-    stride = out.stride(0) if out.dim() == 2 else cols
-    _l.check(_l.load().cuthip_dequant(f, raw.data_ptr(), out.data_ptr(), _l.F16 if dtype == torch.float16 else _l.F32,
-                                      rows, cols, stride, _stream_ptr()))
-    return out
+    return _host().dequantize(raw, fmt, rows, cols, dtype, out)
 
 
 _FMT_NAMES = {_l.Q8_0: "Q8_0", _l.Q4_0: "Q4_0", _l.Q4_K: "Q4_K", _l.Q6_K: "Q6_K"}
@@ -87,93 +92,31 @@ def matmul_gguf(a: torch.Tensor, w_blocks: torch.Tensor, fmt, N: int, K: int, ou
     byte tensor from matmul_gguf_workspace) the call goes through
     cuthip_matmul_gguf_ws, which opens variant 4 (dequantize once, dense GEMM).
     swiglu_pairs: weight rows 2i / 2i+1 are gate_i / up_i and the result is [M, N/2] = silu(gate) * up (M <= 8)."""
-    f = _fmt(fmt)
-    if a.dim() == 1:
-        a2 = a.unsqueeze(0)
-    elif a.dim() == 2:
-        a2 = a
-    else:
-        raise _l.CutHipError("matmul: A must be 1D or 2D")
-    M = a2.shape[0]
-    if a2.shape[1] != K:
-        raise _l.CutHipError(f"matmul: B rows ({K}) must match A cols ({a2.shape[1]})")
-    if a2.dtype not in (torch.float32, torch.float16) or a2.stride(1) != 1:
-        raise _l.CutHipError("matmul: A must be float32/float16 with unit inner stride")
-    if w_blocks.numel() < n_bytes(f, N, K):
-        raise _l.CutHipError("matmul: weight tensor too small for [N, K]")
-    odt = out_dtype or a2.dtype
-    if out is None:
-        out = torch.empty((M, N // 2 if swiglu_pairs else N), dtype=odt, device=a.device)
-    epi, op, dptr = _l.EPI_NONE, 0, None
-    if swiglu_pairs:
-        epi = _l.EPI_SWIGLU_PAIRS
-    elif unary is not None:
-        epi, op = _l.EPI_UNARY, _l.UNARY[unary]
-    elif binary is not None:
-        if d is None or d.shape != out.shape or d.dtype != out.dtype or d.stride(0) != out.stride(0):
-            raise _l.CutHipError("matmul: binary epilogue needs D with the shape, dtype and stride of C")
-        epi, op, dptr = _l.EPI_BINARY, _l.BINARY[binary], d.data_ptr()
-    adt = _l.F16 if a2.dtype == torch.float16 else _l.F32
-    cdt = _l.F16 if out.dtype == torch.float16 else _l.F32
-    if _tuning is not None and variant == -1 and epi == _l.EPI_NONE and workspace is not None:
-        variant = _tuning.select("MatMulGguf" + _FMT_NAMES[f], [M, K, N], -1)
+    if _tuning is not None and variant == -1 and unary is None and binary is None and not swiglu_pairs and workspace is not None:
+        variant = _tuning.select("MatMulGguf" + _FMT_NAMES[_fmt(fmt)], [a.shape[0] if a.dim() == 2 else 1, K, N], -1)
         # a rule may name a variant this process cannot run (the vendor-GEMM variant without its library): the
         # hand-written two-pass GEMM takes its place
         if variant >= 0 and _l.load().cuthip_variant_available(_l.OP_MATMUL_GGUF, variant) != 1:
             variant = 4 if variant == 5 else -1
-    if workspace is not None:
-        _l.check(_l.load().cuthip_matmul_gguf_ws(
-            f, w_blocks.data_ptr(), a2.data_ptr(), adt, out.data_ptr(), cdt, M, K, N, a2.stride(0), out.stride(0), epi, op,
-            dptr, variant, workspace.data_ptr(), workspace.numel() * workspace.element_size(), _stream_ptr()))
-    else:
-        _l.check(_l.load().cuthip_matmul_gguf(
-            f, w_blocks.data_ptr(), a2.data_ptr(), adt, out.data_ptr(), cdt, M, K, N, a2.stride(0), out.stride(0), epi, op,
-            dptr, variant, _stream_ptr()))
-    return out
+    return _host().matmul_gguf(a, w_blocks, fmt, N, K, out_dtype, out, unary, binary, d, variant, workspace, swiglu_pairs)
 
 
 def norm_carry(sumsq_parts: torch.Tensor | None = None, eps: float = 0.0, next_norm_weight: torch.Tensor | None = None,
                next_x16: torch.Tensor | None = None, next_sumsq_parts: torch.Tensor | None = None) -> "_l.NormCarry":
     """cuthip_norm_carry_t from device tensors (float32 [K/8] / [N] / [N/8], fp16 [N] output)."""
-    def ptr(t, dtype):
-        if t is None:
-            return None
-        if t.dtype != dtype or not t.is_contiguous():
-            raise _l.CutHipError("norm_carry: wrong dtype or non-contiguous tensor")
-        return t.data_ptr()
-    return _l.NormCarry(ptr(sumsq_parts, torch.float32), eps, ptr(next_norm_weight, torch.float32), ptr(next_x16, torch.float16),
-                        ptr(next_sumsq_parts, torch.float32))
+    return _host().norm_carry(_l.NormCarry, sumsq_parts, eps, next_norm_weight, next_x16, next_sumsq_parts)
 
 
 def matmul_gguf_carry(a: torch.Tensor, w_blocks: torch.Tensor, fmt, N: int, K: int, out: torch.Tensor, carry, binary: str | None = None,
                       d: torch.Tensor | None = None, swiglu_pairs: bool = False) -> torch.Tensor:
     """Batch-1 matmul taking part in a carried RMSNorm (cuthip_matmul_gguf_carry); a [K], out [N] (or [N/2])."""
-    f = _fmt(fmt)
-    if a.numel() != K or a.dtype not in (torch.float32, torch.float16) or not a.is_contiguous() or not out.is_contiguous():
-        raise _l.CutHipError("matmul_carry: A must be a contiguous float32/float16 vector of K elements, out contiguous")
-    if w_blocks.numel() < n_bytes(f, N, K) or out.numel() != (N // 2 if swiglu_pairs else N):
-        raise _l.CutHipError("matmul_carry: weight tensor too small or output of the wrong size")
-    epi, op, dptr = _l.EPI_NONE, 0, None
-    if swiglu_pairs:
-        epi = _l.EPI_SWIGLU_PAIRS
-    elif binary is not None:
-        if d is None or d.numel() != N or d.dtype != out.dtype:
-            raise _l.CutHipError("matmul_carry: binary epilogue needs D with the size and dtype of C")
-        epi, op, dptr = _l.EPI_BINARY, _l.BINARY[binary], d.data_ptr()
-    import ctypes
-    _l.check(_l.load().cuthip_matmul_gguf_carry(f, w_blocks.data_ptr(), a.data_ptr(), _dt(a), out.data_ptr(), _dt(out), K, N, epi,
-                                                op, dptr, ctypes.byref(carry) if carry is not None else None, _stream_ptr()))
-    return out
+    return _host().matmul_gguf_carry(a, w_blocks, fmt, N, K, out, carry, binary, d, swiglu_pairs)
 
 
 def rope_append(runtime_params: torch.Tensor, cos_t: torch.Tensor, sin_t: torch.Tensor, q_out: torch.Tensor, k_cache: torch.Tensor,
                 v_cache: torch.Tensor, q_dim: int, head_dim: int) -> "_l.RopeAppend":
     """cuthip_rope_append_t for matmul_gguf_pair: rotated q to q_out, rotated k and v to the cache row of the position."""
-    if k_cache.dtype != torch.float16 or v_cache.dtype != torch.float16 or k_cache.stride(0) != v_cache.stride(0):
-        raise _l.CutHipError("rope_append: caches must be fp16 with one row stride")
-    return _l.RopeAppend(runtime_params.data_ptr(), cos_t.data_ptr(), sin_t.data_ptr(), q_out.data_ptr(), _dt(q_out),
-                         k_cache.data_ptr(), v_cache.data_ptr(), q_dim, head_dim, k_cache.stride(0),
-                         min(k_cache.shape[0], cos_t.shape[0]))
+    return _host().rope_append(_l.RopeAppend, runtime_params, cos_t, sin_t, q_out, k_cache, v_cache, q_dim, head_dim)
 
 
 def interleave_rope_rows(w_blocks: torch.Tensor, n_rows: int, head_dim: int) -> torch.Tensor:
@@ -189,22 +132,7 @@ def matmul_gguf_pair(a: torch.Tensor, wa: torch.Tensor, fmt_a, Na: int, out_a: t
                      Nb: int, out_b: torch.Tensor | None, K: int, carry=None, rope=None) -> None:
     """out_a = a . dequant(wa)^T and out_b = a . dequant(wb)^T for one activation vector a [K], in one launch where the
     formats allow it (cuthip_matmul_gguf_pair)."""
-    fa, fb = _fmt(fmt_a), _fmt(fmt_b)
-    if a.numel() != K or a.dtype not in (torch.float32, torch.float16) or not a.is_contiguous():
-        raise _l.CutHipError("matmul_pair: A must be a contiguous float32/float16 vector of K elements")
-    if wa.numel() < n_bytes(fa, Na, K) or wb.numel() < n_bytes(fb, Nb, K):
-        raise _l.CutHipError("matmul_pair: weight tensor too small for [N, K]")
-    import ctypes
-    if rope is not None:   # the epilogue writes q_out and the caches; the plain outputs are not used
-        _l.check(_l.load().cuthip_matmul_gguf_pair(
-            fa, wa.data_ptr(), Na, None, fb, wb.data_ptr(), Nb, None, a.data_ptr(), _dt(a), _l.F32, K,
-            ctypes.byref(carry) if carry is not None else None, ctypes.byref(rope), _stream_ptr()))
-        return
-    if out_a.dtype != out_b.dtype or out_a.numel() != Na or out_b.numel() != Nb or not (out_a.is_contiguous() and out_b.is_contiguous()):
-        raise _l.CutHipError("matmul_pair: outputs must be contiguous [Na] and [Nb] of one dtype")
-    _l.check(_l.load().cuthip_matmul_gguf_pair(
-        fa, wa.data_ptr(), Na, out_a.data_ptr(), fb, wb.data_ptr(), Nb, out_b.data_ptr(), a.data_ptr(), _dt(a), _dt(out_a), K,
-        ctypes.byref(carry) if carry is not None else None, None, _stream_ptr()))
+    _host().matmul_gguf_pair(a, wa, fmt_a, Na, out_a, wb, fmt_b, Nb, out_b, K, carry, rope)
 
 
 def matmul_gguf_workspace(fmt, M: int, K: int, N: int, a_dtype: torch.dtype, device) -> torch.Tensor:
@@ -225,14 +153,7 @@ def _dt(t: torch.Tensor) -> int:
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor | None = None,
             out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """x: [rows, dim] or [dim]; weight: fp32 [dim] (RMSNormOpNode of the reference)."""
-    x2 = x if x.dim() == 2 else x.reshape(1, -1)
-    if weight.dtype != torch.float32 or weight.numel() != x2.shape[1] or x2.stride(1) != 1:
-        raise _l.CutHipError("rmsnorm: weight must be fp32 [dim] and x rows contiguous")
-    if out is None:
-        out = torch.empty(x2.shape, dtype=out_dtype or x.dtype, device=x.device)
-    _l.check(_l.load().cuthip_rmsnorm(x2.data_ptr(), _dt(x2), weight.data_ptr(), out.data_ptr(), _dt(out), x2.shape[0],
-                                      x2.shape[1], x2.stride(0), eps, _stream_ptr()))
-    return out
+    return _host().rmsnorm(x, weight, eps, out, out_dtype)
 
 
 def rope_kv_write(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, runtime_params: torch.Tensor, cos_t: torch.Tensor,
@@ -256,11 +177,7 @@ def attn_decode_workspace(n_heads: int, head_dim: int, max_seq_len: int, device)
 def attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, runtime_params: torch.Tensor, n_heads: int,
                 n_kv_heads: int, head_dim: int, scale: float, workspace: torch.Tensor, out: torch.Tensor,
                 max_seq_len: int | None = None) -> torch.Tensor:
-    _l.check(_l.load().cuthip_attn_decode(q.data_ptr(), _dt(q), k_cache.data_ptr(), v_cache.data_ptr(),
-                                          runtime_params.data_ptr(), out.data_ptr(), _dt(out), n_heads, n_kv_heads, head_dim,
-                                          k_cache.stride(0), scale, max_seq_len or k_cache.shape[0], workspace.data_ptr(),
-                                          workspace.numel(), _stream_ptr()))
-    return out
+    return _host().attn_decode(q, k_cache, v_cache, runtime_params, n_heads, n_kv_heads, head_dim, scale, workspace, out, max_seq_len)
 
 
 def attn_decode_static(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, runtime_params: torch.Tensor, n_heads: int,
@@ -327,8 +244,7 @@ def matmul_gguf_attn_merge(records: torch.Tensor, w_blocks: torch.Tensor, fmt, N
 
 
 def silu_mul(gate_up: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-    _l.check(_l.load().cuthip_silu_mul(gate_up.data_ptr(), _dt(gate_up), out.data_ptr(), _dt(out), out.numel(), _stream_ptr()))
-    return out
+    return _host().silu_mul(gate_up, out)
 
 
 def argmax(x: torch.Tensor, out_index: torch.Tensor) -> torch.Tensor:
@@ -370,26 +286,12 @@ def matmul_gguf_argmax(a: torch.Tensor, w_blocks: torch.Tensor, fmt, N: int, K: 
                        carry=None, pen_tokens: torch.Tensor | None = None, pen_factors: torch.Tensor | None = None,
                        workspace: torch.Tensor | None = None) -> torch.Tensor:
     """The output head with the sampling folded in: logits = a . dequant(W)^T, penalty on the listed tokens, arg-max."""
-    f = _fmt(fmt)
-    if a.numel() != K or not a.is_contiguous() or logits.numel() != N or not logits.is_contiguous():
-        raise _l.CutHipError("matmul_gguf_argmax: a is a contiguous vector of K elements, logits one of N")
-    pt, pf, n = _pen_args(pen_tokens, pen_factors)
-    _l.check(_l.load().cuthip_matmul_gguf_argmax(f, w_blocks.data_ptr(), a.data_ptr(), _dt(a), logits.data_ptr(), _dt(logits), K, N,
-                                                 C.byref(carry) if carry is not None else None, pt, pf, n,
-                                                 workspace.data_ptr() if workspace is not None else None,
-                                                 workspace.numel() if workspace is not None else 0, out_index.data_ptr(),
-                                                 _stream_ptr()))
-    return out_index
+    return _host().matmul_gguf_argmax(a, w_blocks, fmt, N, K, logits, out_index, carry, pen_tokens, pen_factors, workspace)
 
 
 def embedding_rows(w_blocks: torch.Tensor, fmt, token_ids: torch.Tensor, n_rows: int, dim: int, out: torch.Tensor) -> torch.Tensor:
     """out[i] = dequant(row token_ids[i]) of a GGUF table [n_rows, dim]; token_ids int32/uint32 on the device."""
-    if token_ids.dtype not in (torch.int32, torch.uint32) or out.stride(-1) != 1 or out.numel() < token_ids.numel() * dim:
-        raise _l.CutHipError("embedding_rows: token ids are 32-bit integers, out holds one row of dim per id")
-    out2 = out if out.dim() == 2 else out.view(token_ids.numel(), -1)
-    _l.check(_l.load().cuthip_embedding_rows(_fmt(fmt), w_blocks.data_ptr(), token_ids.data_ptr(), token_ids.numel(), n_rows, dim,
-                                             out2.data_ptr(), _dt(out2), out2.stride(0), _stream_ptr()))
-    return out
+    return _host().embedding_rows(w_blocks, fmt, token_ids, n_rows, dim, out)
 
 
 def embedding_col(indices: torch.Tensor, matrix: torch.Tensor, scales: torch.Tensor | None, emb_dim: int, vocab: int,
@@ -414,32 +316,7 @@ def matmul_sep(a: torch.Tensor, b: torch.Tensor, scales: torch.Tensor, N: int, q
     """Operations::matmul(a, packedB, scalesB) of the reference on its own layout: a fp32 [M, K]; b int8 [K, N]
     (q4: uint8 [K, N/2], even column in the low nibble); scales fp16 [K/32, N] ([2K/32, N] when affine).
     variant: the reference's `spec` (an index of its MatMulQ8 / MatMulQ4 variant tables), -1 = by shape."""
-    a2 = a if a.dim() == 2 else a.reshape(1, -1)
-    M, K = a2.shape
-    if a2.dtype != torch.float32 or scales.dtype != torch.float16 or b.element_size() != 1 or b.dim() != 2 or scales.dim() != 2:
-        raise _l.CutHipError("matmul_sep: a must be fp32, b a 2-D 1-byte tensor and scales a 2-D fp16 tensor")
-    rows_s = (2 if affine else 1) * (K // 32)
-    if b.shape[0] != K or scales.shape[0] != rows_s or b.shape[1] < ((N + 1) // 2 if q4 else N) or scales.shape[1] < N:
-        raise _l.CutHipError(f"matmul_sep: shapes do not match K = {K}, N = {N} (b {tuple(b.shape)}, scales {tuple(scales.shape)})")
-    if out is None:
-        out = torch.empty((M, N), dtype=torch.float32, device=a.device)
-    epi, op, dptr = _l.EPI_NONE, 0, None
-    if unary is not None:
-        epi, op = _l.EPI_UNARY, _l.UNARY[unary]
-    elif binary is not None:
-        if d is None or d.shape != out.shape or d.dtype != torch.float32 or d.stride(0) != out.stride(0):
-            raise _l.CutHipError("matmul_sep: binary epilogue needs an fp32 D with the shape and stride of C")
-        epi, op, dptr = _l.EPI_BINARY, _l.BINARY[binary], d.data_ptr()
-    lib = _l.load()
-    ws_bytes = lib.cuthip_matmul_sep_workspace_bytes_for(_l.OP_MATMUL_Q4 if q4 else _l.OP_MATMUL_Q8, variant, M, K, N)
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=a.device)
-    common = (a2.data_ptr(), b.data_ptr(), scales.data_ptr(), dptr, out.data_ptr(), M, K, N, a2.stride(0), b.stride(0),
-              out.stride(0), scales.stride(0), epi, op)
-    if q4:
-        _l.check(lib.cuthip_matmul_q4_sep(*common, int(affine), variant, ws.data_ptr(), ws_bytes, _stream_ptr()))
-    else:
-        _l.check(lib.cuthip_matmul_q8_sep(*common, variant, ws.data_ptr(), ws_bytes, _stream_ptr()))
-    return out
+    return _host().matmul_sep(a, b, scales, N, q4, affine, out, unary, binary, d, variant)
 
 
 def matmul_dense_f16(a: torch.Tensor, w16: torch.Tensor, out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None,
@@ -506,23 +383,7 @@ def prepare_sep(w_blocks: torch.Tensor, fmt, N: int, K: int, stride_b: int | Non
     Q8_0 -> int8 [K, N] + fp16 [K/32, N]; Q4_0 -> nibbles uint8 [K, N/2] + fp16 [K/32, N]; Q4_K -> affine Q4, nibbles
     + fp16 [2K/32, N] (scales then minima: requantizeQ4KToAffine).  Row strides default to the reference's padding
     to multiples of 4 elements (MatMulOp.cpp:514-541)."""
-    f = _fmt(fmt)
-    if f not in (_l.Q8_0, _l.Q4_0, _l.Q4_K):
-        raise _l.CutHipError("prepare_sep: only Q8_0, Q4_0 and Q4_K have a separated layout")
-    q4 = f != _l.Q8_0
-    width = (N // 2) if q4 else N
-    sb = stride_b if stride_b is not None else (width + 3) & ~3
-    ss = scale_stride if scale_stride is not None else (N + 3) & ~3
-    rows_s = (2 if f == _l.Q4_K else 1) * (K // 32)
-    B = torch.empty((K, sb), dtype=torch.uint8 if q4 else torch.int8, device=w_blocks.device)
-    S = torch.empty((rows_s, ss), dtype=torch.float16, device=w_blocks.device)
-    # the kernel writes every column up to the width; the padding beyond it is zero
-    if sb > width:
-        B[:, width:].zero_()
-    if ss > N:
-        S[:, N:].zero_()
-    _l.check(_l.load().cuthip_prepare_sep(f, w_blocks.data_ptr(), N, K, B.data_ptr(), sb, S.data_ptr(), ss, _stream_ptr()))
-    return B, S
+    return _host().prepare_sep(w_blocks, fmt, N, K, stride_b, scale_stride)
 
 
 def transpose_q4_nibble(packed: torch.Tensor, N: int, K: int) -> torch.Tensor:
