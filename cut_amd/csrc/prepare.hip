@@ -15,7 +15,8 @@
 // only 2-byte aligned), all of them before the first use, and puts the quants into LDS without the scales between them;
 // then a thread reads a 16-byte piece of 4 (int8) or 8 (nibble) neighbouring rows, transposes 4 x 4 bytes at a time with
 // v_perm_b32 and writes 16 (32) dwords.  14336 x 4096, us: Q8_0 52 -> 25, Q4_0 34 -> 15, Q4_K 38 -> 13.5 (before: 2-byte
-// loads, one dword per row read from LDS, runs of 64 bytes for nibbles), all three 154 -> 67, 3.9 TB/s.
+// loads, one dword per row read from LDS, runs of 64 bytes for nibbles), all three 154 -> 67; with stores past the caches
+// (nothing here reads the outputs back) 65, 4.0 TB/s.
 #include <cstdint>
 
 #include "common.hpp"
@@ -116,7 +117,7 @@ template <int MODE> __global__ void __launch_bounds__(kPrepThreads) prepare_sep_
   auto put = [&](uint32_t k, uint32_t v) {   // columns col .. col + 3 of row k0 + k
     uint8_t *dst = p.B + (size_t)(k0 + k) * p.strideB + col;
     if (words && col + 3 < cols) {
-      *reinterpret_cast<uint32_t *>(dst) = v;
+      __builtin_nontemporal_store(v, reinterpret_cast<uint32_t *>(dst));   // nothing here reads it back
     } else {
       for (uint32_t j = 0; j < 4 && col + j < cols; ++j) dst[j] = (uint8_t)(v >> (8 * j));
     }
@@ -157,7 +158,7 @@ template <int MODE> __global__ void __launch_bounds__(kPrepThreads) prepare_sep_
 #pragma unroll
     for (int it = 0; it < 8 * G::ROWS / kPrepThreads; ++it) {
       const uint32_t i = it * kPrepThreads + tid, blk = i / G::ROWS, n = n0 + i % G::ROWS;
-      if (n < p.N && blk * 32 < kt) p.S[(size_t)(k0 / 32 + blk) * p.scaleStride + n] = sc[i];
+      if (n < p.N && blk * 32 < kt) __builtin_nontemporal_store(sc[i], &p.S[(size_t)(k0 / 32 + blk) * p.scaleStride + n]);
     }
   }
   if constexpr (MODE == PREP_Q4_K_AFFINE) {   // one thread per row: scales and minima of its eight sub-blocks
@@ -181,8 +182,8 @@ template <int MODE> __global__ void __launch_bounds__(kPrepThreads) prepare_sep_
         const float scale = d * (float)s;
         const float minv = 8.0f * scale - dmin * (float)m;
         const size_t b = k0 / 32 + j;
-        p.S[b * p.scaleStride + n] = (uint16_t)f32_to_f16bits_any(scale);
-        p.S[(blocksK + b) * p.scaleStride + n] = (uint16_t)f32_to_f16bits_any(minv);
+        __builtin_nontemporal_store((uint16_t)f32_to_f16bits_any(scale), &p.S[b * p.scaleStride + n]);
+        __builtin_nontemporal_store((uint16_t)f32_to_f16bits_any(minv), &p.S[(blocksK + b) * p.scaleStride + n]);
       }
     }
   }
