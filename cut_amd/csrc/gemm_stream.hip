@@ -5,25 +5,29 @@
 // Supersedes MatMulQ4GemvKPar8.cu / MatMulQ4TiledReg.cu (operators/impl/matmul) at these batch sizes.
 //
 // Two waves share 16 weight rows and each walks half of the workgroup's K range in steps of one 256-element
-// super-block; per 32-element sub-block one v_mfma_f32_16x16x32_f16 multiplies the 16 (or 32) activation rows with
-// the 16 weight rows: lane l holds the 8 weights k = 8 (l >> 4) .. + 7 of row l & 15, which are 8 consecutive bytes of
-// the block (low nibbles: sub-block 2g, high nibbles: sub-block 2g + 1).  The nibbles are turned into fp16 without a conversion: an integer below 1024 in the low bits
-// of a half IS the subnormal integer * 2^-24.  The 6-bit sub-block scale is multiplied in as an integer
-// (v_pk_mul_lo_u16: 15 * 63 < 1024, still exact), so all eight sub-blocks of a super-block accumulate in one MFMA
-// chain and the fp32 super-block scale d * 2^24 is applied once per step.  The "- dmin * m" term is a second chain on
-// the same activation fragments against fragments that hold the 6-bit min of the sub-block in every element:
-// sum_k x[k] * m[sub(k)], exact for the same reason.  Products and sums are therefore those of the fp32 reference
-// expression (d * sc) * q - dmin * m up to the order of the fp32 additions.
+// super-block.  v_mfma_f32_16x16x32_f16 multiplies the 16 (or 32) activation rows with the 16 weight rows: lane l holds weights
+// of row l & 15, 16 bytes of either half of the quants (32 nibbles of two sub-blocks each).  The nibbles are turned into fp16
+// without a conversion: an integer q in the low bits of a half IS the subnormal q * 2^-24, and four bits up q * 2^-20; the 6-bit
+// scale of the sub-block (for the upper nibbles a sixteenth of it) is multiplied in as fp16, q * sc below 1024 in units of 2^-24, exact.
+// A mask thus takes two weights out of a dword, the eighth byte apart (the activations lie in LDS in that order), and all eight
+// sub-blocks accumulate in one MFMA chain; the fp32 super-block scale d * 2^24 is applied once per step.  The "- dmin * m" term needs
+// only the activations' sums over the sub-blocks: they are formed once, while the activations are staged, as two halves of 11 bits
+// each, and one MFMA multiplies those of a super-block with the eight 6-bit minima.  Products and sums are therefore those of the
+// fp32 reference expression (d * sc) * q - dmin * m up to the order of the fp32 additions: 3e-7 normwise against 64 bits, where a
+// chain of products with the minima, which cancels against the first, had 1e-6 to 3e-6.
 //
 // Activations are staged once per workgroup as fp16 rows in LDS (fp32 inputs rounded to nearest even), row pitch
 // = range + 16 bytes so that the 16 rows of a fragment read hit different banks; the K range of a workgroup is
-// bounded by LDS (132 KB), longer rows are split over workgroups (fp32 partial products, summed by the reduce kernel
+// bounded by LDS (132 KB of activations), longer rows are split over workgroups (fp32 partial products, summed by the reduce kernel
 // of the two-pass GEMM, which applies the epilogue).  After the staging barrier the loop has no barrier: each lane
 // keeps kStreamDepth steps of weight loads in flight in a register ring and waits only for the step it multiplies.
 //
-// Measured (MI355X, HIP-graph replay, Q4_K 14336 x 4096): 15.0 us at 9-16 rows (two passes of the 8-row GEMV: 25),
-// 21 us at 17-32 rows (row-tile matmul: 16, on rounded weights); at 8 rows and fewer the 8-row GEMV is the faster one (13 us):
-// both spend about 0.05 vector instructions per weight on the unpack, which bounds them well before HBM does.
+// Bound by the vector instructions of the unpack and by the staging, well before HBM.  Measured (MI355X, HIP-graph replay, fp16
+// activations): Q4_K 14336 x 4096 at 9 / 16 / 24 / 32 rows 12.5 / 13.1 / 17.0 / 17.9 us (with eight pieces of 8 bytes per lane, integer
+// products and the minima as a second chain of eight products 14.1 / 14.5 / 19.7 / 19.9), 28672 x 4096 22.1 / 23.2 / 28.4 / 30.0
+// (25.3 / 25.9 / 33.7 / 34.1), 2048 x 2048 7.8 / 7.9 / 9.6 / 10.2 (8.8 / 9.1 / 11.0 / 11.2).  A sum per piece as it is staged, every
+// fourth thread storing one, took back 1.5 us of it at 16 rows and 2 at 32: hence four pieces at a time, a sum to every thread.
+// At 8 rows and fewer the 8-row GEMV is as fast for the widest matrices and faster for all others.
 #include <type_traits>
 
 #include "common.hpp"
@@ -50,11 +54,18 @@ typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) uint8_t lds_u8s;
 
 constexpr int kStreamDepth = 2;   // steps of weight loads in flight per lane (waves have 4 to 8 steps: 15.0 us against 16.5 with four)
-constexpr uint32_t kStripBytes = 192 * 16;          // LDS per wave for the blocks of a step
-constexpr uint32_t kStreamLdsMax = 132 * 1024;     // staged activations: 16 rows of 4096 (the strips of eight waves take 24 KB more)
+constexpr uint32_t kStripBytes = 144 * 16;          // LDS per wave for the blocks of a step
+constexpr uint32_t kStreamLdsMax = 132 * 1024;     // staged activations: 16 rows of 4096 (the strips of eight waves and the sums take 26 KB more)
 
-// two 4-bit fields at bits 0 and 16 times a 6-bit scale: no carry between the fields, one full-rate 24-bit multiply
-__device__ __forceinline__ uint32_t pk_mul_u16(uint32_t a, uint32_t b) { return __umul24(a, b); }
+__device__ __forceinline__ half2_t as_pair(uint32_t v) { return __builtin_bit_cast(half2_t, v); }
+__device__ __forceinline__ uint32_t bits(half2_t v) { return __builtin_bit_cast(uint32_t, v); }
+// the value of the lane whose number differs in bit 0 (quad_perm 1 0 3 2) / bit 1 (2 3 0 1)
+__device__ __forceinline__ float lane_xor1(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float lane_xor2(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true));
+}
 __device__ __forceinline__ half8_t as_frag(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
   return __builtin_bit_cast(half8_t, u32x4{a, b, c, d});
 }
@@ -71,7 +82,9 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
   const uint32_t s_lo = split * p.range_steps, nsteps = p.K / 256;
   const uint32_t rcnt = min(p.range_steps, nsteps - s_lo);   // steps of this workgroup; the host launches no empty range
   const uint32_t range_k = rcnt * 256, pitch = range_k * 2 + 16;   // bytes per staged activation row
-  const uint32_t strip0 = 16 * MT * (p.range_steps * 512 + 16);     // the weight strips lie behind the activations
+  // behind the activations: the sums of their sub-blocks, [row][step][lane group][4 halves], then the weight strips
+  const uint32_t sums0 = 16 * MT * (p.range_steps * 512 + 16), spitch = range_k / 8 + 16;
+  const uint32_t strip0 = sums0 + 16 * MT * (p.range_steps * 32 + 16);
   const uint32_t sb = rcnt * kw / KW, cnt = rcnt * (kw + 1) / KW - sb;   // this wave's steps: [sb, sb + cnt) of the range
 
   const uint32_t n = (bid * RG + rg) * 16 + (lane & 15), kq = lane >> 4;
@@ -98,11 +111,12 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
   constexpr int kSB = 16;
   const uint32_t cpr = range_k / 8, chunks = p.M * cpr;   // 8-element pieces per row, in all
   const uint32_t k_lo = s_lo * 256;
+  const uint32_t inv = 0xFFFFFFFFu / cpr + 1;   // c / cpr = c inv >> 32: exact, as c (inv cpr - 2^32) < chunks cpr < 2^32
   u32x4 xa[kSB], xb[kSB];
   auto stage_load = [&](uint32_t base) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kSB; ++i) {
-      const uint32_t c = min(base + (uint32_t)i * THREADS + (uint32_t)tid, chunks - 1), r = c / cpr, col = c - r * cpr;
+      const uint32_t c = min(base + (uint32_t)i * THREADS + (uint32_t)tid, chunks - 1), r = __umulhi(c, inv), col = c - r * cpr;
       const size_t off = (size_t)r * p.strideA + k_lo + col * 8;
       if (p.a_f16) {
         xa[i] = ld_u32x4(reinterpret_cast<const uint8_t *>(p.A) + off * 2);
@@ -112,19 +126,47 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
       }
     }
   };
+  // Four pieces of a thread at a time: four neighbouring threads hold the four pieces of four sub-blocks of 32, and each of
+  // them takes one sub-block's sum
   auto stage_store = [&](uint32_t base) __attribute__((always_inline)) {
+    const half2_t one{(half_t)1.0f, (half_t)1.0f};
+    const bool b0 = tid & 1, b1 = tid & 2;
 #pragma unroll
-    for (int i = 0; i < kSB; ++i) {
-      const uint32_t c = base + (uint32_t)i * THREADS + (uint32_t)tid;
-      if (c < chunks) {
-        const uint32_t r = c / cpr, col = c - r * cpr;
+    for (int i0 = 0; i0 < kSB; i0 += 4) {
+      if (base + (uint32_t)i0 * THREADS >= chunks) break;
+      float sum[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + j;
+        const uint32_t c = base + (uint32_t)i * THREADS + (uint32_t)tid;
         u32x4 o = xa[i];
         if (!p.a_f16) {
           const f32x4 lo = __builtin_bit_cast(f32x4, xa[i]), hi = __builtin_bit_cast(f32x4, xb[i]);
           const half8_t h{(half_t)lo.x, (half_t)lo.y, (half_t)lo.z, (half_t)lo.w, (half_t)hi.x, (half_t)hi.y, (half_t)hi.z, (half_t)hi.w};
           o = __builtin_bit_cast(u32x4, h);
         }
-        *reinterpret_cast<u32x4 *>(lds + (size_t)r * pitch + col * 16) = o;
+        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.x), one, 0.0f, false);
+        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.y), one, sum[j], false);
+        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.z), one, sum[j], false);
+        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.w), one, sum[j], false);
+        if (c < chunks) {
+          const uint32_t r = __umulhi(c, inv), col = c - r * cpr;
+          // elements 0 2 1 3 4 6 5 7, the order in which a mask takes two nibbles out of a dword
+          *reinterpret_cast<u32x4 *>(lds + r * pitch + col * 16) =
+              u32x4{__builtin_amdgcn_perm(o.y, o.x, 0x05040100u), __builtin_amdgcn_perm(o.y, o.x, 0x07060302u),
+                    __builtin_amdgcn_perm(o.w, o.z, 0x05040100u), __builtin_amdgcn_perm(o.w, o.z, 0x07060302u)};
+        }
+      }
+      const float s01 = (b0 ? sum[1] : sum[0]) + lane_xor1(b0 ? sum[0] : sum[1]), s23 = (b0 ? sum[3] : sum[2]) + lane_xor1(b0 ? sum[2] : sum[3]);
+      const float s = ((b1 ? s23 : s01) + lane_xor2(b1 ? s01 : s23)) * 0.03125f;   // of this thread's sub-block, / 32
+      const uint32_t c = base + (uint32_t)(i0 + (tid & 3)) * THREADS + (uint32_t)(tid & ~3);
+      if (c < chunks) {
+        // in two parts of 11 bits: part h of sub-block j of a step to lane group 2 ((j >> 1) & 1) + h
+        const uint32_t r = __umulhi(c, inv), col = c - r * cpr, j = (col >> 2) & 7;
+        half_t *dst = reinterpret_cast<half_t *>(lds + sums0 + r * spitch + (col >> 5) * 32 + 16 * ((j >> 1) & 1)) + 2 * (j >> 2) + (j & 1);
+        const half_t lead = (half_t)s;
+        dst[0] = lead;
+        dst[4] = (half_t)((s - (float)lead) * 2048.0f);
       }
     }
   };
@@ -145,70 +187,73 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
   f32x4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = f32x4{0, 0, 0, 0};
-  // fragment of activation tile t, sub-block s of a step: row 16 t + (lane & 15), k = 32 s + 8 kq .. + 7; rows at
-  // and beyond M hold whatever the LDS held: their products land in accumulator rows that are never stored
-  const lds_u8s *xbase = (const lds_u8s *)(lds) + (size_t)(lane & 15) * pitch + kq * 16;
+  // Lane (n, kq) multiplies bytes 16 kq .. + 15 of each half (64 bytes) of its row's quants: in half t sub-blocks 4 t + 2 p (low
+  // nibbles) and 4 t + 2 p + 1, p = kq >> 1, elements 16 (kq & 1) .. + 15.  Fragment f = 4 t + 2 (high nibbles) + u of activation tile
+  // i: row 16 i + (lane & 15), elements 128 t + 64 p + 32 (high) + 16 (kq & 1) + 8 u .. + 7 of the step; rows at and beyond M
+  // hold whatever the LDS held: their products land in accumulator rows that are never stored
+  const lds_u8s *xbase = (const lds_u8s *)(lds) + (size_t)(lane & 15) * pitch + 128 * (kq >> 1) + 32 * (kq & 1);
+  const lds_u8s *sbase = (const lds_u8s *)(lds) + sums0 + (size_t)(lane & 15) * spitch + 8 * kq;
+  const half_t part = (half_t)(kq & 1 ? 1.0f : 2048.0f);
 
-  // wave-private strip: 144 pieces + the 48 duplicates that the lanes past piece 143 hold (written to the end, never read)
+  // wave-private strip: the 144 pieces of a step
   lds_u8s *strip = (lds_u8s *)(lds) + strip0 + (size_t)wave * kStripBytes;
-  struct Blk { u32x4 hdr; u32x2 q[4]; };   // what a lane multiplies in a step: its row's header, 8 bytes of each group
+  struct Blk { u32x4 hdr, q[2]; };   // what a lane multiplies in a step: its row's header, 16 bytes of each half of the quants
   // pieces of a step -> strip -> the lane's operands (same wave, LDS in order: the strip's earlier reads are done);
   // issuing this a step ahead of the products measured no different
   auto deliver = [&](const Raw &raw, Blk &r) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-      *reinterpret_cast<__attribute__((address_space(3))) u32x4 *>(strip + ((size_t)lane + 64 * j) * 16) = raw.c[j];
+    for (int j = 0; j < 2; ++j) *reinterpret_cast<lds_u32x4 *>(strip + ((size_t)lane + 64 * j) * 16) = raw.c[j];
+    if (lane < 16) *reinterpret_cast<lds_u32x4 *>(strip + ((size_t)lane + 128) * 16) = raw.c[2];
     __builtin_amdgcn_wave_barrier();
     const lds_u8s *blk = strip + (size_t)(lane & 15) * 144;
-    r.hdr = *reinterpret_cast<const __attribute__((address_space(3))) u32x4 *>(blk);
+    r.hdr = *reinterpret_cast<const lds_u32x4 *>(blk);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) r.q[g] = *reinterpret_cast<const __attribute__((address_space(3))) u32x2 *>(blk + 16 + 32 * g + 8 * kq);
+    for (int t = 0; t < 2; ++t) r.q[t] = *reinterpret_cast<const lds_u32x4 *>(blk + 16 + 64 * t + 16 * kq);
     __builtin_amdgcn_wave_barrier();
   };
   auto do_step = [&](const Blk &r, uint32_t step) __attribute__((always_inline)) {
-    const float d = f16bits_to_f32(r.hdr.x & 0xFFFF) * 16777216.0f, dmin = f16bits_to_f32(r.hdr.x >> 16) * 16777216.0f;
-    uint32_t sc4[2], m4[2];
-    q4k_scales(r.hdr.y, r.hdr.z, r.hdr.w, sc4[0], sc4[1], m4[0], m4[1]);
+    // scales and minima of the lane's four sub-blocks: bytes 2 p, 2 p + 1 of either half of the header's 6-bit fields
+    const uint32_t sh = 16 * (kq >> 1), a0 = r.hdr.y >> sh, a1 = r.hdr.z >> sh, a2 = r.hdr.w >> sh;
+    const uint32_t s6[2] = {a0 & 0x3F3Fu, (a2 & 0x0F0Fu) | ((a0 >> 2) & 0x3030u)};
+    const uint32_t m6[2] = {a1 & 0x3F3Fu, ((a2 >> 4) & 0x0F0Fu) | ((a1 >> 2) & 0x3030u)};
+    half2_t sc[2];   // (scale, scale / 16): 1024 + s in the low bits of a half
+    uint32_t mn[2];  // min * 2^-24, or for the leading parts of the sums * 2^-13
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      sc[t] = __builtin_elementwise_fma(as_pair(__builtin_amdgcn_perm(0x64646464u, s6[t], 0x04010400u)), half2_t{(half_t)1.0f, (half_t)0.0625f},
+                                        half2_t{(half_t)-1024.0f, (half_t)-64.0f});
+      mn[t] = bits(as_pair(__builtin_amdgcn_perm(0u, m6[t], 0x0C010C00u)) * half2_t{part, part});
+    }
+    const lds_u8s *xs = xbase + (size_t)(sb + step) * 512, *ss = sbase + (size_t)(sb + step) * 32;
     f32x4 t_main[MT], t_min[MT];
+    const f32x4 zero = {0, 0, 0, 0};
 #pragma unroll
-    for (int t = 0; t < MT; ++t) t_main[t] = t_min[t] = f32x4{0, 0, 0, 0};
-    const lds_u8s *xs = xbase + (size_t)(sb + step) * 512;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      // (scale | scale << 16) and (min | min << 16) of sub-blocks 2g and 2g + 1: byte (2g) & 3 / (2g + 1) & 3 of dword g >> 1
-      const uint32_t scw = sc4[g >> 1], mw = m4[g >> 1];
-      const uint32_t sel0 = (g & 1) ? 0x0c060c06u : 0x0c040c04u, sel1 = (g & 1) ? 0x0c070c07u : 0x0c050c05u;
-      const uint32_t sc0 = (scw >> (16 * (g & 1))) & 0xFFu, sc1 = (scw >> (16 * (g & 1) + 8)) & 0xFFu;
-      const uint32_t mn0 = __builtin_amdgcn_perm(mw, 0, sel0), mn1 = __builtin_amdgcn_perm(mw, 0, sel1);
-      // bytes b0..b3 of a dword -> halves (b0, b1) and (b2, b3), so that the 8 weights stay in the order of k
-      const uint32_t w0 = r.q[g].x, w1 = r.q[g].y;
-      const uint32_t p0 = __builtin_amdgcn_perm(w0, 0, 0x0c050c04u), p1 = __builtin_amdgcn_perm(w0, 0, 0x0c070c06u);
-      const uint32_t p2 = __builtin_amdgcn_perm(w1, 0, 0x0c050c04u), p3 = __builtin_amdgcn_perm(w1, 0, 0x0c070c06u);
-      constexpr uint32_t kNib = 0x000F000Fu;
-      const half8_t lo = as_frag(pk_mul_u16(p0 & kNib, sc0), pk_mul_u16(p1 & kNib, sc0), pk_mul_u16(p2 & kNib, sc0),
-                                 pk_mul_u16(p3 & kNib, sc0));
-      const half8_t hi = as_frag(pk_mul_u16((p0 >> 4) & kNib, sc1), pk_mul_u16((p1 >> 4) & kNib, sc1),
-                                 pk_mul_u16((p2 >> 4) & kNib, sc1), pk_mul_u16((p3 >> 4) & kNib, sc1));
-      const half8_t mlo = as_frag(mn0, mn0, mn0, mn0), mhi = as_frag(mn1, mn1, mn1, mn1);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const lds_u8s *xt = xs + (size_t)t * 16 * pitch + g * 128;
-        const half8_t x0 = *reinterpret_cast<const __attribute__((address_space(3))) half8_t *>(xt);
-        const half8_t x1 = *reinterpret_cast<const __attribute__((address_space(3))) half8_t *>(xt + 64);
-        t_main[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x0, lo, t_main[t], 0, 0, 0);
-        t_min[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x0, mlo, t_min[t], 0, 0, 0);
-        t_main[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x1, hi, t_main[t], 0, 0, 0);
-        t_min[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x1, mhi, t_min[t], 0, 0, 0);
-      }
+    for (int i = 0; i < MT; ++i) {
+      const u32x2 x = *reinterpret_cast<const __attribute__((address_space(3))) u32x2 *>(ss + (size_t)i * 16 * spitch);
+      t_min[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_frag(x.x, x.y, 0, 0), as_frag(mn[0], mn[1], 0, 0), zero, 0, 0, 0);
     }
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int f = 0; f < 8; ++f) {
+      // nibbles of bits 0-3 are q 2^-24, of bits 4-7 q 2^-20; times the scale (scale / 16) an integer below 1024 times 2^-24
+      const uint32_t mask = f & 2 ? 0x00F000F0u : 0x000F000Fu;
+      const half_t k = sc[f >> 2][(f >> 1) & 1];
+      const uint32_t w0 = r.q[f >> 2][2 * (f & 1)], w1 = r.q[f >> 2][2 * (f & 1) + 1];
+      const half2_t kk{k, k};
+      const half8_t w = as_frag(bits(as_pair(w0 & mask) * kk), bits(as_pair((w0 >> 8) & mask) * kk), bits(as_pair(w1 & mask) * kk), bits(as_pair((w1 >> 8) & mask) * kk));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[t][e] = fmaf(d, t_main[t][e], acc[t][e]);
-        acc[t][e] = fmaf(-dmin, t_min[t][e], acc[t][e]);
+      for (int i = 0; i < MT; ++i) {
+        const half8_t x = *reinterpret_cast<const __attribute__((address_space(3))) half8_t *>(xs + (size_t)i * 16 * pitch + 256 * (f >> 2) + 64 * ((f >> 1) & 1) + 16 * (f & 1));
+        t_main[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, w, f == 0 ? zero : t_main[i], 0, 0, 0);
       }
+    }
+    // the sums are of x / 32, in units of 2^-13
+    const float d = f16bits_to_f32(r.hdr.x & 0xFFFF) * 16777216.0f, dmin = f16bits_to_f32(r.hdr.x >> 16) * 262144.0f;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(-dmin, t_min[i][e], fmaf(d, t_main[i][e], acc[i][e]));
   };
 
   // Ring slot i % D holds the pieces of step i.  Every refill is issued, past the end of the range at the range's
@@ -267,8 +312,8 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
 // activations), more while the grid has fewer workgroups than CUs and a range keeps at least 8 steps
 // (and the scratch memory holds the partial products of twice as many)
 // Weight rows per workgroup: 64 (four row groups, two waves each), or with two activation tiles 128 (eight row groups
-// of one wave: half as many workgroups stage the activations; 14336 x 4096 at 32 rows 21 us against 26) wherever that
-// still leaves a workgroup for every second CU (4096 x 4096: 18 us against 14 otherwise)
+// of one wave: half as many workgroups stage the activations; 14336 x 4096 at 32 rows 17.9 us) wherever that
+// still leaves a workgroup for every second CU (4096 x 4096 at 32 rows: 12.6 us with 64)
 static uint32_t stream_block_rows(uint32_t M, uint32_t K, uint32_t N) {
   if (M <= 16) return 64;
   const uint32_t ks_lds = (K / 256 + 7) / 8;   // ranges of at most eight steps with 32 staged rows
@@ -316,7 +361,7 @@ int launch_stream_gemm(const void *W, const void *A, int a_f16, void *C, int c_f
     return CUTHIP_ERR_INVALID;
   }
   const uint32_t mt = (M + 15) / 16;
-  const size_t lds = (size_t)16 * mt * ((size_t)p.range_steps * 512 + 16) + 8 * kStripBytes;
+  const size_t lds = (size_t)16 * mt * ((size_t)p.range_steps * 544 + 32) + 8 * kStripBytes;
   // four row groups: two waves each once a wave keeps at least two steps
   const bool two = block_rows == 64 && p.range_steps >= 4;
   auto kern = block_rows == 128 ? gemm_stream_q4k_kernel<2, 1, 8>

@@ -392,6 +392,27 @@ def test_streaming_mfma_matmul(ops, M, N, K):
         assert normwise_rel_err(alone.cpu().numpy(), want) < TOL_F16_ACT
 
 
+@pytest.mark.parametrize("M,K", [(1, 256), (9, 4096), (16, 4352), (17, 2048), (31, 2304), (32, 4096)])
+@pytest.mark.parametrize("scale", [1e-4, 1.0, 2000.0])
+def test_streaming_mfma_matmul_minima_do_not_cancel(ops, M, K, scale):
+    """The minima of variant 6 come from sums of the staged activations: rows that all lean to one side, so that the minima's
+    term is as large as the products', with fp16 subnormals among them or sums beyond fp16's range, and ragged N.  Exact
+    products, sums of 22 bits: the error stays below 2^-21 of the two terms (2^-22 of the sums' split, as much again for
+    the fp32 additions)."""
+    N, fmt = 83, oracle.Q4_K
+    W = quantized_weights(fmt, N, K, seed=M + K)
+    A = (np.abs(gauss_acts((M, K), seed=M + 7)) * scale).astype(np.float16)
+    ws = ops.matmul_gguf_workspace(fmt, M, K, N, torch.float16, "cuda")
+    got = ops.matmul_gguf(torch.from_numpy(A).cuda(), torch.from_numpy(W).cuda(), fmt, N, K, out_dtype=torch.float32, workspace=ws, variant=6)
+    torch.cuda.synchronize()
+    w = oracle.dequant(fmt, W, N * K).reshape(N, K).astype(np.float64)
+    want = A.astype(np.float64) @ w.T
+    b = W.reshape(N, K // 256, 144)
+    dmin = b[:, :, 2:4].copy().view(np.float16)[:, :, 0].astype(np.float64)
+    size = (A.astype(np.float64).sum(1)[:, None] * 63 * np.abs(dmin).max(1)[None]) + A.astype(np.float64) @ np.abs(w).T
+    assert (np.abs(got.cpu().numpy() - want) <= 2.0 ** -21 * size).all()
+
+
 def test_streaming_mfma_matmul_refusals(ops):
     from cut_amd import lib
     K, N = 512, 64
