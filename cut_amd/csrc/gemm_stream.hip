@@ -1,10 +1,10 @@
-// Streaming matmul on Q4_K blocks for a handful of activation rows (5 <= M <= 32):
+// Streaming matmul on Q4_K and Q8_0 blocks for a handful of activation rows (M <= 32):
 //   C[m,n] = sum_k A[m,k] * dequant(W)[n,k]
 // between the 8-row GEMV (whose matrix-core path spends three quarters of every product on mismatched pieces)
 // and the row-tile matmul (which rounds every weight to fp16).
 // Supersedes MatMulQ4GemvKPar8.cu / MatMulQ4TiledReg.cu (operators/impl/matmul) at these batch sizes.
 //
-// Two waves share 16 weight rows and each walks half of the workgroup's K range in steps of one 256-element
+// Q4_K.  Two waves share 16 weight rows and each walks half of the workgroup's K range in steps of one 256-element
 // super-block.  v_mfma_f32_16x16x32_f16 multiplies the 16 (or 32) activation rows with the 16 weight rows: lane l holds weights
 // of row l & 15, 16 bytes of either half of the quants (32 nibbles of two sub-blocks each).  The nibbles are turned into fp16
 // without a conversion: an integer q in the low bits of a half IS the subnormal q * 2^-24, and four bits up q * 2^-20; the 6-bit
@@ -15,6 +15,10 @@
 // each, and one MFMA multiplies those of a super-block with the eight 6-bit minima.  Products and sums are therefore those of the
 // fp32 reference expression (d * sc) * q - dmin * m up to the order of the fp32 additions: 3e-7 normwise against 64 bits, where a
 // chain of products with the minima, which cancels against the first, had 1e-6 to 3e-6.
+//
+// Q8_0.  A step is eight blocks of 34 bytes.  Lane l holds bytes 8 (l >> 4) .. + 7 of a block, as the halves 1024 + (q + 128) less 1152,
+// one MFMA multiplies a block, and its four sums are scaled by the block's fp32 d: again the reference's expression, 1e-7 to 3e-7
+// against 64 bits (the row-tile matmul, on d q rounded to fp16: 2e-4).
 //
 // Activations are staged once per workgroup as fp16 rows in LDS (fp32 inputs rounded to nearest even), row pitch
 // = range + 16 bytes so that the 16 rows of a fragment read hit different banks; the K range of a workgroup is
@@ -27,7 +31,9 @@
 // products and the minima as a second chain of eight products 14.1 / 14.5 / 19.7 / 19.9), 28672 x 4096 22.1 / 23.2 / 28.4 / 30.0
 // (25.3 / 25.9 / 33.7 / 34.1), 2048 x 2048 7.8 / 7.9 / 9.6 / 10.2 (8.8 / 9.1 / 11.0 / 11.2).  A sum per piece as it is staged, every
 // fourth thread storing one, took back 1.5 us of it at 16 rows and 2 at 32: hence four pieces at a time, a sum to every thread.
-// At 8 rows and fewer the 8-row GEMV is as fast for the widest matrices and faster for all others.
+// Q8_0 14336 x 4096 at 8 / 16 / 24 / 32 rows 17.4 / 18.0 / 22.0 / 22.6 us (8-row GEMV 19.8, row-tile matmul 22.7 / 22.6 / 23.0),
+// 4096 x 14336 19.6 / 20.1 / 22.2 / 22.7 (21.6; 22.6 / 23.1 / 23.8), 28672 x 4096 at 8 / 16 rows 34.2 / 34.8 (37.9; 37.3).
+// Q4_K at 8 rows and fewer: the 8-row GEMV is as fast for the widest matrices and faster for all others.
 #include <type_traits>
 
 #include "common.hpp"
@@ -73,18 +79,20 @@ __device__ __forceinline__ half8_t as_frag(uint32_t a, uint32_t b, uint32_t c, u
 // MT: activation tiles of 16 rows (1 or 2); RG: groups of 16 weight rows per workgroup; KW: waves that share a group,
 // each on its own part of the steps.  RG x KW = 8 waves wherever the range is long enough (two waves per SIMD: one
 // wave alone cannot hide its own LDS and matrix-core latencies).
-template <int MT, int KW, int RG>
-__global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamParams p) {
+template <int FMT, int MT, int KW, int RG>
+__global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int D = kStreamDepth, THREADS = 64 * RG * KW;
+  constexpr bool Q4K = FMT == CUTHIP_Q4_K;
+  constexpr int NP = Q4K ? 3 : 5;   // 16-byte pieces per lane and step
   const uint32_t split = blockIdx.x / p.nblocks, bid = blockIdx.x - split * p.nblocks;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rg = wave % RG, kw = wave / RG;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), rg = wave % RG, kw = wave / RG;
   const uint32_t s_lo = split * p.range_steps, nsteps = p.K / 256;
   const uint32_t rcnt = min(p.range_steps, nsteps - s_lo);   // steps of this workgroup; the host launches no empty range
   const uint32_t range_k = rcnt * 256, pitch = range_k * 2 + 16;   // bytes per staged activation row
   // behind the activations: the sums of their sub-blocks, [row][step][lane group][4 halves], then the weight strips
   const uint32_t sums0 = 16 * MT * (p.range_steps * 512 + 16), spitch = range_k / 8 + 16;
-  const uint32_t strip0 = sums0 + 16 * MT * (p.range_steps * 32 + 16);
+  const uint32_t strip0 = sums0 + (Q4K ? 16 * MT * (p.range_steps * 32 + 16) : 0);
   const uint32_t sb = rcnt * kw / KW, cnt = rcnt * (kw + 1) / KW - sb;   // this wave's steps: [sb, sb + cnt) of the range
 
   const uint32_t n = (bid * RG + rg) * 16 + (lane & 15), kq = lane >> 4;
@@ -94,16 +102,21 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
   // once.  (Fetched in the operand layout - 8 bytes per lane, the four lanes of a row 16 lanes apart - every line
   // was requested four times: 17.6 us against 15.7 for 14336 x 4096 at 16 rows.)  The pieces go through a wave-private
   // strip of LDS, from which each lane picks its row's header and its 8 bytes of every 32-byte group.
-  const uint8_t *piece[3];
+  // Q8_0 (17 pieces a row): parts 0-7, parts 9-16 and, by 16 lanes, part 8 of every row, as the strip holds half a step at a time.
+  constexpr uint32_t kStepBytes = Q4K ? 144 : 272;
+  const uint8_t *piece[NP];
+  uint32_t slot[NP];   // where the piece goes in the strip: 144 bytes a row
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    const uint32_t c = min((uint32_t)lane + 64u * j, 143u), r = c / 9, part = c - 9 * r;
-    piece[j] = p.W + (size_t)min((bid * RG + rg) * 16 + r, p.N - 1) * p.row_bytes + (size_t)(s_lo + sb) * 144 + 16 * part;
+  for (int j = 0; j < NP; ++j) {
+    const uint32_t c = min((uint32_t)lane + 64u * j, Q4K ? 143u : 271u);
+    const uint32_t r = Q4K ? c / 9 : j < 4 ? c / 8 % 16 : c - 256, part = Q4K ? c - 9 * r : j < 4 ? c % 8 + (j < 2 ? 0 : 9) : 8;
+    piece[j] = p.W + (size_t)min((bid * RG + rg) * 16 + r, p.N - 1) * p.row_bytes + (size_t)(s_lo + sb) * kStepBytes + 16 * part;
+    slot[j] = r * 144 + 16 * (part < 9 ? part : part - 8);
   }
-  struct Raw { u32x4 c[3]; };
+  struct Raw { u32x4 c[NP]; };
   auto load = [&](Raw &r, uint32_t step) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 3; ++j) r.c[j] = ld_u32x4(piece[j] + (size_t)step * 144);
+    for (int j = 0; j < NP; ++j) r.c[j] = ld_u32x4(piece[j] + (size_t)step * kStepBytes);
   };
 
   // activations first (they must not queue behind the weight loads), in batches of kSB 16-byte pieces per thread;
@@ -145,18 +158,21 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
           const half8_t h{(half_t)lo.x, (half_t)lo.y, (half_t)lo.z, (half_t)lo.w, (half_t)hi.x, (half_t)hi.y, (half_t)hi.z, (half_t)hi.w};
           o = __builtin_bit_cast(u32x4, h);
         }
-        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.x), one, 0.0f, false);
-        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.y), one, sum[j], false);
-        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.z), one, sum[j], false);
-        sum[j] = __builtin_amdgcn_fdot2(as_pair(o.w), one, sum[j], false);
+        if (Q4K) {
+          sum[j] = __builtin_amdgcn_fdot2(as_pair(o.x), one, 0.0f, false);
+          sum[j] = __builtin_amdgcn_fdot2(as_pair(o.y), one, sum[j], false);
+          sum[j] = __builtin_amdgcn_fdot2(as_pair(o.z), one, sum[j], false);
+          sum[j] = __builtin_amdgcn_fdot2(as_pair(o.w), one, sum[j], false);
+        }
         if (c < chunks) {
           const uint32_t r = __umulhi(c, inv), col = c - r * cpr;
-          // elements 0 2 1 3 4 6 5 7, the order in which a mask takes two nibbles out of a dword
-          *reinterpret_cast<u32x4 *>(lds + r * pitch + col * 16) =
+          // Q4_K: elements 0 2 1 3 4 6 5 7, the order in which a mask takes two nibbles out of a dword
+          *reinterpret_cast<u32x4 *>(lds + r * pitch + col * 16) = !Q4K ? o :
               u32x4{__builtin_amdgcn_perm(o.y, o.x, 0x05040100u), __builtin_amdgcn_perm(o.y, o.x, 0x07060302u),
                     __builtin_amdgcn_perm(o.w, o.z, 0x05040100u), __builtin_amdgcn_perm(o.w, o.z, 0x07060302u)};
         }
       }
+      if (!Q4K) continue;
       const float s01 = (b0 ? sum[1] : sum[0]) + lane_xor1(b0 ? sum[0] : sum[1]), s23 = (b0 ? sum[3] : sum[2]) + lane_xor1(b0 ? sum[2] : sum[3]);
       const float s = ((b1 ? s23 : s01) + lane_xor2(b1 ? s01 : s23)) * 0.03125f;   // of this thread's sub-block, / 32
       const uint32_t c = base + (uint32_t)(i0 + (tid & 3)) * THREADS + (uint32_t)(tid & ~3);
@@ -256,6 +272,56 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
       for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(-dmin, t_min[i][e], fmaf(d, t_main[i][e], acc[i][e]));
   };
 
+  // Q8_0, half a step (four blocks of 34 bytes) at a time: the first half lies in parts 0-8 of a row, the second 8 bytes into parts 8-16.
+  // Lane (n, kq) multiplies bytes 8 kq .. + 7 of every block with elements 32 b + 8 kq .. + 7 of the step.
+  auto q8_step = [&](const Raw &raw, uint32_t step) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    const lds_u8s *xs = (const lds_u8s *)(lds) + (size_t)(lane & 15) * pitch + 16 * kq + (size_t)(sb + step) * 512;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 2; ++j) *reinterpret_cast<lds_u32x4 *>(strip + slot[2 * h + j]) = raw.c[2 * h + j];
+      if (lane < 16) *reinterpret_cast<lds_u32x4 *>(strip + slot[NP - 1] - 128 * h) = raw.c[NP - 1];
+      __builtin_amdgcn_wave_barrier();
+      uint32_t q[4][3];
+      float d[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const lds_u8s *blk = strip + (size_t)(lane & 15) * 144 + 8 * h + 34 * b;
+        d[b] = f16bits_to_f32(*reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>(blk));
+        // the quants begin two bytes into a dword in the even blocks
+#pragma unroll
+        for (int w = 0; w < (b & 1 ? 2 : 3); ++w) q[b][w] = *reinterpret_cast<const lds_u32 *>(blk + (b & 1 ? 2 : 0) + 8 * kq + 4 * w);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        // a byte q + 128 below 0x64 is the half 1024 + q + 128
+        const half2_t bias{(half_t)-1152.0f, (half_t)-1152.0f};
+        uint32_t u[3];
+#pragma unroll
+        for (int w = 0; w < (b & 1 ? 2 : 3); ++w) u[w] = q[b][w] ^ 0x80808080u;
+        uint32_t f[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t w = b & 1 ? u[k / 2] : u[(k + 1) / 2];
+          const bool upper = b & 1 ? k & 1 : !(k & 1);
+          f[k] = bits(as_pair(__builtin_amdgcn_perm(0x64646464u, w, upper ? 0x04030402u : 0x04010400u)) + bias);
+        }
+        const half8_t w = as_frag(f[0], f[1], f[2], f[3]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const half8_t x = *reinterpret_cast<const __attribute__((address_space(3))) half8_t *>(xs + (size_t)i * 16 * pitch + 256 * h + 64 * b);
+          const f32x4 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, w, f32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(d[b], t[e], acc[i][e]);
+        }
+      }
+    }
+  };
+
   // Ring slot i % D holds the pieces of step i.  Every refill is issued, past the end of the range at the range's
   // last step again (a few redundant loads of valid memory): with no load under a condition the compiler counts the
   // loads in flight exactly and every step waits for its own pieces only, also in ranges shorter than 2 D steps.
@@ -265,9 +331,13 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
     for (int u = 0; u < D; ++u) {
       const uint32_t i = i0 + u;
       if (i < cnt) {           // uniform; no global load inside
-        Blk blk;
-        deliver(buf[u], blk);
-        do_step(blk, i);
+        if constexpr (Q4K) {
+          Blk blk;
+          deliver(buf[u], blk);
+          do_step(blk, i);
+        } else {
+          q8_step(buf[u], i);
+        }
       }
       load(buf[u], min(i + D, last));
       __builtin_amdgcn_sched_barrier(0);
@@ -294,7 +364,17 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
         for (int e = 0; e < 4; ++e) acc[t][e] += red[((size_t)(w - 1) * RG * 64 * MT * 4) + (t * 4 + e) * 64];
   }
   // accumulator register e of lane l, tile t: row 16 t + 4 (l >> 4) + e, column (weight row) n
-  if (n < p.N) {
+  if (p.epi.kind == CUTHIP_EPI_SWIGLU_PAIRS) {   // (never with several K ranges) gate in the even weight rows, up in the odd ones
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t m = 16 * t + 4 * kq + e;
+        const float up = lane_xor1(acc[t][e]);
+        if ((n & 1) == 0 && n + 1 < p.N && m < p.M)
+          store_plain(p.C, p.c_f16, (size_t)m * p.strideC + n / 2, apply_unary(CUTHIP_UNARY_SILU, acc[t][e]) * up);
+      }
+  } else if (n < p.N) {
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -309,8 +389,11 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_q4k_kernel(StreamPar
 }
 
 // K ranges of the streaming kernel: as few as LDS allows (one range of up to kStreamLdsMax bytes of staged
-// activations), more while the grid has fewer workgroups than CUs and a range keeps at least 8 steps
-// (and the scratch memory holds the partial products of twice as many)
+// activations), more while the grid has fewer workgroups than CUs and a range keeps at least 8 steps, or 4 where the workgroups
+// still run at once (Q4_K at 16 / 32 rows, one range in the place of two: 4096 x 4096 10.3 / 12.4 us and 9.4 / 10.7, 2048 x 8192 10.3 / 12.4 and
+// 9.4 / 10.8; of eight steps in all only with two activation tiles: 4096 x 2048 8.0 / 10.0 and 8.4 / 9.7), and the scratch memory
+// holds the partial products of twice as many.  (A workgroup that stages one range after the other, without partial
+// products, needs the registers of the staging beside those of the loop: 35.9 us against 30.0 for 28672 x 4096 at 32 rows.)
 // Weight rows per workgroup: 64 (four row groups, two waves each), or with two activation tiles 128 (eight row groups
 // of one wave: half as many workgroups stage the activations; 14336 x 4096 at 32 rows 17.9 us) wherever that
 // still leaves a workgroup for every second CU (4096 x 4096 at 32 rows: 12.6 us with 64)
@@ -323,14 +406,26 @@ static void stream_layout(uint32_t M, uint32_t K, uint32_t N, size_t scratch_byt
   const uint32_t mt = (M + 15) / 16, nsteps = K / 256, nblocks = (N + stream_block_rows(M, K, N) - 1) / stream_block_rows(M, K, N);
   const uint32_t max_steps = (kStreamLdsMax / (16 * mt) - 16) / 512;
   uint32_t ks = (nsteps + max_steps - 1) / max_steps;
-  while (ks < 16 && nblocks * ks < 192 && nsteps / (2 * ks) >= 8 && scratch_bytes >= (size_t)2 * ks * M * N * sizeof(float)) ks *= 2;
+  auto more = [&] {
+    const uint32_t steps = nsteps / (2 * ks), blocks = nblocks * ks;
+    return (blocks < 192 && steps >= 8) || (2 * blocks <= 256 && steps >= 4 && (mt == 2 || nsteps >= 16));
+  };
+  while (ks < 16 && more() && scratch_bytes >= (size_t)2 * ks * M * N * sizeof(float)) ks *= 2;
   *range_steps = (nsteps + ks - 1) / ks;
   *ksplit = (nsteps + *range_steps - 1) / *range_steps;
 }
 
+// workgroups and K ranges of a launch with this much scratch memory
+uint32_t stream_gemm_grid(uint32_t M, uint32_t K, uint32_t N, size_t scratch_bytes, uint32_t *ksplit) {
+  uint32_t rs;
+  stream_layout(M, K, N, scratch_bytes, &rs, ksplit);
+  const uint32_t rows = stream_block_rows(M, K, N);
+  return (N + rows - 1) / rows * *ksplit;
+}
+
 bool stream_gemm_fits(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A) {
   const size_t asz = a_f16 ? 2 : 4;
-  return fmt == CUTHIP_Q4_K && M >= 1 && M <= 32 && K % 256 == 0 && K >= 256 && (uintptr_t)A % 16 == 0 && (strideA * asz) % 16 == 0 &&
+  return (fmt == CUTHIP_Q4_K || fmt == CUTHIP_Q8_0) && M >= 1 && M <= 32 && K % 256 == 0 && K >= 256 && (uintptr_t)A % 16 == 0 && (strideA * asz) % 16 == 0 &&
          (uint64_t)M * N < 0x7FFFFFFFull;
 }
 // bytes of scratch the launch cannot do without (0: the K range of a workgroup may cover all of K)
@@ -340,7 +435,14 @@ size_t stream_gemm_scratch(uint32_t M, uint32_t K, uint32_t N) {
   return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
 }
 
-int launch_stream_gemm(const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
+template <int FMT>
+static auto stream_kernel(uint32_t mt, uint32_t block_rows, bool two) {
+  return block_rows == 128 ? gemm_stream_kernel<FMT, 2, 1, 8>
+         : mt == 1 ? (two ? gemm_stream_kernel<FMT, 1, 2, 4> : gemm_stream_kernel<FMT, 1, 1, 4>)
+                   : (two ? gemm_stream_kernel<FMT, 2, 2, 4> : gemm_stream_kernel<FMT, 2, 1, 4>);
+}
+
+int launch_stream_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
                        uint32_t strideA, uint32_t strideC, Epilogue epi, void *scratch, size_t scratch_bytes, hipStream_t stream) {
   StreamParams p;
   p.W = reinterpret_cast<const uint8_t *>(W);
@@ -348,7 +450,7 @@ int launch_stream_gemm(const void *W, const void *A, int a_f16, void *C, int c_f
   p.C = C;
   p.epi = epi;
   p.M = M; p.K = K; p.N = N; p.strideA = strideA; p.strideC = strideC;
-  p.row_bytes = K / 256 * 144;
+  p.row_bytes = K / 256 * (fmt == CUTHIP_Q4_K ? 144 : 272);
   p.a_f16 = a_f16; p.c_f16 = c_f16;
   const uint32_t block_rows = stream_block_rows(M, K, N);
   p.nblocks = (N + block_rows - 1) / block_rows;
@@ -364,9 +466,7 @@ int launch_stream_gemm(const void *W, const void *A, int a_f16, void *C, int c_f
   const size_t lds = (size_t)16 * mt * ((size_t)p.range_steps * 544 + 32) + 8 * kStripBytes;
   // four row groups: two waves each once a wave keeps at least two steps
   const bool two = block_rows == 64 && p.range_steps >= 4;
-  auto kern = block_rows == 128 ? gemm_stream_q4k_kernel<2, 1, 8>
-              : mt == 1 ? (two ? gemm_stream_q4k_kernel<1, 2, 4> : gemm_stream_q4k_kernel<1, 1, 4>)
-                        : (two ? gemm_stream_q4k_kernel<2, 2, 4> : gemm_stream_q4k_kernel<2, 1, 4>);
+  auto kern = fmt == CUTHIP_Q4_K ? stream_kernel<CUTHIP_Q4_K>(mt, block_rows, two) : stream_kernel<CUTHIP_Q8_0>(mt, block_rows, two);
   const uint32_t threads = block_rows == 128 || two ? 512 : 256;
   if (lds > 64 * 1024) {
     if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -141,7 +141,8 @@ int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C,
                       int use_blaslt);
 bool stream_gemm_fits(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A);
 size_t stream_gemm_scratch(uint32_t M, uint32_t K, uint32_t N);
-int launch_stream_gemm(const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
+uint32_t stream_gemm_grid(uint32_t M, uint32_t K, uint32_t N, size_t scratch_bytes, uint32_t *ksplit);
+int launch_stream_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
                        uint32_t strideA, uint32_t strideC, Epilogue epi, void *scratch, size_t scratch_bytes, hipStream_t stream);
 bool blaslt_available();
 size_t dense_f16_workspace(uint32_t M, uint32_t K, uint32_t N, int a_f16);
@@ -270,12 +271,30 @@ static int check_matmul_args(int fmt, const void *W, const void *A, int a_dtype,
   return 0;
 }
 
-static bool stream_preferred(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A,
+static bool stream_preferred(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A, int epilogue,
                              const void *scratch, size_t scratch_bytes) {
-  // (few weight rows: too few workgroups for it; 1024 x 4096 at 16-32 rows 11.6-13.3 us against 8.2-8.4 for the row-tile matmul)
-  if (M < 9 || M > 32 || N < 2048 || !cuthip::stream_gemm_fits(fmt, M, K, N, strideA, a_f16, A)) return false;
-  const size_t need = cuthip::stream_gemm_scratch(M, K, N);
-  return need == 0 || (scratch && (uintptr_t)scratch % 16 == 0 && scratch_bytes >= need);
+  if (!scratch || (uintptr_t)scratch % 16 != 0) scratch_bytes = 0;
+  if (M > 32 || !cuthip::stream_gemm_fits(fmt, M, K, N, strideA, a_f16, A)) return false;
+  if (fmt == CUTHIP_Q8_0) {
+    // us, this kernel and the one before it.  Up to 8 rows in place of the 8-row GEMV, which keeps fp32 activations: 8 x 14336 x 4096
+    // 17.4 / 19.8, 8 x 4096 x 14336 19.6 / 21.6, 8 x 4096 x 11264 19.1 / 18.4, 4 x 14336 x 4096 17.2 / 18.6 but 1 x 28672 x 4096 33.0 / 29.8.
+    // 9 rows and more in place of the row-tile matmul (not of 8-row passes with fp32 activations): 16 x 4096 x 4096 11.1 / 11.8,
+    // 16 x 2048 x 2048 9.1 / 9.0; with two activation tiles wherever its workgroups run at once: 32 x 11264 x 2048 13.2 / 13.6,
+    // 32 x 8192 x 8192 23.4 / 26.0, 32 x 4096 x 4096 12.6 / 12.2; 32 x 18432 x 4096 (288 workgroups) 35.8 / 33.1.
+    const uint64_t weights = (uint64_t)N * K;
+    uint32_t ksplit;
+    const uint32_t grid = cuthip::stream_gemm_grid(M, K, N, scratch_bytes, &ksplit);
+    if (M <= 8) {
+      if (!a_f16 || M < 5 || weights < 50000000 || (epilogue == CUTHIP_EPI_SWIGLU_PAIRS && ksplit > 1)) return false;
+    } else {
+      if (weights < (M > 16 ? 22000000 : 16000000) || (M > 16 && grid > 256)) return false;
+      if (!a_f16 && passes_preferred(fmt, M, K, N, scratch, scratch_bytes)) return false;
+    }
+  } else if (M < 9 || N < 2048) {
+    // (few weight rows: too few workgroups for it; 1024 x 4096 at 16-32 rows 11.6-13.3 us against 8.2-8.4 for the row-tile matmul)
+    return false;
+  }
+  return cuthip::stream_gemm_scratch(M, K, N) <= scratch_bytes;
 }
 
 // cuthip_matmul_gguf with optional scratch memory (the workspace of cuthip_matmul_gguf_ws, or none): the row-tile matmul
@@ -320,17 +339,17 @@ static int matmul_gguf_scratch(int fmt, const void *W, const void *A, int a_dtyp
   }
   // the table's default entry is valid for every M: beyond the 8 rows its GEMV takes it is the choice by shape
   if (variant == 0 && M > 8) variant = -1;
-  // 9-32 rows on Q4_K: the streaming MFMA kernel (9-16 rows of 14336 x 4096: 15.8 us against 25 for two 8-row passes,
-  // and like them on weights that are not rounded), wherever the scratch memory it needs for long rows or two activation
+  // up to 32 rows on Q4_K and Q8_0: the streaming MFMA kernel (Q4_K, 9-16 rows of 14336 x 4096: 13 us against 25 for two 8-row
+  // passes, and like them on weights that are not rounded), where it is the faster one and the scratch memory it needs for long rows or two activation
   // tiles is at hand
-  if (variant == -1 && stream_preferred(fmt, M, K, N, strideA, a_dtype == CUTHIP_F16, A, scratch, scratch_bytes)) variant = 6;
-  // variant 6: the streaming MFMA kernel (Q4_K, up to 32 rows); scratch only where K has to be split over workgroups
-  if (variant == 6) {
-    if (!stream_gemm_fits(fmt, M, K, N, strideA, a_dtype == CUTHIP_F16, A)) {
+  const bool stream_mfma = variant == 6 || (variant == -1 && stream_preferred(fmt, M, K, N, strideA, a_dtype == CUTHIP_F16, A, epilogue, scratch, scratch_bytes));
+  // asked for by number it takes Q4_K only; scratch only where K has to be split over workgroups
+  if (stream_mfma) {
+    if ((variant == 6 && fmt != CUTHIP_Q4_K) || !stream_gemm_fits(fmt, M, K, N, strideA, a_dtype == CUTHIP_F16, A)) {
       set_error("cuthip_matmul_gguf: variant 6 takes Q4_K, M <= 32 and 16-byte aligned rows of A (fmt %d, M %u, K %u)", fmt, M, K);
       return CUTHIP_ERR_INVALID;
     }
-    return launch_stream_gemm(W, A, a_dtype == CUTHIP_F16, C, c_dtype == CUTHIP_F16, M, K, N, strideA, strideC, epi, scratch,
+    return launch_stream_gemm(fmt, W, A, a_dtype == CUTHIP_F16, C, c_dtype == CUTHIP_F16, M, K, N, strideA, strideC, epi, scratch,
                               scratch_bytes, reinterpret_cast<hipStream_t>(stream));
   }
   // 9-40 rows, automatic choice: passes of 8 rows through the decode kernels
@@ -653,8 +672,8 @@ int cuthip_matmul_gguf_ws(int fmt, const void *W, const void *A, int a_dtype, vo
                                 reinterpret_cast<hipStream_t>(stream));
   }
   const int a_f16 = a_dtype == CUTHIP_F16;
-  if (variant == -1 && stream_preferred(fmt, M, K, N, strideA, a_f16, A, workspace, workspace ? workspace_bytes : 0))
-    return matmul_gguf_scratch(fmt, W, A, a_dtype, C, c_dtype, M, K, N, strideA, strideC, epilogue, epilogue_op, D, 6, stream,
+  if (variant == -1 && stream_preferred(fmt, M, K, N, strideA, a_f16, A, epilogue, workspace, workspace ? workspace_bytes : 0))
+    return matmul_gguf_scratch(fmt, W, A, a_dtype, C, c_dtype, M, K, N, strideA, strideC, epilogue, epilogue_op, D, -1, stream,
                                workspace, workspace_bytes);
   // Beyond 8 rows, with a workspace at hand: 8-row passes up to the line of precision of dense_line_us; else the cheaper of the
   // two-pass path and one launch on the blocks (both on weights rounded to fp16: 40 x 2048 x 512 on Q8_0 12.7 us and 6.3, 40 x 16384 x 512 22.7 and 7.6).

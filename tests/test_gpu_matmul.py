@@ -413,6 +413,28 @@ def test_streaming_mfma_matmul_minima_do_not_cancel(ops, M, K, scale):
     assert (np.abs(got.cpu().numpy() - want) <= 2.0 ** -21 * size).all()
 
 
+@pytest.mark.parametrize("M,N,K,pairs", [(5, 12290, 4096, True), (8, 3500, 14336, False), (9, 3910, 4096, False), (16, 1200, 14336, False),
+                                         (17, 5450, 4352, False), (32, 10800, 2048, False), (31, 4131, 8192, False)])
+def test_streaming_q8_0_matmul(ops, M, N, K, pairs):
+    """The streaming kernel on Q8_0, as the automatic choice takes it for large matrices: one and two activation tiles, ragged N,
+    one K range and several of unequal length, the SwiGLU row pairs.  Products of int8 and fp16 are exact in fp32, so the bound
+    is that of the fp32 additions (the row-tile matmul, on weights rounded to fp16, is 2e-4 off)."""
+    fmt = oracle.Q8_0
+    W = finite_random_blocks(fmt, N * K // 32, seed=N + K).reshape(-1, 34)
+    W[:, :2] = np.random.default_rng(M).uniform(1e-4, 1e-3, (len(W), 1)).astype(np.float16).view(np.uint8)
+    W = W.reshape(-1)
+    A = (gauss_acts((M, K), seed=M + 9) * 0.05).astype(np.float16)
+    w, a = torch.from_numpy(W).cuda(), torch.from_numpy(A).cuda()
+    want = a.double() @ torch.from_numpy(oracle.dequant(fmt, W, N * K).reshape(N, K)).cuda().double().t()
+    ws = ops.matmul_gguf_workspace(fmt, M, K, N, a.dtype, "cuda")
+    got = ops.matmul_gguf(a, w, fmt, N, K, out_dtype=torch.float32, workspace=ws)
+    assert normwise_rel_err(got.cpu().numpy(), want.cpu().numpy()) < 2e-6
+    if pairs:
+        got = ops.matmul_gguf(a, w, fmt, N, K, out_dtype=torch.float32, workspace=ws, swiglu_pairs=True)
+        want = torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2]
+        assert normwise_rel_err(got.cpu().numpy(), want.cpu().numpy()) < 4e-6
+
+
 def test_streaming_mfma_matmul_refusals(ops):
     from cut_amd import lib
     K, N = 512, 64
