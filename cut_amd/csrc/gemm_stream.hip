@@ -79,7 +79,7 @@ __device__ __forceinline__ half8_t as_frag(uint32_t a, uint32_t b, uint32_t c, u
 // MT: activation tiles of 16 rows (1 or 2); RG: groups of 16 weight rows per workgroup; KW: waves that share a group,
 // each on its own part of the steps.  RG x KW = 8 waves wherever the range is long enough (two waves per SIMD: one
 // wave alone cannot hide its own LDS and matrix-core latencies).
-template <int FMT, int MT, int KW, int RG>
+template <int FMT, int SB, int MT, int KW, int RG>
 __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int D = kStreamDepth, THREADS = 64 * RG * KW;
@@ -119,16 +119,15 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams 
     for (int j = 0; j < NP; ++j) r.c[j] = ld_u32x4(piece[j] + (size_t)step * kStepBytes);
   };
 
-  // activations first (they must not queue behind the weight loads), in batches of kSB 16-byte pieces per thread;
+  // activations first (they must not queue behind the weight loads), in batches of SB 16-byte pieces per thread;
   // the weight ring is requested behind the first batch
-  constexpr int kSB = 16;
   const uint32_t cpr = range_k / 8, chunks = p.M * cpr;   // 8-element pieces per row, in all
   const uint32_t k_lo = s_lo * 256;
   const uint32_t inv = 0xFFFFFFFFu / cpr + 1;   // c / cpr = c inv >> 32: exact, as c (inv cpr - 2^32) < chunks cpr < 2^32
-  u32x4 xa[kSB], xb[kSB];
+  u32x4 xa[SB], xb[SB];
   auto stage_load = [&](uint32_t base) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kSB; ++i) {
+    for (int i = 0; i < SB; ++i) {
       const uint32_t c = min(base + (uint32_t)i * THREADS + (uint32_t)tid, chunks - 1), r = __umulhi(c, inv), col = c - r * cpr;
       const size_t off = (size_t)r * p.strideA + k_lo + col * 8;
       if (p.a_f16) {
@@ -145,7 +144,7 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams 
     const half2_t one{(half_t)1.0f, (half_t)1.0f};
     const bool b0 = tid & 1, b1 = tid & 2;
 #pragma unroll
-    for (int i0 = 0; i0 < kSB; i0 += 4) {
+    for (int i0 = 0; i0 < SB; i0 += 4) {
       if (base + (uint32_t)i0 * THREADS >= chunks) break;
       float sum[4];
 #pragma unroll
@@ -194,7 +193,7 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams 
     __builtin_amdgcn_sched_barrier(0);   // issue order = ring order: step i waits for its own loads only
   }
   stage_store(0);
-  for (uint32_t base = kSB * THREADS; base < chunks; base += kSB * THREADS) {
+  for (uint32_t base = SB * THREADS; base < chunks; base += SB * THREADS) {
     stage_load(base);
     stage_store(base);
   }
@@ -322,27 +321,31 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams 
     }
   };
 
-  // Ring slot i % D holds the pieces of step i.  Every refill is issued, past the end of the range at the range's
-  // last step again (a few redundant loads of valid memory): with no load under a condition the compiler counts the
-  // loads in flight exactly and every step waits for its own pieces only, also in ranges shorter than 2 D steps.
+  // Ring slot i % D holds the pieces of step i.  With no load under a condition the compiler counts the loads in flight exactly and
+  // every step waits for its own pieces only: the last D steps, which request nothing, stand by themselves (requested past
+  // the end of the range, at its last step again, their pieces cost Q8_0 2 to 3 %).
   const uint32_t last = cnt ? cnt - 1 : 0u;
-  for (uint32_t i0 = 0; i0 < cnt; i0 += D) {
+  auto multiply = [&](const Raw &raw, uint32_t i) __attribute__((always_inline)) {
+    if constexpr (Q4K) {
+      Blk blk;
+      deliver(raw, blk);
+      do_step(blk, i);
+    } else {
+      q8_step(raw, i);
+    }
+  };
+  uint32_t i0 = 0;
+  for (; i0 + D < cnt; i0 += D) {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
-      const uint32_t i = i0 + u;
-      if (i < cnt) {           // uniform; no global load inside
-        if constexpr (Q4K) {
-          Blk blk;
-          deliver(buf[u], blk);
-          do_step(blk, i);
-        } else {
-          q8_step(buf[u], i);
-        }
-      }
-      load(buf[u], min(i + D, last));
+      multiply(buf[u], i0 + u);
+      load(buf[u], min(i0 + u + D, last));
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+#pragma unroll
+  for (int u = 0; u < D; ++u)
+    if (i0 + u < cnt) multiply(buf[u], i0 + u);   // uniform
   // the K parts of a row group meet in LDS (the staged activations are no longer needed)
   if constexpr (KW > 1) {
     __syncthreads();
@@ -435,11 +438,11 @@ size_t stream_gemm_scratch(uint32_t M, uint32_t K, uint32_t N) {
   return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
 }
 
-template <int FMT>
+template <int FMT, int SB>
 static auto stream_kernel(uint32_t mt, uint32_t block_rows, bool two) {
-  return block_rows == 128 ? gemm_stream_kernel<FMT, 2, 1, 8>
-         : mt == 1 ? (two ? gemm_stream_kernel<FMT, 1, 2, 4> : gemm_stream_kernel<FMT, 1, 1, 4>)
-                   : (two ? gemm_stream_kernel<FMT, 2, 2, 4> : gemm_stream_kernel<FMT, 2, 1, 4>);
+  return block_rows == 128 ? gemm_stream_kernel<FMT, SB, 2, 1, 8>
+         : mt == 1 ? (two ? gemm_stream_kernel<FMT, SB, 1, 2, 4> : gemm_stream_kernel<FMT, SB, 1, 1, 4>)
+                   : (two ? gemm_stream_kernel<FMT, SB, 2, 2, 4> : gemm_stream_kernel<FMT, SB, 2, 1, 4>);
 }
 
 int launch_stream_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
@@ -466,8 +469,12 @@ int launch_stream_gemm(int fmt, const void *W, const void *A, int a_f16, void *C
   const size_t lds = (size_t)16 * mt * ((size_t)p.range_steps * 544 + 32) + 8 * kStripBytes;
   // four row groups: two waves each once a wave keeps at least two steps
   const bool two = block_rows == 64 && p.range_steps >= 4;
-  auto kern = fmt == CUTHIP_Q4_K ? stream_kernel<CUTHIP_Q4_K>(mt, block_rows, two) : stream_kernel<CUTHIP_Q8_0>(mt, block_rows, two);
   const uint32_t threads = block_rows == 128 || two ? 512 : 256;
+  // Activations are staged in batches of 16 pieces per thread, of 8 where those are all: a batch requests its last piece over and over
+  // (Q4_K 4096 x 4096 at 16 rows 9.0 us against 9.5, 2048 x 2048 7.5 against 7.9; chosen inside the kernel it costs large calls 2 %)
+  const bool few = (uint64_t)M * p.range_steps * 32 <= 8 * threads;
+  auto kern = fmt == CUTHIP_Q4_K ? (few ? stream_kernel<CUTHIP_Q4_K, 8>(mt, block_rows, two) : stream_kernel<CUTHIP_Q4_K, 16>(mt, block_rows, two))
+                                 : (few ? stream_kernel<CUTHIP_Q8_0, 8>(mt, block_rows, two) : stream_kernel<CUTHIP_Q8_0, 16>(mt, block_rows, two));
   if (lds > 64 * 1024) {
     if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                (int)lds),
