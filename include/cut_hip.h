@@ -259,14 +259,15 @@ int cuthip_matmul_gguf(int fmt, const void *W, const void *A, int a_dtype, void 
  *            workgroups where its tiles alone would not fill the chip (fp32 partial products
  *            in the workspace, summed in a second launch);
  *            6 = MatMulGgufStreamMfma (Q4_K, M <= 32, 16-byte aligned rows of A, else an
- *            error): the weights stay packed until they are multiplied (integer-scaled
- *            nibbles as fp16 subnormals into 16x16x32 MFMAs: the products are exact and
+ *            error): the weights stay packed until they are multiplied (nibbles as fp16
+ *            subnormals times their scale into 16x16x32 MFMAs: the products are exact and
  *            the result differs from fp32 FMAs only by the order of the fp32 sums, given
  *            fp16 activations; fp32 activations are rounded to fp16, nearest even, when they
  *            are staged - 2^-11 relative per element, |a| > 65504 becomes inf - as on the 8-row
  *            GEMV and the GEMMs); K above 4096 (2048 beyond 16 rows) is split over
  *            workgroups through the workspace, an error without one.  With variant -1
- *            it is what runs for 9..32 rows of Q4_K.
+ *            it is what runs for 9..32 rows of Q4_K; large matrices of Q8_0 take the same
+ *            kernel at 5..32 rows, with variant -1 only.
  * With variant -1 the workspace also serves batch 2-8 (Q6_K: 3-8) on long rows (K >= 8192) of few (N < 12288): the 8-row GEMV
  * then splits K across workgroups, writes fp32 partial products to the workspace and sums them in a second launch
  * (the unsplit kernel would have to stage all of the activations in every workgroup).  The same for any N where the

@@ -429,6 +429,8 @@ def test_streaming_q8_0_matmul(ops, M, N, K, pairs):
     ws = ops.matmul_gguf_workspace(fmt, M, K, N, a.dtype, "cuda")
     got = ops.matmul_gguf(a, w, fmt, N, K, out_dtype=torch.float32, workspace=ws)
     assert normwise_rel_err(got.cpu().numpy(), want.cpu().numpy()) < 2e-6
+    same = ops.matmul_gguf(a.float(), w, fmt, N, K, out_dtype=torch.float32, workspace=ws)
+    assert torch.equal(got, same)
     if pairs:
         got = ops.matmul_gguf(a, w, fmt, N, K, out_dtype=torch.float32, workspace=ws, swiglu_pairs=True)
         want = torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2]
