@@ -392,9 +392,10 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams 
 }
 
 // K ranges of the streaming kernel: as few as LDS allows (one range of up to kStreamLdsMax bytes of staged
-// activations), more while the grid has fewer workgroups than CUs and a range keeps at least 8 steps, or 4 where the workgroups
-// still run at once (Q4_K at 16 / 32 rows, one range in the place of two: 4096 x 4096 10.3 / 12.4 us and 9.4 / 10.7, 2048 x 8192 10.3 / 12.4 and
-// 9.4 / 10.8; of eight steps in all only with two activation tiles: 4096 x 2048 8.0 / 10.0 and 8.4 / 9.7), and the scratch memory
+// activations), more where the workgroups still run at once, one to a CU, a range keeps at least 4 steps (Q4_K at 16 / 32 rows, one
+// range in the place of two: 4096 x 4096 10.3 / 12.4 us and 9.4 / 10.7, 2048 x 8192 10.3 / 12.4 and 9.4 / 10.8; of eight steps in all only
+// with two activation tiles: 4096 x 2048 8.0 / 10.0 and 8.4 / 9.7; beyond 256 workgroups, which then run in two rounds, 10240 x 4096 at
+// 16 rows 12.6 in one range and 16.5 in two, Q8_0 17.6 and 21.7), and the scratch memory
 // holds the partial products of twice as many.  (A workgroup that stages one range after the other, without partial
 // products, needs the registers of the staging beside those of the loop: 35.9 us against 30.0 for 28672 x 4096 at 32 rows.)
 // Weight rows per workgroup: 64 (four row groups, two waves each), or with two activation tiles 128 (eight row groups
@@ -409,10 +410,7 @@ static void stream_layout(uint32_t M, uint32_t K, uint32_t N, size_t scratch_byt
   const uint32_t mt = (M + 15) / 16, nsteps = K / 256, nblocks = (N + stream_block_rows(M, K, N) - 1) / stream_block_rows(M, K, N);
   const uint32_t max_steps = (kStreamLdsMax / (16 * mt) - 16) / 512;
   uint32_t ks = (nsteps + max_steps - 1) / max_steps;
-  auto more = [&] {
-    const uint32_t steps = nsteps / (2 * ks), blocks = nblocks * ks;
-    return (blocks < 192 && steps >= 8) || (2 * blocks <= 256 && steps >= 4 && (mt == 2 || nsteps >= 16));
-  };
+  auto more = [&] { return 2 * nblocks * ks <= 256 && nsteps / (2 * ks) >= 4 && (mt == 2 || nsteps >= 16); };
   while (ks < 16 && more() && scratch_bytes >= (size_t)2 * ks * M * N * sizeof(float)) ks *= 2;
   *range_steps = (nsteps + ks - 1) / ks;
   *ksplit = (nsteps + *range_steps - 1) / *range_steps;

@@ -413,8 +413,8 @@ def test_streaming_mfma_matmul_minima_do_not_cancel(ops, M, K, scale):
     assert (np.abs(got.cpu().numpy() - want) <= 2.0 ** -21 * size).all()
 
 
-@pytest.mark.parametrize("M,N,K,pairs", [(5, 12290, 4096, True), (8, 3500, 14336, False), (9, 3910, 4096, False), (16, 1200, 14336, False),
-                                         (17, 5450, 4352, False), (32, 10800, 2048, False), (31, 4131, 8192, False)])
+@pytest.mark.parametrize("M,N,K,pairs", [(5, 12290, 4096, True), (8, 3500, 14336, False), (7, 10002, 2048, True), (6, 4100, 5120, False), (9, 3910, 4096, False), (16, 1200, 14336, False),
+                                         (17, 7100, 4352, False), (32, 10800, 2048, False), (31, 5201, 8192, False)])
 def test_streaming_q8_0_matmul(ops, M, N, K, pairs):
     """The streaming kernel on Q8_0, as the automatic choice takes it for large matrices: one and two activation tiles, ragged N,
     one K range and several of unequal length, the SwiGLU row pairs.  Products of int8 and fp16 are exact in fp32, so the bound
