@@ -17,7 +17,9 @@
 
 namespace {
 
-PyObject *g_error = nullptr, *g_formats = nullptr, *g_unary = nullptr, *g_binary = nullptr;   // set once by setup()
+// set once by setup()
+PyObject *g_error = nullptr, *g_formats = nullptr, *g_unary = nullptr, *g_binary = nullptr;
+PyObject *g_norm_carry = nullptr, *g_rope_append = nullptr, *g_ctypes = nullptr;
 
 struct PyError {};   // a Python exception is set
 
@@ -105,20 +107,42 @@ at::Tensor empty(at::IntArrayRef size, at::ScalarType dtype, const at::Tensor &l
   return at::empty(size, at::TensorOptions().dtype(dtype).device(like.device()));
 }
 
-// the address of a ctypes structure (null for None)
+// The address of a ctypes structure of the given class (null for None).  Anything else is refused as ctypes refuses it: what the
+// library reads there are device pointers.
 struct Structure {
   Py_buffer b{};
   void *p = nullptr;
-  explicit Structure(PyObject *o) {
+  Structure(PyObject *o, PyObject *cls, size_t size) {
     if (o == Py_None) return;
+    const int is = PyObject_IsInstance(o, cls);
+    if (is < 0) throw PyError{};
+    if (!is) refuse(o, cls);
     if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE)) throw PyError{};
+    if ((size_t)b.len < size) {
+      PyBuffer_Release(&b);
+      refuse(o, cls);
+    }
     p = b.buf;
   }
   ~Structure() {
     if (p) PyBuffer_Release(&b);
   }
   Structure(const Structure &) = delete;
+
+ private:
+  [[noreturn]] static void refuse(PyObject *o, PyObject *cls) {
+    PyObject *r = PyObject_CallMethod(g_ctypes, "byref", "O", o);   // TypeError for what is no ctypes instance
+    if (!r) throw PyError{};
+    Py_DECREF(r);
+    if (PyObject *e = PyObject_GetAttrString(g_ctypes, "ArgumentError")) {
+      PyErr_Format(e, "expected an instance of %s, got %s", ((PyTypeObject *)cls)->tp_name, Py_TYPE(o)->tp_name);
+      Py_DECREF(e);
+    }
+    throw PyError{};
+  }
 };
+Structure norm_carry_of(PyObject *o) { return {o, g_norm_carry, sizeof(cuthip_norm_carry_t)}; }
+Structure rope_append_of(PyObject *o) { return {o, g_rope_append, sizeof(cuthip_rope_append_t)}; }
 
 PyObject *ref(PyObject *o) {
   Py_INCREF(o);
@@ -271,7 +295,7 @@ PyObject *matmul_gguf_carry(PyObject *const *p) {   // a, w_blocks, fmt, N, K, o
     e.op = lookup(g_binary, p[7]);
     e.d = ptr(d);
   }
-  const Structure carry(p[6]);
+  const Structure carry = norm_carry_of(p[6]);
   check(cuthip_matmul_gguf_carry(f, ptr(w), ptr(a), act_dtype(a), mut(out), act_dtype(out), (uint32_t)K, (uint32_t)N, e.epilogue, e.op,
                                  e.d, (const cuthip_norm_carry_t *)carry.p, stream()));
   return ref(p[5]);
@@ -284,7 +308,7 @@ PyObject *matmul_gguf_pair(PyObject *const *p) {
   const int64_t Na = integer(p[3]), Nb = integer(p[7]), K = integer(p[9]);
   if (a.numel() != K || !activation(a) || !a.is_contiguous()) fail("matmul_pair: A must be a contiguous float32/float16 vector of K elements");
   if (wa.numel() < n_bytes(fa, Na, K) || wb.numel() < n_bytes(fb, Nb, K)) fail("matmul_pair: weight tensor too small for [N, K]");
-  const Structure carry(p[10]), rope(p[11]);
+  const Structure carry = norm_carry_of(p[10]), rope = rope_append_of(p[11]);
   void *ca = nullptr, *cb = nullptr;
   int cdt = CUTHIP_F32;
   if (!rope.p) {   // (with it the epilogue writes q_out and the caches; the plain outputs are not used)
@@ -345,7 +369,7 @@ PyObject *matmul_gguf_argmax(PyObject *const *p) {
     pf = ptr(fac);
     n = (uint32_t)t.numel();
   }
-  const Structure carry(p[7]);
+  const Structure carry = norm_carry_of(p[7]);
   const at::Tensor ws = given(p[10]) ? tensor(p[10]) : at::Tensor();
   check(cuthip_matmul_gguf_argmax(f, ptr(w), ptr(a), act_dtype(a), mut(logits), act_dtype(logits), (uint32_t)K, (uint32_t)N,
                                   (const cuthip_norm_carry_t *)carry.p, (const int32_t *)pt, (const float *)pf, n,
@@ -424,11 +448,14 @@ PyObject *prepare_sep(PyObject *const *p) {   // w_blocks, fmt, N, K, stride_b, 
   return pair;
 }
 
-PyObject *setup(PyObject *const *p) {   // CutHipError, FORMATS, UNARY, BINARY
+PyObject *setup(PyObject *const *p) {   // CutHipError, FORMATS, UNARY, BINARY, NormCarry, RopeAppend, ctypes
   g_error = ref(p[0]);
   g_formats = ref(p[1]);
   g_unary = ref(p[2]);
   g_binary = ref(p[3]);
+  g_norm_carry = ref(p[4]);
+  g_rope_append = ref(p[5]);
+  g_ctypes = ref(p[6]);
   return ref(Py_None);
 }
 
@@ -447,7 +474,7 @@ template <PyObject *(*F)(PyObject *const *), int ARGS> PyObject *entry(PyObject 
 }
 
 #define ENTRY(name, args) {#name, (PyCFunction)(void (*)(void))entry<name, args>, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {ENTRY(setup, 4),           ENTRY(dequantize, 6),   ENTRY(matmul_gguf, 13),      ENTRY(norm_carry, 6),
+PyMethodDef methods[] = {ENTRY(setup, 7),           ENTRY(dequantize, 6),   ENTRY(matmul_gguf, 13),      ENTRY(norm_carry, 6),
                          ENTRY(rope_append, 9),     ENTRY(matmul_gguf_carry, 10), ENTRY(matmul_gguf_pair, 12), ENTRY(rmsnorm, 5),
                          ENTRY(attn_decode, 11),    ENTRY(silu_mul, 2),     ENTRY(matmul_gguf_argmax, 11), ENTRY(embedding_rows, 6),
                          ENTRY(matmul_sep, 11),     ENTRY(prepare_sep, 6),  {nullptr, nullptr, 0, nullptr}};

@@ -30,7 +30,7 @@ def _host():
             from . import _host_ops
         except ImportError as e:
             raise _l.CutHipError(f"cut_amd/_host_ops.so is missing or does not load: build it with `make -C cut_amd/csrc` ({e})") from e
-        _host_ops.setup(_l.CutHipError, _l.FORMATS, _l.UNARY, _l.BINARY)
+        _host_ops.setup(_l.CutHipError, _l.FORMATS, _l.UNARY, _l.BINARY, _l.NormCarry, _l.RopeAppend, C)
         _native = _host_ops
     return _native
 
