@@ -27,7 +27,19 @@ struct PyError {};   // a Python exception is set
   PyErr_SetString(g_error, text);
   throw PyError{};
 }
-void check(int rc) {
+// Other Python threads run while a launch waits (a full queue, the first load of a code object) or memory is allocated: a host
+// callback on the stream may need one of them.
+struct Released {
+  PyThreadState *s = PyEval_SaveThread();
+  ~Released() { PyEval_RestoreThread(s); }
+};
+// a call of the C ABI; its arguments are evaluated before the GIL is given back
+template <class... P, class... A> void call(int (*f)(P...), A... args) {
+  int rc;
+  {
+    const Released r;
+    rc = f(args...);
+  }
   if (rc == 0) return;
   PyErr_Format(g_error, "cut_hip error %d: %s", rc, cuthip_last_error());
   throw PyError{};
@@ -104,7 +116,14 @@ const void *ptr(const at::Tensor &t) { return t.const_data_ptr(); }
 void *mut(const at::Tensor &t) { return t.data_ptr(); }
 void *stream() { return (void *)c10::hip::getCurrentHIPStream().stream(); }
 at::Tensor empty(at::IntArrayRef size, at::ScalarType dtype, const at::Tensor &like) {
+  const Released r;
   return at::empty(size, at::TensorOptions().dtype(dtype).device(like.device()));
+}
+
+at::Tensor matrix(const at::Tensor &t) {   // [rows, dim]; a row for any other number of dimensions (which may copy)
+  if (t.dim() == 2) return t;
+  const Released r;
+  return t.reshape({1, -1});
 }
 
 // The address of a ctypes structure of the given class (null for None).  Anything else is refused as ctypes refuses it: what the
@@ -167,8 +186,8 @@ PyObject *dequantize(PyObject *const *a) {   // raw, fmt, rows, cols, dtype, out
   const at::ScalarType dt = ((THPDtype *)a[4])->scalar_type;
   if (dt != at::kFloat && dt != at::kHalf) fail("dequantize: output dtype must be float32 or float16");
   const at::Tensor out = given(a[5]) ? tensor(a[5]) : empty({rows, cols}, dt, raw);
-  check(cuthip_dequant(f, ptr(raw), mut(out), dt == at::kHalf ? CUTHIP_F16 : CUTHIP_F32, (uint32_t)rows, (uint32_t)cols,
-                       (uint32_t)(out.dim() == 2 ? out.stride(0) : cols), stream()));
+  call(cuthip_dequant, f, ptr(raw), mut(out), dt == at::kHalf ? CUTHIP_F16 : CUTHIP_F32, (uint32_t)rows, (uint32_t)cols,
+                       (uint32_t)(out.dim() == 2 ? out.stride(0) : cols), stream());
   return given(a[5]) ? ref(a[5]) : THPVariable_Wrap(out);
 }
 
@@ -212,12 +231,12 @@ PyObject *matmul_gguf(PyObject *const *p) {
   const int variant = (int)integer(p[10]);
   if (given(p[11])) {
     const at::Tensor &ws = tensor(p[11]);
-    check(cuthip_matmul_gguf_ws(f, ptr(w), ptr(a), f16_or_f32(a), mut(out), f16_or_f32(out), (uint32_t)M, (uint32_t)K, (uint32_t)N,
+    call(cuthip_matmul_gguf_ws, f, ptr(w), ptr(a), f16_or_f32(a), mut(out), f16_or_f32(out), (uint32_t)M, (uint32_t)K, (uint32_t)N,
                                 (uint32_t)outer, (uint32_t)out.stride(0), e.epilogue, e.op, e.d, variant, mut(ws),
-                                (size_t)(ws.numel() * ws.element_size()), stream()));
+                                (size_t)(ws.numel() * ws.element_size()), stream());
   } else {
-    check(cuthip_matmul_gguf(f, ptr(w), ptr(a), f16_or_f32(a), mut(out), f16_or_f32(out), (uint32_t)M, (uint32_t)K, (uint32_t)N,
-                             (uint32_t)outer, (uint32_t)out.stride(0), e.epilogue, e.op, e.d, variant, stream()));
+    call(cuthip_matmul_gguf, f, ptr(w), ptr(a), f16_or_f32(a), mut(out), f16_or_f32(out), (uint32_t)M, (uint32_t)K, (uint32_t)N,
+                             (uint32_t)outer, (uint32_t)out.stride(0), e.epilogue, e.op, e.d, variant, stream());
   }
   return given(p[6]) ? ref(p[6]) : THPVariable_Wrap(out);
 }
@@ -296,8 +315,8 @@ PyObject *matmul_gguf_carry(PyObject *const *p) {   // a, w_blocks, fmt, N, K, o
     e.d = ptr(d);
   }
   const Structure carry = norm_carry_of(p[6]);
-  check(cuthip_matmul_gguf_carry(f, ptr(w), ptr(a), act_dtype(a), mut(out), act_dtype(out), (uint32_t)K, (uint32_t)N, e.epilogue, e.op,
-                                 e.d, (const cuthip_norm_carry_t *)carry.p, stream()));
+  call(cuthip_matmul_gguf_carry, f, ptr(w), ptr(a), act_dtype(a), mut(out), act_dtype(out), (uint32_t)K, (uint32_t)N, e.epilogue, e.op,
+                                 e.d, (const cuthip_norm_carry_t *)carry.p, stream());
   return ref(p[5]);
 }
 
@@ -319,20 +338,20 @@ PyObject *matmul_gguf_pair(PyObject *const *p) {
     cb = mut(ob);
     cdt = act_dtype(oa);
   }
-  check(cuthip_matmul_gguf_pair(fa, ptr(wa), (uint32_t)Na, ca, fb, ptr(wb), (uint32_t)Nb, cb, ptr(a), act_dtype(a), cdt, (uint32_t)K,
-                                (const cuthip_norm_carry_t *)carry.p, (const cuthip_rope_append_t *)rope.p, stream()));
+  call(cuthip_matmul_gguf_pair, fa, ptr(wa), (uint32_t)Na, ca, fb, ptr(wb), (uint32_t)Nb, cb, ptr(a), act_dtype(a), cdt, (uint32_t)K,
+                                (const cuthip_norm_carry_t *)carry.p, (const cuthip_rope_append_t *)rope.p, stream());
   return ref(Py_None);
 }
 
 PyObject *rmsnorm(PyObject *const *p) {   // x, weight, eps, out, out_dtype
   const at::Tensor &x = tensor(p[0]), &w = tensor(p[1]);
-  const at::Tensor x2 = x.dim() == 2 ? x : x.reshape({1, -1});
+  const at::Tensor x2 = matrix(x);
   if (w.scalar_type() != at::kFloat || w.numel() != x2.size(1) || x2.stride(1) != 1) fail("rmsnorm: weight must be fp32 [dim] and x rows contiguous");
   const float eps = real(p[2]);
   if (given(p[4]) && !THPDtype_Check(p[4])) fail("rmsnorm: out_dtype must be a dtype");
   const at::Tensor out = given(p[3]) ? tensor(p[3]) : empty(x2.sizes(), given(p[4]) ? ((THPDtype *)p[4])->scalar_type : x.scalar_type(), x);
-  check(cuthip_rmsnorm(ptr(x2), act_dtype(x2), (const float *)ptr(w), mut(out), act_dtype(out), (uint32_t)x2.size(0), (uint32_t)x2.size(1),
-                       (uint32_t)x2.stride(0), eps, stream()));
+  call(cuthip_rmsnorm, ptr(x2), act_dtype(x2), (const float *)ptr(w), mut(out), act_dtype(out), (uint32_t)x2.size(0), (uint32_t)x2.size(1),
+                       (uint32_t)x2.stride(0), eps, stream());
   return given(p[3]) ? ref(p[3]) : THPVariable_Wrap(out);
 }
 
@@ -340,15 +359,15 @@ PyObject *rmsnorm(PyObject *const *p) {   // x, weight, eps, out, out_dtype
 PyObject *attn_decode(PyObject *const *p) {
   const at::Tensor &q = tensor(p[0]), &k = tensor(p[1]), &v = tensor(p[2]), &par = tensor(p[3]), &ws = tensor(p[8]), &out = tensor(p[9]);
   const int64_t len = given(p[10]) && truth(p[10]) ? integer(p[10]) : k.size(0);
-  check(cuthip_attn_decode(ptr(q), act_dtype(q), ptr(k), ptr(v), (const uint32_t *)ptr(par), mut(out), act_dtype(out), (uint32_t)integer(p[4]),
+  call(cuthip_attn_decode, ptr(q), act_dtype(q), ptr(k), ptr(v), (const uint32_t *)ptr(par), mut(out), act_dtype(out), (uint32_t)integer(p[4]),
                            (uint32_t)integer(p[5]), (uint32_t)integer(p[6]), (uint32_t)k.stride(0), real(p[7]), (uint32_t)len, mut(ws),
-                           (size_t)ws.numel(), stream()));
+                           (size_t)ws.numel(), stream());
   return ref(p[9]);
 }
 
 PyObject *silu_mul(PyObject *const *p) {   // gate_up, out
   const at::Tensor &g = tensor(p[0]), &out = tensor(p[1]);
-  check(cuthip_silu_mul(ptr(g), act_dtype(g), mut(out), act_dtype(out), (uint32_t)out.numel(), stream()));
+  call(cuthip_silu_mul, ptr(g), act_dtype(g), mut(out), act_dtype(out), (uint32_t)out.numel(), stream());
   return ref(p[1]);
 }
 
@@ -371,9 +390,9 @@ PyObject *matmul_gguf_argmax(PyObject *const *p) {
   }
   const Structure carry = norm_carry_of(p[7]);
   const at::Tensor ws = given(p[10]) ? tensor(p[10]) : at::Tensor();
-  check(cuthip_matmul_gguf_argmax(f, ptr(w), ptr(a), act_dtype(a), mut(logits), act_dtype(logits), (uint32_t)K, (uint32_t)N,
+  call(cuthip_matmul_gguf_argmax, f, ptr(w), ptr(a), act_dtype(a), mut(logits), act_dtype(logits), (uint32_t)K, (uint32_t)N,
                                   (const cuthip_norm_carry_t *)carry.p, (const int32_t *)pt, (const float *)pf, n,
-                                  ws.defined() ? mut(ws) : nullptr, ws.defined() ? (size_t)ws.numel() : 0, (uint32_t *)mut(index), stream()));
+                                  ws.defined() ? mut(ws) : nullptr, ws.defined() ? (size_t)ws.numel() : 0, (uint32_t *)mut(index), stream());
   return ref(p[6]);
 }
 
@@ -383,15 +402,15 @@ PyObject *embedding_rows(PyObject *const *p) {   // w_blocks, fmt, token_ids, n_
   if ((ids.scalar_type() != at::kInt && ids.scalar_type() != at::kUInt32) || out.stride(-1) != 1 || out.numel() < ids.numel() * dim)
     fail("embedding_rows: token ids are 32-bit integers, out holds one row of dim per id");
   const at::Tensor out2 = out.dim() == 2 ? out : out.view({ids.numel(), -1});
-  check(cuthip_embedding_rows(format(p[1]), ptr(w), (const uint32_t *)ptr(ids), (uint32_t)ids.numel(), (uint32_t)rows, (uint32_t)dim, mut(out2),
-                              act_dtype(out2), (uint32_t)out2.stride(0), stream()));
+  call(cuthip_embedding_rows, format(p[1]), ptr(w), (const uint32_t *)ptr(ids), (uint32_t)ids.numel(), (uint32_t)rows, (uint32_t)dim, mut(out2),
+                              act_dtype(out2), (uint32_t)out2.stride(0), stream());
   return ref(p[5]);
 }
 
 // a, b, scales, N, q4, affine, out, unary, binary, d, variant
 PyObject *matmul_sep(PyObject *const *p) {
   const at::Tensor &in = tensor(p[0]), &b = tensor(p[1]), &s = tensor(p[2]);
-  const at::Tensor a = in.dim() == 2 ? in : in.reshape({1, -1});
+  const at::Tensor a = matrix(in);
   const int64_t M = a.size(0), K = a.size(1), N = integer(p[3]);
   const bool q4 = truth(p[4]), affine = truth(p[5]);
   if (a.scalar_type() != at::kFloat || s.scalar_type() != at::kHalf || b.element_size() != 1 || b.dim() != 2 || s.dim() != 2)
@@ -421,11 +440,11 @@ PyObject *matmul_sep(PyObject *const *p) {
   const at::Tensor ws = empty({(int64_t)std::max<size_t>(bytes, 1)}, at::kByte, in);
   const uint32_t sa = (uint32_t)a.stride(0), sb = (uint32_t)b.stride(0), sc = (uint32_t)out.stride(0), ss = (uint32_t)s.stride(0);
   if (q4)
-    check(cuthip_matmul_q4_sep((const float *)ptr(a), (const uint8_t *)ptr(b), (const uint16_t *)ptr(s), (const float *)e.d, (float *)mut(out), (uint32_t)M,
-                               (uint32_t)K, (uint32_t)N, sa, sb, sc, ss, e.epilogue, e.op, affine, variant, mut(ws), bytes, stream()));
+    call(cuthip_matmul_q4_sep, (const float *)ptr(a), (const uint8_t *)ptr(b), (const uint16_t *)ptr(s), (const float *)e.d, (float *)mut(out), (uint32_t)M,
+                               (uint32_t)K, (uint32_t)N, sa, sb, sc, ss, e.epilogue, e.op, affine, variant, mut(ws), bytes, stream());
   else
-    check(cuthip_matmul_q8_sep((const float *)ptr(a), (const int8_t *)ptr(b), (const uint16_t *)ptr(s), (const float *)e.d, (float *)mut(out), (uint32_t)M,
-                               (uint32_t)K, (uint32_t)N, sa, sb, sc, ss, e.epilogue, e.op, variant, mut(ws), bytes, stream()));
+    call(cuthip_matmul_q8_sep, (const float *)ptr(a), (const int8_t *)ptr(b), (const uint16_t *)ptr(s), (const float *)e.d, (float *)mut(out), (uint32_t)M,
+                               (uint32_t)K, (uint32_t)N, sa, sb, sc, ss, e.epilogue, e.op, variant, mut(ws), bytes, stream());
   return given(p[6]) ? ref(p[6]) : THPVariable_Wrap(out);
 }
 
@@ -437,10 +456,12 @@ PyObject *prepare_sep(PyObject *const *p) {   // w_blocks, fmt, N, K, stride_b, 
   const bool q4 = f != CUTHIP_Q8_0;
   const int64_t width = q4 ? N / 2 : N, sb = given(p[4]) ? integer(p[4]) : (width + 3) & ~(int64_t)3, ss = given(p[5]) ? integer(p[5]) : (N + 3) & ~(int64_t)3;
   const at::Tensor b = empty({K, sb}, q4 ? at::kByte : at::kChar, w), s = empty({(f == CUTHIP_Q4_K ? 2 : 1) * (K / 32), ss}, at::kHalf, w);
-  // the kernel writes every column up to the width; the padding beyond it is zero
-  if (sb > width) b.slice(1, width).zero_();
-  if (ss > N) s.slice(1, N).zero_();
-  check(cuthip_prepare_sep(f, ptr(w), (uint32_t)N, (uint32_t)K, mut(b), (uint32_t)sb, (uint16_t *)mut(s), (uint32_t)ss, stream()));
+  {   // the kernel writes every column up to the width; the padding beyond it is zero
+    const Released r;
+    if (sb > width) b.slice(1, width).zero_();
+    if (ss > N) s.slice(1, N).zero_();
+  }
+  call(cuthip_prepare_sep, f, ptr(w), (uint32_t)N, (uint32_t)K, mut(b), (uint32_t)sb, (uint16_t *)mut(s), (uint32_t)ss, stream());
   PyObject *pair = PyTuple_New(2);
   if (!pair) throw PyError{};
   PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(b));

@@ -1,5 +1,8 @@
 """The native host side of the operators (cut_amd/csrc/host_ops.cpp): what it refuses, before anything reaches the GPU."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -32,3 +35,47 @@ def test_carry_and_rope_take_their_own_structure_only(bad, error):
         ops.matmul_gguf_pair(a, w, "Q8_0", 8, o, w, "Q8_0", 8, o, 32, carry=for_norm)
     with pytest.raises(error):
         ops.matmul_gguf_pair(a, w, "Q8_0", 8, o, w, "Q8_0", 8, o, 32, carry=norm, rope=for_rope)
+
+
+STUB = """
+#include <poll.h>
+#include <unistd.h>
+int stub_fd = -1;
+volatile int stub_entered = 0;
+/* stands for a launch that waits until the other thread of the test has written to the pipe */
+int cuthip_silu_mul(const void *a, int b, void *c, int d, unsigned n, void *s) {
+  struct pollfd p = {stub_fd, POLLIN, 0};
+  stub_entered = 1;
+  return poll(&p, 1, 5000) == 1 ? 0 : 7;
+}
+/* the current stream, where there is no device */
+struct stream { long a, b; } _ZN3c103hip19getCurrentHIPStreamEa(signed char d) { struct stream s = {0, 0}; return s; }
+void *_ZNK3c103hip9HIPStream6streamEv(const void *s) { return 0; }
+"""
+WAITING = """
+import ctypes, os, sys, threading, time
+import torch
+stub = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)   # ahead of the library for the extension that is loaded next
+from cut_amd import ops
+r, w = os.pipe()
+ctypes.c_int.in_dll(stub, "stub_fd").value = r
+entered = ctypes.c_int.in_dll(stub, "stub_entered")
+def other():
+    while not entered.value:
+        time.sleep(0.001)
+    os.write(w, b"x")
+threading.Thread(target=other, daemon=True).start()
+ops.silu_mul(torch.zeros(8), torch.zeros(4))
+print("launched")
+"""
+
+
+def test_other_threads_run_while_a_launch_waits(tmp_path):
+    """A launch that can only go on when another Python thread has run (a full queue behind a host callback): the GIL is not held
+    across the C ABI.  The entry point is a stub that waits at most 5 s; no device is needed."""
+    src, so = tmp_path / "stub.c", tmp_path / "stub.so"
+    src.write_text(STUB)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-O1", str(src), "-o", str(so)])
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", WAITING, str(so)], cwd=root, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "launched" in r.stdout, r.stderr[-2000:]
