@@ -120,6 +120,21 @@ at::Tensor empty(at::IntArrayRef size, at::ScalarType dtype, const at::Tensor &l
   return at::empty(size, at::TensorOptions().dtype(dtype).device(like.device()));
 }
 
+// Whether a launch that writes `rows` rows of `width` elements, stride(0) apart, stays inside the tensor's own rows.
+bool holds(const at::Tensor &t, int64_t rows, int64_t width) {
+  if (t.dim() == 0) return false;
+  if (t.dim() == 1) return rows <= 1 && t.size(0) >= width && (t.size(0) <= 1 || t.stride(0) == 1);
+  int64_t run = 1;
+  for (int64_t d = t.dim() - 1; d > 0; run *= t.size(d--))
+    if (t.size(d) != 1 && t.stride(d) != run) return false;
+  return t.size(0) >= rows && run >= width;
+}
+void require(bool ok, const char *what, int64_t rows, int64_t width) {
+  if (ok) return;
+  PyErr_Format(g_error, "%s %lld rows of %lld", what, (long long)rows, (long long)width);
+  throw PyError{};
+}
+
 at::Tensor matrix(const at::Tensor &t) {   // [rows, dim]; a row for any other number of dimensions (which may copy)
   if (t.dim() == 2) return t;
   const Released r;
@@ -186,6 +201,8 @@ PyObject *dequantize(PyObject *const *a) {   // raw, fmt, rows, cols, dtype, out
   const at::ScalarType dt = ((THPDtype *)a[4])->scalar_type;
   if (dt != at::kFloat && dt != at::kHalf) fail("dequantize: output dtype must be float32 or float16");
   const at::Tensor out = given(a[5]) ? tensor(a[5]) : empty({rows, cols}, dt, raw);
+  require(out.scalar_type() == dt && (out.dim() == 2 ? holds(out, rows, cols) : out.is_contiguous() && out.numel() >= rows * cols),
+       "dequantize: out must have the output dtype and contiguous room for", rows, cols);
   call(cuthip_dequant, f, ptr(raw), mut(out), dt == at::kHalf ? CUTHIP_F16 : CUTHIP_F32, (uint32_t)rows, (uint32_t)cols,
                        (uint32_t)(out.dim() == 2 ? out.stride(0) : cols), stream());
   return given(a[5]) ? ref(a[5]) : THPVariable_Wrap(out);
@@ -213,6 +230,9 @@ PyObject *matmul_gguf(PyObject *const *p) {
     if (given(p[5]) && !THPDtype_Check(p[5])) fail("matmul: out_dtype must be a dtype");
     out = empty({M, pairs ? N / 2 : N}, given(p[5]) ? ((THPDtype *)p[5])->scalar_type : a.scalar_type(), a);
   }
+  const int dtype = act_dtype(out);
+  const int64_t width = pairs ? N / 2 : N;
+  require(holds(out, M, width), "matmul: out must have contiguous room for", M, width);
   Op e;
   if (pairs) {
     e.epilogue = CUTHIP_EPI_SWIGLU_PAIRS;
@@ -223,7 +243,7 @@ PyObject *matmul_gguf(PyObject *const *p) {
     const char *bad = "matmul: binary epilogue needs D with the shape, dtype and stride of C";
     if (!given(p[9])) fail(bad);
     const at::Tensor &d = tensor(p[9]);
-    if (d.sizes() != out.sizes() || d.scalar_type() != out.scalar_type() || d.stride(0) != out.stride(0)) fail(bad);
+    if (d.sizes() != out.sizes() || d.scalar_type() != out.scalar_type() || d.stride(0) != out.stride(0) || !holds(d, M, width)) fail(bad);
     e.epilogue = CUTHIP_EPI_BINARY;
     e.op = lookup(g_binary, p[8]);
     e.d = ptr(d);
@@ -231,11 +251,11 @@ PyObject *matmul_gguf(PyObject *const *p) {
   const int variant = (int)integer(p[10]);
   if (given(p[11])) {
     const at::Tensor &ws = tensor(p[11]);
-    call(cuthip_matmul_gguf_ws, f, ptr(w), ptr(a), f16_or_f32(a), mut(out), f16_or_f32(out), (uint32_t)M, (uint32_t)K, (uint32_t)N,
+    call(cuthip_matmul_gguf_ws, f, ptr(w), ptr(a), f16_or_f32(a), mut(out), dtype, (uint32_t)M, (uint32_t)K, (uint32_t)N,
                                 (uint32_t)outer, (uint32_t)out.stride(0), e.epilogue, e.op, e.d, variant, mut(ws),
                                 (size_t)(ws.numel() * ws.element_size()), stream());
   } else {
-    call(cuthip_matmul_gguf, f, ptr(w), ptr(a), f16_or_f32(a), mut(out), f16_or_f32(out), (uint32_t)M, (uint32_t)K, (uint32_t)N,
+    call(cuthip_matmul_gguf, f, ptr(w), ptr(a), f16_or_f32(a), mut(out), dtype, (uint32_t)M, (uint32_t)K, (uint32_t)N,
                              (uint32_t)outer, (uint32_t)out.stride(0), e.epilogue, e.op, e.d, variant, stream());
   }
   return given(p[6]) ? ref(p[6]) : THPVariable_Wrap(out);
@@ -270,6 +290,7 @@ PyObject *rope_append(PyObject *const *p) {   // RopeAppend, runtime_params, cos
   const at::Tensor &k = tensor(p[5]), &v = tensor(p[6]), &cos = tensor(p[2]), &q = tensor(p[4]);
   if (k.scalar_type() != at::kHalf || v.scalar_type() != at::kHalf || k.stride(0) != v.stride(0))
     fail("rope_append: caches must be fp16 with one row stride");
+  if (!q.is_contiguous() || q.numel() < integer(p[7])) fail("rope_append: q_out must hold q_dim contiguous elements");
   cuthip_rope_append_t r{};
   r.runtime_params = (decltype(r.runtime_params))ptr(tensor(p[1]));
   r.cos_table = (decltype(r.cos_table))ptr(cos);
@@ -349,9 +370,19 @@ PyObject *rmsnorm(PyObject *const *p) {   // x, weight, eps, out, out_dtype
   if (w.scalar_type() != at::kFloat || w.numel() != x2.size(1) || x2.stride(1) != 1) fail("rmsnorm: weight must be fp32 [dim] and x rows contiguous");
   const float eps = real(p[2]);
   if (given(p[4]) && !THPDtype_Check(p[4])) fail("rmsnorm: out_dtype must be a dtype");
-  const at::Tensor out = given(p[3]) ? tensor(p[3]) : empty(x2.sizes(), given(p[4]) ? ((THPDtype *)p[4])->scalar_type : x.scalar_type(), x);
-  call(cuthip_rmsnorm, ptr(x2), act_dtype(x2), (const float *)ptr(w), mut(out), act_dtype(out), (uint32_t)x2.size(0), (uint32_t)x2.size(1),
-                       (uint32_t)x2.stride(0), eps, stream());
+  // rows of x and out lie equally far apart
+  const int64_t rows = x2.size(0), dim = x2.size(1), stride = x2.stride(0);
+  at::Tensor out;
+  if (given(p[3])) {
+    out = tensor(p[3]);
+    require((holds(out, rows, dim) && (rows <= 1 || out.stride(0) == stride)) || (out.is_contiguous() && out.numel() >= (rows - 1) * stride + dim),
+         "rmsnorm: out must have contiguous room, as far apart as the rows of x, for", rows, dim);
+  } else {
+    const at::ScalarType dtype = given(p[4]) ? ((THPDtype *)p[4])->scalar_type : x.scalar_type();
+    out = rows > 1 && stride > dim ? empty({rows, stride}, dtype, x).slice(1, 0, dim) : empty(x2.sizes(), dtype, x);
+  }
+  call(cuthip_rmsnorm, ptr(x2), act_dtype(x2), (const float *)ptr(w), mut(out), act_dtype(out), (uint32_t)rows, (uint32_t)dim,
+                       (uint32_t)stride, eps, stream());
   return given(p[3]) ? ref(p[3]) : THPVariable_Wrap(out);
 }
 
@@ -359,6 +390,7 @@ PyObject *rmsnorm(PyObject *const *p) {   // x, weight, eps, out, out_dtype
 PyObject *attn_decode(PyObject *const *p) {
   const at::Tensor &q = tensor(p[0]), &k = tensor(p[1]), &v = tensor(p[2]), &par = tensor(p[3]), &ws = tensor(p[8]), &out = tensor(p[9]);
   const int64_t len = given(p[10]) && truth(p[10]) ? integer(p[10]) : k.size(0);
+  require(out.is_contiguous() && out.numel() >= integer(p[4]) * integer(p[6]), "attn_decode: out must have contiguous room for", integer(p[4]), integer(p[6]));
   call(cuthip_attn_decode, ptr(q), act_dtype(q), ptr(k), ptr(v), (const uint32_t *)ptr(par), mut(out), act_dtype(out), (uint32_t)integer(p[4]),
                            (uint32_t)integer(p[5]), (uint32_t)integer(p[6]), (uint32_t)k.stride(0), real(p[7]), (uint32_t)len, mut(ws),
                            (size_t)ws.numel(), stream());
@@ -367,6 +399,7 @@ PyObject *attn_decode(PyObject *const *p) {
 
 PyObject *silu_mul(PyObject *const *p) {   // gate_up, out
   const at::Tensor &g = tensor(p[0]), &out = tensor(p[1]);
+  if (!out.is_contiguous() || !g.is_contiguous() || g.numel() < 2 * out.numel()) fail("silu_mul: gate_up must hold two contiguous halves of the size of out");
   call(cuthip_silu_mul, ptr(g), act_dtype(g), mut(out), act_dtype(out), (uint32_t)out.numel(), stream());
   return ref(p[1]);
 }
@@ -402,6 +435,7 @@ PyObject *embedding_rows(PyObject *const *p) {   // w_blocks, fmt, token_ids, n_
   if ((ids.scalar_type() != at::kInt && ids.scalar_type() != at::kUInt32) || out.stride(-1) != 1 || out.numel() < ids.numel() * dim)
     fail("embedding_rows: token ids are 32-bit integers, out holds one row of dim per id");
   const at::Tensor out2 = out.dim() == 2 ? out : out.view({ids.numel(), -1});
+  require(holds(out2, ids.numel(), dim), "embedding_rows: out must have contiguous room for", ids.numel(), dim);
   call(cuthip_embedding_rows, format(p[1]), ptr(w), (const uint32_t *)ptr(ids), (uint32_t)ids.numel(), (uint32_t)rows, (uint32_t)dim, mut(out2),
                               act_dtype(out2), (uint32_t)out2.stride(0), stream());
   return ref(p[5]);
@@ -422,6 +456,7 @@ PyObject *matmul_sep(PyObject *const *p) {
     throw PyError{};
   }
   const at::Tensor out = given(p[6]) ? tensor(p[6]) : empty({M, N}, at::kFloat, in);
+  require(out.scalar_type() == at::kFloat && holds(out, M, N), "matmul_sep: out must be fp32 and have contiguous room for", M, N);
   Op e;
   if (given(p[7])) {
     e.epilogue = CUTHIP_EPI_UNARY;
@@ -430,7 +465,7 @@ PyObject *matmul_sep(PyObject *const *p) {
     const char *bad = "matmul_sep: binary epilogue needs an fp32 D with the shape and stride of C";
     if (!given(p[9])) fail(bad);
     const at::Tensor &d = tensor(p[9]);
-    if (d.sizes() != out.sizes() || d.scalar_type() != at::kFloat || d.stride(0) != out.stride(0)) fail(bad);
+    if (d.sizes() != out.sizes() || d.scalar_type() != at::kFloat || d.stride(0) != out.stride(0) || !holds(d, M, N)) fail(bad);
     e.epilogue = CUTHIP_EPI_BINARY;
     e.op = lookup(g_binary, p[8]);
     e.d = ptr(d);

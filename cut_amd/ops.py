@@ -55,6 +55,13 @@ def n_bytes(fmt, rows: int, cols: int) -> int:
     return rows * (cols // _l.BLOCK_ELEMS[f]) * _l.BLOCK_BYTES[f]
 
 
+def _holds(t: torch.Tensor, rows: int, width: int) -> bool:
+    """Whether a launch that writes rows of `width` elements, stride(0) apart, stays inside the rows of t."""
+    if t.dim() < 2:
+        return t.dim() == 1 and rows <= 1 and t.shape[0] >= width and (t.shape[0] <= 1 or t.stride(0) == 1)
+    return t.shape[0] >= rows and t.numel() >= t.shape[0] * width and (t.numel() == 0 or t[0].is_contiguous())
+
+
 def dequantize(raw: torch.Tensor, fmt, rows: int, cols: int, dtype: torch.dtype = torch.float32,
                out: torch.Tensor | None = None) -> torch.Tensor:
     """raw: 1-D uint8/int8 device tensor of GGUF blocks -> [rows, cols]."""
@@ -256,7 +263,10 @@ def repetition_penalty(logits: torch.Tensor, factors: torch.Tensor, out: torch.T
     """RepetitionPenaltyOpNode on the dense fp32 factor vector (1 for tokens that are not penalised)."""
     if logits.dtype != torch.float32 or factors.dtype != torch.float32 or logits.numel() != factors.numel():
         raise _l.CutHipError("RepetitionPenalty: logits and penaltyFactors must be fp32 tensors of the same shape")
-    out = torch.empty_like(logits) if out is None else out
+    if out is None:
+        out = torch.empty_like(logits)
+    elif out.dtype != torch.float32 or not out.is_contiguous() or out.numel() < logits.numel():
+        raise _l.CutHipError(f"RepetitionPenalty: out must hold {logits.numel()} contiguous fp32 elements")
     _l.check(_l.load().cuthip_repetition_penalty(logits.data_ptr(), factors.data_ptr(), out.data_ptr(), logits.numel(), _stream_ptr()))
     return out
 
@@ -303,6 +313,8 @@ def embedding_col(indices: torch.Tensor, matrix: torch.Tensor, scales: torch.Ten
         raise _l.CutHipError("embedding_col: matrix is 2-D fp16 (no scales) or int8 (fp16 scales), indices 32-bit integers")
     if out is None:
         out = torch.empty((indices.numel(), emb_dim), dtype=torch.float32, device=matrix.device)
+    elif out.dtype != torch.float32 or not _holds(out, indices.numel(), emb_dim):
+        raise _l.CutHipError(f"embedding_col: out must be fp32 and have contiguous room for {indices.numel()} rows of {emb_dim}")
     _l.check(_l.load().cuthip_embedding_col(indices.data_ptr(), matrix.data_ptr(), scales.data_ptr() if fmt else None, out.data_ptr(),
                                             indices.numel(), emb_dim, matrix.stride(0), scales.stride(0) if fmt else 0, out.stride(0),
                                             vocab, fmt, _stream_ptr()))
@@ -333,6 +345,8 @@ def matmul_dense_f16(a: torch.Tensor, w16: torch.Tensor, out_dtype: torch.dtype 
         raise _l.CutHipError("matmul_dense_f16: a must be fp32 / fp16 with contiguous rows")
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype or a2.dtype, device=a.device)
+    elif not _holds(out, M, N):
+        raise _l.CutHipError(f"matmul_dense_f16: out must have contiguous room for {M} rows of {N}")
     epi, op, dptr = _l.EPI_NONE, 0, None
     if unary is not None:
         epi, op = _l.EPI_UNARY, _l.UNARY[unary]
@@ -361,6 +375,8 @@ def matmul_q8_i8(a: torch.Tensor, w_blocks: torch.Tensor, N: int, K: int, out_dt
         raise _l.CutHipError(f"matmul_q8_i8: a must be fp32 / fp16 [M, {K}] with contiguous rows")
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype or a2.dtype, device=a.device)
+    elif not _holds(out, M, N):
+        raise _l.CutHipError(f"matmul_q8_i8: out must have contiguous room for {M} rows of {N}")
     epi, op, dptr = _l.EPI_NONE, 0, None
     if unary is not None:
         epi, op = _l.EPI_UNARY, _l.UNARY[unary]

@@ -79,3 +79,72 @@ def test_other_threads_run_while_a_launch_waits(tmp_path):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, "-c", WAITING, str(so)], cwd=root, capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "launched" in r.stdout, r.stderr[-2000:]
+
+
+M, K, N = 4, 32, 8
+# outputs the launch would write past: too few rows, too narrow ones, the columns of a wider one, the wrong strides, rows in one piece
+ROOM = {"rows": lambda n, **k: torch.zeros(M - 1, n, **k), "narrow": lambda n, **k: torch.zeros(M, n - 1, **k),
+        "part": lambda n, **k: torch.zeros(M, n, **k)[:, :n - 1], "columns": lambda n, **k: torch.zeros(n, M, **k).t(),
+        "every other": lambda n, **k: torch.zeros(M, 2 * n, **k)[:, ::2], "one block": lambda n, **k: torch.zeros(1, M * n, **k),
+        "batch": lambda n, **k: torch.zeros(1, M, n, **k)}
+
+
+@pytest.mark.parametrize("room", list(ROOM))
+def test_outputs_without_room_are_refused(room):
+    """Every operator that takes its output from the caller, before any launch."""
+    out, wide = ROOM[room](N), ROOM[room](32 * N)
+    a, w = torch.zeros(M, K), torch.zeros(M * N * K, dtype=torch.uint8)
+    ids = torch.zeros(M, dtype=torch.int32)
+    for call in (lambda: ops.matmul_gguf(a, w, "Q8_0", N, K, out=out), lambda: ops.matmul_gguf(a, w, "Q8_0", 2 * N, K, out=out, swiglu_pairs=True),
+                 lambda: ops.matmul_gguf(a, w, "Q8_0", N, K, out=out, binary="add", d=out),
+                 lambda: ops.matmul_sep(a, torch.zeros(K, N, dtype=torch.int8), torch.zeros(1, N, dtype=torch.float16), N, out=out),
+                 lambda: ops.rmsnorm(torch.zeros(M, 2 * N)[:, :N], torch.zeros(N), 1e-5, out=out),
+                 lambda: ops.matmul_dense_f16(a, torch.zeros(N, K, dtype=torch.float16), out=out), lambda: ops.matmul_q8_i8(a, w, N, K, out=out),
+                 lambda: ops.embedding_col(ids, torch.zeros(32 * N, 4, dtype=torch.float16), None, 32 * N, 4, out=wide)):
+        with pytest.raises(L.CutHipError):
+            call()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("room", list(ROOM))
+def test_dequantize_without_room_is_refused(room):
+    w = torch.zeros(M * 34, dtype=torch.uint8, device="cuda")
+    for dt, more in ((torch.float32, {}), (torch.float16, {}), (torch.float32, dict(dtype=torch.float16))):
+        out = ROOM[room](32, device="cuda", dtype=dt)
+        with pytest.raises(L.CutHipError):
+            ops.dequantize(w, "Q8_0", M, 32, **({"dtype": dt} | more), out=out)
+
+
+@pytest.mark.gpu
+def test_rmsnorm_of_rows_with_a_pitch_makes_its_own_output():
+    """The launch keeps the pitch of x: an output that the operator makes has it too."""
+    x = torch.randn(5, 24, device="cuda")
+    got = ops.rmsnorm(x[:, :16], torch.ones(16, device="cuda"), 1e-5)
+    want = x[:, :16] / torch.sqrt((x[:, :16].double() ** 2).mean(-1, keepdim=True) + 1e-5)
+    assert got.shape == (5, 16)
+    torch.testing.assert_close(got.double(), want, rtol=2e-6, atol=1e-7)
+
+
+def test_outputs_of_other_types_are_refused():
+    a, w = torch.zeros(M, K), torch.zeros(M * N * K, dtype=torch.uint8)
+    for dt in (torch.bfloat16, torch.int16, torch.int8, torch.float64):
+        with pytest.raises(L.CutHipError):
+            ops.matmul_gguf(a, w, "Q8_0", N, K, out_dtype=dt)
+        with pytest.raises(L.CutHipError):
+            ops.matmul_gguf(a, w, "Q8_0", N, K, out=torch.zeros(M, N, dtype=dt))
+        with pytest.raises(L.CutHipError):
+            ops.matmul_sep(a, torch.zeros(K, N, dtype=torch.int8), torch.zeros(1, N, dtype=torch.float16), N, out=torch.zeros(M, N, dtype=dt))
+
+
+def test_vectors_without_room_are_refused():
+    a, w, o = vectors()
+    x = torch.zeros(64)
+    with pytest.raises(L.CutHipError):
+        ops.silu_mul(x, torch.zeros(33))
+    with pytest.raises(L.CutHipError):
+        ops.attn_decode(x, x.half().view(1, 64), x.half().view(1, 64), torch.zeros(2, dtype=torch.int32), 1, 1, 64, 1.0,
+                        torch.zeros(4096, dtype=torch.uint8), torch.zeros(63))
+    with pytest.raises(L.CutHipError):
+        ops.repetition_penalty(x, x, out=torch.zeros(63))
+    with pytest.raises(L.CutHipError):
+        ops.embedding_rows(w, "Q8_0", torch.zeros(2, dtype=torch.int32), 8, 32, torch.zeros(1, 64))
