@@ -77,7 +77,14 @@ int lookup(PyObject *table, PyObject *key) {
   return (int)integer(v);
 }
 int format(PyObject *o) {
-  if (!PyUnicode_Check(o)) return (int)integer(o);
+  if (!PyUnicode_Check(o)) {   // any number, as int() takes it
+    PyObject *number = PyNumber_Long(o);
+    if (!number) throw PyError{};
+    const int64_t f = PyLong_AsLongLong(number);
+    Py_DECREF(number);
+    if (f == -1 && PyErr_Occurred()) throw PyError{};
+    return f == (int)f ? (int)f : -1;
+  }
   PyObject *v = PyDict_GetItemWithError(g_formats, o);
   if (!v) {
     if (!PyErr_Occurred()) PyErr_Format(g_error, "unknown quantization format %R", o);

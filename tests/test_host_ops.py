@@ -4,6 +4,7 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -148,3 +149,17 @@ def test_vectors_without_room_are_refused():
         ops.repetition_penalty(x, x, out=torch.zeros(63))
     with pytest.raises(L.CutHipError):
         ops.embedding_rows(w, "Q8_0", torch.zeros(2, dtype=torch.int32), 8, 32, torch.zeros(1, 64))
+
+
+def test_formats_are_names_or_numbers():
+    """As int() takes them; what follows is another check's error."""
+    raw = torch.zeros(144, dtype=torch.uint8)
+    for fmt in (2, 2.0, np.int64(2), np.float32(2.0), torch.tensor(2), True, "Q4_K"):
+        with pytest.raises(L.CutHipError, match="device tensor"):
+            ops.dequantize(raw, fmt, 1, 256)
+        assert ops.n_bytes(fmt, 1, 256) == 144
+    with pytest.raises(L.CutHipError, match="unknown quantization format"):
+        ops.dequantize(raw, "Q5_K", 1, 256)
+    for fmt, error in ((None, TypeError), (float("nan"), ValueError), (2.0j, TypeError)):
+        with pytest.raises(error):
+            ops.dequantize(raw, fmt, 1, 256)
