@@ -99,9 +99,13 @@ void block_of(int f, int64_t &elems, int64_t &bytes) {
   case CUTHIP_Q4_K: elems = 256; bytes = 144; return;
   case CUTHIP_Q6_K: elems = 256; bytes = 210; return;
   }
-  PyErr_SetObject(PyExc_KeyError, PyLong_FromLong(f));
+  if (PyObject *key = PyLong_FromLong(f)) {
+    PyErr_SetObject(PyExc_KeyError, key);
+    Py_DECREF(key);
+  }
   throw PyError{};
 }
+// more than any tensor holds for counts that are negative or whose product needs more than 64 bits
 int64_t n_bytes(int f, int64_t rows, int64_t cols) {
   int64_t elems, bytes;
   block_of(f, elems, bytes);
@@ -109,7 +113,9 @@ int64_t n_bytes(int f, int64_t rows, int64_t cols) {
     PyErr_Format(g_error, "cols (%lld) must be a multiple of the block size %lld", (long long)cols, (long long)elems);
     throw PyError{};
   }
-  return rows * (cols / elems) * bytes;
+  int64_t n;
+  if (rows < 0 || cols < 0 || __builtin_mul_overflow(cols / elems, bytes, &n) || __builtin_mul_overflow(rows, n, &n)) return INT64_MAX;
+  return n;
 }
 bool activation(const at::Tensor &t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kFloat; }
 int act_dtype(const at::Tensor &t) {

@@ -163,3 +163,11 @@ def test_formats_are_names_or_numbers():
     for fmt, error in ((None, TypeError), (float("nan"), ValueError), (2.0j, TypeError)):
         with pytest.raises(error):
             ops.dequantize(raw, fmt, 1, 256)
+
+
+@pytest.mark.parametrize("n", [2 ** 62, 2 ** 63 - 1, -1])
+def test_row_counts_that_no_tensor_holds(n):
+    """2^62 rows of 34 bytes are a negative number in 64 bits; the launch takes the lower 32 of what passes."""
+    a, w, _ = vectors()
+    with pytest.raises(L.CutHipError, match="too small"):
+        ops.matmul_gguf_pair(a, w, "Q8_0", n, None, w, "Q8_0", n, None, 32, rope=L.RopeAppend())
