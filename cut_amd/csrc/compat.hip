@@ -559,8 +559,12 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
   p.M = M; p.K = K; p.N = N; p.strideA = strideA; p.strideB = strideB; p.strideC = strideC; p.scaleStride = scaleStride;
   p.affine = affine;
   p.nsplit = (K + kSepWaves * kSepKC - 1) / (kSepWaves * kSepKC);
-  if (p.nsplit > 1 && (!workspace || workspace_bytes < (size_t)p.nsplit * M * N * sizeof(float))) {
-    set_error("%s: workspace of %zu bytes, need %zu", who, workspace_bytes, (size_t)p.nsplit * M * N * sizeof(float));
+  // Partial sums of all rows at once need `full` bytes; what cuthip_matmul_sep_workspace_bytes_for says may be less, from 32 rows on,
+  // where it is meant for the fp16 route and rows of A that are not 16-byte aligned end here.
+  const size_t bytes = workspace ? workspace_bytes : 0, per_row = p.nsplit > 1 ? (size_t)p.nsplit * N * sizeof(float) : 0, full = per_row * M;
+  const size_t said = cuthip_matmul_sep_workspace_bytes_for(q4 ? CUTHIP_OP_MATMUL_Q4 : CUTHIP_OP_MATMUL_Q8, variant, M, K, N);
+  if (bytes < per_row || (bytes < full && bytes < said)) {
+    set_error("%s: workspace of %zu bytes, need %zu", who, workspace_bytes, std::min(full, said));
     return CUTHIP_ERR_INVALID;
   }
   // One or two rows stay on the vector ALU: 14336 x 4096, us, both launches, vector kernel / matrix cores: int8 one row 16.9 / 19.2,
@@ -572,11 +576,20 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
       return r.nsplit == 1 ? CUTHIP_OK : launch_sep_reduce(r.partial, C, p.epi, M, N, strideC, 0, M, r.nsplit, stream);
     }
   }
-  // passes of up to 4 rows of A (8 rows would spill registers)
-  if (q4) return M == 1 ? launch_sep<true, 1>(p, workspace, stream) : M == 2 ? launch_sep<true, 2>(p, workspace, stream)
-                                                                             : launch_sep<true, 4>(p, workspace, stream);
-  return M == 1 ? launch_sep<false, 1>(p, workspace, stream) : M == 2 ? launch_sep<false, 2>(p, workspace, stream)
-                                                                      : launch_sep<false, 4>(p, workspace, stream);
+  // passes of up to 4 rows of A (8 rows would spill registers), as many rows at a time as the workspace holds
+  const uint32_t rows = bytes < full ? (uint32_t)(bytes / per_row) : M;
+  for (uint32_t m0 = 0; m0 < M; m0 += rows) {
+    p.M = std::min(rows, M - m0);
+    p.A = A + (size_t)m0 * strideA;
+    p.C = C + (size_t)m0 * strideC;
+    p.epi.D = D ? D + (size_t)m0 * strideC : nullptr;
+    const int rc = q4 ? (M == 1 ? launch_sep<true, 1>(p, workspace, stream) : M == 2 ? launch_sep<true, 2>(p, workspace, stream)
+                                                                                 : launch_sep<true, 4>(p, workspace, stream))
+                      : (M == 1 ? launch_sep<false, 1>(p, workspace, stream) : M == 2 ? launch_sep<false, 2>(p, workspace, stream)
+                                                                                  : launch_sep<false, 4>(p, workspace, stream));
+    if (rc) return rc;
+  }
+  return CUTHIP_OK;
 }
 
 }  // namespace cuthip

@@ -383,7 +383,7 @@ int cuthip_matmul_gguf_pro(int fmt, const void *W, const void *A, int a_dtype, v
  * epilogue / epilogue_op / D as in cuthip_matmul_gguf (MatMulFusion).
  * workspace: device scratch of cuthip_matmul_sep_workspace_bytes(M, K, N)
  * bytes, 256-byte aligned (may be NULL when that is 0).  Below 32 rows of A
- * (or when K is not a multiple of 128) the weights are streamed once per 32 rows
+ * (or when K is not a multiple of 128 or rows of A are not 16-byte aligned) the weights are streamed once per 32 rows
  * (N not a multiple of 8: per 4 rows) and the workspace holds split-K partial sums;
  * from 32 rows on the products are those of fp16 operands, fp32 accumulate (within
  * 1e-3 of the fp32 loop, normwise): with weights decoded as they are needed, or, where

@@ -153,6 +153,32 @@ def test_rows_on_rounded_operands(ops, kind, ks, M, K, N):
     assert normwise_rel_err(added - D, want) < 4e-6
 
 
+@pytest.mark.parametrize("kind", ["q8", "q4", "affine"])
+@pytest.mark.parametrize("N", [1040, 1036])
+@pytest.mark.parametrize("view", ["offset", "pitch"])
+def test_many_rows_that_are_not_aligned(ops, kind, N, view):
+    """Rows of A off the 16 bytes that the fp16 route from 32 rows on reads: exact products in the workspace of that route, which is
+    smaller than the vector kernel's partial sums of all rows (K / 128 x M x N x 4 bytes).  Columns in multiples of eight
+    take the matrix cores, others the vector kernel, some rows at a time.  Bounds as below 32 rows."""
+    M, K = 512, 4096
+    g = torch.Generator("cuda").manual_seed(N)
+    buf = torch.randn((M, K + 8), generator=g, device="cuda")
+    A = buf[:, 1:K + 1] if view == "offset" else torch.randn((M, K + 1), generator=g, device="cuda")[:, :K]
+    q4, affine = kind != "q8", kind == "affine"
+    B = torch.randint(0, 256, (K, N // 2 if q4 else N), generator=g, device="cuda", dtype=torch.uint8)
+    S = (torch.rand(((2 if affine else 1) * (K // 32), N), generator=g, device="cuda") * 0.02 + 0.001).half()
+    q = torch.stack((B & 15, B >> 4), -1).reshape(K, N).double() - 8 if q4 else B.view(torch.int8).double()
+    w = q * S[:K // 32].double().repeat_interleave(32, 0)
+    if affine:
+        w += S[K // 32:].double().repeat_interleave(32, 0)
+    want = (A.double() @ w).cpu().numpy()
+    B = B if q4 else B.view(torch.int8)
+    assert normwise_rel_err(ops.matmul_sep(A, B, S, N, q4=q4, affine=affine).cpu().numpy(), want) < 2e-6
+    D = torch.randn((M, N), generator=g, device="cuda")
+    got = ops.matmul_sep(A, B, S, N, q4=q4, affine=affine, binary="add", d=D)
+    assert normwise_rel_err((got - D).cpu().numpy(), want) < 4e-6
+
+
 def test_rows_on_the_matrix_cores_extreme_activations(ops):
     """Magnitudes from the smallest normal numbers to the largest, and an infinity: it reaches its own row alone, as infinity
     where the weight is not zero."""
