@@ -2,8 +2,8 @@
 //   C[m,n] = sum_k A[m,k] * w[k,n]
 // on the matrix cores, with products as exact as fp32 fused multiply-adds have them: an integer of 8 bits or less is a bf16
 // number, and an fp32 activation is the sum of three (its leading, middle and last eight significant bits), so the three
-// v_mfma_f32_16x16x32_bf16 of a fragment multiply without rounding and add in fp32.  One matrix instruction's k range is one
-// quantization block, whose sum is scaled in fp32 as in the vector kernel.
+// v_mfma_f32_16x16x32_bf16 of a fragment multiply without rounding and add in fp32 (below 2^-110 times 2^24: see split3).  One matrix
+// instruction's k range is one quantization block, whose sum is scaled in fp32 as in the vector kernel.
 //
 //   * A wave owns 128 columns and a range of blocks.  Lane (c, g) loads columns 8 c .. 8 c + 7 of the k-rows 8 g .. 8 g + 7
 //     of a block: 128 (nibbles: 64) contiguous bytes of each k-row per load.  Byte f of the eight rows is the lane's part of
@@ -45,26 +45,41 @@ __device__ __forceinline__ uint32_t upper_pair(float a, float b) {
 __device__ __forceinline__ float upper(float v) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u); }
 
 // Eight activations as three bf16 operands whose sum they are (8 + 8 + 8 significant bits, truncated each time, so that the
-// differences are exact).  An infinity is its first part alone: infinity minus itself would make the others NaN.
-__device__ __forceinline__ void split3(f32x4 x, f32x4 y, u32x4 &hi, u32x4 &mid, u32x4 &lo) {
-  float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]}, r[8], s[8];
-  bool inf = false;
+// differences are exact).  True for one of which that does not hold: a third part that is a NaN (infinity minus itself) or
+// subnormal (bf16 ends at 2^-133, so that below 2^-110 the last bits may be lost).
+__device__ __forceinline__ bool split3(f32x4 x, f32x4 y, u32x4 &hi, u32x4 &mid, u32x4 &lo) {
+  const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  float r[8], s[8];
+  bool odd = false;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     r[e] = v[e] - upper(v[e]);
-    inf |= __builtin_isinf(v[e]);
+    s[e] = r[e] - upper(r[e]);
+    odd |= __builtin_amdgcn_classf(s[e], 0x1 | 0x2 | 0x10 | 0x80);
   }
-  if (__builtin_amdgcn_ballot_w64(inf) != 0) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = __builtin_isinf(v[e]) ? 0.0f : r[e];
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) s[e] = r[e] - upper(r[e]);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     hi[e] = upper_pair(v[2 * e], v[2 * e + 1]);
     mid[e] = upper_pair(r[2 * e], r[2 * e + 1]);
     lo[e] = upper_pair(s[2 * e], s[2 * e + 1]);
+  }
+  return odd;
+}
+// For waves that hold such values: times `up` (2^24 makes every part of a subnormal number normal), and an infinity as its first
+// part alone.
+__device__ __forceinline__ void split3_odd(f32x4 x, f32x4 y, float up, u32x4 &hi, u32x4 &mid, u32x4 &lo) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float v[2], r[2], s[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      v[h] = (e < 2 ? x[2 * e + h] : y[2 * e + h - 4]) * up;
+      r[h] = __builtin_isinf(v[h]) ? 0.0f : v[h] - upper(v[h]);
+      s[h] = r[h] - upper(r[h]);
+    }
+    hi[e] = upper_pair(v[0], v[1]);
+    mid[e] = upper_pair(r[0], r[1]);
+    lo[e] = upper_pair(s[0], s[1]);
   }
 }
 
@@ -227,15 +242,51 @@ __global__ void __launch_bounds__(512, T == 1 ? 4 : 2) sep_rows_kernel(SepRowsPa
     for (int f = 0; f < 8; ++f) acc[t][f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 
+  // Where a wave holds numbers that split3 does not split exactly, activations and sums are held times 2^24, unless it also
+  // holds numbers that have no room above them (32 products of 2^64 2^24 127 times a scale of 2^16, sums of 2^100 times 2^24):
+  // beside those the small ones keep what bf16 has.
+  // (Kept over the blocks, or scaled back behind each: as the registers allow.  The other way round spills 59 of them on int8 and 2
+  // on affine weights with one tile; with two, nibbles take 3 % longer.)
+  constexpr bool kKeepUp = T > 1 || KIND == kSepQ8;
+  float up = 1.0f;
+  auto rescale = [&](float by) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int f = 0; f < 8; ++f) acc[t][f] *= by;
+  };
+
   auto work = [&](int d) __attribute__((always_inline)) {
     u32x4 hi[T], mid[T], lo[T];
     f32x4 sx[T];
+    auto sum = [&](int t) __attribute__((always_inline)) {   // of x over the block, in every column
+      const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+      if constexpr (Q4) sx[t] = mfma_bf16(hi[t], ones, mfma_bf16(mid[t], ones, mfma_bf16(lo[t], ones, zero)));
+    };
+    bool odd = false;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      split3(a[d][t][0], a[d][t][1], hi[t], mid[t], lo[t]);
-      if constexpr (Q4) {   // sums of x over the block, in every column
-        const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-        sx[t] = mfma_bf16(hi[t], ones, mfma_bf16(mid[t], ones, mfma_bf16(lo[t], ones, zero)));
+      odd |= split3(a[d][t][0], a[d][t][1], hi[t], mid[t], lo[t]);
+      sum(t);   // (one tile's beside the split of the next: behind both, 17 to 31 rows of nibbles take 4 % longer)
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) != 0 || up != 1.0f, 0)) {
+      bool large = false;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) large |= !(__builtin_fabsf(a[d][t][e >> 2][e & 3]) < 0x1p64f);
+#pragma unroll
+        for (int f = 0; f < 8; ++f)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) large |= !(__builtin_fabsf(acc[t][f][i]) < 0x1p100f);
+      }
+      const float was = up;
+      up = __builtin_amdgcn_ballot_w64(large) ? 1.0f : 0x1p24f;
+      if (up != was) rescale(up == 1.0f ? 0x1p-24f : 0x1p24f);
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        split3_odd(a[d][t][0], a[d][t][1], up, hi[t], mid[t], lo[t]);
+        sum(t);
       }
     }
     uint32_t n[8][2];   // Q4: nibbles of the even and the odd columns, a byte each
@@ -269,9 +320,14 @@ __global__ void __launch_bounds__(512, T == 1 ? 4 : 2) sep_rows_kernel(SepRowsPa
         }
       }
     }
+    if (!kKeepUp && __builtin_expect(up != 1.0f, 0)) {
+      rescale(0x1p-24f);
+      up = 1.0f;
+    }
   };
 
   sep_walk(s.b0, s.b1, request, work);
+  if (kKeepUp && __builtin_expect(up != 1.0f, 0)) rescale(0x1p-24f);
   sep_finish<T>(p, s, acc, lds);
 }
 

@@ -180,8 +180,8 @@ def test_many_rows_that_are_not_aligned(ops, kind, N, view):
 
 
 def test_rows_on_the_matrix_cores_extreme_activations(ops):
-    """Magnitudes from the smallest normal numbers to the largest, and an infinity: it reaches its own row alone, as infinity
-    where the weight is not zero."""
+    """Magnitudes from 1e-30 to 1e30 in one row tile, and an infinity: it reaches its own row alone, as infinity where the
+    weight is not zero."""
     M, K, N = 5, 64, 32
     rng = np.random.default_rng(5)
     A = (rng.standard_normal((M, K)) * np.array([1e-30, 1e-8, 1.0, 1e8, 1e30])[:, None]).astype(np.float32)
@@ -197,6 +197,37 @@ def test_rows_on_the_matrix_cores_extreme_activations(ops):
     np.testing.assert_array_equal(np.delete(inf, 2, 0), np.delete(got, 2, 0))
     with np.errstate(invalid="ignore"):
         np.testing.assert_array_equal(inf[2], np.where(B[9] == 0, np.nan, np.inf * B[9].astype(np.float32)))
+
+
+@pytest.mark.parametrize("kind", ["q8", "q4", "affine"])
+@pytest.mark.parametrize("M", [6, 20])
+def test_rows_on_the_matrix_cores_small_activations(ops, kind, M):
+    """Down to the smallest subnormal numbers, beside ordinary rows: 24 bits of every activation, as the fp32 multiply-adds have
+    them.  (Parts of such numbers lie below the smallest bf16; scales of 64 keep the results normal.)  One block for a wave and
+    several.  Then rows whose magnitude changes inside the range of a wave, from one to which the waves scale up to one that has no
+    room for that and back: what they hold is scaled with it."""
+    rng = np.random.default_rng(M)
+    N, q4, affine = 264, kind != "q8", kind == "affine"
+    size = np.array([1.0, 1e-34, 1e-36, 2e-38, 1e-40, 1e-43])[np.arange(M) % 6]
+    for K in (96, 4160):
+        S = np.full(((2 if affine else 1) * (K // 32), N), 64.0, np.float32)
+        if q4:
+            B = rng.integers(0, 256, (K, N // 2)).astype(np.uint8)
+            q = np.stack((B & 15, B >> 4), -1).reshape(K, N).astype(np.float64) - 8
+        else:
+            B = rng.integers(-127, 128, (K, N)).astype(np.int8)
+            q = B.astype(np.float64)
+        w = q * 64 + (64 if affine else 0)
+        A = (rng.standard_normal((M, K)) * size[:, None]).astype(np.float32)
+        for rows in (slice(None), slice(1, None, 6), slice(3, None, 6)):   # and rows of one size by themselves
+            a = np.ascontiguousarray(np.repeat(A[rows], 3, 0)[:M])
+            want, got = a.astype(np.float64) @ w, run(ops, a, B, S, N, q4=q4, affine=affine, variant=1)
+            for m in range(len(a)):
+                assert normwise_rel_err(got[m], want[m]) < 2e-6, (K, m, np.abs(a[m]).max())
+        for sizes in ((1e-36, 1.0, 1e25), (1e25, 1e-36, 1.0), (1e25, 1.0, 1e-36), (1e-36, 1e25, 1e-36)):
+            a = (A / size[:, None] * np.repeat(np.resize(sizes, K // 32), 32)[None]).astype(np.float32)
+            want, got = a.astype(np.float64) @ w, run(ops, a, B, S, N, q4=q4, affine=affine, variant=1)
+            assert normwise_rel_err(got, want) < 2e-6, (K, sizes)
 
 
 def test_affine_layout_from_q4k_requantizer(ops):
