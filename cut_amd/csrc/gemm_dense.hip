@@ -601,6 +601,9 @@ int launch_splitk_reduce(const float *partial, uint32_t ksplit, uint32_t M, uint
   return check_hip(hipGetLastError(), "split-K reduce launch");
 }
 
+// tiles that exist with 32 x 32 x 16 MFMAs too
+constexpr bool dense_has_mfma32(int bn, int wm) { return wm == 2 || bn == 224; }
+
 template <int BM, int BN, int WM = 2> static int launch_dense_bm(DenseParams p, hipStream_t stream) {
   p.mtiles = (p.M + BM - 1) / BM;
   p.ntiles = (p.N + BN - 1) / BN;
@@ -616,12 +619,14 @@ template <int BM, int BN, int WM = 2> static int launch_dense_bm(DenseParams p, 
     return CUTHIP_ERR_INVALID;
   }
   // the 16 x 16 x 32 kernel unless the tuning key dense_mfma16 = 0 asks for the 32 x 32 x 16 one (kept for comparison)
-  const bool mfma16 = g_tuning.dense_mfma16 != 0;
-  constexpr bool kBoth = WM == 2 || BN == 224;
-  if constexpr (kBoth) {
-    if (!mfma16) hipLaunchKernelGGL((gemm_dense_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
+  if (g_tuning.dense_mfma16 != 0) {
+    hipLaunchKernelGGL((gemm_dense16_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
+  } else if constexpr (dense_has_mfma32(BN, WM)) {
+    hipLaunchKernelGGL((gemm_dense_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
+  } else {   // (only where that tile is forced as well)
+    set_error("dense GEMM: the tile %d,%d has no 32 x 32 x 16 kernel (dense_mfma16 = 0)", BM, BN);
+    return CUTHIP_ERR_INVALID;
   }
-  if (mfma16 || !kBoth) hipLaunchKernelGGL((gemm_dense16_kernel<BM, BN, WM>), dim3((uint32_t)grid), dim3(256), 0, stream, p);
   return check_hip(hipGetLastError(), "dense gemm launch");
 }
 
@@ -658,6 +663,7 @@ static DenseShape pick_dense_shape(uint32_t M, uint32_t K, uint32_t N, int c_byt
   const double mn = (double)M * N;
   DenseShape best{0, 0, 1, 1e30};
   for (const auto &t : kTiles) {
+    if (g_tuning.dense_mfma16 == 0 && !g_tuning.dense_bn && !dense_has_mfma32(t.bn, t.bm == 256 && t.bn < 256 ? 4 : 2)) continue;
     for (uint32_t ks = 1; ks <= 8; ks *= 2) {
       if (g_tuning.dense_bn && (t.bm != g_tuning.dense_bm || t.bn != g_tuning.dense_bn || ks != (uint32_t)g_tuning.dense_ks) &&
           K % ((uint32_t)g_tuning.dense_ks * 128) == 0)

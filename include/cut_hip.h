@@ -114,9 +114,12 @@ int cuthip_init(int device);
 const char *cuthip_last_error(void);
 /* Forces a launch shape for tests and tuning sweeps, process-wide, until changed; value NULL or "" restores the
  * library's own choice.  Keys: "rows8_shape" = "rwg,kw" (8-row GEMV: row groups per workgroup, K ranges 1/2/4/8),
- * "gemv_shape" = "kp,waves" (fallback GEMV), "gemm_ksplit" = "n" (K ranges of the row-tile matmul, 1..16),
+ * "gemv_shape" = "kp,waves" (fallback GEMV), "gemm_ksplit" = "n" (K ranges of the row-tile matmul and of the
+ * several-row matmul on the separated layout, 1..16),
  * "rows_tile" = "t,nw" (row-tile matmul: 32 t rows of A and 32 nw weight rows per workgroup: nw 4 with t 1..4, nw 2 with t 1..2),
- * "dense_tile" = "bm,bn[,ksplit]" (256,224 / 128,448 / 128,256 / 256,256), "dense_mfma16" = "0" | "1",
+ * "dense_tile" = "bm,bn[,ksplit]" (256,128 / 256,160 / 256,192 / 256,224 / 256,256 / 128,256 / 128,448), "dense_mfma16" =
+ * "1" | "0" (16x16x32 or 32x32x16 MFMAs; the tiles of 256 by less than 224 exist with the former only: not chosen, and
+ * an error where they are forced, with "0"),
  * "dense_pf" = prefetch distance in slices.  Not synchronised with launches in flight on other threads.  The
  * reference's counterpart is the per-operator `spec` argument that its tests and op_bench pass
  * (operators/impl/matmul/MatMulOp.cpp:336-374); an unknown key or a malformed value is CUTHIP_ERR_INVALID. */

@@ -74,3 +74,21 @@ def test_line_between_row_tiles_and_two_passes(fmt, M, N, K, a_f16, rows, dense)
     f = FORMATS[fmt]
     row_tiles = cost("rows", f, M, K, N, a_f16, SCRATCH) + 0.12e-6 * M * N * (2 if a_f16 else 4)
     assert (cost("dense", f, M, K, N, a_f16) < row_tiles) == (dense < rows)
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 5120, 4096), (1024, 5120, 4096), (2048, 11008, 4096), (700, 5632, 2048)])
+def test_tiles_without_the_32x32x16_kernel_are_not_chosen_for_it(M, N, K):
+    """These shapes take tiles of 256 by 128, 160 or 192; a comparison of the two kernels compares them on a tile that both have."""
+    both = ("256,224", "128,448", "256,256", "128,256")
+    try:
+        best = cost("dense", lib.Q4_K, M, K, N, 1)
+        lib.set_tuning("dense_mfma16", "0")
+        without = cost("dense", lib.Q4_K, M, K, N, 1)
+        forced = []
+        for tile in both:
+            lib.set_tuning("dense_tile", tile)
+            forced.append(cost("dense", lib.Q4_K, M, K, N, 1))
+    finally:
+        lib.set_tuning("dense_mfma16", None)
+        lib.set_tuning("dense_tile", None)
+    assert best < without == min(forced)
