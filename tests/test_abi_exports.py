@@ -4,6 +4,7 @@ tables, argument validation).  No compute call is made here."""
 import ctypes as C
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -183,3 +184,14 @@ def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(L, "LIB_PATH", "/nonexistent/libcut_hip.so")
     with pytest.raises(L.CutHipError):
         L.load()
+
+
+def test_the_library_builds_without_torch():
+    """A caller of the C ABI needs the library alone: without torch in python3 make builds it and leaves the Python extension out."""
+    csrc = os.path.join(ROOT, "cut_amd", "csrc")
+
+    def plan(*more):
+        return subprocess.run(["make", "-n", "-B", "-C", csrc, *more], capture_output=True, text=True, check=True).stdout
+    assert "host_ops.cpp" in plan()
+    without = plan("TORCH=")
+    assert "host_ops.cpp" not in without and "-o ../libcut_hip.so" in without
