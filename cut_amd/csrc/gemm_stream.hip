@@ -416,12 +416,35 @@ static void stream_layout(uint32_t M, uint32_t K, uint32_t N, size_t scratch_byt
   *ksplit = (nsteps + *range_steps - 1) / *range_steps;
 }
 
-// workgroups and K ranges of a launch with this much scratch memory
-uint32_t stream_gemm_grid(uint32_t M, uint32_t K, uint32_t N, size_t scratch_bytes, uint32_t *ksplit) {
-  uint32_t rs;
-  stream_layout(M, K, N, scratch_bytes, &rs, ksplit);
-  const uint32_t rows = stream_block_rows(M, K, N);
-  return (N + rows - 1) / rows * *ksplit;
+// Whether Q8_0 takes this kernel by itself, with this much scratch memory.  Figures: us, the kernel that ran before this one / this one;
+// both round fp32 activations to fp16.
+bool stream_q8_preferred(uint32_t M, uint32_t K, uint32_t N, int a_f16, bool pairs, size_t scratch_bytes) {
+  uint32_t range_steps, ksplit;
+  stream_layout(M, K, N, scratch_bytes, &range_steps, &ksplit);
+  const uint64_t weights = (uint64_t)N * K;
+  const uint32_t rows = stream_block_rows(M, K, N), grid = (N + rows - 1) / rows * ksplit;
+  if (M <= 8) {
+    // In place of the 8-row GEMV (exact products as here).  8 rows: 14336 x 4096 19.8 / 17.0 (fp32 20.5 / 18.4), 4096 x 14336 20.7 / 18.7,
+    // 5120 x 5120 18.7 / 13.0, 10240 x 2048 11.1 / 9.9, but 4096 x 4096 8.7 / 10.4, 1 x 28672 x 4096 29.8 / 33.0.  Not with few
+    // workgroups: 8192 x 2560 (128) 9.7 / 10.6 (fp32 11.6 / 11.2), 8192 x 4096 without scratch 13.4 / 14.9, 7168 x 3584 (112) 12.9 / 14.9;
+    if (M < 5 || weights < 20000000 || grid < (a_f16 && ksplit == 1 ? 144u : 128u)) return false;
+    // nor on a short K that the GEMV takes in one round: 14336 x 1536 9.4 / 9.8, 16384 x 1536 9.6 / 10.2 (20480 x 1536 16.6 / 16.3);
+    if (K < 2048 && grid <= 256) return false;
+    if (ksplit == 1) return true;
+    // a split only where its workgroups nearly run at once (13824 x 5120, 432 of two ranges, 23.9 / 26.2), and not where the GEMV's own
+    // split suits it: 8192 x 4096 14.0 / 14.4 (fp32 16.8 / 14.6), 4096 x 5120 10.8 / 11.3 (12.8 / 11.7), 2048 x 11008 11.7 / 12.3.
+    if (grid > 320 || pairs) return false;
+    if (a_f16 && (K <= 4096 || (K <= 5120 && N <= 4096))) return false;
+    return ksplit <= 4 || weights >= 25000000;
+  }
+  // In place of the row-tile matmul (weights rounded to fp16, 2e-4 of the norm) or of 8-row passes: 16 x 4096 x 4096 11.8 / 10.6,
+  // 16 x 2048 x 2048 9.0 / 9.1, 16 x 9216 x 5120 (288 workgroups of two K ranges) 22.1 / 24.0; with two activation tiles from where
+  // its workgroups run at once and fill the chip: 32 x 11264 x 2048 13.6 / 13.2, 32 x 8192 x 8192 26.0 / 23.4; below that the two
+  // are level (17 / 24 / 32 rows of 5120 x 4096 14.1 / 13.6, 13.5 / 13.8, 14.0 / 14.4; of 4096 x 5120 13.9 / 13.2, 14.7 / 14.1, 15.5 / 14.3; of
+  // 8192 x 2048 12.2 / 11.6, 11.4 / 11.9, 11.5 / 12.1; 32 x 4096 x 4096 12.6 / 12.1).  32 x 18432 x 4096 (288 workgroups) 33.1 / 35.8,
+  // 32 x 6144 x 6144 (144) 20.5 / 21.3.  Exact weights are kept inside these lines also where they cost time: 16 x 20480 x 1024
+  // 10.8 / 12.5, 16 x 32000 x 2048 19.1 / 20.1, 32 x 10240 x 2560 13.6 / 15.8, 32 x 12288 x 2048 with fp32 activations 13.2 / 14.3.
+  return weights >= (M > 16 ? 22000000u : 16000000u) && (M <= 16 || grid >= 160) && (grid <= 256 || (M <= 16 && ksplit == 1));
 }
 
 bool stream_gemm_fits(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A) {

@@ -141,7 +141,7 @@ int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C,
                       int use_blaslt);
 bool stream_gemm_fits(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A);
 size_t stream_gemm_scratch(uint32_t M, uint32_t K, uint32_t N);
-uint32_t stream_gemm_grid(uint32_t M, uint32_t K, uint32_t N, size_t scratch_bytes, uint32_t *ksplit);
+bool stream_q8_preferred(uint32_t M, uint32_t K, uint32_t N, int a_f16, bool pairs, size_t scratch_bytes);
 int launch_stream_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
                        uint32_t strideA, uint32_t strideC, Epilogue epi, void *scratch, size_t scratch_bytes, hipStream_t stream);
 bool blaslt_available();
@@ -276,24 +276,7 @@ static bool stream_preferred(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32
   if (!scratch || (uintptr_t)scratch % 16 != 0) scratch_bytes = 0;
   if (M > 32 || !cuthip::stream_gemm_fits(fmt, M, K, N, strideA, a_f16, A)) return false;
   if (fmt == CUTHIP_Q8_0) {
-    // us, this kernel and the one before it (both round fp32 activations).  Up to 8 rows in place of the 8-row GEMV: 8 x 14336 x 4096
-    // 17.0 / 19.8 (fp32 18.4 / 20.5), 8 x 4096 x 14336 19.0 / 21.6, 8 x 5120 x 5120 14.6 / 20.0, 8 x 10240 x 2048 10.2 / 11.4, but
-    // 8 x 4096 x 4096 10.4 / 8.7, with fp16 activations and a split of a short K 8 x 8192 x 4096 14.4 / 14.0 (fp32 14.6 / 16.8), and
-    // 8 x 7168 x 3584 (112 workgroups) 14.9 / 12.9, 8 x 13824 x 5120 (432 of two K ranges) 26.2 / 23.9, 1 x 28672 x 4096 33.0 / 29.8.
-    // 9 rows and more in place of the row-tile matmul or of 8-row passes: 16 x 4096 x 4096 10.6 / 11.8,
-    // 16 x 2048 x 2048 9.1 / 9.0, 16 x 9216 x 5120 (288 workgroups of two K ranges) 24.0 / 22.1; with two activation tiles wherever its
-    // workgroups run at once and fill the chip: 32 x 11264 x 2048 13.2 / 13.6,
-    // 32 x 8192 x 8192 23.4 / 26.0, 32 x 4096 x 4096 12.6 / 12.2; 32 x 18432 x 4096 (288 workgroups) 35.8 / 33.1,
-    // 32 x 6144 x 6144 (144) 21.3 / 20.5.
-    const uint64_t weights = (uint64_t)N * K;
-    uint32_t ksplit;
-    const uint32_t grid = cuthip::stream_gemm_grid(M, K, N, scratch_bytes, &ksplit);
-    if (M <= 8) {
-      if (M < 5 || weights < 20000000 || grid < 128) return false;
-      if (ksplit > 1 && (grid > 320 || (a_f16 && K <= 4096) || epilogue == CUTHIP_EPI_SWIGLU_PAIRS)) return false;
-    } else {
-      if (weights < (M > 16 ? 22000000 : 16000000) || (M > 16 && grid < 160) || (grid > 256 && (M > 16 || ksplit > 1))) return false;
-    }
+    if (!cuthip::stream_q8_preferred(M, K, N, a_f16, epilogue == CUTHIP_EPI_SWIGLU_PAIRS, scratch_bytes)) return false;
   } else if (M < 9 || N < 2048) {
     // (few weight rows: too few workgroups for it; 1024 x 4096 at 16-32 rows 11.6-13.3 us against 8.2-8.4 for the row-tile matmul)
     return false;

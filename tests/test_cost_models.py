@@ -92,3 +92,18 @@ def test_tiles_without_the_32x32x16_kernel_are_not_chosen_for_it(M, N, K):
         lib.set_tuning("dense_mfma16", None)
         lib.set_tuning("dense_tile", None)
     assert best < without == min(forced)
+
+
+# measured: (rows, N, K, fp16 activations, scratch memory, 8-row GEMV, streaming matmul)
+STREAM_LINE = [(8, 14336, 4096, 1, 1, 19.7, 16.9), (8, 14336, 4096, 0, 1, 19.4, 16.9), (8, 4096, 14336, 1, 1, 20.7, 18.7), (8, 5120, 5120, 1, 1, 18.7, 13.0),
+               (5, 10240, 2048, 1, 0, 11.1, 10.0), (8, 3072, 11008, 1, 1, 19.9, 16.6), (8, 2560, 8192, 1, 1, 17.3, 11.8), (8, 20480, 1536, 1, 1, 16.6, 16.3),
+               (8, 8192, 2560, 1, 1, 9.8, 10.7), (8, 8192, 2560, 0, 1, 11.7, 11.3), (5, 8192, 3072, 1, 0, 10.1, 11.5), (8, 8192, 4096, 1, 0, 13.4, 14.9),
+               (6, 14336, 1536, 0, 1, 9.6, 10.2), (8, 16384, 1536, 1, 1, 9.6, 10.2), (8, 4096, 5120, 1, 1, 10.8, 11.3), (8, 4096, 5120, 0, 1, 12.8, 11.7),
+               (8, 2048, 11008, 1, 1, 11.7, 12.3), (8, 2048, 11008, 0, 1, 12.1, 12.7), (8, 2048, 14336, 1, 1, 14.3, 13.2)]
+
+
+@pytest.mark.parametrize("M,N,K,a_f16,scratch,gemv,stream", STREAM_LINE)
+def test_line_between_the_8_row_gemv_and_the_streaming_matmul_on_q8_0(M, N, K, a_f16, scratch, gemv, stream):
+    f = lib.load()._ZN6cuthip19stream_q8_preferredEjjjibm
+    f.restype, f.argtypes = C.c_bool, [C.c_uint32, C.c_uint32, C.c_uint32, C.c_int, C.c_bool, C.c_size_t]
+    assert f(M, K, N, a_f16, False, SCRATCH if scratch else 0) == (stream < gemv)
