@@ -351,7 +351,6 @@ int launch_dense_gemm(int fmt, const void *W, const void *A, int a_f16, void *C,
 int launch_cvt_rows(const float *A, half_t *A16, uint32_t M, uint32_t K, uint32_t strideA, hipStream_t stream);
 int launch_splitk_reduce(const float *partial, uint32_t ksplit, uint32_t M, uint32_t N, void *C, uint32_t strideC, Epilogue epi,
                          int c_f16, hipStream_t stream);
-double sep_two_pass_us(uint32_t M, uint32_t K, uint32_t N);
 
 static size_t sep_w16_bytes(uint32_t K, uint32_t N) { return ((size_t)N * K * 2 + 255) & ~(size_t)255; }
 static bool sep_dense_fits(uint32_t K, uint32_t N, uint32_t M) {
@@ -531,7 +530,7 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
       SepRowsParams r{A, reinterpret_cast<const uint8_t *>(B), reinterpret_cast<const uint16_t *>(S), C,
                       reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(workspace) + a16), epi, M, K, N, strideA, strideB, strideC,
                       scaleStride, reinterpret_cast<const half_t *>(workspace)};
-      if (sep_rows16_cut(r, q4, affine != 0, workspace_bytes - a16) && r.cost_us < sep_two_pass_us(M, K, N)) {
+      if (sep_rows16_preferred(r, q4, affine != 0, workspace_bytes - a16)) {
         if (int rc = launch_cvt_rows(A, reinterpret_cast<half_t *>(workspace), M, K, strideA, stream)) return rc;
         if (int rc = launch_sep_rows16(r, q4, affine != 0, stream)) return rc;
         return r.nsplit == 1 ? CUTHIP_OK : launch_splitk_reduce(r.partial, r.nsplit, M, N, C, strideC, epi, 0, stream);

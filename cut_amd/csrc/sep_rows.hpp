@@ -22,6 +22,7 @@ struct SepRowsParams {
 // more than K / 128 rounded up).
 bool sep_rows_cut(SepRowsParams &p, size_t partial_bytes);
 bool sep_rows16_cut(SepRowsParams &p, bool q4, bool affine, size_t partial_bytes);
+bool sep_rows16_preferred(SepRowsParams &p, bool q4, bool affine, size_t partial_bytes);   // cut, and the cheaper of the two ways
 int launch_sep_rows(const SepRowsParams &p, bool q4, bool affine, hipStream_t stream);
 int launch_sep_rows16(const SepRowsParams &p, bool q4, bool affine, hipStream_t stream);
 

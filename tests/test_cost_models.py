@@ -107,3 +107,25 @@ def test_line_between_the_8_row_gemv_and_the_streaming_matmul_on_q8_0(M, N, K, a
     f = lib.load()._ZN6cuthip19stream_q8_preferredEjjjibm
     f.restype, f.argtypes = C.c_bool, [C.c_uint32, C.c_uint32, C.c_uint32, C.c_int, C.c_bool, C.c_size_t]
     assert f(M, K, N, a_f16, False, SCRATCH if scratch else 0) == (stream < gemv)
+
+
+class SepRowsParams(C.Structure):
+    _fields_ = ([(n, C.c_void_p) for n in ("A", "B", "S", "C", "partial")] + [("kind", C.c_int), ("op", C.c_int), ("D", C.c_void_p)] +
+                [(n, C.c_uint32) for n in ("M", "K", "N", "strideA", "strideB", "strideC", "scaleStride")] + [("A16", C.c_void_p)] +
+                [(n, C.c_uint32) for n in ("t", "nsplit", "per", "tiles", "passes")] + [("cost_us", C.c_double)])
+
+
+# measured: (layout, rows, N, K, two passes, weights decoded as they are needed)
+SEP_LINE = [("q8", 64, 256, 256, 12.9, 16.6), ("q8", 512, 512, 256, 14.5, 17.5), ("q4", 128, 96, 256, 13.5, 14.7), ("affine", 64, 512, 256, 13.3, 15.3),
+            ("q8", 64, 512, 512, 15.5, 15.3), ("q8", 512, 512, 512, 18.0, 16.7), ("q4", 512, 14336, 4096, 110.0, 114.7), ("q4", 384, 14336, 4096, 106.4, 113.2),
+            ("affine", 384, 14336, 4096, 110.5, 118.9), ("q8", 64, 14336, 4096, 86, 34), ("q8", 256, 4096, 4096, 47, 32), ("q4", 512, 1024, 512, 18.4, 16.3)]
+
+
+@pytest.mark.parametrize("layout,M,N,K,two,direct", SEP_LINE)
+def test_line_between_two_passes_and_direct_decoding_on_the_separated_layout(layout, M, N, K, two, direct):
+    so, q4 = lib.load(), layout != "q8"
+    f = so._ZN6cuthip20sep_rows16_preferredERNS_13SepRowsParamsEbbm
+    f.restype, f.argtypes = C.c_bool, [C.POINTER(SepRowsParams), C.c_bool, C.c_bool, C.c_size_t]
+    p = SepRowsParams(M=M, K=K, N=N, strideA=K, strideB=N // 2 if q4 else N, strideC=N, scaleStride=N)
+    room = so.cuthip_matmul_sep_workspace_bytes_for(lib.OP_MATMUL_Q4 if q4 else lib.OP_MATMUL_Q8, -1, M, K, N) - ((M * K * 2 + 255) & ~255)
+    assert f(C.byref(p), q4, layout == "affine", room) == (direct < two)
