@@ -653,7 +653,9 @@ constexpr size_t kDenseScratch = (size_t)32 << 20;
 // weight shapes from 1024 x 4096 to 32000 x 2048, every tile forced in turn, graph replay; 6 % rms, the shape chosen is 0.7 % slower
 // than the best of them on average).  Microseconds: a part for each round of 256 workgroups, K x the tile's area x its cost per
 // multiply-add, once more a little of it for a full chip (clocks), C; a K split writes and reads its partial products and is a
-// second launch.  Edge tiles count in full, so that narrower tiles win where they fit the rows of W or the CUs better (us, widest
+// second launch (its two terms fitted to 1,325 more of 1 .. 768 rows on 16 weight shapes from 256 x 256 to 4096 x 14336, where the
+// shape chosen is 0.5 % slower than the best, with those of the larger calls 2.0 %; us, without the split / with it: 1 x 512 x 512
+// 10.1 / 8.8, 64 x 512 x 512 11.0 / 10.0, 200 fp32 rows 15.3 / 13.2).  Edge tiles count in full, so that narrower tiles win where they fit the rows of W or the CUs better (us, widest
 // tiles in the order of one panel per eight XCDs -> this): 2048 x 5120 x 4096 107 -> 73 (256 x 160), 1024 x 5120 x 4096 105 -> 57
 // (256 x 128), 512 x 11008 x 4096 117 -> 59, 2048 x 11008 x 4096 222 -> 167 (256 x 192), 2048 x 2560 x 2560 63 -> 40,
 // 700 x 5632 x 2048 59 -> 34; 2048 x 14336 x 4096 stays with 256 x 224.
@@ -674,7 +676,7 @@ static DenseShape pick_dense_shape(uint32_t M, uint32_t K, uint32_t N, int c_byt
       if (ks > 1 && (K % (ks * 128) != 0 || (!g_tuning.dense_bn && (t.bm != 128 || t.bn != 256 || tiles > 256 || ks * mn * 4 > (double)kDenseScratch)))) break;
       const double full = (double)((tiles - 1) / 256), part = (tiles - 256.0 * full) / 256.0;
       double us = 0.3 + 5.25 * (full + 1.0) + 0.37e-6 * mn * c_bytes + (double)K / ks * t.bm * t.bn * (t.mac * (full + 1.0) + t.full * (full + part));
-      if (ks > 1) us += 5.2 + 0.95e-6 * ks * mn;
+      if (ks > 1) us += 2.5 + 1.5e-6 * ks * mn;
       if (us < best.us) best = DenseShape{t.bm, t.bn, ks, us};
     }
   }

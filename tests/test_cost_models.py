@@ -117,7 +117,7 @@ class SepRowsParams(C.Structure):
 
 # measured: (layout, rows, N, K, two passes, weights decoded as they are needed)
 SEP_LINE = [("q8", 64, 256, 256, 12.9, 16.6), ("q8", 512, 512, 256, 14.5, 17.5), ("q4", 128, 96, 256, 13.5, 14.7), ("affine", 64, 512, 256, 13.3, 15.3),
-            ("q8", 64, 512, 512, 15.5, 15.3), ("q8", 512, 512, 512, 18.0, 16.7), ("q4", 512, 14336, 4096, 110.0, 114.7), ("q4", 384, 14336, 4096, 106.4, 113.2),
+            ("q8", 64, 512, 512, 14.5, 15.5), ("q8", 48, 512, 512, 14.0, 13.7), ("q8", 200, 1024, 512, 16.6, 16.2), ("q4", 512, 14336, 4096, 110.0, 114.7), ("q4", 384, 14336, 4096, 106.4, 113.2),
             ("affine", 384, 14336, 4096, 110.5, 118.9), ("q8", 64, 14336, 4096, 86, 34), ("q8", 256, 4096, 4096, 47, 32), ("q4", 512, 1024, 512, 18.4, 16.3)]
 
 
@@ -129,3 +129,20 @@ def test_line_between_two_passes_and_direct_decoding_on_the_separated_layout(lay
     p = SepRowsParams(M=M, K=K, N=N, strideA=K, strideB=N // 2 if q4 else N, strideC=N, scaleStride=N)
     room = so.cuthip_matmul_sep_workspace_bytes_for(lib.OP_MATMUL_Q4 if q4 else lib.OP_MATMUL_Q8, -1, M, K, N) - ((M * K * 2 + 255) & ~255)
     assert f(C.byref(p), q4, layout == "affine", room) == (direct < two)
+
+
+# measured on resident fp16 weights: (rows, N, K, K split, us, one range, us)
+SPLIT_LINE = [(1, 512, 512, "128,256,4", 8.8, "256,128", 10.1), (64, 512, 512, "128,256,4", 10.0, "256,128", 11.0), (64, 1024, 1024, "128,256,4", 12.2, "128,256", 16.4)]
+
+
+@pytest.mark.parametrize("M,N,K,split,us,whole,more", SPLIT_LINE)
+def test_small_problems_split_k(M, N, K, split, us, whole, more):
+    try:
+        chosen = cost("dense", lib.Q4_K, M, K, N, 1)
+        forced = {}
+        for tile in (split, whole):
+            lib.set_tuning("dense_tile", tile)
+            forced[tile] = cost("dense", lib.Q4_K, M, K, N, 1)
+    finally:
+        lib.set_tuning("dense_tile", None)
+    assert chosen <= forced[split] < forced[whole]
