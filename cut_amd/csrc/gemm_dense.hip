@@ -710,12 +710,13 @@ static double two_pass_us(double decode_us, uint32_t M, uint32_t K, uint32_t N, 
 
 double dense_cost_us(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16) {
   // The factor sets this sum against the estimate of the row-tile matmul: over 1,040 calls of 224 .. 2048 rows on ten weight shapes
-  // (four formats, both activation types) the sum comes out 6 per cent high and that estimate 6 per cent low; Q6_K, whose 210-byte
-  // blocks are slower to take apart, is held at the row tiles where the two are level (640 x 11008 x 4096 94 us either way).  The
-  // choice is 0.3 per cent slower than the better of the two on average.  The row-tile matmul decodes every weight once per 128
-  // rows and this path once, so the line runs at about 450 rows on wide matrices and 32000 x 2048, at 600 on 4096 x 14336, at
-  // 1,300 on 4096 x 4096.
-  return (fmt == CUTHIP_Q6_K ? 1.01 : 0.88) *
+  // (four formats, both activation types) the sum comes out 6 per cent high and that estimate 6 per cent low; on Q6_K, whose 210-byte
+  // blocks are slower to take apart, less so.  Over 1,536 more (200 .. 2048 rows, 15 shapes) the choice is 0.1 to 0.2 per cent slower
+  // (Q6_K 0.3) than the better of the two on average and 12 at most; with Q6_K held at the row tiles (1.01) it was 0.6 and 19 there (us, row
+  // tiles / two passes: 512 x 14336 x 4096 98 / 90, 2048 x 2048 x 2048 with fp32 activations 50.5 / 43.8, 768 x 8192 x 2048 47.8 / 42.8).
+  // The row-tile matmul decodes every weight once per 128 rows and this path once, so the line runs at about 450 rows on wide
+  // matrices and 32000 x 2048, at 600 on 4096 x 14336, at 1,300 on 4096 x 4096.
+  return (fmt == CUTHIP_Q6_K ? 0.95 : 0.88) *
          two_pass_us(5.0 + (double)N * K * ((double)fmt_bytes(fmt) / fmt_elems(fmt) + 2.0) / 5.14e6, M, K, N, a_f16);
 }
 
