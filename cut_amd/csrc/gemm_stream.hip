@@ -11,8 +11,8 @@
 // scale of the sub-block (for the upper nibbles a sixteenth of it) is multiplied in as fp16, q * sc below 1024 in units of 2^-24, exact.
 // A mask thus takes two weights out of a dword, the eighth byte apart (the activations lie in LDS in that order), and all eight
 // sub-blocks accumulate in one MFMA chain; the fp32 super-block scale d * 2^24 is applied once per step.  The "- dmin * m" term needs
-// only the activations' sums over the sub-blocks: they are formed once, while the activations are staged, as two halves of 11 bits
-// each, and one MFMA multiplies those of a super-block with the eight 6-bit minima.  Products and sums are therefore those of the
+// only the activations' sums over the sub-blocks: they are formed once, while the activations are staged, as two halves (the second
+// what rounding to the first leaves, with its sign: 24 bits together), and one MFMA multiplies those of a super-block with the eight 6-bit minima.  Products and sums are therefore those of the
 // fp32 reference expression (d * sc) * q - dmin * m up to the order of the fp32 additions: 3e-7 normwise against 64 bits, where a
 // chain of products with the minima, which cancels against the first, had 1e-6 to 3e-6.
 //
@@ -26,14 +26,16 @@
 // of the two-pass GEMM, which applies the epilogue).  After the staging barrier the loop has no barrier: each lane
 // keeps kStreamDepth steps of weight loads in flight in a register ring and waits only for the step it multiplies.
 //
-// Bound by the vector instructions of the unpack and by the staging, well before HBM.  Measured (MI355X, HIP-graph replay, fp16
-// activations): Q4_K 14336 x 4096 at 9 / 16 / 24 / 32 rows 12.5 / 13.1 / 17.0 / 17.9 us (with eight pieces of 8 bytes per lane, integer
-// products and the minima as a second chain of eight products 14.1 / 14.5 / 19.7 / 19.9), 28672 x 4096 22.1 / 23.2 / 28.4 / 30.0
-// (25.3 / 25.9 / 33.7 / 34.1), 2048 x 2048 7.8 / 7.9 / 9.6 / 10.2 (8.8 / 9.1 / 11.0 / 11.2).  A sum per piece as it is staged, every
-// fourth thread storing one, took back 1.5 us of it at 16 rows and 2 at 32: hence four pieces at a time, a sum to every thread.
-// Q8_0 14336 x 4096 at 8 / 16 / 24 / 32 rows 17.4 / 18.0 / 22.0 / 22.6 us (8-row GEMV 19.8, row-tile matmul 22.7 / 22.6 / 23.0),
-// 4096 x 14336 19.6 / 20.1 / 22.2 / 22.7 (21.6; 22.6 / 23.1 / 23.8), 28672 x 4096 at 8 / 16 rows 34.2 / 34.8 (37.9; 37.3).
-// Q4_K at 8 rows and fewer: the 8-row GEMV is as fast for the widest matrices and faster for all others.
+// Q4_K is bound by the vector instructions of the unpack (47 % of the time at 16 and at 32 rows) and by the staging in front of the loop
+// (waits 43 %), well before HBM (2.6 TB/s); Q8_0 by HBM (3.5 of the 4.8 TB/s of a copy) beside 31 to 34 % of vector instructions and LDS
+// bank conflicts in the strip (15 to 19 %).  Measured (MI355X, HIP-graph replay, fp16 activations): Q4_K 14336 x 4096 at 9 / 16 / 24 / 32
+// rows 12.4 / 12.7 / 17.0 / 17.2 us (with eight pieces of 8 bytes per lane, integer products and the minima as a second chain of eight
+// products 14.1 / 14.5 / 19.7 / 19.9), 28672 x 4096 23.2 / 23.6 / 28.4 / 29.7 (25.3 / 25.9 / 33.7 / 34.1), 4096 x 4096 8.5 / 8.8 / 10.3 /
+// 10.3 (11.2 / 11.6 / 13.2 / 13.7).  A sum per piece as it is staged, every fourth thread storing one, took back 1.5 us of it at 16 rows
+// and 2 at 32: hence four pieces at a time, a sum to every thread.  Q8_0 14336 x 4096 at 8 / 16 / 24 / 32 rows 17.6 / 17.8 / 21.6 / 22.3 us
+// (8-row GEMV 19.8, row-tile matmul 22.7 / 22.6 / 23.0), 4096 x 14336 19.6 / 20.3 / 22.1 / 22.1 (20.7; 22.6 / 23.1 / 23.8), 28672 x 4096
+// at 8 / 16 rows 32.6 / 32.7 (36.1; 37.3).  Q4_K at 8 rows and fewer: the 8-row GEMV is as fast for the widest matrices and faster for
+// all others.
 #include <type_traits>
 
 #include "common.hpp"
@@ -59,7 +61,7 @@ struct StreamParams {
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) uint8_t lds_u8s;
 
-constexpr int kStreamDepth = 2;   // steps of weight loads in flight per lane (14336 x 4096 at 16 rows, two / three / four: Q4_K 13.1 / 13.4 / 14.3 us, Q8_0 17.6 / 19.7 / 19.9)
+constexpr int kStreamDepth = 2;   // steps of weight loads in flight per lane (14336 x 4096 at 16 rows, two / three / four: Q4_K 12.7 / 13.0 / 13.5 us, Q8_0 17.8 / 20.0 / 23.9)
 constexpr uint32_t kStripBytes = 144 * 16;          // LDS per wave for the blocks of a step
 constexpr uint32_t kStreamLdsMax = 132 * 1024;     // staged activations: 16 rows of 4096 (the strips of eight waves and the sums take 26 KB more)
 
@@ -101,7 +103,7 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams 
   // c % 9, by lanes c, c - 64, c - 128: neighbouring lanes read neighbouring bytes, every cache line is requested
   // once.  (Fetched in the operand layout - 8 bytes per lane, the four lanes of a row 16 lanes apart - every line
   // was requested four times: 17.6 us against 15.7 for 14336 x 4096 at 16 rows.)  The pieces go through a wave-private
-  // strip of LDS, from which each lane picks its row's header and its 8 bytes of every 32-byte group.
+  // strip of LDS, from which each lane picks its row's header and its 16 bytes of either half of the quants.
   // Q8_0 (17 pieces a row): parts 0-7, parts 9-16 and, by 16 lanes, part 8 of every row, as the strip holds half a step at a time.
   constexpr uint32_t kStepBytes = Q4K ? 144 : 272;
   const uint8_t *piece[NP];
@@ -176,7 +178,7 @@ __global__ void __launch_bounds__(64 * RG * KW) gemm_stream_kernel(StreamParams 
       const float s = ((b1 ? s23 : s01) + lane_xor2(b1 ? s01 : s23)) * 0.03125f;   // of this thread's sub-block, / 32
       const uint32_t c = base + (uint32_t)(i0 + (tid & 3)) * THREADS + (uint32_t)(tid & ~3);
       if (c < chunks) {
-        // in two parts of 11 bits: part h of sub-block j of a step to lane group 2 ((j >> 1) & 1) + h
+        // in two parts (24 bits together): part h of sub-block j of a step to lane group 2 ((j >> 1) & 1) + h
         const uint32_t r = __umulhi(c, inv), col = c - r * cpr, j = (col >> 2) & 7;
         half_t *dst = reinterpret_cast<half_t *>(lds + sums0 + r * spitch + (col >> 5) * 32 + 16 * ((j >> 1) & 1)) + 2 * (j >> 2) + (j & 1);
         const half_t lead = (half_t)s;

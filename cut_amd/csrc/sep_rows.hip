@@ -12,8 +12,10 @@
 //     barrier until the ranges of the workgroup meet at the end.
 //   * Two blocks of loads are in flight per wave, in a ring of registers.
 //
-// What bounds it: the memory up to 16 rows (about 180 vector instructions and 24 matrix instructions a block and wave, 4 KB of
-// int8), the vector ALU beyond (44 instructions to split 16 rows, 32 to scale their results).  Measured, us, both launches
+// What bounds it (14336 x 4096): int8 up to 16 rows the memory (3.4 of the 4.8 TB/s of a copy, vector ALU 41 % of the time: about 210
+// vector instructions and 24 matrix instructions a block and wave, 4 KB of int8), nibbles the vector ALU (56 to 59 %), and int8 beyond
+// 16 rows it (46 %: 44 instructions to split 16 rows, 32 to scale their results) beside chains of three matrix instructions (28 %).  Measured,
+// us, both launches
 // (graph replay, weights from memory), passes of four rows on the vector ALU -> this kernel:
 //   14336 x 4096  int8     4 rows 22.3 -> 19.7,  8 rows 33.4 -> 20.3,  16 rows 54.5 -> 21.9,  31 rows 96.5 -> 29.5
 //                 nibbles  4 rows 19.3 -> 18.0,  8 rows 31.6 -> 18.4,  16 rows 53.8 -> 19.9,  31 rows 96.0 -> 28.7

@@ -397,8 +397,7 @@ def test_streaming_mfma_matmul(ops, M, N, K):
 def test_streaming_mfma_matmul_minima_do_not_cancel(ops, M, K, scale):
     """The minima of variant 6 come from sums of the staged activations: rows that all lean to one side, so that the minima's
     term is as large as the products', with fp16 subnormals among them or sums beyond fp16's range, and ragged N.  Exact
-    products, sums of 22 bits: the error stays below 2^-21 of the two terms (2^-22 of the sums' split, as much again for
-    the fp32 additions)."""
+    products, sums of 24 bits as two halves: the error stays below 2^-21 of the two terms, the fp32 additions'."""
     N, fmt = 83, oracle.Q4_K
     W = quantized_weights(fmt, N, K, seed=M + K)
     A = (np.abs(gauss_acts((M, K), seed=M + 7)) * scale).astype(np.float16)
