@@ -107,7 +107,7 @@ def test_outputs_without_room_are_refused(room):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("room", list(ROOM))
+@pytest.mark.parametrize("room", [r for r in ROOM if r != "batch"])   # (which is one piece of the right size here)
 def test_dequantize_without_room_is_refused(room):
     w = torch.zeros(M * 34, dtype=torch.uint8, device="cuda")
     for dt, more in ((torch.float32, {}), (torch.float16, {}), (torch.float32, dict(dtype=torch.float16))):
