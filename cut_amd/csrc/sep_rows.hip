@@ -484,11 +484,11 @@ double sep_two_pass_us(uint32_t M, uint32_t K, uint32_t N);
 // That way, or the weights written out as fp16 first (both estimated).  Not on a K below 512, where its waves have a block or two and the
 // row tiles' code is most of the time: 64 x 256 x 256, us, two passes / this: int8 12.9 / 16.6, nibbles 13.1 / 14.7, affine 13.2 / 15.1;
 // on int8 up to 512 x 512: 64 rows 14.5 / 15.5, 200 rows 15.3 / 15.8 (of 1024 x 512 16.6 / 16.2).
-// On nibbles its estimate is low for the largest matrices: 384 rows of 14336 x 4096 106.4 / 113.2 (affine 110.5 / 118.9), 512 rows
-// 110.0 / 114.7; no other of 342 calls lies within that factor of the line.
+// (Nibbles of 11008 x 4096 and 14336 x 4096 from 350 rows on are up to 10 % faster in two passes by themselves, 512 rows 106 / 112, but a
+// layer of 500 rows of the latter is 3 % slower so: the line by the estimates stays.)
 bool sep_rows16_preferred(SepRowsParams &p, bool q4, bool affine, size_t partial_bytes) {
   const bool small = p.K < 512 || (!q4 && p.M >= 64 && p.K == 512 && p.N <= 512);
-  return !small && sep_rows16_cut(p, q4, affine, partial_bytes) && p.cost_us * (q4 ? 1.15 : 1.0) < sep_two_pass_us(p.M, p.K, p.N);
+  return !small && sep_rows16_cut(p, q4, affine, partial_bytes) && p.cost_us < sep_two_pass_us(p.M, p.K, p.N);
 }
 
 template <int KIND> static int launch_kind(const SepRowsParams &p, uint32_t grid, hipStream_t stream) {

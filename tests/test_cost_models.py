@@ -119,8 +119,8 @@ class SepRowsParams(C.Structure):
 
 # measured: (layout, rows, N, K, two passes, weights decoded as they are needed)
 SEP_LINE = [("q8", 64, 256, 256, 12.9, 16.6), ("q8", 512, 512, 256, 14.5, 17.5), ("q4", 128, 96, 256, 13.5, 14.7), ("affine", 64, 512, 256, 13.3, 15.3),
-            ("q8", 64, 512, 512, 14.5, 15.5), ("q8", 48, 512, 512, 14.0, 13.7), ("q8", 200, 1024, 512, 16.6, 16.2), ("q4", 512, 14336, 4096, 110.0, 114.7), ("q4", 384, 14336, 4096, 106.4, 113.2),
-            ("affine", 384, 14336, 4096, 110.5, 118.9), ("q8", 64, 14336, 4096, 86, 34), ("q8", 256, 4096, 4096, 47, 32), ("q4", 512, 1024, 512, 18.4, 16.3)]
+            ("q8", 64, 512, 512, 14.5, 15.5), ("q8", 48, 512, 512, 14.0, 13.7), ("q8", 200, 1024, 512, 16.6, 16.2), ("affine", 500, 5120, 4096, 58.2, 55.1),
+            ("q8", 64, 14336, 4096, 86, 34), ("q8", 256, 4096, 4096, 47, 32), ("q4", 512, 1024, 512, 18.4, 16.3)]
 
 
 @pytest.mark.parametrize("layout,M,N,K,two,direct", SEP_LINE)
