@@ -66,8 +66,8 @@ DENSE_LINE = [("Q4_K", 640, 14336, 4096, 1, 112, 105), ("Q4_K", 768, 14336, 4096
               ("Q8_0", 576, 14336, 4096, 1, 123, 103), ("Q8_0", 512, 14336, 4096, 1, 95, 85), ("Q4_K", 1536, 4096, 4096, 1, 71, 62),
               ("Q4_K", 2048, 4096, 14336, 1, 274, 227), ("Q8_0", 2048, 28672, 4096, 1, 678, 430), ("Q8_0", 384, 14336, 4096, 1, 83, 103),
               ("Q4_K", 512, 14336, 4096, 1, 78, 85), ("Q4_K", 1024, 4096, 4096, 1, 45, 56), ("Q6_K", 350, 11008, 4096, 1, 77, 83),
-              ("Q6_K", 512, 11008, 4096, 1, 92, 84), ("Q6_K", 512, 14336, 4096, 1, 98, 90), ("Q6_K", 2048, 2048, 2048, 0, 50, 44), ("Q6_K", 300, 11008, 4096, 0, 75, 88),
-             
+              ("Q6_K", 512, 11008, 4096, 1, 92, 84), ("Q6_K", 512, 14336, 4096, 1, 98, 90), ("Q6_K", 2048, 2048, 2048, 0, 50, 44),
+              ("Q6_K", 300, 11008, 4096, 0, 75, 88),   # (640 rows of it with fp16 activations: 135 in two passes before tiles of 256 x 192, now 93 either way)
               ("Q8_0", 2048, 1024, 4096, 0, 45, 47), ("Q6_K", 224, 32000, 2048, 0, 81, 119), ("Q4_K", 100, 14336, 4096, 1, 26, 66)]
 
 
