@@ -244,53 +244,7 @@ __global__ void __launch_bounds__(512, T == 1 ? 4 : 2) sep_rows_kernel(SepRowsPa
     for (int f = 0; f < 8; ++f) acc[t][f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 
-  // Where a wave holds numbers that split3 does not split exactly, activations and sums are held times 2^24, unless it also
-  // holds numbers that have no room above them (32 products of 2^64 2^24 127 times a scale of 2^16, sums of 2^100 times 2^24):
-  // beside those the small ones keep what bf16 has.
-  // (Kept over the blocks, or scaled back behind each: as the registers allow.  The other way round spills 59 of them on int8 and 2
-  // on affine weights with one tile; with two, nibbles take 3 % longer.)
-  constexpr bool kKeepUp = T > 1 || KIND == kSepQ8;
-  float up = 1.0f;
-  auto rescale = [&](float by) __attribute__((always_inline)) {
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-      for (int f = 0; f < 8; ++f) acc[t][f] *= by;
-  };
-
-  auto work = [&](int d) __attribute__((always_inline)) {
-    u32x4 hi[T], mid[T], lo[T];
-    f32x4 sx[T];
-    auto sum = [&](int t) __attribute__((always_inline)) {   // of x over the block, in every column
-      const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-      if constexpr (Q4) sx[t] = mfma_bf16(hi[t], ones, mfma_bf16(mid[t], ones, mfma_bf16(lo[t], ones, zero)));
-    };
-    bool odd = false;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      odd |= split3(a[d][t][0], a[d][t][1], hi[t], mid[t], lo[t]);
-      sum(t);   // (one tile's beside the split of the next: behind both, 17 to 31 rows of nibbles take 4 % longer)
-    }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) != 0 || up != 1.0f, 0)) {
-      bool large = false;
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) large |= !(__builtin_fabsf(a[d][t][e >> 2][e & 3]) < 0x1p64f);
-#pragma unroll
-        for (int f = 0; f < 8; ++f)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) large |= !(__builtin_fabsf(acc[t][f][i]) < 0x1p100f);
-      }
-      const float was = up;
-      up = __builtin_amdgcn_ballot_w64(large) ? 1.0f : 0x1p24f;
-      if (up != was) rescale(up == 1.0f ? 0x1p-24f : 0x1p24f);
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-        split3_odd(a[d][t][0], a[d][t][1], up, hi[t], mid[t], lo[t]);
-        sum(t);
-      }
-    }
+  auto multiply = [&](int d, const u32x4 *hi, const u32x4 *mid, const u32x4 *lo, const f32x4 *sx) __attribute__((always_inline)) {
     uint32_t n[8][2];   // Q4: nibbles of the even and the odd columns, a byte each
     if constexpr (Q4) {
 #pragma unroll
@@ -322,14 +276,67 @@ __global__ void __launch_bounds__(512, T == 1 ? 4 : 2) sep_rows_kernel(SepRowsPa
         }
       }
     }
-    if (!kKeepUp && __builtin_expect(up != 1.0f, 0)) {
-      rescale(0x1p-24f);
-      up = 1.0f;
-    }
+  };
+  auto sum = [&](const u32x4 &hi, const u32x4 &mid, const u32x4 &lo) __attribute__((always_inline)) {   // of x over the block, in every column
+    const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    return Q4 ? mfma_bf16(hi, ones, mfma_bf16(mid, ones, mfma_bf16(lo, ones, zero))) : zero;
   };
 
-  sep_walk(s.b0, s.b1, request, work);
-  if (kKeepUp && __builtin_expect(up != 1.0f, 0)) rescale(0x1p-24f);
+  bool odd = false;
+  sep_walk(s.b0, s.b1, request, [&](int d) __attribute__((always_inline)) {
+    u32x4 hi[T], mid[T], lo[T];
+    f32x4 sx[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      odd |= split3(a[d][t][0], a[d][t][1], hi[t], mid[t], lo[t]);
+      sx[t] = sum(hi[t], mid[t], lo[t]);   // (one tile's beside the split of the next: behind both, 17 to 31 rows of nibbles take 4 % longer)
+    }
+    multiply(d, hi, mid, lo, sx);
+  });
+
+  // A wave that met numbers which split3 does not split exactly begins again, with activations and sums times 2^24 in the rows that
+  // hold no number from 2^40 on (2^32 products of it with 127 and a scale of 2^16, times 2^24, stay below 2^119); beside such a number
+  // the small ones of its own row keep what bf16 has.  8 x 14336 x 4096, us, with one such number / in every block: int8 25.2 / 32.2
+  // (without 20.2), nibbles 23.0 / 28.8 (17.8).  Inside the walk, block by block, they take 23.6 there, but 720 calls of 3 to 31
+  // rows without any 1.4 % longer, up to 7 (code and registers beside the loop), or 0.4 % with one scaling for all rows of the wave.
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) != 0, 0)) {
+    uint32_t most[T] = {};   // the largest magnitude of the lane's row, as bits: what is no number is above all
+#pragma unroll 1
+    for (uint32_t b = s.b0; b < s.b1; ++b) {
+      request(0, b);
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) most[t] = max(most[t], __builtin_bit_cast(uint32_t, a[0][t][e >> 2][e & 3]) & 0x7FFFFFFFu);
+    }
+    uint32_t up = 0;   // (uniform) a bit for each row that is scaled
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      uint64_t large = __builtin_amdgcn_ballot_w64(most[t] >= __builtin_bit_cast(uint32_t, 0x1p40f));   // 16 g + row
+      large |= large >> 32;
+      up |= (uint32_t)(~(large | large >> 16) & 0xFFFF) << 16 * t;
+#pragma unroll
+      for (int f = 0; f < 8; ++f) acc[t][f] = zero;
+    }
+    sep_walk(s.b0, s.b1, request, [&](int d) __attribute__((always_inline)) {
+      u32x4 hi[T], mid[T], lo[T];
+      f32x4 sx[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        split3_odd(a[d][t][0], a[d][t][1], up >> (16 * t + s.c) & 1 ? 0x1p24f : 1.0f, hi[t], mid[t], lo[t]);
+        sx[t] = sum(hi[t], mid[t], lo[t]);
+      }
+      multiply(d, hi, mid, lo, sx);
+    });
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float by = up >> (16 * t + 4 * s.g + i) & 1 ? 0x1p-24f : 1.0f;
+#pragma unroll
+        for (int f = 0; f < 8; ++f) acc[t][f][i] *= by;
+      }
+  }
   sep_finish<T>(p, s, acc, lds);
 }
 

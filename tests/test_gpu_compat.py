@@ -230,6 +230,35 @@ def test_rows_on_the_matrix_cores_small_activations(ops, kind, M):
             assert normwise_rel_err(got, want) < 2e-6, (K, sizes)
 
 
+@pytest.mark.parametrize("kind", ["q8", "q4", "affine"])
+@pytest.mark.parametrize("M", [6, 20])
+@pytest.mark.parametrize("beside", [1e25, np.inf, np.nan])
+def test_rows_on_the_matrix_cores_small_rows_beside_large_ones(ops, kind, M, beside):
+    """A row of a tile that has no room above it (large numbers, an infinity, a NaN; in the first block of a wave or in a later one)
+    takes nothing from the rows beside it: 24 bits of their activations however small they are, as in the test before this one."""
+    rng = np.random.default_rng(M)
+    K, N, q4, affine = 4160, 264, kind != "q8", kind == "affine"
+    S = np.full(((2 if affine else 1) * (K // 32), N), 64.0, np.float32)
+    if q4:
+        B = rng.integers(0, 256, (K, N // 2)).astype(np.uint8)
+        q = np.stack((B & 15, B >> 4), -1).reshape(K, N).astype(np.float64) - 8
+    else:
+        B = rng.integers(-127, 128, (K, N)).astype(np.int8)
+        q = B.astype(np.float64)
+    w = q * 64 + (64 if affine else 0)
+    size = np.array([1e-34, 1.0, 1e-36, 2e-38, 1e-40])[np.arange(M) % 5]
+    for row in (0, M - 1):
+        for k in (5, 2600):
+            a = (rng.standard_normal((M, K)) * size[:, None]).astype(np.float32)
+            a[row, k] = beside
+            want, got = a.astype(np.float64) @ w, run(ops, a, B, S, N, q4=q4, affine=affine, variant=1)
+            for m in range(M):
+                if m != row or np.isfinite(beside):
+                    assert normwise_rel_err(got[m], want[m]) < 2e-6, (row, k, m)
+                else:
+                    assert not np.isfinite(got[m]).any()
+
+
 def test_affine_layout_from_q4k_requantizer(ops):
     """Q4_K blocks -> requantizeQ4KToAffine (oracle restatement of llama.cpp:573-619) -> separated affine matmul
     agrees with the matmul over the decoded affine weights."""
