@@ -100,11 +100,15 @@ template <int T> __device__ __forceinline__ SepPlace sep_place(const SepRowsPara
   s.side = wave & 1;
   s.kw = wave >> 1;
   // Ids id, id + 8, ... share an XCD: the passes over one piece of the weights run there one after the other, and all but
-  // the first find it in that XCD's L2.
-  const uint32_t slot = blockIdx.x >> 3, group = __builtin_amdgcn_readfirstlane(slot / p.passes), pass = slot - group * p.passes;
-  const uint32_t piece = group * 8 + (blockIdx.x & 7);
+  // the first find it in that XCD's L2.  Pieces go round the XCDs (neighbours on one XCD: 3 to 31 rows 3 % longer); the passes over
+  // those that are left over, fewer than eight, are shared out (as whole pieces they are a second round of workgroups for
+  // some XCDs: 828 rows of 4816 x 5888 on nibbles, 19 pieces of 13 passes, 140 us, so 81).
+  const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, pieces = p.tiles * p.nsplit, even = (pieces >> 3) * p.passes;
+  const uint32_t item = slot < even ? slot : xcd * (((pieces & 7) * p.passes + 7) >> 3) + slot - even;
+  const uint32_t group = __builtin_amdgcn_readfirstlane(item / p.passes), pass = item - group * p.passes;
+  const uint32_t piece = slot < even ? group * 8 + xcd : (pieces & ~7u) + group;
   s.split = __builtin_amdgcn_readfirstlane(piece / p.tiles);
-  s.any = s.split < p.nsplit;   // the last group of eight may be short
+  s.any = s.split < p.nsplit;   // the last XCD's share may be short
   s.m0 = pass * (16 * T);
   s.c0 = (piece - s.split * p.tiles) * kSepRowsTile + s.side * 128 + 8 * s.c;
   s.live = s.c0 < p.N;
@@ -430,7 +434,10 @@ __global__ void __launch_bounds__(512, 2) sep_rows16_kernel(SepRowsParams p) {
   sep_finish<T>(p, s, acc, lds);
 }
 
-static uint64_t sep_rows_grid(const SepRowsParams &p) { return ((uint64_t)p.tiles * p.nsplit + 7) / 8 * 8 * p.passes; }
+static uint64_t sep_rows_grid(const SepRowsParams &p) {
+  const uint64_t pieces = (uint64_t)p.tiles * p.nsplit;
+  return (pieces / 8 * p.passes + (pieces % 8 * p.passes + 7) / 8) * 8;
+}
 
 // Whole lanes of eight columns; offsets inside a block and inside a pass over the rows of A are 32-bit, and so are the threads
 // of the launch and of the reduce.

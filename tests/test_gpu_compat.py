@@ -120,7 +120,8 @@ def test_rows_on_the_matrix_cores(ops, kind, M, K, N):
 
 @pytest.mark.parametrize("ks", ["", "1", "3"])
 @pytest.mark.parametrize("kind", ["q8", "q4", "affine"])
-@pytest.mark.parametrize("M,K,N", [(32, 128, 8), (33, 384, 264), (64, 640, 136), (65, 1152, 520), (130, 256, 1032), (32, 512, 8), (33, 512, 264), (130, 640, 1032)])
+@pytest.mark.parametrize("M,K,N", [(32, 128, 8), (33, 384, 264), (64, 640, 136), (65, 1152, 520), (130, 256, 1032), (32, 512, 8), (33, 512, 264), (130, 640, 1032), (200, 512, 776),
+                                   (300, 512, 2312)])   # (three and nine column tiles of four and five passes: shared out over the XCDs)
 def test_rows_on_rounded_operands(ops, kind, ks, M, K, N):
     """The default from 32 rows: two, three and four row tiles in one pass and several, sides and lanes without columns, waves
     without blocks, one range and several.  Against the float64 product of the operands rounded to fp16 once each: fp32 sums."""
