@@ -658,12 +658,15 @@ constexpr size_t kDenseScratch = (size_t)32 << 20;
 // 10.1 / 8.8, 64 x 512 x 512 11.0 / 10.0, 200 fp32 rows 15.3 / 13.2).  Edge tiles count in full, so that narrower tiles win where they fit the rows of W or the CUs better (us, widest
 // tiles in the order of one panel per eight XCDs -> this): 2048 x 5120 x 4096 107 -> 73 (256 x 160), 1024 x 5120 x 4096 105 -> 57
 // (256 x 128), 512 x 11008 x 4096 117 -> 59, 2048 x 11008 x 4096 222 -> 167 (256 x 192), 2048 x 2560 x 2560 63 -> 40,
-// 700 x 5632 x 2048 59 -> 34; 2048 x 14336 x 4096 stays with 256 x 224.
+// 700 x 5632 x 2048 59 -> 34; 2048 x 14336 x 4096 stays with 256 x 224.  Where an XCD's share ends inside a panel, the panel's M-tiles,
+// which share its L2 warm-up between them, run on two XCDs, and the smaller tiles take `cut` times as long
+// (1,200 launches of 100 .. 2048 rows on weight shapes drawn at random; us, tile with cut panels / with whole ones: 719 x 1632 x 7552
+// with fp32 C 256 x 128 100 / 128 x 256 82, 790 x 17768 x 5888 128 x 256 215 / 256 x 160 182).
 struct DenseShape { int bm, bn; uint32_t ksplit; double us; };
 static DenseShape pick_dense_shape(uint32_t M, uint32_t K, uint32_t N, int c_bytes) {
-  static const struct { int bm, bn; double mac, full; } kTiles[] = {
-      {256, 224, 2.87e-7, 0.17e-7}, {256, 192, 2.87e-7, 0.39e-7}, {256, 160, 3.01e-7, 0.47e-7}, {256, 128, 3.33e-7, 0.41e-7},
-      {128, 448, 2.96e-7, 0.24e-7}, {256, 256, 2.59e-7, 0.26e-7}, {128, 256, 3.58e-7, 0.42e-7}};
+  static const struct { int bm, bn; double mac, full, cut; } kTiles[] = {
+      {256, 224, 2.87e-7, 0.17e-7, 1.0}, {256, 192, 2.87e-7, 0.39e-7, 1.0}, {256, 160, 3.01e-7, 0.47e-7, 1.05}, {256, 128, 3.33e-7, 0.41e-7, 1.1},
+      {128, 448, 2.96e-7, 0.24e-7, 1.0}, {256, 256, 2.59e-7, 0.26e-7, 1.0}, {128, 256, 3.58e-7, 0.42e-7, 1.1}};
   const double mn = (double)M * N;
   DenseShape best{0, 0, 1, 1e30};
   for (const auto &t : kTiles) {
@@ -675,7 +678,9 @@ static DenseShape pick_dense_shape(uint32_t M, uint32_t K, uint32_t N, int c_byt
       const uint64_t tiles = (uint64_t)((M - 1) / t.bm + 1) * ((N - 1) / t.bn + 1) * ks;
       if (ks > 1 && (K % (ks * 128) != 0 || (!g_tuning.dense_bn && (t.bm != 128 || t.bn != 256 || tiles > 256 || ks * mn * 4 > (double)kDenseScratch)))) break;
       const double full = (double)((tiles - 1) / 256), part = (tiles - 256.0 * full) / 256.0;
-      double us = 0.3 + 5.25 * (full + 1.0) + 0.37e-6 * mn * c_bytes + (double)K / ks * t.bm * t.bn * (t.mac * (full + 1.0) + t.full * (full + part));
+      const uint64_t mtiles = (M - 1) / t.bm + 1, per_xcd = (tiles / ks + 7) / 8;
+      double us = 0.3 + 5.25 * (full + 1.0) + 0.37e-6 * mn * c_bytes +
+                  (per_xcd % mtiles ? t.cut : 1.0) * K / ks * t.bm * t.bn * (t.mac * (full + 1.0) + t.full * (full + part));
       if (ks > 1) us += 2.5 + 1.5e-6 * ks * mn;
       if (us < best.us) best = DenseShape{t.bm, t.bn, ks, us};
     }

@@ -148,3 +148,21 @@ def test_small_problems_split_k(M, N, K, split, us, whole, more):
     finally:
         lib.set_tuning("dense_tile", None)
     assert chosen <= forced[split] < forced[whole]
+
+
+# measured on resident fp16 weights: (rows, N, K, fp16 activations, tile whose panels lie in one XCD each, us, tile whose panels are cut, us)
+CUT_LINE = [(719, 1632, 7552, 0, "128,256", 82, "256,128", 100), (790, 17768, 5888, 0, "256,160", 182, "128,256", 215),
+            (677, 1624, 2176, 1, "128,256", 30, "256,128", 35)]
+
+
+@pytest.mark.parametrize("M,N,K,a_f16,whole,us,cut,more", CUT_LINE)
+def test_tiles_whose_panels_lie_in_one_xcd(M, N, K, a_f16, whole, us, cut, more):
+    try:
+        chosen = cost("dense", lib.Q4_K, M, K, N, a_f16)
+        forced = {}
+        for tile in (whole, cut):
+            lib.set_tuning("dense_tile", tile)
+            forced[tile] = cost("dense", lib.Q4_K, M, K, N, a_f16)
+    finally:
+        lib.set_tuning("dense_tile", None)
+    assert chosen == forced[whole] < forced[cut]
