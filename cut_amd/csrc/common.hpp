@@ -254,5 +254,7 @@ extern Tuning g_tuning;
 // How a launch of the row-tile matmul is cut (gemm_rows.hip): t 32-row tiles of A and 32 nw weight rows per workgroup, K in
 // ksplit x (8 / nw) ranges of per units of 128; cost in microseconds.
 struct RowsLayout { uint32_t t, nw, per, ksplit; double cost; };
+// fp16 rows of A that the row-tile matmul may load straight to LDS: one predicate for the layout and the launch
+inline bool rows_aligned(const void *A, uint32_t strideA) { return (uintptr_t)A % 16 == 0 && strideA % 8 == 0; }
 
 }  // namespace cuthip

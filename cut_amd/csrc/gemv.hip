@@ -127,6 +127,7 @@ GemvShape pick_gemv_shape(uint32_t N, uint32_t nsteps, int mt) {
 int launch_rows_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
                      uint32_t strideA, uint32_t strideC, Epilogue epi, hipStream_t stream, const RowsLayout &l, void *scratch);
 RowsLayout rows_gemm_layout(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16, size_t scratch_bytes);
+RowsLayout rows_gemm_layout_off16(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16, size_t scratch_bytes);
 bool rows_gemm_fits(int fmt, uint32_t K, uint32_t strideA, int a_f16);
 int launch_lds_gemm(int fmt, const void *W, const void *A, int a_f16, void *C, int c_f16, uint32_t M, uint32_t K, uint32_t N,
                     uint32_t strideA, uint32_t strideC, Epilogue epi, hipStream_t stream);
@@ -210,10 +211,12 @@ static bool passes_preferred(int fmt, uint32_t M, uint32_t K, uint32_t N, const 
 // 120 / 57, 512 137 / 100, 1024 203 / 177) and where 32-bit offsets do not reach.  The row-tile matmul's cost was fitted without
 // the store of C, which only counts where K is short: 0.12 us per MB more.
 struct SingleLaunch { bool lds; double cost; cuthip::RowsLayout rows; };
-static SingleLaunch single_launch_choice(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, size_t scratch_bytes) {
+static SingleLaunch single_launch_choice(int fmt, uint32_t M, uint32_t K, uint32_t N, uint32_t strideA, int a_f16, const void *A,
+                                         size_t scratch_bytes) {
   const double lds = cuthip::lds_gemm_cost_us(fmt, M, K, N, a_f16);
   if (!cuthip::rows_gemm_fits(fmt, K, strideA, a_f16)) return {true, lds, {}};
-  const cuthip::RowsLayout l = cuthip::rows_gemm_layout(fmt, M, K, N, a_f16, scratch_bytes);
+  const cuthip::RowsLayout l = cuthip::rows_aligned(A, strideA) ? cuthip::rows_gemm_layout(fmt, M, K, N, a_f16, scratch_bytes)
+                                                                 : cuthip::rows_gemm_layout_off16(fmt, M, K, N, a_f16, scratch_bytes);
   const double rows = l.cost + 0.12e-6 * M * N * (a_f16 ? 2 : 4);
   if (cuthip::g_tuning.rows_t || cuthip::g_tuning.gemm_ksplit) return {false, rows, l};   // a test or a sweep asks for the row-tile matmul
   // up to 64 rows the cost does not tell them apart: one super-block of K (48 x 32000 x 256, us, row tiles / LDS: Q4_K 7.4 / 6.6,
@@ -359,7 +362,7 @@ static int matmul_gguf_scratch(int fmt, const void *W, const void *A, int a_dtyp
     }
     const int a_f16 = a_dtype == CUTHIP_F16;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const SingleLaunch l = chosen ? *chosen : single_launch_choice(fmt, M, K, N, strideA, a_f16,
+    const SingleLaunch l = chosen ? *chosen : single_launch_choice(fmt, M, K, N, strideA, a_f16, A,
                                                                    scratch && (uintptr_t)scratch % 16 == 0 ? scratch_bytes : 0);
     if (l.lds)
       return launch_lds_gemm(fmt, W, A, a_f16, C, c_dtype == CUTHIP_F16, M, K, N, strideA, strideC, epi, s);
@@ -674,7 +677,7 @@ int cuthip_matmul_gguf_ws(int fmt, const void *W, const void *A, int a_dtype, vo
   if (variant == -1 && M > 8 && fits && ws_ok) {
     passes = passes && dense_line_us(fmt, K, N) >= 0.9 * passes_cost_us(fmt, M, K, N);
     if (!passes) {
-      single = single_launch_choice(fmt, M, K, N, strideA, a_f16, workspace_bytes);
+      single = single_launch_choice(fmt, M, K, N, strideA, a_f16, A, workspace_bytes);
       dense_first = dense_cost_us(fmt, M, K, N, a_f16) < single.cost;
       chosen = &single;
     }

@@ -166,3 +166,23 @@ def test_tiles_whose_panels_lie_in_one_xcd(M, N, K, a_f16, whole, us, cut, more)
     finally:
         lib.set_tuning("dense_tile", None)
     assert chosen == forced[whole] < forced[cut]
+
+
+# measured with fp16 rows of A off 16 bytes: (format, rows, N, K, scratch memory, row tiles and panel width, us, with the cut of the kernel that
+# loads A straight to LDS, us)
+OFF16 = [("Q4_K", 49, 14292, 8704, 1, (2, 4), 44.1, 57.4), ("Q4_K", 799, 1523, 6656, 1, (2, 4), 42.6, 49.0),
+         ("Q4_K", 40, 13878, 3584, 1, (1, 4), 24.9, 28.2), ("Q6_K", 51, 6045, 7680, 0, (1, 2), 43.4, 54.5),
+         ("Q6_K", 229, 1673, 10752, 0, (1, 2), 51.8, 64.6), ("Q6_K", 136, 2612, 6400, 0, (1, 2), 37.2, 45.4)]
+
+
+@pytest.mark.parametrize("fmt,M,N,K,scratch,tile,us,other", OFF16)
+def test_rows_off_16_bytes_have_a_layout_of_their_own(fmt, M, N, K, scratch, tile, us, other):
+    """They run through registers: the estimate for A straight to LDS is not theirs."""
+    f = getattr(lib.load(), "_ZN6cuthip22rows_gemm_layout_off16Eijjjim")
+    f.restype, f.argtypes = RowsLayout, [C.c_int, C.c_uint32, C.c_uint32, C.c_uint32, C.c_int, C.c_size_t]
+    room = SCRATCH if scratch else 0
+    own = f(FORMATS[fmt], M, K, N, 1, room)
+    assert (own.t, own.nw) == tile and us < other
+    assert own.cost >= cost("rows", FORMATS[fmt], M, K, N, 1, room)
+    for same in (lib.Q8_0, lib.Q4_0):   # formats without that kernel: one layout
+        assert f(same, M, K, N, 1, room).cost == cost("rows", same, M, K, N, 1, room)
