@@ -36,13 +36,15 @@ static double unit_us(int fmt, uint32_t t, uint32_t nw) {
   return u[nw == 4][t - 1];
 }
 
-// What a unit takes where A goes straight to LDS (rows_direct), against the staging through registers that the table was fitted to: 180 problems
-// (two formats, 40 .. 1024 rows, nine weight shapes, every t and nw forced); the layout chosen is 0.2 % (Q6_K 0.3 %) slower than the best one,
-// without this 0.8 % (1.0 %): 64 x 4096 x 4096 on Q4_K 13.6 us -> 12.3, 400 x 2048 x 8192 28.8 -> 25.6, 100 x 5120 x 4096 on Q6_K 23.2 -> 20.9.
+// What a unit takes where fp16 rows of A lie on 16 bytes, against the table: the direct form (rows_direct), and on Q6_K also the
+// tiles of 32 rows beside it, which the table has 10 % too high for such rows (without a factor of their own they lost to the direct tiles of 64
+// where those are slower, us: 53 x 5788 x 12544 without scratch memory 56.0 -> 63.7, 229 x 1673 x 10752 46.4 -> 51.9, 340 x 1046 x 1792
+// 14.1 -> 16.0).  270 problems (33 .. 1200 rows, every t and nw forced): the layout chosen is 0.4 % (Q6_K 0.8 %) slower than the best one, without
+// these factors 5.3 % (4.3 %); against the layout without them 0.956 (0.969) of the time, 5 of 152 (0 of 118) slower by more than 3 %.
 static double direct_gain(int fmt, uint32_t t, uint32_t nw) {
+  if (fmt == CUTHIP_Q6_K) return t == 1 || (t == 2 && nw == 2) ? 0.9 : 1.0;
   if (!rows_direct(fmt, (int)t, (int)nw)) return 1.0;
-  if (fmt == CUTHIP_Q6_K) return t == 2 ? 0.94 : 1.0;
-  return t == 2 ? 0.88 : t == 3 ? 1.0 : 0.93;
+  return t == 2 ? 0.88 : t == 3 ? 1.0 : 0.96;
 }
 
 static RowsLayout layout_of(int fmt, uint32_t M, uint32_t K, uint32_t N, int a_f16, size_t scratch_bytes, bool aligned) {

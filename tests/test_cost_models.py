@@ -186,3 +186,19 @@ def test_rows_off_16_bytes_have_a_layout_of_their_own(fmt, M, N, K, scratch, til
     assert own.cost >= cost("rows", FORMATS[fmt], M, K, N, 1, room)
     for same in (lib.Q8_0, lib.Q4_0):   # formats without that kernel: one layout
         assert f(same, M, K, N, 1, room).cost == cost("rows", same, M, K, N, 1, room)
+
+
+# measured with fp16 rows of A on 16 bytes: (rows, N, K, scratch memory, tile chosen, us, other tile, us)
+Q6_K_TILE = [(53, 5788, 12544, 0, "1,2", 56.0, "2,2", 63.7), (229, 1673, 10752, 0, "1,2", 46.4, "2,2", 51.9), (64, 5512, 5376, 0, "1,2", 28.7, "2,2", 32.3),
+             (340, 1046, 1792, 1, "1,2", 14.1, "2,2", 16.0), (169, 1387, 2048, 1, "1,2", 13.6, "2,2", 15.1), (317, 929, 4096, 1, "2,2", 18.9, "2,4", 21.4),
+             (481, 1787, 3840, 1, "2,2", 23.4, "4,4", 32.0)]
+
+
+@pytest.mark.parametrize("M,N,K,scratch,tile,us,other,more", Q6_K_TILE)
+def test_tiles_of_q6_k_that_go_straight_to_lds_beside_the_others(rows_tile, M, N, K, scratch, tile, us, other, more):
+    room = SCRATCH if scratch else 0
+    chosen = cost("rows", lib.Q6_K, M, K, N, 1, room)
+    rows_tile(tile)
+    own = cost("rows", lib.Q6_K, M, K, N, 1, room)
+    rows_tile(other)
+    assert chosen == own < cost("rows", lib.Q6_K, M, K, N, 1, room) and us < more
