@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const void *q, const 
   }
 }
 
-// The same for head dimensions of 128 and 64 and up to four query heads (NH) of a KV head; gridDim.z goes through the groups of NH.
+// The same for head dimensions of 128 and 64 and up to four query heads (NH) of a KV head; gridDim.y goes through the groups of NH.
 // Bound: HBM on long contexts, latency on short ones.  K and V stay in the registers that they are loaded into: lane = (row of G, piece
 // of 8 dimensions).  A wave takes 16 positions of a chunk for its heads; its products of 8 dimensions meet across the lanes of a row in halving
 // steps, which leaves each lane the score of one (position, head), so that softmax costs every lane one exponential; the weights
@@ -416,16 +416,18 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const void *q, const 
 // Against 64 bits 1.2 to 2.4e-7 where that kernel has 2.2 to 7.1e-7 (shorter chains of additions).
 template <int HD, int NH, bool ONE>
 __global__ void __launch_bounds__(256) attn_rows_kernel(const void *q, const half_t *kCache, const half_t *vCache, const uint32_t *params,
-                                                        uint32_t alignedKvDim, uint32_t maxSeqLen, uint32_t nHeads, uint32_t nKvHeads,
+                                                        uint32_t alignedKvDim, uint32_t maxSeqLen, uint32_t nRep, uint32_t nKvHeads,
                                                         int q_f16, uint32_t nsplit, float *partial, float scale) {
   constexpr int LPR = HD / 8, G = 64 / LPR, IT = 16 / G, NV = IT * NH;   // NV scores per lane of a row
   static_assert(kAttnChunk == 4 * 16 && NV <= LPR, "four waves of 16 positions; a lane of a row ends with one score");
   __shared__ __attribute__((aligned(16))) float Ps[4][16][NH];
   __shared__ float Os[4][NH * HD], Ms[4][NH], Ls[4][NH];
-  const uint32_t kvH = blockIdx.x, split = blockIdx.y, nRep = nHeads / nKvHeads, rep0 = blockIdx.z * NH;
+  // blockIdx.x: XCD, .y: group of NH query heads, .z: eighths of the (KV head, split) pairs
+  const uint32_t pair = blockIdx.z * 8 + blockIdx.x, split = __builtin_amdgcn_readfirstlane(pair / nKvHeads), kvH = pair - split * nKvHeads;
+  const uint32_t rep0 = blockIdx.y * NH;
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t piece = lane % LPR, row = lane / LPR;
-  if (split >= nsplit) return;   // (the grid is padded)
+  if (split >= nsplit) return;   // (the last eight pairs may be fewer)
 
   // the queries first, then the first positions: one memory round trip for both (attn_partial_kernel)
   u32x4 q_raw[NH][2];
@@ -1183,6 +1185,9 @@ static int attn_check_args(const char *who, const void *q, int q_dtype, const vo
   return CUTHIP_OK;
 }
 
+}  // extern "C"
+
+namespace cuthip {
 // Splits of the context (records per head): one chunk of 64 positions each while that gives at most kAttnWgs workgroups
 // (two per CU; twice as many where a workgroup serves more than four heads; more than eight heads multiply them, not
 // counted), several beyond, so that every workgroup is resident and streams.  Eight layers of an 8B model in all, us, with 8 KV heads of 128 and a context of 16,384 / 8,192 /
@@ -1203,24 +1208,34 @@ static uint32_t attn_splits(uint32_t max_seq_len, uint32_t n_heads, uint32_t n_k
 // 8.2 / 9.1; 64 / 8 1500 (768) 7.3 / 8.1 / 8.4, 2500 (1280) 10.1 / 9.3 / 10.6; more than 32 heads, 71 / 1 30,000: 63 / 60 / 40.
 // Dimension 64: four heads 32 / 8 3000 (quads 376) 6.8 against 6.6, 6000 (752) 7.7 / 8.4; 64 / 8 4096 (1024) 7.8 / 8.6; pairs 32 / 4 1500 (384) 5.9 / 6.4,
 // 3000 (752) 7.2 / 7.0; 32 / 8 64 (16) 4.8 / 4.9, 1024 (256) 5.4 / 5.5, 1500 (384) 5.9 / 5.6.
+// Three, five, six and seven groups of four leave CUs of an XCD idle, which very many heads feel (us, four / attn_partial_kernel): dimension 64,
+// 12,000 positions 96 / 8 heads 19.8 / 22.0, 144 / 12 26.3 / 24.1, 288 / 24 45.5 / 40.0; dimension 128 192 / 16 at 20,000 73 / 80, 384 / 32 at 12,000 103 / 91.
 struct AttnRoute { uint32_t heads, nsplit; };
-static AttnRoute attn_route(uint32_t head_dim, uint32_t n_heads, uint32_t n_kv_heads, uint32_t max_seq_len) {
+AttnRoute attn_route(uint32_t head_dim, uint32_t n_heads, uint32_t n_kv_heads, uint32_t max_seq_len) {
   const uint32_t chunks = (max_seq_len + kAttnChunk - 1) / kAttnChunk, n_rep = n_heads / n_kv_heads;
   const uint64_t work = (uint64_t)chunks * n_kv_heads;
   // as many chunks a workgroup as leave at most one workgroup per CU: its waves stream by themselves, and there is half as much to merge
-  // (the kernel with a barrier per chunk wants two)
+  // (the kernel with a barrier per chunk wants two).  Counted XCD by XCD: the `groups` workgroups of a (KV head, split) share one, and a CU with
+  // two of them ends last.  Counted over the whole chip, three and seven groups put 33 and 35 on the 32 CUs of some XCDs; us, attn_partial_kernel / so
+  // (and with the split padded to a multiple of eight workgroups, see the launch) / now, dimension 128: 48 / 4 heads at 32,000 positions 39.0 / 43.0 /
+  // 32.2, 56 / 2 at 20,000 28.9 / 33.0 / 25.7, 84 / 7 at 20,000 40.8 / 49.2 / 36.7, 144 / 9 60.7 / 75.2 / 52.0, 40 / 5 27.9 / 27.5 / 20.8.
   auto splits = [&](uint64_t groups) {
-    const uint32_t most = (uint32_t)std::max<uint64_t>(1, 256 / (n_kv_heads * groups)), per = (chunks + most - 1) / most;
+    const uint32_t most = (uint32_t)std::max<uint64_t>(1, 8 * (32 / groups) / n_kv_heads), per = (chunks + most - 1) / most;
     return (chunks + per - 1) / per;
   };
-  if (head_dim == 128 || head_dim == 64) {
+  if ((head_dim == 128 || head_dim == 64) && n_kv_heads <= 1u << 16) {   // (65,535 eighths of the pairs)
     if (n_rep <= 2) return {n_rep, work <= 512 ? chunks : splits(1)};
     const uint64_t pairs = work * ((n_rep + 1) / 2), quads = work * ((n_rep + 3) / 4);
     if (pairs <= (head_dim == 128 ? 768u : n_rep <= 4 ? 0u : 512u)) return {2, chunks};
-    if (n_rep <= 32 && (head_dim == 128 || quads > 512)) return {4, splits((n_rep + 3) / 4)};
+    const uint32_t groups = (n_rep + 3) / 4;
+    const bool fills = 32 % groups == 0 || n_heads <= (head_dim == 128 ? 192u : 96u);
+    if (n_rep <= 32 && fills && (head_dim == 128 || quads > 512)) return {4, splits(groups)};
   }
   return {0, attn_splits(max_seq_len, n_heads, n_kv_heads)};
 }
+}  // namespace cuthip
+
+extern "C" {
 
 // The two launches of the split-context attention; `partial` holds cuthip_attn_decode_workspace_bytes() bytes.
 static int attn_launch(const void *q, int q_dtype, const void *k_cache, const void *v_cache, const uint32_t *runtime_params,
@@ -1237,13 +1252,11 @@ static int attn_launch(const void *q, int q_dtype, const void *k_cache, const vo
     };
     auto kernel = head_dim == 128 ? (one ? of(std::integral_constant<int, 128>{}, std::true_type{}) : of(std::integral_constant<int, 128>{}, std::false_type{}))
                                   : (one ? of(std::integral_constant<int, 64>{}, std::true_type{}) : of(std::integral_constant<int, 64>{}, std::false_type{}));
-    // the workgroups of a KV head's further query heads follow the first one's at a multiple of eight: on the same XCD, whose L2 has the
-    // chunk by then
-    const uint32_t groups = (n_rep - 1) / route.heads + 1;
-    const uint32_t even = n_kv_heads % 8 == 0 ? 1 : n_kv_heads % 4 == 0 ? 2 : n_kv_heads % 2 == 0 ? 4 : 8;
-    hipLaunchKernelGGL(kernel, dim3(n_kv_heads, groups == 1 ? nsplit : (nsplit + even - 1) / even * even, groups), dim3(256), 0, s, q,
-                       (const half_t *)k_cache, (const half_t *)v_cache, runtime_params, aligned_kv_dim, max_seq_len, n_heads, n_kv_heads,
-                       (int)(q_dtype == CUTHIP_F16), nsplit, (float *)partial, scale);
+    // the groups of a (KV head, split) follow each other on one XCD, whose L2 has the chunk by then; only the last eight pairs are padded (empty
+    // workgroups between the others, group by group, left CUs with two of them: 84 / 3 heads at 20,000 positions 53.6 us, so 39.2)
+    const uint32_t groups = (n_rep - 1) / route.heads + 1, pairs = n_kv_heads * nsplit;
+    hipLaunchKernelGGL(kernel, dim3(8, groups, (pairs + 7) / 8), dim3(256), 0, s, q, (const half_t *)k_cache, (const half_t *)v_cache, runtime_params,
+                       aligned_kv_dim, max_seq_len, n_rep, n_kv_heads, (int)(q_dtype == CUTHIP_F16), nsplit, (float *)partial, scale);
     if (int rc = check_hip(hipGetLastError(), "attention launch")) return rc;
     return launch_attn_merge(partial, nsplit, n_heads, head_dim, out, out_dtype == CUTHIP_F16, s);
   }

@@ -202,3 +202,25 @@ def test_tiles_of_q6_k_that_go_straight_to_lds_beside_the_others(rows_tile, M, N
     own = cost("rows", lib.Q6_K, M, K, N, 1, room)
     rows_tile(other)
     assert chosen == own < cost("rows", lib.Q6_K, M, K, N, 1, room) and us < more
+
+
+class AttnRoute(C.Structure):
+    _fields_ = [("heads", C.c_uint32), ("nsplit", C.c_uint32)]
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("n_kv", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 16, 20, 32, 40])
+def test_attention_of_four_heads_a_workgroup_has_one_on_every_cu(head_dim, n_kv):
+    """The workgroups of a (KV head, split) share an XCD of 32 CUs: counted over the whole chip, three groups of four heads put 33 on some
+    of them (48 / 4 heads at 32,000 positions 43.0 us, with 30 on each 32.2)."""
+    f = lib.load()._ZN6cuthip10attn_routeEjjjj
+    f.restype, f.argtypes = AttnRoute, [C.c_uint32] * 4
+    taken = 0
+    for n_rep in range(1, 41):
+        for positions in (1, 64, 700, 2500, 6000, 12000, 20000, 32000, 65536):
+            r, chunks = f(head_dim, n_kv * n_rep, n_kv, positions), (positions + 63) // 64
+            assert 1 <= r.nsplit <= min(chunks, 1024)
+            if r.heads == 4 and r.nsplit > 1:
+                taken += 1
+                assert (r.nsplit * n_kv + 7) // 8 * ((n_rep + 3) // 4) <= 32, (n_rep, positions, r.nsplit)
+    assert taken
