@@ -560,7 +560,7 @@ static int matmul_sep(bool q4, const float *A, const void *B, const void *S, con
   // two 17.1 / 19.4; three rows on the general vector kernel 22.3 / 19.7, nibbles 19.3 / 17.2.
   {
     SepRowsParams r{A, p.B, p.S, C, reinterpret_cast<float *>(workspace), p.epi, M, K, N, strideA, strideB, strideC, scaleStride};
-    if (sep_vec_cut(r, q4, bytes)) return launch_sep_vec(r, q4, affine != 0, stream);
+    if (sep_vec_cut(r, q4)) return launch_sep_vec(r, q4, affine != 0, stream);
     if (M > 2 && sep_rows_cut(r, (uintptr_t)workspace % 16 == 0 ? workspace_bytes : 0)) {
       if (int rc = launch_sep_rows(r, q4, affine != 0, stream)) return rc;
       return r.nsplit == 1 ? CUTHIP_OK : launch_sep_reduce(r.partial, C, p.epi, M, N, strideC, 0, M, r.nsplit, stream);

@@ -20,7 +20,7 @@ struct SepRowsParams {
 
 // How the launch is cut; false if it does not fit.  partial_bytes: room for the sums of several K ranges (nsplit is never
 // more than K / 128 rounded up).
-bool sep_vec_cut(SepRowsParams &p, bool q4, size_t partial_bytes);
+bool sep_vec_cut(SepRowsParams &p, bool q4);
 bool sep_rows_cut(SepRowsParams &p, size_t partial_bytes);
 bool sep_rows16_cut(SepRowsParams &p, bool q4, bool affine, size_t partial_bytes);
 bool sep_rows16_preferred(SepRowsParams &p, bool q4, bool affine, size_t partial_bytes);   // cut, and the cheaper of the two ways

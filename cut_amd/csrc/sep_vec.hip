@@ -5,14 +5,16 @@
 // 32 k-rows in turn, two of them in flight in each, and meet in LDS at the end:
 //   * strips of a whole cache line of the weights (128 int8 columns, 256 of nibbles) where there are enough of them: half lines arrive
 //     at a lower rate (14336 x 4096 int8 as 224 workgroups, us: strips of 128 15.8, of 64 19.4, of 32 27, of 16 42);
-//   * as many ranges as fill the 256 CUs once, so that the partial sums that meet in memory are 2 to 16 sets and not one for every 128 k-rows
-//     (16 columns a lane and one block a wave: 32 sets for K = 4096, 112 for 14336);
+//   * as many ranges as fill the 256 CUs once, and at most 16, so that the partial sums that meet in memory are 2 to 16 sets and not one for
+//     every 128 k-rows (16 columns a lane and one block a wave: 32 sets for K = 4096, 112 for 14336); few columns over a long K then run on
+//     16 workgroups for each strip (128 x 14336 7.5, 512 x 14336 8.7, 1024 x 14336 9.5, that form 13.4, 9.3, 10.6);
 //   * a short K in one range: strips of 64 columns and sixteen waves, and no second launch;
 //   * the activations come straight from the caches with the block they belong to: no staging, no barrier ahead of the weights.
 // Against that form, both launches, us, graph replay over 600 MB of weights: int8 one row 14336 x 4096 (N x K) 16.4 -> 15.8, 4096 x 14336
 // 18.2 -> 15.6 (4.0 TB/s), 4096 x 4096 9.9 -> 7.9, 1024 x 4096 7.8 -> 5.7, 4096 x 1024 7.8 -> 4.2, 28672 x 4096 28.2 -> 25.6; two rows
 // 4096 x 14336 20.0 -> 16.5, 4096 x 4096 11.6 -> 8.1; nibbles with minima 4096 x 14336 14.6 -> 12.3, 4096 x 4096 9.2 -> 7.1.
-// Columns in a multiple of eight that is none of 16 took the byte-wise form: 1000 x 2560 51 -> 5.8.
+// Columns in a multiple of eight that is none of 16 took the byte-wise form: 1000 x 2560 51 -> 5.8.  On weights that were written just
+// before, the launches of the seven matmuls of such a layer take 102 -> 92 together, with all caches flushed 137 -> 121.
 #include <algorithm>
 #include <type_traits>
 
@@ -191,7 +193,7 @@ __global__ void __launch_bounds__(64) sep_vec_reduce_kernel(const float *ws, uin
 //   13.2, 4096 x 14336 12.3 / 13.7, 28672 x 4096 19.7 / 20.8; 5120 x 5120 8.8 / 8.8, 4096 x 4096 7.2 / 7.1, 1024 x 4096 5.9 / 5.4;
 //   ranges: as many as leave every wave a block and fit the chip once; two workgroups a CU where that leaves a quarter of it idle and K is
 //   long (20000 x 4096, 157 strips: one range 22.9 / 18.5, three 21.4 / 16.9; 20000 x 2048 one 12.7 / 10.8, three 13.1 / 11.6).
-bool sep_vec_cut(SepRowsParams &p, bool q4, size_t partial_bytes) {
+bool sep_vec_cut(SepRowsParams &p, bool q4) {
   if (p.M > 2 || p.N % 8 != 0 || p.strideB > 1u << 26 || p.N > 1u << 29) return false;
   const uint32_t blocks = p.K / 32, strips64 = (p.N - 1) / 64 + 1;
   const bool one = blocks <= 32 && strips64 <= 256;
@@ -201,8 +203,7 @@ bool sep_vec_cut(SepRowsParams &p, bool q4, size_t partial_bytes) {
   if (blocks > 32) {
     ns = std::max(1u, 256 / p.tiles);
     if (p.tiles * ns <= 192 && p.tiles > 64 && blocks >= 96) ns = 512 / p.tiles;
-    ns = std::min(std::min(ns, blocks / (p.t == 32 ? 4 : 8)), kVecSplits);
-    while (ns > 1 && (uint64_t)ns * p.M * p.N * 4 > partial_bytes) --ns;
+    ns = std::min(std::min(ns, blocks / (p.t == 32 ? 4 : 8)), kVecSplits);   // (the workspace holds blocks / 4 sets of sums: matmul_sep)
   }
   p.per = (blocks - 1) / ns + 1;
   p.nsplit = (blocks - 1) / p.per + 1;
