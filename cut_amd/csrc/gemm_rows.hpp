@@ -142,8 +142,6 @@ template <> struct RowFmt<CUTHIP_Q4_K, true> {
   __device__ static uint32_t off(uint32_t p) { return 16 * p; }
   struct Raw { u32x4 hdr, q[2]; };
   struct Sc { float s[4], o[4]; };
-  __device__ static uint32_t a_off(uint32_t kg) { return 16 * kg; }
-  static constexpr uint32_t j_off(int j) { return 32 * (j >> 1) + 8 * (j & 1); }
   static constexpr uint32_t PART = 64;
   __device__ static uint32_t chunk(uint32_t c) { return 8 * c; }
   __device__ static uint32_t h_off(uint32_t kg) { return 16 * kg; }
@@ -230,7 +228,7 @@ template <bool DIR> struct RowFmt<CUTHIP_Q6_K, DIR> {
 
 // Blocks of 32 with an fp16 scale in front: block 2 kg and 2 kg + 1 of the unit; the quants of the first lie two bytes off
 // a dword boundary.  value = d * q with one rounding to fp16: a packed fp16 product.
-template <bool DIR> struct RowFmt<CUTHIP_Q8_0, DIR> {
+template <> struct RowFmt<CUTHIP_Q8_0, false> {
   static constexpr int GROUP = 1, PIECE = 8, NP = 17, BYTES = 136, IMG = 136;
   __device__ static uint32_t off(uint32_t p) { return 8 * p; }
   struct Raw { uint32_t w[17]; };
@@ -260,7 +258,7 @@ template <bool DIR> struct RowFmt<CUTHIP_Q8_0, DIR> {
   template <int J> __device__ static uint32_t fin(Mid v, const Sc &c) { return __builtin_bit_cast(uint32_t, v * (J < 4 ? c.d0 : c.d1)); }
 };
 
-template <bool DIR> struct RowFmt<CUTHIP_Q4_0, DIR> {
+template <> struct RowFmt<CUTHIP_Q4_0, false> {
   static constexpr int GROUP = 1, PIECE = 8, NP = 9, BYTES = 72, IMG = 72;
   __device__ static uint32_t off(uint32_t p) { return 8 * p; }
   struct Raw { uint32_t w[9]; };
@@ -307,7 +305,8 @@ template <int FMT, int T, int NW, bool DIR> struct RowsGeom {
                        NI = (32 * F::NP + 63) / 64;
   // DIR: a row of one K range is CR chunks of 16 bytes, an instruction of a wave fills RPI rows of it
   static constexpr int CR = SK / 8, RPI = 64 / CR;
-  __device__ static uint32_t key(uint32_t row) { return CR == 16 ? row & 15 : (row >> 1) & 7; }
+  __device__ static uint32_t key(uint32_t row) { return (row >> 1) & 7; }
+  static_assert(!DIR || (SU == 2 && CR == 8), "straight to LDS: slices of half a unit (rows_direct)");
   static_assert(NW * KW == 8 && 512 % CH == 0 && (32 * T * CH) % 512 == 0 && LDS <= 160 * 1024, "tile geometry");
 };
 
@@ -468,7 +467,7 @@ __global__ void __launch_bounds__(512, 2) gemm_rows_kernel(RowsParams p) {
     for (int v = 0; v < G::CPT; ++v) {
       constexpr uint32_t per_kw = 32 * T / G::RPI;
       const uint32_t i = 8 * v + wave, dkw = i / per_kw, row = (i % per_kw) * G::RPI + lane / G::CR;
-      const uint32_t c = (lane % G::CR) ^ G::key(row), beg = (split * KW + dkw) * p.per * 128 + (SU == 1 ? 8 * c : F::chunk(c));
+      const uint32_t c = (lane % G::CR) ^ G::key(row), beg = (split * KW + dkw) * p.per * 128 + F::chunk(c);
       doff[v] = (min(row, rows - 1) * p.strideA + beg) * 2;
     }
   }
@@ -495,7 +494,9 @@ __global__ void __launch_bounds__(512, 2) gemm_rows_kernel(RowsParams p) {
   constexpr int BAR = FR - L + 2;                // the barrier stands in front of this MFMA: the last read is two MFMAs old
   constexpr int TRIP = 2 * SU > P ? 2 * SU : P;   // slices per loop trip: everything indexed by a slice or unit is static in it
   static_assert(TRIP * FR % RING == 0 && TRIP % (2 * SU) == 0 && TRIP % P == 0, "compile-time slots over a loop trip");
-  const uint32_t aread = r32 * G::PITCH + kw * (G::SK * 2) + (SU == 1 ? F::a_off(kg) : F::h_off(kg)) * 2;
+  uint32_t aread = r32 * G::PITCH + kw * (G::SK * 2);
+  if constexpr (SU == 1) aread += F::a_off(kg) * 2;
+  else aread += F::h_off(kg) * 2;
   half8_t ring[RING];
   typename F::Raw raw[2];
   typename F::Sc sc;
@@ -506,7 +507,7 @@ __global__ void __launch_bounds__(512, 2) gemm_rows_kernel(RowsParams p) {
   if constexpr (DIR) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      joff[j] = (kw * 32 * T + r32) * (G::SK * 2) + ((((SU == 1 ? F::a_off(kg) + F::j_off(j) : F::h_off(kg) + F::hj_off(j)) / 8) ^ G::key(r32)) * 16);
+      joff[j] = (kw * 32 * T + r32) * (G::SK * 2) + (((F::h_off(kg) + F::hj_off(j)) / 8) ^ G::key(r32)) * 16;
   }
   // LDS offsets of the buffers of the present slice, the next one and the one after that
   uint32_t bufr = 0, bufn = G::BUF, bufw = 2 * G::BUF;
@@ -514,8 +515,11 @@ __global__ void __launch_bounds__(512, 2) gemm_rows_kernel(RowsParams p) {
     if constexpr (DIR) {
       if (f % T == 0) jaddr = joff[f / T] + buf;
       return lds_get<half8_t>(lds + jaddr + (f % T) * 32 * G::SK * 2);
+    } else if constexpr (SU == 1) {
+      return lds_get<half8_t>(lds + buf * G::BUF + aread + (f % T) * 32 * G::PITCH + F::j_off(f / T) * 2);
+    } else {
+      return lds_get<half8_t>(lds + buf * G::BUF + aread + (f % T) * 32 * G::PITCH + F::hj_off(f / T) * 2);
     }
-    return lds_get<half8_t>(lds + buf * G::BUF + aread + (f % T) * 32 * G::PITCH + (SU == 1 ? F::j_off(f / T) : F::hj_off(f / T)) * 2);
   };
   auto prep = [&](auto uc, const typename F::Raw &r, uint32_t i) __attribute__((always_inline)) {   // i: unit of this wave's range
     const uint32_t u = u0 + i;
