@@ -1244,11 +1244,11 @@ static int attn_launch(const void *q, int q_dtype, const void *k_cache, const vo
   const AttnRoute route = attn_route(head_dim, n_heads, n_kv_heads, max_seq_len);
   const uint32_t nsplit = route.nsplit, n_rep = n_heads / n_kv_heads;
   if (route.heads) {
-    const bool one = nsplit * (uint64_t)kAttnChunk >= max_seq_len;   // a chunk per workgroup
+    const bool one = nsplit * (uint64_t)kAttnChunk >= max_seq_len;   // a chunk per workgroup (four heads: only past 1,500 query heads)
     auto of = [&](auto hd, auto o) {
       constexpr int HD = decltype(hd)::value;
       constexpr bool ONE = decltype(o)::value;
-      return route.heads == 1 ? attn_rows_kernel<HD, 1, ONE> : route.heads == 2 ? attn_rows_kernel<HD, 2, ONE> : attn_rows_kernel<HD, 4, ONE>;
+      return route.heads == 1 ? attn_rows_kernel<HD, 1, ONE> : route.heads == 2 ? attn_rows_kernel<HD, 2, ONE> : attn_rows_kernel<HD, 4, false>;
     };
     auto kernel = head_dim == 128 ? (one ? of(std::integral_constant<int, 128>{}, std::true_type{}) : of(std::integral_constant<int, 128>{}, std::false_type{}))
                                   : (one ? of(std::integral_constant<int, 64>{}, std::true_type{}) : of(std::integral_constant<int, 64>{}, std::false_type{}));
@@ -1261,7 +1261,7 @@ static int attn_launch(const void *q, int q_dtype, const void *k_cache, const vo
     return launch_attn_merge(partial, nsplit, n_heads, head_dim, out, out_dtype == CUTHIP_F16, s);
   }
   const bool two = n_rep > 4;
-  auto kernel = head_dim == 128  ? attn_partial_kernel<128, 2>   // (more than 32 query heads per KV head)
+  auto kernel = head_dim == 128  ? attn_partial_kernel<128, 2>   // (more than 32 query heads per KV head, or very many in all)
                 : head_dim == 64 ? (two ? attn_partial_kernel<64, 2> : attn_partial_kernel<64, 1>)
                                  : (two ? attn_partial_kernel<0, 2> : attn_partial_kernel<0, 1>);
   hipLaunchKernelGGL(kernel, dim3(n_kv_heads, nsplit, (n_rep + 7) / 8), dim3(256), 0, s, q, (const half_t *)k_cache,
