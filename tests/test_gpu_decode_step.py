@@ -3,6 +3,7 @@ RoPE + KV write, GQA decode attention, SiLU * up, arg-max) through the C ABI
 against the CPU oracle, and of a whole small decode step (two layers + head)
 against the same chain composed from oracle calls.  Floating point: each
 assert states its tolerance; the KV cache write is bit-exact."""
+import ctypes
 import math
 
 import numpy as np
@@ -254,6 +255,39 @@ def test_attention_of_head_pairs(ops, n_heads, n_kv, hd, seq, max_ctx):
         ops.attn_decode(dev(q), dev(K), dev(V), dev(np.array([seq - 1, seq], np.int32)), n_heads, n_kv, hd, scale, ws, out)
         torch.cuda.synchronize()
         assert bool((out == 0).all())
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,seq,heads,chunks", [(2, 2, 128, 200, 1, 1), (32, 32, 128, 1300, 1, 3), (8, 2, 128, 300, 2, 1), (32, 16, 128, 2500, 2, 3),
+                                                             (32, 8, 128, 4000, 4, 2), (14, 2, 128, 12000, 4, 3), (3, 3, 64, 300, 1, 1), (40, 40, 64, 1500, 1, 4),
+                                                             (20, 4, 64, 500, 2, 1), (40, 20, 64, 3001, 2, 4), (20, 4, 64, 9000, 4, 5), (12, 1, 64, 20000, 4, 4)])
+@pytest.mark.parametrize("blind", [0, 1])
+def test_attention_one_head_of_a_group_sees_nothing_of_a_wave(ops, n_heads, n_kv, hd, seq, heads, chunks, blind):
+    """Scores of -inf (a product that overflows) for one query head of every group over the 16 positions of a wave, in its first chunk: that head
+    starts later than the others whose sums lie in the same lanes.  Then over all positions: it attends nothing, the others everything.
+    heads, chunks: query heads a workgroup has, chunks it goes through."""
+    route = ops._l.load()._ZN6cuthip10attn_routeEjjjj
+    route.restype = ctypes.c_uint64
+    r = route(hd, n_heads, n_kv, seq)
+    assert (r & 0xFFFFFFFF, -(-((seq + 63) // 64) // (r >> 32))) == (heads, chunks)
+    rng, n_rep, scale = np.random.default_rng(n_heads + seq), n_heads // n_kv, 1 / math.sqrt(hd)
+    h = np.arange(n_kv) * n_rep + min(blind, n_rep - 1)
+    q = rng.standard_normal((n_heads, hd)).astype(np.float32)
+    K = (rng.standard_normal((seq, n_kv * hd)) * 0.5).astype(np.float16)
+    V = rng.standard_normal((seq, n_kv * hd)).astype(np.float16)
+    q[:, 0], K[:, ::hd] = 0, 0
+    attend = lambda at: oracle.attention_decode(q.ravel(), K[at].view(np.uint16), V[at].view(np.uint16), len(at), n_heads, n_kv, hd, scale).reshape(n_heads, hd)
+    want, without = attend(np.arange(seq)), attend(np.r_[0:32, 48:seq])
+    q[h, 0] = 1e36
+    ws = ops.attn_decode_workspace(n_heads, hd, seq, "cuda")
+    out = torch.full((n_heads * hd,), np.nan, dtype=torch.float32, device="cuda")
+    for rows, of_blind in ((slice(32, 48), without[h]), (slice(0, seq), np.zeros((n_kv, hd)))):
+        K[rows, ::hd] = -65504
+        ops.attn_decode(dev(q.ravel()), dev(K), dev(V), dev(np.array([seq - 1, seq], np.int32)), n_heads, n_kv, hd, scale, ws, out)
+        torch.cuda.synchronize()
+        got, want[h] = out.cpu().numpy().reshape(n_heads, hd), of_blind
+        for head in range(n_heads):   # fp32 sums in any order, as above
+            err = np.linalg.norm(got[head] - want[head])
+            assert err <= 2e-6 * np.linalg.norm(want[head]), (head, err)
 
 
 @pytest.mark.parametrize("records", [1, 3, 4, 5, 8, 31, 32, 33, 64, 65])
