@@ -10,11 +10,14 @@
 // The attention differs from the reference in structure, not in result: the
 // reference runs one workgroup per query head over the whole context (every
 // K/V row is read nRep times, scores staged in 8 KB of shared memory).  Here
-// a workgroup owns one KV head and a chunk of 64 positions; its four waves
-// are the (up to four at a time) query heads sharing that KV head, so K and V
-// are read from HBM once, staged in LDS, and the softmax is carried as
-// (max, sum, weighted V) partials (the usual split-context decode attention).
-// A second, small kernel merges the partials.  Merging inside the first kernel
+// a workgroup owns one KV head and chunks of 64 positions, and leaves (max,
+// sum, weighted V) partials of its query heads (the usual split-context decode
+// attention).  Two kernels do that: attn_rows_kernel (head dimensions 128 and
+// 64) keeps K and V in the registers that they are loaded into, 16 positions a
+// wave for one, two or four query heads; attn_partial_kernel (the other
+// dimensions, and where attn_route says so) stages a chunk in LDS, and its four
+// waves are four query heads.  A third, small kernel merges the partials.
+// Merging inside the first kernel
 // (the workgroup that draws the last ticket of a KV head's counter reads the
 // records back; all workgroups of a head placed on one XCD so that records
 // and tickets stay in that XCD's L2; no fences) was built and measured: the
@@ -231,12 +234,12 @@ constexpr int kAttnRow = kAttnMaxHd + 8;   // LDS row in halfs: +16 bytes keeps 
 // Bound: HBM on long contexts (K and V once), latency on short ones.  Split s takes the 64-position chunks s, s + nsplit,
 // s + 2 nsplit, ...: a workgroup that has several keeps (m, l, o) of its heads in registers and requests the next chunk
 // while it works on the present one, so that memory does not idle between workgroups and a long context leaves 64
-// records per head to merge instead of 256 (attn_splits draws the line).  A 16,384-position context of 8 KV heads of 128:
-// partials and merge 30.6 us before, about 20 now.
+// records per head to merge instead of 256 (attn_splits draws the line).  32 / 8 heads of 128 over 16,384 positions, partials and merge: a chunk
+// per workgroup 30.6 us, several 21 (that shape is attn_rows_kernel's now, 18 us).
 // HD: the head dimension where it is 128 or 64 (loops over it unroll and their LDS reads overlap), 0 = any
 // NG: query heads of a KV head in groups of four (one per wave); gridDim.z covers the heads beyond 4 * NG, each of its
-// workgroups with its own reading of K and V (the L2 serves all but one): one KV head of 128 with 32 query heads over 16,384
-// positions 34.8 -> 18.2 us against one workgroup that went through all heads, with 71 over 65,536 143 -> 84.
+// workgroups with its own reading of K and V (the L2 serves all but one): one KV head of 128 with 71 query heads over 65,536
+// positions 143 -> 84 us against one workgroup that went through all heads.
 // The arguments that the first loads need (up to and including headDimArg: 14 dwords) lead the list: with
 // kernel-argument preloading they arrive in SGPRs with the wave, and the loads of q, K and V wait for no scalar load.
 template <int HD, int NG>
@@ -1190,7 +1193,8 @@ static int attn_check_args(const char *who, const void *q, int q_dtype, const vo
 namespace cuthip {
 // Splits of the context (records per head): one chunk of 64 positions each while that gives at most kAttnWgs workgroups
 // (two per CU; twice as many where a workgroup serves more than four heads; more than eight heads multiply them, not
-// counted), several beyond, so that every workgroup is resident and streams.  Eight layers of an 8B model in all, us, with 8 KV heads of 128 and a context of 16,384 / 8,192 /
+// counted), several beyond, so that every workgroup is resident and streams.  attn_partial_kernel, when it served these shapes: eight layers of an
+// 8B model in all, us, with 8 KV heads of 128 and a context of 16,384 / 8,192 /
 // 4,096: one chunk per workgroup 420 / 344 / 300, at most 1024 workgroups 401 / 344 / 298, 512 384 / 332 / 300, 256
 // 411 / 340 / 305; 32 KV heads at 8,192: 560 / 512 / 496 / 573; 4 KV heads (eight query heads each) at 16,384: 363 / 363 /
 // 372 / 400.  (One chunk each, one group of threads per merge and no prefetch: 464 / 363 / 318; 534; 446.)
@@ -1202,7 +1206,9 @@ static uint32_t attn_splits(uint32_t max_seq_len, uint32_t n_heads, uint32_t n_k
 }
 
 // Which kernel: attn_rows_kernel with `heads` query heads of a KV head per workgroup, or (0) attn_partial_kernel.  A group of more than two is
-// served in pairs, a chunk each, while these are few: each reads K and V again, from the L2.  Then four heads at a time over several chunks.  us, in
+// served in pairs, a chunk each, while these are few: each reads K and V again, from the L2.  Then four heads at a time over several chunks.  (In a
+// decode step of twelve layers with 32 / 8 heads, all routes in one library, us a layer, pairs / attn_partial_kernel / four: 1024 positions 43.6 /
+// 44.8 / 44.3, 2048 44.6 / 44.9 / 44.7, 3000 45.8 / 46.2 / 46.2, 3500 46.6 / 46.4 / 46.2.)  us by themselves, in
 // pairs / four / attn_partial_kernel (query / KV heads, dimension 128; workgroups in pairs): 32 / 8 1500 positions (384) 6.5 / 7.2 / 6.8, 2048 (512) 7.1 /
 // 7.4 / 7.4, 3000 (752) 8.4 / 8.4 / 8.7, 4096 (1024) 9.8 / 9.2 / 9.4, 16,384 25.7 / 17.7 / 21.2; 32 / 4 2500 (640) 7.5 / 8.0 / 8.5, 3500 (880) 8.9 /
 // 8.2 / 9.1; 64 / 8 1500 (768) 7.3 / 8.1 / 8.4, 2500 (1280) 10.1 / 9.3 / 10.6; more than 32 heads, 71 / 1 30,000: 63 / 60 / 40.
